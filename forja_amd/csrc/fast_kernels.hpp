@@ -144,9 +144,31 @@ struct KsplitRouted {
   uint32_t inner, columns;
   const uint32_t *sorted_routes, *blocks, *n_blocks;
   uint32_t max_blocks, tile_rows, route_div;
-  bool wide;                // f32 activations and results; tiles of 16 routes only
+  bool wide;                // f32 activations and results (launch_ksplit_routed: tiles of 16 routes only)
 };
 bool launch_ksplit_routed(fh_backend *backend, const KsplitRouted &problem);
+
+// ---- qmm_rows.hip: products over up to 64 activation rows per weight, weights unpacked once for
+// all of them.  Operands as above, K a multiple of 256, columns of 16; rows of bf16, or f32 (`wide`: f32 residual
+// and result; the only form that takes 8-bit weights).
+struct RowsDense {
+  const void *x;
+  uint64_t x_row_stride;
+  const uint32_t *packed;
+  const uint16_t *scales, *biases;
+  void *out;
+  uint64_t out_row_stride;
+  uint32_t out_f32;
+  const void *residual;     // rows of the activations' dtype
+  uint64_t residual_row_stride;
+  uint32_t rows, inner, columns, bits;
+  bool wide;
+};
+// False when the operands do not fit: nothing was launched.
+bool launch_rows_dense(fh_backend *backend, const RowsDense &problem);
+uint32_t rows_route_tile(bool wide);   // routes per tile of the routed form
+bool rows_routed_supports(uint32_t inner, uint32_t columns);
+bool launch_rows_routed(fh_backend *backend, const KsplitRouted &problem);
 
 // A row-wise RMS normalisation the next dispatch applies to the rows a weighted sum produces:
 // out[r,:] = rows[r,:] * rsqrt(mean(rows[r,:]^2) + eps) * weight[r,:], everything bf16 or

@@ -845,8 +845,8 @@ bool rows_contiguous(const View &v, uint32_t rank) {
 }
 
 bool weights_eligible(const View &packed, const View &scales, const View &biases, uint32_t rank,
-                      uint32_t inner, uint32_t bits, uint32_t group) {
-  if (bits != 4 || group != kGroup || inner % 256 != 0) return false;
+                      uint32_t inner, uint32_t bits, uint32_t group, uint32_t accepted_bits = 4) {
+  if (bits != accepted_bits || group != kGroup || inner % 256 != 0) return false;
   if (scales.dtype != FH_BF16 || biases.dtype != FH_BF16) return false;
   if (!rows_contiguous(packed, rank) || !rows_contiguous(scales, rank) ||
       !rows_contiguous(biases, rank))
@@ -1084,17 +1084,17 @@ const uint16_t *u16_ptr(const View &v) { return (const uint16_t *)v.base + v.off
 
 namespace {
 
+constexpr uint32_t kRowsKernelWide = 9;
+
 // f32 activations (the engines' own activation dtype) on the matrix cores: each value goes in as
-// three bf16 pieces that add up to it exactly, so nothing of it is rounded away before the f32
-// accumulation.  Decode batches of at most 32 rows, f32 results.
+// three bf16 or f16 pieces that add up to it, so that f32 accumulation sees all of it.  f32 results.
+// Decode batches of at most 32 rows through the K-split kernels, more rows and 8-bit weights through
+// the row-tile kernels (fewer than nine rows of what neither takes: the vector-ALU kernel for few rows,
+// 12 us for the 8-bit router of 8 rows).
 bool try_wide_quant_matmul(fh_backend *backend, const QmmProblem &p) {
   if (p.out.dtype != FH_F32 || p.out.stride[1] != 1) return false;
-  if (!weights_eligible(p.packed, p.scales, p.biases, 2, p.inner, p.bits, p.group)) return false;
+  if (!weights_eligible(p.packed, p.scales, p.biases, 2, p.inner, p.bits, p.group, p.bits == 8 ? 8 : 4)) return false;
   if (p.x.stride[1] != 1 || p.x.stride[0] % 4 != 0 || p.x.offset % 4 != 0) return false;
-  // K = 4096 (three pieces of so long a slice do not fit the registers): two launches over half
-  // the K each, the second adding to what the first stored
-  const uint32_t ranges = p.inner == 4096 ? 2 : 1, range = p.inner / ranges;
-  if (!ksplit_dense_supports(p.rows, range, p.columns, true)) return false;
   const float *residual = nullptr;
   uint64_t residual_row_stride = 0;
   if (p.residual) {
@@ -1102,6 +1102,16 @@ bool try_wide_quant_matmul(fh_backend *backend, const QmmProblem &p) {
     if (r.dtype != FH_F32 || r.stride[1] != 1) return false;
     residual = (const float *)r.base + r.offset;
     residual_row_stride = r.stride[0];
+  }
+  // K = 4096 (three pieces of so long a slice do not fit the registers): two launches over half
+  // the K each, the second adding to what the first stored
+  const uint32_t ranges = p.inner == 4096 ? 2 : 1, range = p.inner / ranges;
+  if (p.bits == 8 || !ksplit_dense_supports(p.rows, range, p.columns, true)) {
+    if (p.rows < kRowsKernelWide) return false;
+    RowsDense d{(const float *)p.x.base + p.x.offset, p.x.stride[0], u32_ptr(p.packed), u16_ptr(p.scales),
+                u16_ptr(p.biases), (float *)p.out.base + p.out.offset, p.out.stride[0], 1, residual,
+                residual_row_stride, p.rows, p.inner, p.columns, p.bits, true};
+    return launch_rows_dense(backend, d);
   }
   float *out = (float *)p.out.base + p.out.offset;
   for (uint32_t i = 0; i < ranges; ++i) {
@@ -1155,8 +1165,22 @@ bool try_fast_quant_matmul(fh_backend *backend, const QmmProblem &p) {
                   a.out_f32, residual, residual_row_stride, p.rows, p.inner, p.columns};
     if (launch_ksplit_dense(backend, d)) return true;
   }
-  // Decode rows.  When one workgroup per compute unit covers the output, the single-kernel tile
-  // product; wider outputs go through the K slabs.
+  // More rows, or a longer K, than the K-split kernels hold: row tiles, the weights unpacked once for
+  // all rows of a tile.  (48 x 34816 x 5120 66 us against 101 through the streaming kernel, 48 x 5120 x
+  // 17408 34 against 75 through the tile product; 1 row against 34816 x 5120 43 and 64.)  Two shapes are
+  // faster elsewhere: vocabulary-sized matrices at more than 64 rows, which the GEMM's 128-row tiles
+  // read once (128 x 151936 x 2048 127 us against 175), and few rows against so little weight that the
+  // second launch, which adds the K ranges, shows (1 x 5120 x 5120 11.5 us through the tile product
+  // against 13.4, 16 rows 16 against 14).
+  const bool vocabulary = p.rows > 64 && p.columns >= 32768;
+  const bool little = p.rows <= 8 && p.inner <= 6144 && (p.columns + 31) / 32 <= backend_compute_units(backend);
+  if (p.rows <= 128 && !vocabulary && !little) {
+    RowsDense d{a.x, a.x_row_stride, a.packed[0], a.scales[0], a.biases[0], a.out, a.out_row_stride,
+                a.out_f32, residual, residual_row_stride, p.rows, p.inner, p.columns, 4, false};
+    if (launch_rows_dense(backend, d)) return true;
+  }
+  // Columns that are no multiple of 16, and the little products: when one workgroup per compute unit
+  // covers the output, the single-kernel tile product; wider outputs go through the K slabs.
   if (p.rows <= 128 &&
       (uint64_t)((p.columns + 31) / 32) * ((p.rows + 31) / 32) <= 3 * backend_compute_units(backend)) {
     launch_tile_product(backend, a, residual, residual_row_stride);
@@ -1173,7 +1197,7 @@ bool try_fast_quant_matmul(fh_backend *backend, const QmmProblem &p) {
   // (also a full decode batch against a vocabulary-sized matrix: 128 x 151936 x 2048 takes 132 us
   // through the GEMM's 128 x 128 tiles and 224 us through the streaming kernel, which reads the
   // weights once per 64 rows)
-  if (p.rows > 128 || (p.rows > 64 && p.columns >= 32768)) {
+  if (p.rows > 128 || vocabulary) {
     // the tiled GEMM, followed by the any-range kernel conditioned on the GEMM's refusal
     const uint32_t *refused = nullptr;
     if (launch_quant_gemm(backend, p, &refused)) {
@@ -1258,15 +1282,29 @@ void launch_routed(hipStream_t stream, const QmmArgs &a, uint32_t max_blocks, ui
   launch_qmm<kPair, true>(stream, a, max_blocks, 1);
 }
 
-// Route tile of the K-split kernels: 16 rows while an expert sees few routes on average (an
-// expert with more gets a second tile and its weights are read again), else 32; 0 when the
-// kernels do not take this K.
-uint32_t ksplit_route_tile(const GatherProblem &p, bool pair) {
-  if (!ksplit_supports(p.inner, p.columns, pair, true)) return 0;
-  return (uint64_t)p.rows * p.k <= 10ull * p.experts ? 16 : 32;
+// Routes per tile (an expert with more gets further tiles, and its weights are read again for
+// each); 0 when neither the K-split nor the row-tile kernels take the problem.  16 through the
+// K-split kernels while an expert sees few routes on average.  Beyond that f32 rows take the row-tile
+// kernels, and bf16 rows tiles of 32 through the K-split kernels up to 25 routes per expert (gate/up
+// and down together, 128 experts of 768 x 2048: 15 routes 111 us against 122 through the row-tile
+// kernels, 20 routes 116 and 128), the row-tile kernels from there (30 routes 131 against 151, 45
+// routes 143 and 203, 130 routes 324 and 435).
+uint32_t route_tile(const GatherProblem &p, bool pair, bool wide) {
+  const uint64_t routes = (uint64_t)p.rows * p.k;
+  const bool ksplit = ksplit_supports(p.inner, p.columns, pair, true);
+  if (routes <= 10ull * p.experts) return ksplit ? 16 : 0;
+  if (!wide && ksplit && routes <= 25ull * p.experts) return 32;
+  const bool small = p.rows * p.x.stride[0] * (wide ? 4 : 2) <= 0xffffffffull;   // a lane's row offset is 32 bits
+  if (small && rows_routed_supports(p.inner, p.columns)) return rows_route_tile(wide);
+  return ksplit && !wide ? 32 : 0;
 }
 
-bool launch_routed_ksplit(fh_backend *backend, const QmmArgs &a, bool pair, uint32_t max_blocks, uint32_t tile) {
+// The kernel that goes with route_tile's answer.
+bool launch_tiles(fh_backend *backend, const KsplitRouted &r) {
+  return r.tile_rows == rows_route_tile(r.wide) ? launch_rows_routed(backend, r) : launch_ksplit_routed(backend, r);
+}
+
+bool launch_routed_tiles(fh_backend *backend, const QmmArgs &a, bool pair, uint32_t max_blocks, uint32_t tile) {
   KsplitRouted r{};
   r.x = a.x;
   r.x_row_stride = a.x_row_stride;
@@ -1286,7 +1324,7 @@ bool launch_routed_ksplit(fh_backend *backend, const QmmArgs &a, bool pair, uint
   r.max_blocks = max_blocks;
   r.tile_rows = tile;
   r.route_div = a.route_div;
-  return launch_ksplit_routed(backend, r);
+  return launch_tiles(backend, r);
 }
 
 bool gather_eligible(const GatherProblem &p, int projections) {
@@ -1326,12 +1364,12 @@ void launch_combine_routes(hipStream_t stream, const float *partial, const Gathe
 
 namespace {
 
-// The routed products on f32 activations (three bf16 pieces a value, see try_wide_quant_matmul):
-// tiles of 16 routes, so only while an expert sees few routes on average -- the decode batches of
-// a few lanes the engines run.  `x_rows` input rows of `x_row_stride` elements, `route_div` routes
+// The routed products on f32 activations (three pieces a value, see try_wide_quant_matmul):
+// the decode batches of a few lanes and the prompt chunks the engines run.  `x_rows` input rows of `x_row_stride` elements, `route_div` routes
 // per input row; results are f32 rows of `p.columns`.
 bool launch_wide_routed(fh_backend *backend, const GatherProblem &p, int projections, const float *x,
-                        uint64_t x_row_stride, uint32_t route_div, float *out, const RoutePlan &plan) {
+                        uint64_t x_row_stride, uint32_t route_div, float *out, const RoutePlan &plan,
+                        uint32_t tile) {
   KsplitRouted r{};
   r.x = x;
   r.x_row_stride = x_row_stride;
@@ -1349,25 +1387,27 @@ bool launch_wide_routed(fh_backend *backend, const GatherProblem &p, int project
   r.blocks = plan.blocks;
   r.n_blocks = plan.n_blocks;
   r.max_blocks = plan.max_blocks;
-  r.tile_rows = 16;
+  r.tile_rows = tile;
   r.route_div = route_div;
   r.wide = true;
   KernelTimer timer(backend, FH_KC_MOE_KERNEL);
-  return launch_ksplit_routed(backend, r);
+  return launch_tiles(backend, r);
 }
 
-bool wide_gather_eligible(const GatherProblem &p, int projections) {
-  if (p.x.dtype != FH_F32) return false;
+// The route tile, 0 when the operands do not fit.
+uint32_t wide_route_tile(const GatherProblem &p, int projections) {
+  if (p.x.dtype != FH_F32) return 0;
   for (int pj = 0; pj < projections; ++pj)
     if (!weights_eligible(p.packed[pj], p.scales[pj], p.biases[pj], 3, p.inner, p.bits, p.group))
-      return false;
-  if ((uint64_t)p.rows * p.k > (1u << 24) || p.experts > 512) return false;
-  return ksplit_route_tile(p, projections == 2) == 16;
+      return 0;
+  if ((uint64_t)p.rows * p.k > (1u << 24) || p.experts > 512) return 0;
+  return route_tile(p, projections == 2, true);
 }
 
 bool try_wide_gather_projection(fh_backend *backend, const GatherProblem &p, int projections,
                                 bool swiglu, ErrorSlot *error) {
-  if (!wide_gather_eligible(p, projections) || (projections == 2 && !swiglu)) return false;
+  const uint32_t tile = wide_route_tile(p, projections);
+  if (!tile || (projections == 2 && !swiglu)) return false;
   if (p.out.dtype != FH_F32) return false;
   if (p.x.stride[1] != 1 || p.x.stride[0] % 4 != 0 || p.x.offset % 4 != 0) return false;
   if (p.out.stride[2] != 1 || p.out.stride[1] != p.columns ||
@@ -1377,25 +1417,26 @@ bool try_wide_gather_projection(fh_backend *backend, const GatherProblem &p, int
   // first when an earlier plan is reused (see try_fast_gather_projection)
   RoutePlan plan;
   float *out = (float *)p.out.base + p.out.offset;
-  if (!plan_routes(backend, p, 0, error, &plan, (uint32_t *)out, p.columns, 16)) return false;
+  if (!plan_routes(backend, p, 0, error, &plan, (uint32_t *)out, p.columns, tile)) return false;
   if (plan.reused)
     launch_fill_u32(backend_stream(backend), (uint32_t *)out, (uint64_t)p.rows * p.k * p.columns, 0);
   return launch_wide_routed(backend, p, projections, (const float *)p.x.base + p.x.offset, p.x.stride[0],
-                            p.k, out, plan);
+                            p.k, out, plan, tile);
 }
 
 bool try_wide_gather_weighted(fh_backend *backend, const GatherProblem &p, const View *residual,
                               ErrorSlot *error) {
-  if (!wide_gather_eligible(p, 1)) return false;
+  const uint32_t tile = wide_route_tile(p, 1);
+  if (!tile) return false;
   if (p.x.stride[2] != 1 || p.x.stride[1] % 4 != 0 || p.x.offset % 4 != 0 ||
       p.x.stride[0] != (uint64_t)p.k * p.x.stride[1])
     return false;
   const uint64_t partial_bytes = (uint64_t)p.rows * p.k * p.columns * sizeof(float);
   RoutePlan plan;
-  if (!plan_routes(backend, p, partial_bytes, error, &plan, nullptr, 0, 16)) return false;
+  if (!plan_routes(backend, p, partial_bytes, error, &plan, nullptr, 0, tile)) return false;
   float *partial = (float *)plan.rest;
   if (!launch_wide_routed(backend, p, 1, (const float *)p.x.base + p.x.offset, p.x.stride[1], 1, partial,
-                          plan))
+                          plan, tile))
     return false;
   auto rows_of_eight = [](const View &v) {   // f32 [rows, columns] in 16-byte aligned pieces of 8
     return v.dtype == FH_F32 && v.stride[1] == 1 && v.stride[0] % 8 == 0 && v.offset % 8 == 0;
@@ -1431,10 +1472,10 @@ bool try_fast_gather_projection(fh_backend *backend, const GatherProblem &p, int
   // packs, and the whole output is cleared first.
   RoutePlan plan;
   const bool row_words = p.columns % 2 == 0 && p.out.offset % 2 == 0;
-  const uint32_t ksplit_tile = ksplit_route_tile(p, projections == 2);
+  const uint32_t tile = route_tile(p, projections == 2, false);
   if (!plan_routes(backend, p, 0, error, &plan,
                    row_words ? (uint32_t *)((uint16_t *)p.out.base + p.out.offset) : nullptr,
-                   p.columns / 2, ksplit_tile ? ksplit_tile : kRouteTile))
+                   p.columns / 2, tile ? tile : kRouteTile))
     return false;
   hipStream_t stream = backend_stream(backend);
   if (plan.reused || !row_words)
@@ -1462,7 +1503,7 @@ bool try_fast_gather_projection(fh_backend *backend, const GatherProblem &p, int
   a.route_div = p.k;
   a.split_below = backend_compute_units(backend) / 2;
   KernelTimer timer(backend, FH_KC_MOE_KERNEL);
-  if (ksplit_tile && launch_routed_ksplit(backend, a, projections == 2, plan.max_blocks, ksplit_tile)) return true;
+  if (tile && launch_routed_tiles(backend, a, projections == 2, plan.max_blocks, tile)) return true;
   if (projections == 2)
     launch_routed<true>(stream, a, plan.max_blocks, backend_compute_units(backend));
   else
@@ -1480,8 +1521,8 @@ bool try_fast_gather_weighted(fh_backend *backend, const GatherProblem &p, const
     return false;
   uint64_t partial_bytes = (uint64_t)p.rows * p.k * p.columns * sizeof(float);
   RoutePlan plan;
-  const uint32_t ksplit_tile = ksplit_route_tile(p, false);
-  if (!plan_routes(backend, p, partial_bytes, error, &plan, nullptr, 0, ksplit_tile ? ksplit_tile : kRouteTile))
+  const uint32_t tile = route_tile(p, false, false);
+  if (!plan_routes(backend, p, partial_bytes, error, &plan, nullptr, 0, tile ? tile : kRouteTile))
     return false;
   hipStream_t stream = backend_stream(backend);
   float *partial = (float *)plan.rest;
@@ -1506,7 +1547,7 @@ bool try_fast_gather_weighted(fh_backend *backend, const GatherProblem &p, const
   a.split_below = backend_compute_units(backend) / 2;
   {
     KernelTimer timer(backend, FH_KC_MOE_KERNEL);
-    if (!(ksplit_tile && launch_routed_ksplit(backend, a, false, plan.max_blocks, ksplit_tile)))
+    if (!(tile && launch_routed_tiles(backend, a, false, plan.max_blocks, tile)))
       launch_routed<false>(stream, a, plan.max_blocks, backend_compute_units(backend));
   }
   uint64_t work = (uint64_t)p.rows * p.columns;

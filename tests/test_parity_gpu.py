@@ -255,6 +255,73 @@ def test_routed_products_on_f32_activations_that_use_their_whole_mantissa(cpu, h
     differential(cpu, hip, build)
 
 
+@pytest.mark.parametrize("rows,n,k,bits,dtype,padded", [
+    # row tiles of 16, 32, 48 and 64 and their remainders; 16-column tiles past a block's edge; K ranges
+    # of an odd number of 256-value quads; K that no other matrix-core kernel for few rows takes
+    (1, 8224, 1280, 4, DType.BF16, False), (9, 144, 1280, 4, DType.BF16, True),
+    (17, 272, 6400, 4, DType.BF16, False), (33, 16, 256, 4, DType.BF16, True),
+    (48, 400, 3328, 4, DType.BF16, False), (49, 128, 1280, 4, DType.BF16, False),
+    (64, 144, 2304, 4, DType.BF16, True), (127, 256, 3840, 4, DType.BF16, False),
+    # f32 rows: tiles of 32, 4- and 8-bit weights
+    (33, 272, 256, 4, DType.F32, True), (65, 528, 1280, 4, DType.F32, False),
+    (9, 16, 768, 8, DType.F32, False), (70, 272, 2048, 8, DType.F32, True),
+])
+def test_quant_matmul_in_row_tiles(cpu, hip, rows, n, k, bits, dtype, padded):
+    """`padded`: results into rows that no 16-byte store fits.  f32 inputs use their whole mantissa."""
+    weights = Quantised(27, 300 + n + k, (n, k), bits=bits)
+    x_values = orc.fill_normal_f32(27, 1, rows * k).reshape(rows, k) if dtype == DType.F32 else normal_bf16(27, 1, (rows, k))
+    extra_values = normal_bf16(27, 2, (rows, n))
+
+    def build(backend):
+        x, extra = upload(backend, x_values, dtype), upload(backend, extra_values, dtype)
+        plain, whole = backend.alloc(dtype, (rows, n)), upload(backend, np.zeros((rows, n + 3)), dtype)
+        added = whole.narrow(1, 1, n) if padded else whole.narrow(1, 0, n)
+        triple = weights.upload(backend)
+        commands = CommandList()
+        commands.dispatch(Op.quant_matmul(bits, 64), [x, *triple], plain)
+        commands.dispatch_epilogue(Op.quant_matmul(bits, 64), [x, *triple], added,
+                                   backend.prepare_epilogue(programs.add_elements()), [extra])
+        return commands, [plain, whole]
+    differential(cpu, hip, build)
+
+
+@pytest.mark.parametrize("rows,k,experts,n,inner,dtype", [
+    (60, 8, 8, 144, 256, DType.BF16),      # 60 routes per expert: a 64-row tile and its remainder
+    (130, 2, 5, 272, 512, DType.BF16),     # 52: columns past a block's edge, two quads
+    (45, 4, 7, 784, 768, DType.BF16),      # odd numbers of quads
+    (17, 8, 8, 144, 256, DType.F32), (70, 4, 7, 272, 768, DType.F32),
+])
+def test_routed_products_in_row_tiles(cpu, hip, rows, k, experts, n, inner, dtype):
+    """More routes per expert than the K-split kernels take, with bad routes among them."""
+    gate, up = (Quantised(28, 1 + i, (n, inner), experts=experts) for i in range(2))
+    down = Quantised(28, 21, (512, inner), experts=experts)
+    indices = routed_case(28, rows, k, experts, n, inner, bad=((3, 1, experts), (rows - 1, 0, experts + 7)))
+    x_values, wide_values = normal_bf16(28, 40, (rows, inner)), normal_bf16(28, 43, (rows, k, inner))
+    if dtype == DType.F32:
+        x_values = orc.fill_normal_f32(28, 40, rows * inner).reshape(rows, inner)
+    logits = orc.fill_normal_f32(28, 41, rows * k).reshape(rows, k)
+    w_values = np.exp(logits) / np.exp(logits).sum(axis=1, keepdims=True)
+
+    def pair(backend):
+        x, idx = upload(backend, x_values, dtype), upload(backend, indices, DType.U32)
+        activated = backend.alloc(dtype, (rows, k, n))
+        commands = CommandList()
+        commands.dispatch_epilogue(Op.gather_quant_matmul(4, 64), [x, *gate.upload(backend), *up.upload(backend), idx],
+                                   activated, backend.prepare_epilogue(programs.silu_mul_elements()), [])
+        return commands, [activated]
+
+    def summed(backend):
+        x, idx = upload(backend, wide_values, dtype), upload(backend, indices, DType.U32)
+        combined = backend.alloc(dtype, (rows, 512))
+        commands = CommandList()
+        commands.dispatch(Op.gather_quant_matmul(4, 64),
+                          [x, *down.upload(backend), idx, upload(backend, w_values, dtype)], combined)
+        return commands, [combined]
+
+    for build in (pair, summed):
+        differential(cpu, hip, build, expect_error={Status.INDEX_OUT_OF_RANGE, Status.DEVICE_ERROR_FLAG})
+
+
 @pytest.mark.parametrize("dtype,bits,group", [(DType.F32, 4, 64), (DType.F16, 8, 32), (DType.BF16, 4, 128)])
 def test_quant_matmul_with_f16_scales_and_a_residual_in_other_dtypes(cpu, hip, dtype, bits, group):
     """f16 affine parameters (the reference allows f16 or bf16, quantized.rs:78-121) and the
