@@ -1578,10 +1578,14 @@ bool same_lane_shape(const LaneMember &a, const LaneMember &b) {
          same_tensor(a.value_pool, b.value_pool);
 }
 
-// Longest fusable run of per-lane attention starting at `first`; false when there is none of at
-// least two lanes.  `run->dispatches` then still says how many dispatches were examined, so that
-// the caller does not examine the tail of a refused run again.
-bool find_lane_run(const fh_dispatch *d, uint32_t count, uint32_t first, LaneRun *run) {
+// Longest fusable run of per-lane attention starting at `first`; false when there is none.  A run of
+// one lane is a step recorded for a single sequence: its layers then share one gather and one plan,
+// and the attention kernel stores the new row itself (48 layers of one lane at 6000 keys: the plan
+// per layer 12 us, the two copies 9).  It is taken only where the member stands alone (`alone`: not
+// behind a member that was not fused; nor before one), because members next to each other that make
+// no run are an order that the caller wants kept.  `run->dispatches` says how many dispatches were
+// examined also when false, so that the caller does not examine the tail of a refused run again.
+bool find_lane_run(const fh_dispatch *d, uint32_t count, uint32_t first, bool alone, LaneRun *run) {
   *run = LaneRun{};
   LaneMember member;
   if (!lane_member_at(d, count, first, &member)) return false;
@@ -1609,7 +1613,8 @@ bool find_lane_run(const fh_dispatch *d, uint32_t count, uint32_t first, LaneRun
     run->members.push_back(member);
     run->dispatches += member.dispatches;
   }
-  if (run->members.size() < 2) return false;
+  if (run->members.size() < 2 && (!alone || (first + run->dispatches < count && lane_member_at(d, count, first + run->dispatches, &member))))
+    return false;
   // Nothing a member writes may be something another member reads or writes.
   const LaneMember &head = run->members[0];
   std::unordered_set<uint64_t> read;
@@ -1709,8 +1714,8 @@ fh_status run_lane_group(fh_backend *b, const LaneRun &run, ErrorSlot *errors, b
     // on the gathered tables, once per set of tables (not per layer); the verdict is needed here,
     // so the stream is waited for.
     uint32_t *flag = cu + lanes + 1;
-    b->lane_conflict = true;
-    if (launch_lane_conflict_check(b->stream, tables, activity, starts, lanes, table_pages,
+    b->lane_conflict = lanes > 1;   // (a lane alone has no other to meet)
+    if (lanes > 1 && launch_lane_conflict_check(b->stream, tables, activity, starts, lanes, table_pages,
                                    head.page_tokens, flag)) {
       if (hipMemcpyAsync(b->host_flag, flag, sizeof(uint32_t), hipMemcpyDeviceToHost, b->stream) != hipSuccess ||
           hipStreamSynchronize(b->stream) != hipSuccess)
@@ -2730,6 +2735,7 @@ static fh_status submit_locked(fh_backend *b, const fh_dispatch *dispatches, uin
   };
   fh_status status = FH_OK;
   uint32_t no_run_before = 0;  // dispatches already examined as part of a run that was refused
+  uint32_t unfused_end = 0;    // where the last per-lane member that was not fused ended
   for (uint32_t i = 0; i < count && status == FH_OK;) {
     uint32_t consumed = 1;
     LaneRun run;
@@ -2738,11 +2744,12 @@ static fh_status submit_locked(fh_backend *b, const fh_dispatch *dispatches, uin
                            i >= no_run_before;
     // a run that brings prefill chunks first (it takes one-row members too), else one of one-row members
     const bool with_chunks = candidate && find_chunk_run(dispatches, count, i, &run);
-    bool fused = with_chunks || (candidate && find_lane_run(dispatches, count, i, &run));
+    bool fused = with_chunks || (candidate && find_lane_run(dispatches, count, i, i != unfused_end || i == 0, &run));
     if (fused)
       consumed = run.dispatches;
     else if (run.members.size() > 1)
       no_run_before = i + run.dispatches;
+    if (!fused && !run.members.empty()) unfused_end = i + run.dispatches;
     for (uint32_t member = 0; member < consumed; ++member) s->ops[i + member] = dispatches[i + member].op;
     hipEvent_t t0 = nullptr, t1 = nullptr;
     if (b->profiling >= 2 || profiled) {
