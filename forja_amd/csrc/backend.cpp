@@ -1710,12 +1710,12 @@ fh_status run_lane_group(fh_backend *b, const LaneRun &run, ErrorSlot *errors, b
       launch_gather_lane_metadata(b->stream, sources, base, chunk, lanes, table_words, tables,
                                   activity, starts, cu);
     }
-    // The one thing the tensors cannot show: an append into a slot another lane attends.  Checked
+    // The one thing the tensors cannot show: an append into a slot attended elsewhere.  Checked
     // on the gathered tables, once per set of tables (not per layer); the verdict is needed here,
     // so the stream is waited for.
     uint32_t *flag = cu + lanes + 1;
-    b->lane_conflict = lanes > 1;   // (a lane alone has no other to meet)
-    if (lanes > 1 && launch_lane_conflict_check(b->stream, tables, activity, starts, lanes, table_pages,
+    b->lane_conflict = true;
+    if (launch_lane_conflict_check(b->stream, tables, activity, starts, lanes, table_pages,
                                    head.page_tokens, flag)) {
       if (hipMemcpyAsync(b->host_flag, flag, sizeof(uint32_t), hipMemcpyDeviceToHost, b->stream) != hipSuccess ||
           hipStreamSynchronize(b->stream) != hipSuccess)

@@ -44,9 +44,10 @@ __global__ __launch_bounds__(256) void gather_lane_metadata_kernel(
 }
 
 // One workgroup per lane (the reader): does any OTHER active lane append into a slot this lane
-// attends?  A fused run performs every append before every attention; lane by lane, a reader
-// that comes first sees the slot's old contents, and two lanes that append to one slot each see
-// their own value.  The host keeps pages copy-on-write, so this does not happen
+// attends, or this lane itself into one that its table names at another position too?  A fused run
+// performs every append before, or while, any lane attends; lane by lane, a reader that comes first
+// sees the slot's old contents, two lanes that append to one slot each see their own value, and a
+// lane whose page appears twice sees its new row at both positions.  The host keeps pages copy-on-write, so this does not happen
 // (crates/forja-host/src/lib.rs:5408-5470); tables are caller data all the same, so it is checked
 // and a run with such an overlap is executed dispatch by dispatch instead.
 // Dynamic LDS: 2 * lanes words (each lane's destination page and slot).
@@ -73,7 +74,8 @@ __global__ __launch_bounds__(256) void lane_conflict_kernel(const uint32_t *tabl
   for (uint32_t logical = threadIdx.x; logical < limit; logical += blockDim.x) {
     const uint32_t page = tables[((uint64_t)reader * table_pages + logical) * 2];
     for (uint32_t writer = 0; writer < lanes; ++writer)
-      if (writer != reader && slots[writer] != kNone && pages[writer] == page &&
+      if ((writer != reader || logical != starts[reader] / page_tokens) && slots[writer] != kNone &&
+          pages[writer] == page &&
           (uint64_t)logical * page_tokens + slots[writer] < attended)
         found = true;
   }

@@ -287,6 +287,32 @@ def test_tables_that_share_a_tail_page_run_dispatch_by_dispatch(cpu, hip, case, 
     assert hip.fusion_stats()[0] == before[0] + 1
 
 
+@pytest.mark.parametrize("idiom", ["append", "copies"])
+def test_a_lane_alone_runs_fused_and_keeps_the_serial_order(cpu, hip, idiom):
+    """A step recorded for one sequence is a run of one lane.  Where its table names the page of the
+    new row at an earlier position too, the row is attended at both, as in serial execution: such a
+    step stays dispatch by dispatch."""
+    for context, aliased in ((0, False), (16, False), (437, False), (437, True)):
+        results = []
+        for backend in (cpu, hip):
+            batch = LaneBatch(backend, [context], 8, 4, 16, seed=92, layers=2)
+            if aliased:
+                table = batch.host_tables[0].copy()
+                table[3] = table[context // 16]
+                backend.write(batch.tables[0], table.tobytes())
+            before = hip.fusion_stats()
+            commands, kept = CommandList(), []
+            for layer in range(2):
+                attended, rows = batch.record_layer(commands, layer, idiom=idiom)
+                commands.dispatch(Op.copy(), [attended], backend.alloc(DType.BF16, attended.shape))
+                kept += [attended, *rows, *batch.pools[layer]]
+            run(backend, commands)
+            if backend is hip:
+                assert hip.fusion_stats()[0] - before[0] == (0 if aliased else 2)
+            results.append(kept)
+        check(cpu, hip, results[0], results[1], exact=(2, 3, 6, 7))
+
+
 def _random_scenario(rng):
     """A decode batch recorded with random deviations from the regular pattern; every list is
     valid dispatch by dispatch, only some of it can be fused."""
