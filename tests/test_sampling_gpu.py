@@ -117,6 +117,28 @@ def test_f32_f16_and_strided_rows_and_a_single_row(cpu, hip):
     assert np.frombuffer(results[1][0], np.uint32)[1] == np.frombuffer(results[1][1], np.uint32)[0]
 
 
+@pytest.mark.parametrize("kind", ["long_tie", "flat", "two_peaks", "nan_peak", "inf_peak"])
+@pytest.mark.parametrize("dtype", [DType.BF16, DType.F32])
+def test_cuts_that_the_shortened_orderings_cannot_bound(cpu, hip, kind, dtype):
+    """`long_tie`: more columns share the bound of the selected candidates than are ranked at once.
+    The others, over a whole row: every column within reach of the largest; a sum that only columns
+    far below the largest complete (top_p close to one); a largest value that is no number."""
+    values = normal_bf16(104, 1, (3, 9001)).astype(np.float32)
+    if kind == "long_tie":
+        values[:, ::4] = 4.0
+    elif kind == "flat":
+        values *= 0.01
+    else:
+        values[:, 17], values[:, 4096] = 40.0, 39.5
+        if kind != "two_peaks":
+            values[1, 5000] = np.nan if kind == "nan_peak" else np.inf
+    for number, (temperature, top_k, top_p) in enumerate([(1.0, 20, 0.8), (0.7, 256, 0.95), (1.0, 0, 0.5), (0.6, 0, 0.95),
+                                                          (1.0, 0, 0.99999994), (1.0, 2000, 0.99999994)]):
+        words = orc.sampling_words(temperature, top_k, top_p, 31 + number)
+        expected, actual = sample_both(cpu, hip, values, words, 5, dtype=dtype)
+        assert expected.tolist() == actual.tolist(), (temperature, top_k, top_p)
+
+
 def test_distribution_on_the_device_matches_the_known_probabilities(hip):
     """The reference's chi-squared check (crates/forja-cpu/src/lib.rs:3283-3306) on the device:
     20000 positions of the 4-way case with top_k 3 and top_p 0.95."""
