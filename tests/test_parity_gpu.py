@@ -1646,6 +1646,23 @@ def test_quant_embed_copy_matmul_rms_norm_rope(cpu, hip):
     differential(cpu, hip, build, abs_=2e-2)
 
 
+@pytest.mark.parametrize("dtype", [DType.BF16, DType.F32])
+def test_quant_embed_rows_of_every_alignment(cpu, hip, dtype):
+    """Output rows that take the eight-value stores, dense and strided, and rows that start off them."""
+    table, ids_values = Quantised(83, 1, (37, 320)), np.array([36, 0, 3, 5, 36, 11, 2], dtype=np.uint32)
+
+    def build(backend):
+        ids, triple = upload(backend, ids_values, DType.U32), table.upload(backend)
+        plain = backend.alloc(dtype, (7, 320))
+        whole = upload(backend, np.ones((7, 339)), dtype)
+        wide = upload(backend, np.ones((7, 336)), dtype)
+        commands = CommandList()
+        for out in (plain, whole.narrow(1, 1, 320), wide.narrow(1, 8, 320)):
+            commands.dispatch(Op.quant_embed(4, 64), [*triple, ids], out)
+        return commands, [plain, whole, wide]
+    differential(cpu, hip, build)
+
+
 def test_quant_embed_zeroes_bad_rows_and_reports_the_lowest_bad_id(cpu, hip):
     """lib.rs:3020-3037 for the quantised table"""
     table = Quantised(82, 1, (300, 128))
