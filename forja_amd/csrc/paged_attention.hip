@@ -266,6 +266,7 @@ typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 constexpr uint32_t kMinSplitTokens = 128, kMaxSplitTokens = 1024;  // split length bounds
+constexpr uint32_t kFillingGroups = 512, kFilledSplitTokens = 512;  // see ragged_plan_kernel
 // Groups of several query tokens (prefill) are many and each split of theirs costs a merge of
 // `members x heads` partial rows: they are split only beyond this many keys.
 constexpr uint32_t kPrefillSplitTokens = 2048;
@@ -405,13 +406,13 @@ __global__ __launch_bounds__(256) void ragged_validate_kernel(const uint32_t *cu
 __global__ __launch_bounds__(256) void ragged_plan_kernel(FastRagged p, ErrorSlot *error) {
   __shared__ uint32_t class_items[kSizeClasses];   // items per class, then the class's cursor
   __shared__ unsigned long long total_attended;
-  __shared__ uint32_t merge_count, malformed_lane, longest_keys, trial_items;
+  __shared__ uint32_t merge_count, malformed_lane, longest_keys, longest_group, trial_items;
   constexpr uint32_t kKeysHeld = 4096;   // tokens whose key counts the split search keeps in LDS
   __shared__ uint32_t keys_held[kKeysHeld];
   for (uint32_t c = threadIdx.x; c < kSizeClasses; c += 256) class_items[c] = 0;
   if (threadIdx.x == 0) {
     total_attended = 0;
-    longest_keys = 0;
+    longest_keys = longest_group = 0;
     merge_count = 0;
     malformed_lane = 0xffffffffu;
   }
@@ -445,7 +446,7 @@ __global__ __launch_bounds__(256) void ragged_plan_kernel(FastRagged p, ErrorSlo
   uint32_t split_tokens = p.split_tokens;
   if (split_tokens == 0) {
     unsigned long long mine = 0;
-    uint32_t mine_longest = 0;
+    uint32_t mine_longest = 0, mine_group = 0;
     for (uint32_t token = threadIdx.x; token < p.tokens; token += 256) {
       const TokenPlan whole = plan_token(p, token, 1u << 30);
       // the keys of the token's group in whole tiles, for the search below: a decode batch has
@@ -455,15 +456,24 @@ __global__ __launch_bounds__(256) void ragged_plan_kernel(FastRagged p, ErrorSlo
       else if (p.item_slots) p.plans[token].chunk = keys;
       mine += whole.attended / p.group_tokens;
       mine_longest = max(mine_longest, keys);
+      if (whole.members > 1) mine_group = max(mine_group, keys);
     }
     for (int offset = 32; offset > 0; offset >>= 1) mine += __shfl_xor(mine, offset, 64);
     if ((threadIdx.x & 63) == 0) atomicAdd(&total_attended, mine);
     atomicMax(&longest_keys, mine_longest);
+    if (mine_group) atomicMax(&longest_group, mine_group);
     __syncthreads();
     if (p.item_slots == 0) {
       unsigned long long per_item = total_attended / kTargetItems;
       split_tokens = (uint32_t)((per_item + kTile - 1) / kTile * kTile);
-      if (split_tokens < kMinSplitTokens) split_tokens = kMinSplitTokens;
+      // Decode rows beside groups that fill the device twice over by themselves: items shorter than the
+      // longest group's shorten nothing and cost a start-up and a merge each.  (2000 prompt rows in
+      // four chunks and 48 decode rows of 128 to 4096 keys, 28 layers: 10.07 ms with items of 128 keys,
+      // 9.92 with 256, 9.75 with 512, 10.0 with 1024; 90 prompt rows and 5 such decode rows, four layers,
+      // which fill nothing: 1.33, 1.36, 1.40 and 1.50 ms.)
+      const bool filled = p.tokens / p.group_tokens * p.kv_heads >= kFillingGroups;
+      const uint32_t least = filled ? min(max(longest_group, kMinSplitTokens), kFilledSplitTokens) : kMinSplitTokens;
+      if (split_tokens < least) split_tokens = least;
       if (split_tokens > kMaxSplitTokens) split_tokens = kMaxSplitTokens;
     } else if (longest_keys <= p.max_splits * kTile &&
                2 * (total_attended / kTile + p.tokens) <= p.item_slots) {

@@ -1177,6 +1177,21 @@ def test_ragged_attention_equals_the_per_lane_sequence(cpu, hip, contexts, count
     assert cpu.read(cpu_out[1]) == hip.read(hip_out[1]) and cpu.read(cpu_out[2]) == hip.read(hip_out[2])
 
 
+@pytest.mark.parametrize("contexts,counts", [
+    # six tokens to a group of five heads, eight kv heads: 63 and 64 groups, the second with decode rows
+    # in items of the longest group's length, the third with groups shorter than the shortest items
+    ([0, 1500, 513], [381, 1, 1]), ([0, 1500, 513], [382, 1, 1]), ([0] * 8 + [1500, 31], [48] * 8 + [1, 1])])
+def test_decode_rows_beside_prefill_groups_that_fill_the_device(cpu, hip, contexts, counts):
+    def build(backend):
+        t, inputs = ragged_case(backend, contexts, counts, 40, 8, 16, seed=62)
+        commands = CommandList()
+        commands.dispatch_many(Op.paged_attention_ragged(1.0 / math.sqrt(128), 16), inputs,
+                               [t["out"], t["keys"], t["values"]])
+        return commands, [t["out"], t["keys"], t["values"]]
+    (cpu_out, _), (hip_out, _) = differential(cpu, hip, build)
+    assert cpu.read(cpu_out[1]) == hip.read(hip_out[1]) and cpu.read(cpu_out[2]) == hip.read(hip_out[2])
+
+
 DTYPE_MIXES = [
     # query and new rows, pools, output
     (DType.F32, DType.F16, DType.F32),      # the qwen3-coder engine
