@@ -453,18 +453,23 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a, Er
     // ---- general case: order the allowed columns.  A weight below 2^-25 changes no f32 sum that
     // starts with the largest column's weight of one, so for the nucleus the columns that far below the
     // largest can stay out of the ordering, unless the sum of what is left does not reach top_p: then
-    // all are ordered.  (NaN columns stay in: their weight makes the sum NaN.)
+    // all are ordered.  So they are where a column holds a NaN of negative sign: it sorts behind the
+    // columns left out, and makes the sum NaN if and only if top_k reaches it.  (A positive one is the
+    // largest column.)
     uint64_t largest = 0;
+    bool nan_behind = false;
     if (top_p < 1.0f) {
       row.for_each_allowed([&](uint32_t index, float value) {
         const uint64_t mine = candidate(value, index);
         largest = mine > largest ? mine : largest;
+        nan_behind |= __float_as_uint(value) > 0xff800000u;
       });
       largest = block_max(largest, s);
+      nan_behind = __syncthreads_or(nan_behind) != 0;
     }
     const float maximum = top_p < 1.0f ? row.value((uint32_t)(largest - 1)) : 0.0f;
     uint32_t count = 0;
-    for (bool filtered = top_p < 1.0f && is_finite(maximum);; filtered = false) {
+    for (bool filtered = top_p < 1.0f && is_finite(maximum) && !nan_behind;; filtered = false) {
       // Start from descending index so that the stable passes leave equal values in descending
       // index order.
       __syncthreads();

@@ -139,6 +139,24 @@ def test_cuts_that_the_shortened_orderings_cannot_bound(cpu, hip, kind, dtype):
         assert expected.tolist() == actual.tolist(), (temperature, top_k, top_p)
 
 
+NEGATIVE_NAN = np.array(0xffc00000, np.uint32).view(np.float32)   # x86's default NaN: sorts below every number
+
+
+@pytest.mark.parametrize("dtype", [DType.BF16, DType.F32])
+def test_a_nan_that_sorts_last_stays_outside_top_k(cpu, hip, dtype):
+    """Fewer columns than top_k lie within reach of the two peaks, but more columns than top_k sort before the
+    NaN: the cut leaves it out, and the nucleus is the two peaks' (0.62 and 0.38)."""
+    values = normal_bf16(105, 1, (4, 9001)).astype(np.float32)
+    values[:, 17], values[:, 4096], values[:, 600] = 40.0, 39.5, NEGATIVE_NAN
+    drawn = set()
+    for seed in range(12):
+        words = orc.sampling_words(1.0, 1000, 0.95, seed)
+        expected, actual = sample_both(cpu, hip, values, words, seed, dtype=dtype)
+        assert expected.tolist() == actual.tolist(), seed
+        drawn |= set(expected.tolist())
+    assert drawn == {17, 4096}
+
+
 def test_distribution_on_the_device_matches_the_known_probabilities(hip):
     """The reference's chi-squared check (crates/forja-cpu/src/lib.rs:3283-3306) on the device:
     20000 positions of the 4-way case with top_k 3 and top_p 0.95."""
