@@ -283,6 +283,9 @@ __device__ inline void scatter_tile(bool valid, uint32_t digit, uint2 element, u
 template <typename WeightAt>
 __device__ inline uint32_t top_p_keep(uint32_t count, float top_p, WeightAt weight_at,
                                       SampleShared &s) {
+  // A NaN of negative sign sorts last; it makes the sum NaN, also where the walk below ends before it.
+  const float last = weight_at(count - 1);
+  if (last != last) return 1;
   const float4 *staged = (const float4 *)s.stage;
   float total = 0.0f;
   for (uint32_t first = 0; first < count; first += kStage) {
@@ -301,7 +304,8 @@ __device__ inline uint32_t top_p_keep(uint32_t count, float top_p, WeightAt weig
         total += v.z;
         total += v.w;
       }
-      // The weights descend: once one no longer changes the sum, none behind it does.
+      // The weights descend (none is NaN, or the first is and the sum with it): once one no longer
+      // changes the sum, none behind it does.
       s.word[0] = total + s.stage[chunk - 1] == total ? 1u : 0u;
     }
     __syncthreads();

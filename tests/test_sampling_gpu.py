@@ -157,6 +157,20 @@ def test_a_nan_that_sorts_last_stays_outside_top_k(cpu, hip, dtype):
     assert drawn == {17, 4096}
 
 
+@pytest.mark.parametrize("dtype", [DType.BF16, DType.F32])
+def test_a_nan_that_sorts_last_makes_a_long_sum_nan(cpu, hip, dtype):
+    """More ordered columns than are staged at a time, whose weights stop to change the sum long before
+    the last: the NaN there still leaves the largest column as the only candidate, where top_k reaches it."""
+    values = normal_bf16(106, 1, (4, 60000)).astype(np.float32) * 3.0
+    values[:3, 11111] = NEGATIVE_NAN            # the fourth row has none
+    for number, top_k in enumerate((0, 60000, 59999, 5000) * 3):
+        words = orc.sampling_words(1.0, top_k, 0.9, 41 + number)
+        expected, actual = sample_both(cpu, hip, values, words, number, dtype=dtype)
+        assert expected.tolist() == actual.tolist(), (number, top_k)
+        if top_k in (0, 60000):
+            assert np.all(values[np.arange(3), expected[:3]] == np.nanmax(values[:3], axis=1))
+
+
 def test_distribution_on_the_device_matches_the_known_probabilities(hip):
     """The reference's chi-squared check (crates/forja-cpu/src/lib.rs:3283-3306) on the device:
     20000 positions of the 4-way case with top_k 3 and top_p 0.95."""
