@@ -480,30 +480,57 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
   constexpr uint32_t kOutCols = 16 * CT, kLanes = kOutCols / 4, kRows = 64 / kLanes;   // of a piece of 64 lanes
   __syncthreads();
   float *blocks = (float *)staged;
-  const uint32_t piece_row = lane / kLanes, piece_column = lane % kLanes * 4;
+  // (counted anew: the thread's index need not stay in a register through the loop)
+  const uint32_t out_lane = __builtin_amdgcn_mbcnt_hi(0xffffffffu, __builtin_amdgcn_mbcnt_lo(0xffffffffu, 0u));
+  const uint32_t piece_row = out_lane / kLanes, piece_column = out_lane % kLanes * 4;
   const uint32_t column = col_block * kBlockCols + wc * kOutCols + piece_column;
   auto put_block = [&](int rt) {
-    float *mine = blocks + ((wk * WC + wc) * kBlocks + rt % kBlocks) * kBlock + 4 * g * kLine + n;
+    float *mine = blocks + ((wk * WC + wc) * kBlocks + rt % kBlocks) * kBlock + 4 * (out_lane >> 4) * kLine + (out_lane & 15);
 #pragma unroll
     for (int tp = 0; tp < kColTiles; ++tp)
 #pragma unroll
       for (int i = 0; i < 4; ++i) mine[i * kLine + 16 * tp] = acc[tp][rt][i];
+  };
+  // Four results that are no numbers, value by value: a row that holds an infinity has it subtracted from
+  // itself by its pieces and by its group sum, and values next to f32's largest overflow on the way (a
+  // group sum by 128 of them).  What the products themselves give is the reference's infinity, or NaN.
+  auto by_value = [&](const f32x4 &value, int pj, uint32_t row) -> f32x4 {
+    bool number = true;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) number &= (__float_as_uint(value[i]) & 0x7f800000u) != 0x7f800000u;
+    if (__builtin_expect(number, 1)) return value;
+    const uint64_t in_row = kRouted ? row_ids[row] / a.route_div : tile_first + row;
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (uint32_t k = first_quad * kQuad; k < last_quad * kQuad; ++k) {
+      const uint64_t x_at = in_row * a.x_row_stride + k;
+      const float x = XP == 1 ? low_bf16(((const uint16_t *)a.x)[x_at]) : ((const float *)a.x)[x_at];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint64_t group = expert * a.expert_groups + (uint64_t)(column + i) * groups_per_row + k / kGroup;
+        const uint32_t word = a.packed[pj][expert * a.expert_words + (uint64_t)(column + i) * words_per_row + k / (32 / BITS)];
+        const float q = (float)(word >> (k % (32 / BITS) * BITS) & ((1u << BITS) - 1));
+        sum[i] += x * (low_bf16(a.scales[pj][group]) * q + low_bf16(a.biases[pj][group]));
+      }
+    }
+    return sum;
   };
   auto finish_block = [&](int rt) {
     const float *from = blocks + (wc * kBlocks + rt % kBlocks) * kBlock + piece_column;
 #pragma unroll 1
     for (uint32_t step = wk; step < 16 / kRows; step += WK) {
       const uint32_t in_tile = step * kRows + piece_row, row = 16 * rt + in_tile;
+      if (row >= tile_count || column >= a.columns) continue;
       f32x4 value = *(const f32x4 *)(from + in_tile * kLine);
 #pragma unroll
       for (int part = 1; part < WK; ++part)
         value += *(const f32x4 *)(from + part * WC * kBlocks * kBlock + in_tile * kLine);
+      value = by_value(value, 0, row);
       if constexpr (kPair) {
-        const f32x4 up = *(const f32x4 *)(from + in_tile * kLine + kOutCols);
+        const f32x4 up = by_value(*(const f32x4 *)(from + in_tile * kLine + kOutCols), 1, row);
 #pragma unroll
         for (int i = 0; i < 4; ++i) value[i] = value[i] * (1.0f / (1.0f + __expf(-value[i]))) * up[i];
       }
-      if (row >= tile_count || column >= a.columns) continue;
       if (!kRouted && a.splits > 1) {
         *(f32x4 *)((float *)a.out + ((uint64_t)split * a.rows + tile_first + row) * a.columns + column) = value;
         continue;

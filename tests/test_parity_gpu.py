@@ -322,6 +322,64 @@ def test_routed_products_in_row_tiles(cpu, hip, rows, k, experts, n, inner, dtyp
         differential(cpu, hip, build, expect_error={Status.INDEX_OUT_OF_RANGE, Status.DEVICE_ERROR_FLAG})
 
 
+def rows_with_infinities(seed, rows, k, dtype):
+    """Rows 1 to 5: an infinity of either sign, two that agree, two that do not, a NaN; row 6 (f32 only):
+    values next to the largest of f32, whose sum over a group by 128 is past it."""
+    values = orc.fill_normal_f32(seed, 1, rows * k).reshape(rows, k) if dtype == DType.F32 else normal_bf16(seed, 1, (rows, k))
+    values[1, 7], values[2, k - 1], values[3, [0, 70]] = np.inf, -np.inf, np.inf
+    values[4, 5], values[4, 200], values[5, 64] = np.inf, -np.inf, np.nan
+    if dtype == DType.F32:
+        values[6] *= np.float32(2.0 ** 120)
+    return values
+
+
+def same_kinds(expected, actual, dtype):
+    """The same infinities and NaNs; elsewhere sums of the same products: f32 ones that differ by their order
+    (1e-5 of the row's typical value, as in assert_close), rounded once more to bf16."""
+    for kind in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(kind(expected), kind(actual))
+    finite = np.isfinite(expected)
+    assert finite.any() and not finite.all()
+    e, a = (np.where(finite, v, 0).astype(np.float64) for v in (expected, actual))
+    rel, of_row = (1e-4, 1e-5) if dtype == DType.F32 else (1e-2, 1e-2)
+    typical = np.sqrt(np.mean(np.square(e), axis=tuple(range(1, e.ndim)), keepdims=True))
+    assert np.all(np.abs(a - e) <= of_row * typical + rel * np.abs(e))
+
+
+@pytest.mark.parametrize("rows,n,k,bits,dtype", [(40, 272, 1280, 4, DType.F32), (9, 4112, 2048, 4, DType.F32),
+                                                 (40, 272, 768, 8, DType.F32), (48, 400, 3328, 4, DType.BF16)])
+def test_infinities_in_row_tiles_reach_the_results_as_the_products_give_them(cpu, hip, rows, n, k, bits, dtype):
+    weights, values = Quantised(27, 300 + n + k, (n, k), bits=bits), rows_with_infinities(29, rows, k, dtype)
+    results = []
+    for backend in (cpu, hip):
+        out = backend.alloc(dtype, (rows, n))
+        commands = CommandList()
+        commands.dispatch(Op.quant_matmul(bits, 64), [upload(backend, values, dtype), *weights.upload(backend)], out)
+        run(backend, commands)
+        results.append(to_f32(backend.read(out), dtype).reshape(rows, n))
+    same_kinds(*results, dtype)
+
+
+@pytest.mark.parametrize("dtype", [DType.F32, DType.BF16])
+def test_infinities_in_routed_row_tiles(cpu, hip, dtype):
+    rows, k, experts, n, inner = 70, 4, 7, 272, 768
+    gate, up = (Quantised(28, 1 + i, (n, inner), experts=experts) for i in range(2))
+    indices, values = routed_case(28, rows, k, experts, n, inner), rows_with_infinities(29, rows, inner, dtype)
+    results = []
+    for backend in (cpu, hip):
+        x, idx = upload(backend, values, dtype), upload(backend, indices, DType.U32)
+        plain, activated = backend.alloc(dtype, (rows, k, n)), backend.alloc(dtype, (rows, k, n))
+        g, u = gate.upload(backend), up.upload(backend)
+        commands = CommandList()
+        commands.dispatch(Op.gather_quant_matmul(4, 64), [x, *g, idx], plain)
+        commands.dispatch_epilogue(Op.gather_quant_matmul(4, 64), [x, *g, *u, idx], activated,
+                                   backend.prepare_epilogue(programs.silu_mul_elements()), [])
+        run(backend, commands)
+        results.append([to_f32(backend.read(out), dtype).reshape(rows, k, n) for out in (plain, activated)])
+    for expected, actual in zip(*results):
+        same_kinds(expected, actual, dtype)
+
+
 @pytest.mark.parametrize("dtype,bits,group", [(DType.F32, 4, 64), (DType.F16, 8, 32), (DType.BF16, 4, 128)])
 def test_quant_matmul_with_f16_scales_and_a_residual_in_other_dtypes(cpu, hip, dtype, bits, group):
     """f16 affine parameters (the reference allows f16 or bf16, quantized.rs:78-121) and the
