@@ -491,14 +491,75 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) mine[i * kLine + 16 * tp] = acc[tp][rt][i];
   };
-  // Four results that are no numbers, value by value: a row that holds an infinity has it subtracted from
-  // itself by its pieces and by its group sum, and values next to f32's largest overflow on the way (a
-  // group sum by 128 of them).  What the products themselves give is the reference's infinity, or NaN.
-  auto by_value = [&](const f32x4 &value, int pj, uint32_t row) -> f32x4 {
-    bool number = true;
+  auto swiglu = [](f32x4 &value, const f32x4 &up) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) number &= (__float_as_uint(value[i]) & 0x7f800000u) != 0x7f800000u;
-    if (__builtin_expect(number, 1)) return value;
+    for (int i = 0; i < 4; ++i) value[i] = value[i] * (1.0f / (1.0f + __expf(-value[i]))) * up[i];
+  };
+  auto store = [&](uint32_t row, f32x4 value) {
+    if (!kRouted && a.splits > 1) {
+      *(f32x4 *)((float *)a.out + ((uint64_t)split * a.rows + tile_first + row) * a.columns + column) = value;
+      return;
+    }
+    if (!kRouted && a.residual) {
+      const uint64_t at = (uint64_t)(tile_first + row) * a.residual_row_stride + column;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        value[i] += XP == 1 ? low_bf16(((const uint16_t *)a.residual)[at + i]) : ((const float *)a.residual)[at + i];
+    }
+    const uint64_t at = (uint64_t)(kRouted ? row_ids[row] : tile_first + row) * a.out_row_stride + column;
+    if (a.out_f32) {
+      float *to = (float *)a.out + at;
+      if (a.out_aligned)
+        *(f32x4 *)to = value;
+      else
+        for (int i = 0; i < 4; ++i) to[i] = value[i];
+    } else {
+      uint16_t *to = (uint16_t *)a.out + at;
+      const u32x2 packed = {pack_bf16(value[0], value[1]), pack_bf16(value[2], value[3])};
+      if (a.out_aligned)
+        *(u32x2 *)to = packed;
+      else
+        for (int i = 0; i < 4; ++i) to[i] = (uint16_t)(packed[i / 2] >> (16 * (i % 2)));
+    }
+  };
+  // Results that are computed again value by value, after the others (one copy of the code), a bit for each
+  // four that are no numbers: a row that holds an infinity has it subtracted from itself by its pieces and
+  // by its group sum, and values next to f32's largest overflow on the way (a group sum by 128 of them).
+  // What the products themselves give is the reference's infinity, or NaN.
+  // So too results of f32 rows that are next to nothing, all four below 2^-80: where every value of a row is
+  // below 2^-104 or so, the pieces of the group sums and the products of factor and scale lose bits below the
+  // smallest normal number, and only such rows (or weights no larger than 2^-40) end there.  (Rows of 4096
+  // values at 2^-126: error 3e-4 through the pieces, 4e-7 value by value.  Looking at the values instead of
+  // the results costs the loop 2 % of the time.)
+  constexpr uint32_t kSteps = 16 / kRows;
+  uint32_t again = 0;
+  auto is_number = [](const f32x4 &value) {
+    uint32_t largest = 0;   // bits of the largest of the four; a NaN's are above an infinity's
+#pragma unroll
+    for (int i = 0; i < 4; ++i) largest = max(largest, __float_as_uint(value[i]) & 0x7fffffffu);
+    return XP == 1 ? largest < 0x7f800000u : largest - (47u << 23) < 0x7f800000u - (47u << 23) || largest == 0;
+  };
+  auto finish_block = [&](int rt) {
+    const float *from = blocks + (wc * kBlocks + rt % kBlocks) * kBlock + piece_column;
+#pragma unroll 1
+    for (uint32_t step = wk; step < kSteps; step += WK) {
+      const uint32_t in_tile = step * kRows + piece_row, row = 16 * rt + in_tile;
+      f32x4 value = *(const f32x4 *)(from + in_tile * kLine);
+#pragma unroll
+      for (int part = 1; part < WK; ++part)
+        value += *(const f32x4 *)(from + part * WC * kBlocks * kBlock + in_tile * kLine);
+      bool number = is_number(value);
+      if constexpr (kPair) {
+        const f32x4 up = *(const f32x4 *)(from + in_tile * kLine + kOutCols);
+        number &= is_number(up);
+        swiglu(value, up);
+      }
+      if (row >= tile_count || column >= a.columns) continue;
+      if (!number) again |= 1u << (rt * kSteps + step);
+      store(row, value);
+    }
+  };
+  auto by_value = [&](int pj, uint32_t row) -> f32x4 {
     const uint64_t in_row = kRouted ? row_ids[row] / a.route_div : tile_first + row;
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
@@ -515,49 +576,6 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
     }
     return sum;
   };
-  auto finish_block = [&](int rt) {
-    const float *from = blocks + (wc * kBlocks + rt % kBlocks) * kBlock + piece_column;
-#pragma unroll 1
-    for (uint32_t step = wk; step < 16 / kRows; step += WK) {
-      const uint32_t in_tile = step * kRows + piece_row, row = 16 * rt + in_tile;
-      if (row >= tile_count || column >= a.columns) continue;
-      f32x4 value = *(const f32x4 *)(from + in_tile * kLine);
-#pragma unroll
-      for (int part = 1; part < WK; ++part)
-        value += *(const f32x4 *)(from + part * WC * kBlocks * kBlock + in_tile * kLine);
-      value = by_value(value, 0, row);
-      if constexpr (kPair) {
-        const f32x4 up = by_value(*(const f32x4 *)(from + in_tile * kLine + kOutCols), 1, row);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) value[i] = value[i] * (1.0f / (1.0f + __expf(-value[i]))) * up[i];
-      }
-      if (!kRouted && a.splits > 1) {
-        *(f32x4 *)((float *)a.out + ((uint64_t)split * a.rows + tile_first + row) * a.columns + column) = value;
-        continue;
-      }
-      if (!kRouted && a.residual) {
-        const uint64_t at = (uint64_t)(tile_first + row) * a.residual_row_stride + column;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          value[i] += XP == 1 ? low_bf16(((const uint16_t *)a.residual)[at + i]) : ((const float *)a.residual)[at + i];
-      }
-      const uint64_t at = (uint64_t)(kRouted ? row_ids[row] : tile_first + row) * a.out_row_stride + column;
-      if (a.out_f32) {
-        float *to = (float *)a.out + at;
-        if (a.out_aligned)
-          *(f32x4 *)to = value;
-        else
-          for (int i = 0; i < 4; ++i) to[i] = value[i];
-      } else {
-        uint16_t *to = (uint16_t *)a.out + at;
-        const u32x2 packed = {pack_bf16(value[0], value[1]), pack_bf16(value[2], value[3])};
-        if (a.out_aligned)
-          *(u32x2 *)to = packed;
-        else
-          for (int i = 0; i < 4; ++i) to[i] = (uint16_t)(packed[i / 2] >> (16 * (i % 2)));
-      }
-    }
-  };
   if constexpr (WK > 1) {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) put_block(rt);
@@ -572,6 +590,13 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
       finish_block(rt);
       __builtin_amdgcn_wave_barrier();
     }
+  }
+#pragma unroll 1
+  for (; again; again &= again - 1) {
+    const uint32_t bit = (uint32_t)__ffs((int)again) - 1, row = 16 * (bit / kSteps) + bit % kSteps * kRows + piece_row;
+    f32x4 value = by_value(0, row);
+    if constexpr (kPair) swiglu(value, by_value(1, row));
+    store(row, value);
   }
 }
 

@@ -380,6 +380,56 @@ def test_infinities_in_routed_row_tiles(cpu, hip, dtype):
         same_kinds(expected, actual, dtype)
 
 
+def rows_of_every_magnitude(seed, rows, k):
+    """Rows at 2^-130 to 2^120, a row of zeros, rows with groups of zeros, of values far below the row's
+    others, and of 1e6 beside 1e-3; every value uses its whole mantissa."""
+    values = orc.fill_normal_f32(seed, 1, rows * k).reshape(rows, k)
+    exponents = (-130, -126, -120, -112, -100, -90, -60, 60, 100, 118)
+    for row, exponent in enumerate(exponents):
+        values[row] = np.ldexp(values[row], exponent)
+    values[10], values[11, :64], values[12, 64:192] = 0, 0, values[12, 64:192] * np.float32(2.0 ** -120)
+    values[13, ::2] *= np.float32(1e6)
+    values[13, 1::2] *= np.float32(1e-3)
+    values[14] = np.ldexp(np.abs(values[14]), -126)
+    return values
+
+
+def close_row_by_row(actual, values, dense, k):
+    """Against 64 bits.  f32 sums of K products: K roundings of 2^-24 of the running sum, which add up like sqrt(K) in
+    the 2-norm over a row of results.  The running sum is at most about the larger of the sum itself (terms of one
+    sign) and the root of its squared terms; and every addition below 2^-126 rounds to 2^-149."""
+    expected = values.astype(np.float64) @ np.swapaxes(dense, -1, -2)
+    size = np.maximum(np.abs(expected), np.sqrt(values.astype(np.float64) ** 2 @ np.swapaxes(dense, -1, -2) ** 2))
+    error = np.linalg.norm(actual - expected, axis=-1)
+    bound = math.sqrt(k) * 2.0 ** -24 * np.linalg.norm(size, axis=-1) + 2.0 ** -149 * k ** 0.5 * dense.shape[-2] ** 0.5
+    assert np.all(error <= bound), (error / bound).max()
+
+
+@pytest.mark.parametrize("rows,n,k,bits", [(40, 272, 1280, 4), (16, 4112, 2048, 4), (40, 272, 768, 8)])
+def test_f32_rows_of_every_magnitude_in_row_tiles(hip, rows, n, k, bits):
+    weights, values = Quantised(27, 300 + n + k, (n, k), bits=bits), rows_of_every_magnitude(29, rows, k)
+    out = hip.alloc(DType.F32, (rows, n))
+    commands = CommandList()
+    commands.dispatch(Op.quant_matmul(bits, 64), [upload(hip, values, DType.F32), *weights.upload(hip)], out)
+    run(hip, commands)
+    close_row_by_row(to_f32(hip.read(out), DType.F32).reshape(rows, n).astype(np.float64), values, weights.dequantised(), k)
+
+
+def test_f32_rows_of_every_magnitude_in_routed_row_tiles(hip):
+    rows, k, experts, n, inner = 70, 4, 7, 272, 768
+    weights = Quantised(28, 1, (n, inner), experts=experts)
+    indices, values = routed_case(28, rows, k, experts, n, inner), rows_of_every_magnitude(29, rows, inner)
+    out = hip.alloc(DType.F32, (rows, k, n))
+    commands = CommandList()
+    commands.dispatch(Op.gather_quant_matmul(4, 64), [upload(hip, values, DType.F32), *weights.upload(hip),
+                                                      upload(hip, indices, DType.U32)], out)
+    run(hip, commands)
+    actual, dense = to_f32(hip.read(out), DType.F32).reshape(rows, k, n).astype(np.float64), weights.dequantised()
+    for slot in range(k):
+        for row in range(rows):
+            close_row_by_row(actual[row:row + 1, slot], values[row:row + 1], dense[indices[row, slot]], inner)
+
+
 @pytest.mark.parametrize("dtype,bits,group", [(DType.F32, 4, 64), (DType.F16, 8, 32), (DType.BF16, 4, 128)])
 def test_quant_matmul_with_f16_scales_and_a_residual_in_other_dtypes(cpu, hip, dtype, bits, group):
     """f16 affine parameters (the reference allows f16 or bf16, quantized.rs:78-121) and the
