@@ -1581,7 +1581,10 @@ bool same_lane_shape(const LaneMember &a, const LaneMember &b) {
 // Longest fusable run of per-lane attention starting at `first`; false when there is none.  A run of
 // one lane is a step recorded for a single sequence: its layers then share one gather and one plan,
 // and the attention kernel stores the new row itself (48 layers of one lane at 6000 keys: the plan
-// per layer 12 us, the two copies 9).  It is taken only where the member stands alone (`alone`: not
+// per layer 12 us, the two copies 9), and nothing waits for the device, since the one thing that the
+// tables decide (a page named twice) is read there.  Sequences whose layers alternate in one submission are
+// such runs too, each with a gather and a plan of its own (3000 and 900 keys, f32 rows: 34 us a layer and
+// sequence, 39 dispatch by dispatch, 48 when each waited for a verdict).  It is taken only where the member stands alone (`alone`: not
 // behind a member that was not fused; nor before one), because members next to each other that make
 // no run are an order that the caller wants kept.  `run->dispatches` says how many dispatches were
 // examined also when false, so that the caller does not examine the tail of a refused run again.
@@ -1676,9 +1679,10 @@ fh_status run_lane_group(fh_backend *b, const LaneRun &run, ErrorSlot *errors, b
 
   // What the gathered metadata depends on; equal keys mean the gather of an earlier layer holds.
   std::vector<uint64_t> key;
-  key.reserve(5ull * lanes + 2);
+  key.reserve(5ull * lanes + 3);
   key.push_back(lanes);
   key.push_back(table_words);
+  key.push_back(head.page_tokens);
   for (const LaneMember &m : run.members) {
     key.push_back(m.table.buffer);
     key.push_back(m.table.offset);
@@ -1707,16 +1711,16 @@ fh_status run_lane_group(fh_backend *b, const LaneRun &run, ErrorSlot *errors, b
         }
         sources.start[local] = m.q_start;
       }
-      launch_gather_lane_metadata(b->stream, sources, base, chunk, lanes, table_words, tables,
-                                  activity, starts, cu);
+      launch_gather_lane_metadata(b->stream, sources, base, chunk, lanes, table_words,
+                                  head.page_tokens, tables, activity, starts, cu);
     }
     // The one thing the tensors cannot show: an append into a slot attended elsewhere.  Checked
     // on the gathered tables, once per set of tables (not per layer); the verdict is needed here,
-    // so the stream is waited for.
+    // so the stream is waited for.  A lane alone needs no verdict: the attention reads the flag.
     uint32_t *flag = cu + lanes + 1;
-    b->lane_conflict = true;
-    if (launch_lane_conflict_check(b->stream, tables, activity, starts, lanes, table_pages,
-                                   head.page_tokens, flag)) {
+    b->lane_conflict = lanes > 1;
+    if (lanes > 1 && launch_lane_conflict_check(b->stream, tables, activity, starts, lanes, table_pages,
+                                                head.page_tokens, flag)) {
       if (hipMemcpyAsync(b->host_flag, flag, sizeof(uint32_t), hipMemcpyDeviceToHost, b->stream) != hipSuccess ||
           hipStreamSynchronize(b->stream) != hipSuccess)
         return FH_DEVICE_EXECUTION_FAILED;
@@ -1784,6 +1788,7 @@ fh_status run_lane_group(fh_backend *b, const LaneRun &run, ErrorSlot *errors, b
   problem.error_stride = head.dispatches;
   problem.attention_error_offset = head.attention_at;
   problem.one_row_per_lane = 1;   // by construction: every member is one query row of its own lane
+  problem.row_twice = lanes == 1 ? cu + lanes + 1 : nullptr;
   if (!run_ragged_attention(b, problem, errors)) return FH_ALLOCATION_FAILED;
 
   for (uint32_t base = 0; base < lanes; base += kLaneChunk) {

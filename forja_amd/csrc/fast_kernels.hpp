@@ -247,6 +247,9 @@ struct RaggedAttention {
   // the work plan is built; a violation is reported).  The attention kernel can then store a
   // lane's new key and value row itself, because no other row's attention reads them.
   uint32_t one_row_per_lane;
+  // Null, or (one lane, whose table nothing has checked) a device word: non-zero where the table names the
+  // page of the new row at an earlier position too, so that the row is to be stored before anything is read.
+  const uint32_t *row_twice;
 };
 // Always handles the problem (specialised kernel when the layout allows, generic otherwise);
 // false only when workspace allocation fails.

@@ -115,11 +115,12 @@ struct LaneRows {
   void *second[kLaneChunk];  // a second copy of it, or null
 };
 // Lanes [first, first + count) of `lanes`: tables [lanes, table_words], activity/starts [lanes],
-// cu [lanes + 1] (one query row per lane) followed by one word, cleared here, that
-// launch_lane_conflict_check raises.
+// cu [lanes + 1] (one query row per lane) followed by one word.  Of several lanes it is cleared here and
+// launch_lane_conflict_check raises it; of a lane alone it is set here, to whether the lane's table names
+// the slot of the new row at another attended position too.
 void launch_gather_lane_metadata(hipStream_t s, const LaneSources &sources, uint32_t first,
                                  uint32_t count, uint32_t lanes, uint32_t table_words,
-                                 uint32_t *tables, uint32_t *activity, uint32_t *starts,
+                                 uint32_t page_tokens, uint32_t *tables, uint32_t *activity, uint32_t *starts,
                                  uint32_t *cu);
 // Sets *conflict to 1 when an active lane appends into a slot another active lane attends (the
 // gathered arrays of launch_gather_lane_metadata; tables as (page, generation) pairs).  False,

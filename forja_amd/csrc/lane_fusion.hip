@@ -22,16 +22,26 @@ namespace fh {
 
 namespace {
 
-// One workgroup per lane: copies the lane's block table and writes its scalars.
+// One workgroup per lane: copies the lane's block table and writes its scalars.  A lane alone (nothing
+// has to be decided for it on the host, and no kernel of its own is spent on it) is also looked through for
+// the slot of its new row at another attended position, see FastRagged::row_twice.
 __global__ __launch_bounds__(256) void gather_lane_metadata_kernel(
     LaneSources sources, uint32_t first, uint32_t count, uint32_t lanes, uint32_t table_words,
-    uint32_t *tables, uint32_t *activity, uint32_t *starts, uint32_t *cu) {
+    uint32_t page_tokens, uint32_t *tables, uint32_t *activity, uint32_t *starts, uint32_t *cu) {
   const uint32_t local = blockIdx.x;
   if (local >= count) return;
   const uint32_t lane = first + local;
-  if (lane == 0 && threadIdx.x == 0) cu[lanes + 1] = 0;   // the overlap flag of lane_conflict_kernel
   const uint32_t *table = sources.table[local];
   uint32_t *target = tables + (uint64_t)lane * table_words;
+  bool twice = false;
+  if (lanes == 1) {
+    const uint32_t start = sources.start[local], own = start / page_tokens;
+    if (own < table_words / 2)
+      for (uint32_t logical = threadIdx.x; logical < own; logical += blockDim.x)   // (no page behind is attended)
+        twice |= table[2 * logical] == table[2 * own];
+  }
+  twice = __syncthreads_or(twice) != 0;
+  if (lane == 0 && threadIdx.x == 0) cu[lanes + 1] = twice;   // several lanes: lane_conflict_kernel raises it
   for (uint32_t word = threadIdx.x; word < table_words; word += blockDim.x)
     target[word] = table[word];
   if (threadIdx.x == 0) {
@@ -253,12 +263,12 @@ void launch_fold_chunk_errors(hipStream_t stream, ErrorSlot *staged, ErrorSlot *
 
 void launch_gather_lane_metadata(hipStream_t stream, const LaneSources &sources, uint32_t first,
                                  uint32_t count, uint32_t lanes, uint32_t table_words,
-                                 uint32_t *tables, uint32_t *activity, uint32_t *starts,
-                                 uint32_t *cu) {
-  if (count == 0 || count > kLaneChunk || first + count > lanes) return;
+                                 uint32_t page_tokens, uint32_t *tables, uint32_t *activity,
+                                 uint32_t *starts, uint32_t *cu) {
+  if (count == 0 || count > kLaneChunk || first + count > lanes || page_tokens == 0) return;
   gather_lane_metadata_kernel<<<dim3(count), 256, 0, stream>>>(sources, first, count, lanes,
-                                                                table_words, tables, activity,
-                                                                starts, cu);
+                                                                table_words, page_tokens, tables,
+                                                                activity, starts, cu);
 }
 
 bool launch_lane_conflict_check(hipStream_t stream, const uint32_t *tables, const uint32_t *activity,

@@ -316,6 +316,10 @@ struct FastRagged {
   const void *k_new, *v_new;   // q_dtype elements
   uint64_t kn_stride_t, kn_stride_h, vn_stride_t, vn_stride_h;
   uint32_t append_in_kernel, append_error_back;
+  // Null, or (a lane alone, whose table nothing has checked) a device word: non-zero where the table names
+  // the page of the new row at an earlier position too.  Every split then stores the row, the same bytes,
+  // before it reads: the split that meets it at the other position sees it, as after an append of its own.
+  const uint32_t *row_twice;
   uint32_t promised;   // one query row per lane, vouched for by the caller: verified by the plan
 };
 
@@ -762,9 +766,10 @@ __device__ inline void ragged_attention_body(const FastRagged &p, ErrorSlot *err
   const uint32_t end = min(longest, begin + plan.chunk);
   const uint32_t pt = p.page_tokens;
   const uint32_t *table = p.tables + (uint64_t)plan.lane * p.table_pages * 2;
-  if (NT == 1 && p.append_in_kernel && split + 1 == plan.splits) {
+  if (NT == 1 && p.append_in_kernel &&
+      (split + 1 == plan.splits || (p.row_twice != nullptr && p.row_twice[0] != 0))) {
     // This wave's kv head of the lane's new row goes into the pool before anything is read: the
-    // row sits at the last attended position, which only this workgroup's range contains.
+    // row sits at the last attended position, which only the last split's range contains.
     const uint32_t position = plan.attended - 1, logical = position / pt;
     uint32_t physical;
     if (entry_ok(table, p.generations, logical, p.table_pages, p.physical_pages, &physical)) {
@@ -1453,6 +1458,7 @@ bool run_ragged_attention(fh_backend *backend, const RaggedAttention &p, ErrorSl
     f.vn_stride_t = p.v_new.stride[0];
     f.vn_stride_h = p.v_new.stride[1];
     f.append_error_back = p.attention_error_offset;
+    f.row_twice = p.row_twice;
     if (!reuse) launch_plan(stream, f, error);
   }
   if (fast && f.append_in_kernel) {

@@ -202,7 +202,10 @@ FH_API fh_status fh_prepare_program(fh_backend *backend, uint32_t kind /* 0 map,
 FH_API fh_status fh_release_program(fh_backend *backend, fh_program program);
 
 /* Backend::submit (lib.rs:1419-1516): validates every tensor and operand shape, then enqueues the
- * dispatches in order on the backend's stream.  Returns without waiting. */
+ * dispatches in order on the backend's stream.  Returns without waiting, with one exception: a list
+ * that holds the attention of several sequences recorded one by one next to each other is executed as
+ * one launch only if no sequence appends into a page that another attends, which the device has to
+ * have found out before the rest is enqueued. */
 FH_API fh_status fh_submit(fh_backend *backend, const fh_dispatch *dispatches, uint32_t count,
                     fh_submission **out);
 /* fh_submit for callers that cannot allocate.  It has no counterpart in the reference: it exists

@@ -5,6 +5,7 @@ allocation (crates/forja-host/src/lib.rs:4466-4480) and a fresh output row
 activation.  The library executes such a run as one ragged launch; these tests hold the result to
 the CPU oracle's serial execution and to the library's own dispatch-by-dispatch execution."""
 import math
+import time
 
 import numpy as np
 import pytest
@@ -290,8 +291,7 @@ def test_tables_that_share_a_tail_page_run_dispatch_by_dispatch(cpu, hip, case, 
 @pytest.mark.parametrize("idiom", ["append", "copies"])
 def test_a_lane_alone_runs_fused_and_keeps_the_serial_order(cpu, hip, idiom):
     """A step recorded for one sequence is a run of one lane.  Where its table names the page of the
-    new row at an earlier position too, the row is attended at both, as in serial execution: such a
-    step stays dispatch by dispatch."""
+    new row at an earlier position too, the row is attended at both, as in serial execution."""
     for context, aliased in ((0, False), (16, False), (437, False), (437, True)):
         results = []
         for backend in (cpu, hip):
@@ -308,9 +308,44 @@ def test_a_lane_alone_runs_fused_and_keeps_the_serial_order(cpu, hip, idiom):
                 kept += [attended, *rows, *batch.pools[layer]]
             run(backend, commands)
             if backend is hip:
-                assert hip.fusion_stats()[0] - before[0] == (0 if aliased else 2)
+                assert hip.fusion_stats()[0] - before[0] == 2
             results.append(kept)
         check(cpu, hip, results[0], results[1], exact=(2, 3, 6, 7))
+
+
+@pytest.mark.parametrize("idiom", ["append", "copies"])
+@pytest.mark.parametrize("lanes", [1, 2])
+def test_a_submission_of_lanes_alone_returns_before_its_work_is_done(cpu, hip, idiom, lanes):
+    """Sequences whose attention is not next to each other, layer by layer, in one submission: each is a
+    run of one lane, equal to serial execution, and submitting it waits for nothing (there are tens of
+    milliseconds of products in front)."""
+    results = []
+    for backend in (cpu, hip):
+        batch = LaneBatch(backend, [437, 90][:lanes], 8, 4, 16, seed=92, layers=3)
+        before, commands, kept = hip.fusion_stats(), CommandList(), []
+        if backend is hip:
+            x, out = backend.alloc(DType.BF16, (2048, 8192)), backend.alloc(DType.BF16, (2048, 8192))
+            weights = [backend.alloc(DType.U32, (8192, 1024)), *(backend.alloc(DType.BF16, (8192, 128)) for _ in "sb")]
+            for _ in range(100):
+                commands.dispatch(Op.quant_matmul(4, 64), [x, *weights], out)
+        for layer in range(3):
+            for lane in range(lanes):
+                attended, rows = batch.record_layer(commands, layer, idiom=idiom, lanes=[lane])
+                commands.dispatch(Op.copy(), [attended.narrow(0, lane, 1)], backend.alloc(DType.BF16, (1, 8 * WIDTH)))
+                kept += rows
+            kept += batch.pools[layer]
+        start = time.perf_counter()
+        submission = backend.submit(commands)
+        submitted = time.perf_counter() - start
+        submission.wait()
+        if backend is hip:
+            assert hip.fusion_stats()[0] - before[0] == 3 * lanes
+            assert submitted < 0.5 * (time.perf_counter() - start)
+            for tensor in (x, out, *weights):
+                backend.release(tensor)
+        results.append(kept)
+    pools = [i for i in range(len(results[0])) if i % (lanes + 2) >= lanes]
+    check(cpu, hip, *results, exact=pools)
 
 
 def _random_scenario(rng):
