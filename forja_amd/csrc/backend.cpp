@@ -1554,6 +1554,7 @@ bool lane_member_at(const fh_dispatch *d, uint32_t count, uint32_t at, LaneMembe
   }
   if (m->k_new.dtype != m->q.dtype || m->v_new.dtype != m->q.dtype) return false;
   if (!dense_head_rows(m->out) || !is_contiguous(m->table)) return false;
+  if (may_overlap(m->key_pool, m->value_pool)) return false;   // the second copy's row is the one that stays
   if (m->has_activity && element_count(m->activity) != 1) return false;
   if (at + m->dispatches < count && copies_attended_row(m->out, d[at + m->dispatches])) {
     m->has_copy = true;

@@ -313,6 +313,23 @@ def test_a_lane_alone_runs_fused_and_keeps_the_serial_order(cpu, hip, idiom):
         check(cpu, hip, results[0], results[1], exact=(2, 3, 6, 7))
 
 
+@pytest.mark.parametrize("pool_dtype", [DType.BF16, DType.F32])
+@pytest.mark.parametrize("lanes", [1, 2])
+def test_keys_and_values_in_one_pool_run_dispatch_by_dispatch(cpu, hip, lanes, pool_dtype):
+    """Two copies into one pool: the second row replaces the first, and is attended as key and value."""
+    results = []
+    for backend in (cpu, hip):
+        batch = LaneBatch(backend, [437, 90][:lanes], 8, 4, 16, seed=94, pool_dtype=pool_dtype)
+        batch.pools = [(batch.pools[0][0], batch.pools[0][0])]
+        before, commands = hip.fusion_stats(), CommandList()
+        attended, rows = batch.record_layer(commands, 0, idiom="copies")
+        run(backend, commands)
+        if backend is hip:
+            assert hip.fusion_stats()[0] == before[0]
+        results.append([attended, *rows, batch.pools[0][0]])
+    check(cpu, hip, *results, exact=(len(results[0]) - 1,))
+
+
 @pytest.mark.parametrize("idiom", ["append", "copies"])
 @pytest.mark.parametrize("lanes", [1, 2])
 def test_a_submission_of_lanes_alone_returns_before_its_work_is_done(cpu, hip, idiom, lanes):
