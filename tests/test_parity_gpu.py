@@ -285,6 +285,25 @@ def test_quant_matmul_in_row_tiles(cpu, hip, rows, n, k, bits, dtype, padded):
     differential(cpu, hip, build)
 
 
+@pytest.mark.parametrize("rows,n,k,dtype", [(17, 272, 6400, DType.BF16), (64, 400, 3328, DType.BF16),
+                                            (33, 16, 256, DType.BF16), (40, 272, 1280, DType.F32)])
+def test_row_tiles_under_an_epilogue_that_is_not_fused(cpu, hip, rows, n, k, dtype):
+    """The product itself stays f32, of bf16 rows too: added up from several K ranges, and from one."""
+    weights = Quantised(27, 300 + n + k, (n, k))
+    x_values, extra_values = normal_bf16(27, 1, (rows, k)), normal_bf16(27, 2, (rows, n))
+    builder = ProgramBuilder(ProgramKind.MAP)
+    builder.output(0, builder.mul(builder.input(0), builder.input(1)))
+    program = builder.finish()
+
+    def build(backend):
+        out = backend.alloc(dtype, (rows, n))
+        commands = CommandList()
+        commands.dispatch_epilogue(Op.quant_matmul(4, 64), [upload(backend, x_values, dtype), *weights.upload(backend)], out,
+                                   backend.prepare_epilogue(program), [upload(backend, extra_values, dtype)])
+        return commands, [out]
+    differential(cpu, hip, build)
+
+
 @pytest.mark.parametrize("rows,k,experts,n,inner,dtype", [
     (60, 8, 8, 144, 256, DType.BF16),      # 60 routes per expert: a 64-row tile and its remainder
     (130, 2, 5, 272, 512, DType.BF16),     # 52: columns past a block's edge, two quads

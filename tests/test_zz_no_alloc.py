@@ -88,6 +88,20 @@ def test_accumulators_programs_sampling_and_packing_match(hip):
         assert results[0] == results[1]
 
 
+def test_row_tile_products_match_whatever_room_their_partial_sums_have(hip):
+    """64 rows by 151936 columns: one K range's sums are 39 MB, two do not fit the fixed array.  17 by 272: several
+    ranges in either form."""
+    for rows, n, k in ((64, 151936, 1280), (17, 272, 6400)):
+        x, weights = upload(hip, normal_bf16(34, 1, (rows, k)), DType.BF16), Quantised(34, 2, (n, k)).upload(hip)
+        outs = [hip.alloc(DType.BF16, (rows, n)) for _ in range(2)]
+        for out, submit in zip(outs, (lambda c: hip.submit(c).wait(), hip.submit_static)):
+            commands = CommandList()
+            commands.dispatch(Op.quant_matmul(4, 64), [x, *weights], out)
+            submit(commands)
+        expected, got = (hip.read(out) for out in outs)
+        assert np.frombuffer(expected, np.uint16).any() and expected == got
+
+
 def test_enqueue_only_form_and_data_dependent_errors(hip):
     """`error` null: the call only enqueues; a later synchronisation sees the results.  `error`
     given: a stale page is reported as fh_wait reports it, with the same zero row."""
