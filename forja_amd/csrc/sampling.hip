@@ -283,9 +283,6 @@ __device__ inline void scatter_tile(bool valid, uint32_t digit, uint2 element, u
 template <typename WeightAt>
 __device__ inline uint32_t top_p_keep(uint32_t count, float top_p, WeightAt weight_at,
                                       SampleShared &s) {
-  // A NaN of negative sign sorts last; it makes the sum NaN, also where the walk below ends before it.
-  const float last = weight_at(count - 1);
-  if (last != last) return 1;
   const float4 *staged = (const float4 *)s.stage;
   float total = 0.0f;
   for (uint32_t first = 0; first < count; first += kStage) {
@@ -313,7 +310,9 @@ __device__ inline uint32_t top_p_keep(uint32_t count, float top_p, WeightAt weig
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    s.real[0] = total;
+    // (a NaN of negative sign sorts last; it makes the sum NaN, also where the walk has ended before it)
+    const float last = weight_at(count - 1);
+    s.real[0] = last != last ? last : total;
     s.word[0] = 0xffffffffu;
   }
   __syncthreads();
@@ -461,23 +460,21 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a, Er
     // columns left out, and makes the sum NaN if and only if top_k reaches it.  (A positive one is the
     // largest column.)
     uint64_t largest = 0;
-    bool nan_behind = false;
     if (top_p < 1.0f) {
       row.for_each_allowed([&](uint32_t index, float value) {
         const uint64_t mine = candidate(value, index);
         largest = mine > largest ? mine : largest;
-        nan_behind |= __float_as_uint(value) > 0xff800000u;
       });
       largest = block_max(largest, s);
-      nan_behind = __syncthreads_or(nan_behind) != 0;
     }
     const float maximum = top_p < 1.0f ? row.value((uint32_t)(largest - 1)) : 0.0f;
     uint32_t count = 0;
-    for (bool filtered = top_p < 1.0f && is_finite(maximum) && !nan_behind;; filtered = false) {
+    for (bool filtered = top_p < 1.0f && is_finite(maximum);; filtered = false) {
       // Start from descending index so that the stable passes leave equal values in descending
       // index order.
       __syncthreads();
       if (threadIdx.x < 256) s.base[threadIdx.x] = 0;
+      if (threadIdx.x == 0) s.word[3] = 0;
       __syncthreads();
       for (uint32_t first = 0; first < a.width; first += kSampleThreads) {
         const uint32_t at = first + threadIdx.x;
@@ -488,10 +485,14 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a, Er
         if (valid) {
           const float value = row.value(index);
           element.x = ~ordered_key(value);
-          if (filtered && (value - maximum) / temperature < -17.5f) valid = false;   // exp(-17.5) < 2^-25
+          if (filtered && !((value - maximum) / temperature >= -17.5f)) {   // exp(-17.5) < 2^-25
+            valid = false;
+            if (value != value) s.word[3] = 1;
+          }
         }
         scatter_tile(valid, 0, element, sorted, s);
       }
+      if (s.word[3] != 0) continue;
       const uint32_t ordered = s.base[0];
       uint2 *from = sorted, *to = other;
       // (the lower half of a bf16 value's key follows from its sign: two passes order it)
