@@ -583,8 +583,8 @@ __global__ __launch_bounds__(1024) void argmax_rows_kernel(const void *in, uint6
 // ---------------------------------------------------------------- glue
 
 // The same rows of a 4-bit table into dense bf16 or f32 rows, a word's eight values per thread: the
-// general kernel's thread per value spends its time on addresses and index arithmetic (8256 x 5120:
-// 264 us, 42 MB/s of the table and 85 MB written; this one 27).  Same arithmetic, same results.
+// general kernel's thread per value spends its time on addresses and index arithmetic (8256 x 5120, 24 MB
+// read and 85 MB written: 264 us; this one 27).  Same arithmetic, same results.
 __global__ __launch_bounds__(256) void quant_embed_words_kernel(View packed, View scales, View biases, View ids,
                                                                 View out, uint32_t id_count, uint32_t vocab,
                                                                 uint32_t packed_width, uint32_t words_per_group,

@@ -1087,7 +1087,8 @@ namespace {
 constexpr uint32_t kRowsKernelWide = 9;
 
 // f32 activations (the engines' own activation dtype) on the matrix cores: each value goes in as
-// three bf16 or f16 pieces that add up to it, so that f32 accumulation sees all of it.  f32 results.
+// three pieces, of bf16 (K-split kernels: they add up to it) or of f16 (row tiles: they add up to it to 2^-38 of
+// the largest value of its group of 64), so that f32 accumulation sees what it would keep.  f32 results.
 // Decode batches of at most 32 rows through the K-split kernels, more rows and 8-bit weights through
 // the row-tile kernels (fewer than nine rows of what neither takes: the vector-ALU kernel for few rows,
 // 12 us for the 8-bit router of 8 rows).
@@ -1167,11 +1168,13 @@ bool try_fast_quant_matmul(fh_backend *backend, const QmmProblem &p) {
   }
   // More rows, or a longer K, than the K-split kernels hold: row tiles, the weights unpacked once for
   // all rows of a tile.  (48 x 34816 x 5120 66 us against 101 through the streaming kernel, 48 x 5120 x
-  // 17408 34 against 75 through the tile product; 1 row against 34816 x 5120 43 and 64.)  Two shapes are
-  // faster elsewhere: vocabulary-sized matrices at more than 64 rows, which the GEMM's 128-row tiles
-  // read once (128 x 151936 x 2048 127 us against 175), and few rows against so little weight that the
-  // second launch, which adds the K ranges, shows (1 x 5120 x 5120 11.5 us through the tile product
-  // against 13.4, 16 rows 16 against 14).
+  // 17408 33 against 75 through the tile product; 1 row against 34816 x 5120 43 and 64; 128 x 2048 x 4096
+  // with the launch that adds its K ranges 17.6 against 19.0, in the decode step's trace 11.8 + 4.6 against 17.9.)
+  // Two shapes go elsewhere: vocabulary-sized matrices at more than 64 rows, which the GEMM's 128-row tiles
+  // read once (128 x 151936 x 2048 127 us against 175); and at most 8 rows against so little weight that a
+  // launch's fixed costs are most of the time: there the two are close (1 x 5120 x 5120 11.8 us through the
+  // tile product and 11.2 through row tiles, 8 rows 13.4 and 11.7), and one
+  // launch needs no room for partial sums.
   const bool vocabulary = p.rows > 64 && p.columns >= 32768;
   const bool little = p.rows <= 8 && p.inner <= 6144 && (p.columns + 31) / 32 <= backend_compute_units(backend);
   if (p.rows <= 128 && !vocabulary && !little) {

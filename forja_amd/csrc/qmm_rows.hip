@@ -6,19 +6,20 @@
 //   y[m,n] = sum_g scale[n,g] * (sum_{k in g} x[m,k] * (q - c)[n,k]) + (bias + c * scale)[n,g] * sum_{k in g} x[m,k]
 // (affine_quant_dot, crates/forja-cpu/src/lib.rs:1277-1310).  bf16 rows meet 16 + q in bf16 (c = -16);
 // f32 rows, brought into f16's range by a power of two per row and group, go in as three f16 pieces of
-// eleven bits that make up each value, against q - 8 (4 bits) or q - 128 (8 bits) in f16: centred,
+// eleven bits that make up each value (to 2^-38 of the group's largest), against q - 8 (4 bits) or q - 128 (8 bits) in f16: centred,
 // because what 16 + q adds to a group's sum only to be taken off again costs f32 results their last
 // bits.  Error of 512 x 512 x 2048 on f32 N(0,1) rows against 64 bits (2-norm): 1.0e-7, on rows of mean 1
 // 2.7e-7 (the vector-ALU kernels, value by value: 2.9e-7 both; bf16 pieces against 16 + q: 5.2e-7, 2.5e-6).
 //
-// What bounds such a product is neither the weights alone nor the matrix cores but instruction issue
-// (48 x 34816 x 5120: the matrix cores are busy a quarter of the time, and taking out the loads, the
-// staging or the matrix instructions alone each gains a tenth to a quarter): a weight is used for 16 to 64 rows,
-// so its unpacking (8 instructions a word) and its share of activation traffic have to be spread over
-// all of them.  A wave therefore owns 64 weight columns and every row of the tile: the weights go
+// No one unit bounds such a product (48 x 34816 x 5120, counters: while two waves share a SIMD, its vector ALU is
+// busy 0.46 of the cycles and its matrix cores 0.22, and a wave issues for a third of its life, is ready but not
+// issued for half and waits for the rest; taking out the loads, the staging or the matrix instructions
+// alone each gains a tenth to a quarter; and its 544 workgroups are 32 more than have a place at once, which
+// costs little less than half of the 61 us).  A weight is used for 16 to 64 rows, so its unpacking (8
+// instructions a word) and its share of activation traffic have to be spread over all of them.  A wave therefore owns 64 weight columns and every row of the tile: the weights go
 // straight from memory to the wave's registers, 16 rows x 64 bytes per load, a pair of groups ahead of
 // the arithmetic, and are unpacked once; the activations, which the column waves of a workgroup share,
-// are staged through LDS in operand order (one ds_read_b128 per operand, no conflicts on either side),
+// are staged through LDS in operand order (one ds_read_b128 per operand, few bank conflicts),
 // split and summed per group on the way in.  K is divided over WK waves of a workgroup and, where the
 // output has too few tiles for the device, over workgroups whose f32 partial sums a second launch
 // adds in order.
@@ -256,7 +257,8 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
       } else {
         // A power of two takes the largest of the row's group into [2^14, 2^15); then three f16
         // pieces, each the leading eleven bits of what the ones before left, make up every value to
-        // 2^-39 of that largest (pieces are cut off, not rounded, so that the rest is exact).
+        // 2^-38 of that largest: the smallest step of f16 is 2^-24 (pieces are cut off, not rounded, so that
+        // the rest is exact).
         uint32_t largest = 0;
 #pragma unroll
         for (int half = 0; half < 2; ++half)
@@ -670,7 +672,7 @@ bool launch_rows_dense(fh_backend *backend, const RowsDense &d) {
   // K over workgroups where that shortens the launch.  Measured (microseconds, 48 x 5120 x 17408 and
   // 48 x 34816 x 5120 bf16, 512 x 5120 x 2048 f32): a workgroup alone on its compute unit takes
   // `alone` per quad of its longest K wave and 2.4 beyond that, two that share one take `shared` each
-  // (bf16 rows, bound by instruction issue, gain nothing from sharing; f32 rows, which meet at two
+  // (bf16 rows gain nothing from sharing; f32 rows, which meet at two
   // barriers a pair of groups, do).  Splits cost their partial sums and the launch that adds them.
   const uint32_t quads = d.inner / kQuad, waves_k = d.wide ? 1 : 2;
   const uint64_t tiles = (uint64_t)a.row_blocks * a.col_blocks, units_cu = backend_compute_units(backend);

@@ -1,6 +1,7 @@
 // Quantised matmul on the vector ALUs, in f32: the path of everything the matrix-core kernels do
-// not take (f32 or f16 activations, 8-bit weights, groups of 32 or 128, f16 scales) as long as
-// rows are contiguous.  The reference holds f32 products to its f32 tolerance
+// not take (f16 activations, bf16 ones against 8-bit weights, fewer than nine f32 rows against 8-bit weights or
+// a K that the K-split kernels do not hold, groups of 32 or 128, f16 scales, columns that are no multiple
+// of 16) as long as rows are contiguous.  The reference holds f32 products to its f32 tolerance
 // (crates/forja-metal/tests/quant_matmul.rs:108-120), so nothing here is rounded below f32.
 //
 // Arithmetic of affine_quant_dot (crates/forja-cpu/src/lib.rs:1277-1310): the weight is formed

@@ -14,9 +14,11 @@
 //     their own value as score.
 //
 // One workgroup of 1024 threads per row.  Ordering work is only done when the cut needs it: no
-// ordering for "all candidates, top_p = 1"; up to 256 candidates are extracted largest first by
-// repeated block-wide maxima; more than that takes a stable LSD radix sort of (value key, index)
-// pairs in global scratch, after which one lane walks the sums through LDS-staged weights.
+// ordering for "all candidates, top_p = 1"; up to 256 candidates are selected at once (select_largest;
+// where more than 1024 columns tie at their bound, they are extracted largest first by repeated
+// block-wide maxima); more than that takes a stable LSD radix sort of (value key, index) pairs in global
+// scratch, two passes for bf16 rows and four for others, of the columns whose weight can change the
+// nucleus's sums, or of all; after it one lane walks the sums through LDS-staged weights.
 // exp and ln are evaluated in f64 and rounded to f32, i.e. the correctly rounded f32 functions up
 // to double rounding; an f32 libm may differ from that in the last place.
 #include <hip/hip_runtime.h>
