@@ -1585,10 +1585,11 @@ bool same_lane_shape(const LaneMember &a, const LaneMember &b) {
 // per layer 12 us, the two copies 9), and nothing waits for the device, since the one thing that the
 // tables decide (a page named twice) is read there.  Sequences whose layers alternate in one submission are
 // such runs too, each with a gather and a plan of its own (3000 and 900 keys, f32 rows: 34 us a layer and
-// sequence, 39 dispatch by dispatch, 48 when each waited for a verdict).  It is taken only where the member stands alone (`alone`: not
-// behind a member that was not fused; nor before one), because members next to each other that make
-// no run are an order that the caller wants kept.  `run->dispatches` says how many dispatches were
-// examined also when false, so that the caller does not examine the tail of a refused run again.
+// sequence, 39 dispatch by dispatch, 48 when each waited for a verdict).  It is taken only where the
+// member stands alone (`alone`: not behind a member that was not fused; nor before one), because members
+// next to each other that make no run are an order that the caller wants kept.  `run->dispatches` says
+// how many dispatches were examined also when false, so that the caller does not examine the tail of a
+// refused run again.
 bool find_lane_run(const fh_dispatch *d, uint32_t count, uint32_t first, bool alone, LaneRun *run) {
   *run = LaneRun{};
   LaneMember member;

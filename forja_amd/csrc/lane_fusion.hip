@@ -57,9 +57,9 @@ __global__ __launch_bounds__(256) void gather_lane_metadata_kernel(
 // attends, or this lane itself into one that its table names at another position too?  A fused run
 // performs every append before, or while, any lane attends; lane by lane, a reader that comes first
 // sees the slot's old contents, two lanes that append to one slot each see their own value, and a
-// lane whose page appears twice sees its new row at both positions.  The host keeps pages copy-on-write, so this does not happen
-// (crates/forja-host/src/lib.rs:5408-5470); tables are caller data all the same, so it is checked
-// and a run with such an overlap is executed dispatch by dispatch instead.
+// lane whose page appears twice sees its new row at both positions.  The host keeps pages copy-on-write,
+// so this does not happen (crates/forja-host/src/lib.rs:5408-5470); tables are caller data all the same,
+// so it is checked and a run with such an overlap is executed dispatch by dispatch instead.
 // Dynamic LDS: 2 * lanes words (each lane's destination page and slot).
 __global__ __launch_bounds__(256) void lane_conflict_kernel(const uint32_t *tables, const uint32_t *activity,
                                                             const uint32_t *starts, uint32_t lanes,

@@ -266,7 +266,8 @@ typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 constexpr uint32_t kMinSplitTokens = 128, kMaxSplitTokens = 1024;  // split length bounds
-constexpr uint32_t kFillingGroups = 512, kFilledSplitTokens = 512;  // (512 groups: two for each of the 256 compute units) see ragged_plan_kernel
+// see ragged_plan_kernel (512 groups: two for each of the 256 compute units)
+constexpr uint32_t kFillingGroups = 512, kFilledSplitTokens = 512;
 // Groups of several query tokens (prefill) are many and each split of theirs costs a merge of
 // `members x heads` partial rows: they are split only beyond this many keys.
 constexpr uint32_t kPrefillSplitTokens = 2048;
