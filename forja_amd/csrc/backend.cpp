@@ -1407,6 +1407,100 @@ bool find_norm_tail(fh_backend *b, const fh_dispatch &d, const fh_dispatch &next
   return norm_tail_of(program->second.fast, args, produced, tail);
 }
 
+// ---------------------------------------------------------------- what stands around a dense product
+//
+// A dense layer's products have row programs in front of them (the RMS normalisation, with or without
+// the residual sum) and silu(gate) * up behind the stacked gate/up projection.  Over a few rows each is a
+// launch of about 3 us for bytes that the product's own workgroups read and write in passing: the
+// kernel of a product with few rows takes them in.  Same rule as above: every dispatch is the one it is (the list
+// has been validated), the product reads what the normalisation writes element for element, and nothing
+// one of them writes is read or written by another in any other way, since the workgroups of one
+// kernel do it all in no order.
+//
+// Executes the normalisation, product and element program that start at `first` in one launch and
+// returns how many dispatches that were (2 or 3), or returns 0 having done nothing.
+uint32_t run_dense_group(fh_backend *b, const fh_dispatch *d, uint32_t count, uint32_t first) {
+  if (b->static_mode || first + 1 >= count) return 0;
+  auto program_at = [&](uint32_t at, int kind_a, int kind_b) -> Program * {
+    if (at >= count || d[at].op != FH_OP_PROGRAM) return nullptr;
+    auto it = b->programs.find(d[at].program);
+    if (it == b->programs.end()) return nullptr;
+    const int kind = it->second.fast.kind;
+    return kind == kind_a || kind == kind_b ? &it->second : nullptr;
+  };
+  Program *norm = program_at(first, kProgramRmsNorm, kProgramResidualNorm);
+  const uint32_t at = norm ? first + 1 : first;
+  const fh_dispatch &product = d[at];
+  if (product.op != FH_OP_QUANT_MATMUL || product.n_outputs != 1 || product.n_inputs < 4 ||
+      product.inputs[0].dtype != FH_BF16 || product.inputs[0].rank != 2 || product.inputs[0].shape[0] > 32)
+    return 0;
+  const fh_tensor &x = product.inputs[0], &out = product.outputs[0];
+  const bool adds = product.epilogue != 0;
+  if (adds) {
+    auto it = b->programs.find(product.epilogue);
+    if (it == b->programs.end() || !it->second.add_epilogue || product.accumulator_count != 1 ||
+        product.n_extras != 1 || product.n_inputs != 5 || !shape_is(product.inputs[4], {out.shape[0], out.shape[1]}))
+      return 0;
+  }
+  Program *silu = adds ? nullptr : program_at(at + 1, kProgramSiluMul, kProgramSiluMul);
+  if (!norm && !silu) return 0;
+  // binds dispatch `which` as the row program it is
+  auto bind = [&](const fh_dispatch &which, Program &program, ProgramArgs *args) {
+    View in[kMaxProgramInputs], made[kMaxProgramOutputs];
+    if (which.n_inputs > kMaxProgramInputs || which.n_outputs > kMaxProgramOutputs) return false;
+    for (uint32_t i = 0; i < which.n_inputs; ++i)
+      if (make_view(b, which.inputs[i], false, &in[i]) != FH_OK) return false;
+    for (uint32_t i = 0; i < which.n_outputs; ++i)
+      if (make_view(b, which.outputs[i], true, &made[i]) != FH_OK) return false;
+    return bind_program(b, program, which.inputs, which.n_inputs, in, which.outputs, which.n_outputs, made,
+                        which.outputs[0].shape, which.outputs[0].rank, args) == FH_OK;
+  };
+  auto overlaps_any = [](const fh_tensor &written, const fh_tensor *others, uint32_t n) {
+    for (uint32_t i = 0; i < n; ++i)
+      if (may_overlap(written, others[i])) return true;
+    return false;
+  };
+  NormHead head{};
+  if (norm) {
+    const fh_dispatch &n = d[first];
+    const fh_tensor &rows = n.outputs[n.n_outputs - 1];
+    bool same = rows.buffer == x.buffer && rows.offset == x.offset && rows.rank == 2 && rows.dtype == x.dtype;
+    for (uint32_t axis = 0; same && axis < 2; ++axis)
+      same = rows.shape[axis] == x.shape[axis] && rows.stride[axis] == x.stride[axis];
+    bool apart = same && !overlaps_any(out, n.inputs, n.n_inputs) && !overlaps_any(out, n.outputs, n.n_outputs);
+    for (uint32_t o = 0; apart && o < n.n_outputs; ++o)
+      apart = !overlaps_any(n.outputs[o], product.inputs + 1, product.n_inputs - 1);
+    // (the sum is not the tensor the product reads)
+    if (apart && n.n_outputs == 2) apart = !may_overlap(n.outputs[0], x);
+    ProgramArgs args;
+    if (!apart || !bind(n, *norm, &args) || !norm_head_of(norm->fast, args, &head))
+      return 0;   // it runs by itself; the product is looked at again with what follows it
+  }
+  View views[5], made;
+  for (uint32_t i = 0; i < product.n_inputs && i < 5; ++i)
+    if (make_view(b, product.inputs[i], false, &views[i]) != FH_OK) return 0;
+  if (make_view(b, out, true, &made) != FH_OK) return 0;
+  QmmProblem problem{views[0], views[1], views[2], views[3], made, x.shape[0], x.shape[1], out.shape[1],
+                     product.bits, product.group_size};
+  if (adds) problem.residual = &views[4];
+  if (problem.rows == 0 || problem.columns == 0) return 0;
+  View activated;
+  if (silu) {
+    const fh_dispatch &s = d[at + 1];
+    bool apart = s.n_outputs == 1 && !overlaps_any(s.outputs[0], product.inputs, product.n_inputs);
+    if (apart && norm)
+      apart = !overlaps_any(s.outputs[0], d[first].inputs, d[first].n_inputs) &&
+              !overlaps_any(s.outputs[0], d[first].outputs, d[first].n_outputs);
+    ProgramArgs args;
+    if (!apart || !bind(s, *silu, &args) || !silu_of_halves(silu->fast, args, made) ||
+        make_view(b, s.outputs[0], true, &activated) != FH_OK)
+      silu = nullptr;
+  }
+  if (silu && try_fused_quant_matmul(b, problem, norm ? &head : nullptr, &activated)) return norm ? 3 : 2;
+  if (norm && try_fused_quant_matmul(b, problem, &head, nullptr)) return 2;
+  return 0;
+}
+
 // ---------------------------------------------------------------- fusion of per-lane attention
 //
 // The engines record a decode batch lane by lane (engines/qwen3-coder/src/lib.rs:917-935): for
@@ -2775,6 +2869,10 @@ static fh_status submit_locked(fh_backend *b, const fh_dispatch *dispatches, uin
           note_outputs(dispatches[i + member]);
         }
       }
+    } else if (const uint32_t together = op == FH_OP_PROGRAM || op == FH_OP_QUANT_MATMUL
+                                             ? run_dense_group(b, dispatches, count, i) : 0) {
+      consumed = together;
+      for (uint32_t member = 1; member < consumed; ++member) s->ops[i + member] = dispatches[i + member].op;
     } else {
       NormTail tail;
       bool tail_taken = false;

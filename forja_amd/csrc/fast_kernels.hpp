@@ -112,6 +112,15 @@ void backend_prepared_verdict(fh_backend *backend, const PreparedKey &key);
 // 16 or 32 rows) and the output columns are whole batches of the kernel (32 or 64 columns; 16 or
 // 32 per projection of a pair).
 bool ksplit_supports(uint32_t inner, uint32_t columns, bool pair, bool routed);
+// A row-wise RMS normalisation in front of a product, computed by the product's workgroups:
+// normed[r,:] = v * rsqrt(mean(v^2) + eps) * weight, v = x[r,:] (+ update[r,:], and then
+// added[r,:] = v too).  Everything bf16, strides in elements per row, rows in 16-byte pieces.
+struct NormHead {
+  const void *x, *update, *weight;
+  void *added, *normed;
+  uint64_t x_stride, update_stride, added_stride, normed_stride;
+  float eps;
+};
 struct KsplitDense {
   const void *x;            // bf16 rows, or f32 rows with `wide`
   uint64_t x_row_stride;
@@ -127,7 +136,15 @@ struct KsplitDense {
   // Non-zero: `inner` is a range of the K of weight rows `weight_inner` long; x, packed, scales and
   // biases point at the range's first element.
   uint32_t weight_inner;
+  // Null, or the dispatch in front whose rows (x) this product's kernel makes (ksplit_fuses).
+  const NormHead *norm;
+  // Null, or: the matrix has 2 * columns columns, both halves' results go to `out` (row length
+  // 2 * columns or more) and silu(first) * second of the stored results here (ksplit_fuses).
+  uint16_t *activated;
+  uint64_t activated_row_stride;
 };
+// Whether the fused forms of the dense kernel take a product (columns: of one half with `pair`).
+bool ksplit_fuses(uint32_t rows, uint32_t inner, uint32_t columns, bool pair);
 // Whether launch_ksplit_dense takes a product of `rows` rows: at most 128, in row tiles of 16 or
 // 32, and more than one tile only for weights small enough to stay cached between the tiles.
 bool ksplit_dense_supports(uint32_t rows, uint32_t inner, uint32_t columns, bool wide = false);
@@ -273,6 +290,16 @@ bool try_fast_program(hipStream_t stream, const ProgramClass &cls, const Program
 // that norm_rows_kernel would run, reading exactly `produced`; fills `tail` if so.
 bool norm_tail_of(const ProgramClass &cls, const ProgramArgs &args, const View &produced,
                   NormTail *tail);
+// Whether the program is an RMS normalisation (after a residual sum) of bf16 rows that
+// norm_rows_kernel would run; fills `head` if so.
+bool norm_head_of(const ProgramClass &cls, const ProgramArgs &args, NormHead *head);
+// Whether it is silu(in0) * in1 of bf16 rows that map_pair_kernel would run, in0 and in1 the two
+// halves of `produced`'s columns.
+bool silu_of_halves(const ProgramClass &cls, const ProgramArgs &args, const View &produced);
+// A dense product together with what stands around it (either may be null): false, and nothing
+// launched, when the kernels do not take it.  `activated`: the element program's output rows.
+bool try_fused_quant_matmul(fh_backend *backend, const QmmProblem &problem, const NormHead *norm,
+                            const View *activated);
 // combine_routes_rows_kernel followed by that normalisation, one workgroup per row: `out` gets
 // the sums (+ residual), `tail.out` their normalisation.  columns <= 2048, a multiple of 8;
 // routes <= 8; rows of the tail's dtype with 16-byte aligned pieces of 8 elements.

@@ -317,6 +317,46 @@ bool typed_rows(const View &v, uint32_t rank, uint32_t dtype) {
   return v.dtype == dtype && v.rank == rank && v.stride[rank - 1] == 1;
 }
 
+// The operands of norm_rows_kernel, when the program is one it runs.
+bool norm_rows_args(const ProgramClass &cls, const ProgramArgs &p, RowArgs *out, bool *residual_norm, bool *wide_rows) {
+  if ((cls.kind != kProgramRmsNorm && cls.kind != kProgramResidualNorm) || cls.axis + 1 != p.rank) return false;
+  const bool residual = cls.kind == kProgramResidualNorm;
+  if (p.rank != 2 || p.n_inputs != (residual ? 3u : 2u)) return false;
+  const uint32_t n_out = residual ? 2 : 1;
+  const uint32_t dtype = p.inputs[0].dtype;
+  if (dtype != FH_BF16 && dtype != FH_F32) return false;
+  auto ptr = [](const View &v) { return (void *)(v.base + v.offset * dtype_size(v.dtype)); };
+  auto whole_pieces = [](const View &v) { return v.offset % 8 == 0 && v.stride[0] % 8 == 0; };
+  for (uint32_t i = 0; i < p.n_inputs; ++i)
+    if (!typed_rows(p.inputs[i], 2, dtype) || !whole_pieces(p.inputs[i])) return false;
+  for (uint32_t i = 0; i < n_out; ++i)
+    if (!typed_rows(p.outputs[i], 2, dtype) || !whole_pieces(p.outputs[i])) return false;
+  if (p.shape[1] % 8 != 0) return false;
+  RowArgs a{};
+  a.x = ptr(p.inputs[0]);
+  a.x_stride = p.inputs[0].stride[0];
+  const View &w = p.inputs[residual ? 2 : 1];
+  a.weight = ptr(w);
+  a.weight_stride = w.stride[0];
+  if (residual) {
+    a.update = ptr(p.inputs[1]);
+    a.update_stride = p.inputs[1].stride[0];
+  }
+  // out_slot maps pairs to output tensors; pairs are (slot, value) with slot = output index
+  a.out0 = ptr(p.outputs[0]);
+  a.out0_stride = p.outputs[0].stride[0];
+  if (residual) {
+    a.out1 = ptr(p.outputs[1]);
+    a.out1_stride = p.outputs[1].stride[0];
+  }
+  a.width = p.shape[1];
+  a.eps = cls.c[0];
+  *out = a;
+  *residual_norm = residual;
+  *wide_rows = dtype == FH_F32;
+  return true;
+}
+
 }  // namespace
 
 ProgramClass classify_program(uint32_t kind, const fh_inst *insts, uint32_t n_insts,
@@ -429,38 +469,9 @@ bool try_fast_program(hipStream_t stream, const ProgramClass &cls, const Program
   }
   if (cls.axis != rank - 1) return false;
   if (cls.kind == kProgramRmsNorm || cls.kind == kProgramResidualNorm) {
-    const bool residual = cls.kind == kProgramResidualNorm;
-    if (rank != 2 || p.n_inputs != (residual ? 3u : 2u)) return false;
-    const uint32_t n_out = residual ? 2 : 1;
-    const uint32_t dtype = p.inputs[0].dtype;
-    if (dtype != FH_BF16 && dtype != FH_F32) return false;
-    const bool wide = dtype == FH_F32;
-    auto ptr = [](const View &v) { return (void *)(v.base + v.offset * dtype_size(v.dtype)); };
-    for (uint32_t i = 0; i < p.n_inputs; ++i)
-      if (!typed_rows(p.inputs[i], 2, dtype) || !aligned(p.inputs[i])) return false;
-    for (uint32_t i = 0; i < n_out; ++i)
-      if (!typed_rows(p.outputs[i], 2, dtype) || !aligned(p.outputs[i])) return false;
-    const uint32_t width = p.shape[1];
-    if (width % 8 != 0) return false;
     RowArgs a{};
-    a.x = ptr(p.inputs[0]);
-    a.x_stride = p.inputs[0].stride[0];
-    const View &w = p.inputs[residual ? 2 : 1];
-    a.weight = ptr(w);
-    a.weight_stride = w.stride[0];
-    if (residual) {
-      a.update = ptr(p.inputs[1]);
-      a.update_stride = p.inputs[1].stride[0];
-    }
-    // out_slot maps pairs to output tensors; pairs are (slot, value) with slot = output index
-    a.out0 = ptr(p.outputs[0]);
-    a.out0_stride = p.outputs[0].stride[0];
-    if (residual) {
-      a.out1 = ptr(p.outputs[1]);
-      a.out1_stride = p.outputs[1].stride[0];
-    }
-    a.width = width;
-    a.eps = cls.c[0];
+    bool residual = false, wide = false;
+    if (!norm_rows_args(cls, p, &a, &residual, &wide)) return false;
     auto *kernel = residual ? (wide ? norm_rows_kernel<true, true> : norm_rows_kernel<true, false>)
                             : (wide ? norm_rows_kernel<false, true> : norm_rows_kernel<false, false>);
     kernel<<<dim3(p.shape[0]), 256, 0, stream>>>(a);
@@ -513,6 +524,30 @@ bool try_fast_program(hipStream_t stream, const ProgramClass &cls, const Program
     return true;
   }
   return false;
+}
+
+bool norm_head_of(const ProgramClass &cls, const ProgramArgs &p, NormHead *head) {
+  RowArgs a{};
+  bool residual = false, wide = false;
+  if (!norm_rows_args(cls, p, &a, &residual, &wide) || wide || a.weight_stride != 0) return false;
+  *head = NormHead{a.x, a.update, a.weight, residual ? a.out0 : nullptr, residual ? a.out1 : a.out0,
+                   a.x_stride, a.update_stride, a.out0_stride,
+                   residual ? a.out1_stride : a.out0_stride, a.eps};
+  return true;
+}
+
+bool silu_of_halves(const ProgramClass &cls, const ProgramArgs &p, const View &produced) {
+  if (cls.kind != kProgramSiluMul || p.rank != 2 || p.n_inputs != 2 || p.shape[1] % 8 != 0) return false;
+  for (const View *v : {&p.inputs[0], &p.inputs[1], &p.outputs[0]})
+    if (!bf16_rows(*v, 2) || v->offset % 8 || v->stride[0] % 8) return false;
+  if (!bf16_rows(produced, 2) || produced.shape[0] != p.shape[0] || produced.shape[1] != 2 * p.shape[1]) return false;
+  for (int half = 0; half < 2; ++half) {
+    const View &v = p.inputs[half];
+    if (v.base != produced.base || v.offset != produced.offset + (uint64_t)half * p.shape[1] ||
+        v.stride[0] != produced.stride[0])
+      return false;
+  }
+  return true;
 }
 
 bool norm_tail_of(const ProgramClass &cls, const ProgramArgs &p, const View &produced, NormTail *tail) {

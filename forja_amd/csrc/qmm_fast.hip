@@ -1214,6 +1214,37 @@ bool try_fast_quant_matmul(fh_backend *backend, const QmmProblem &p) {
   return true;
 }
 
+bool try_fused_quant_matmul(fh_backend *backend, const QmmProblem &p, const NormHead *norm, const View *activated) {
+  if (p.x.dtype != FH_BF16 || p.out.dtype != FH_BF16) return false;
+  if (!weights_eligible(p.packed, p.scales, p.biases, 2, p.inner, p.bits, p.group)) return false;
+  if (p.x.stride[1] != 1 || p.x.stride[0] % 8 != 0 || p.x.offset % 8 != 0 || p.out.stride[1] != 1) return false;
+  const uint32_t columns = activated ? p.columns / 2 : p.columns;
+  if (!ksplit_fuses(p.rows, p.inner, columns, activated != nullptr)) return false;
+  KsplitDense d{};
+  d.x = u16_ptr(p.x);
+  d.x_row_stride = p.x.stride[0];
+  d.packed = u32_ptr(p.packed);
+  d.scales = u16_ptr(p.scales);
+  d.biases = u16_ptr(p.biases);
+  d.out = (uint16_t *)p.out.base + p.out.offset;
+  d.out_row_stride = p.out.stride[0];
+  d.rows = p.rows;
+  d.inner = p.inner;
+  d.columns = columns;
+  if (p.residual) {
+    const View &r = *p.residual;
+    if (activated || r.dtype != FH_BF16 || r.stride[1] != 1 || r.stride[0] % 4 != 0 || r.offset % 4 != 0) return false;
+    d.residual = u16_ptr(r);
+    d.residual_row_stride = r.stride[0];
+  }
+  d.norm = norm;
+  if (activated) {
+    d.activated = (uint16_t *)activated->base + activated->offset;
+    d.activated_row_stride = activated->stride[0];
+  }
+  return launch_ksplit_dense(backend, d);
+}
+
 namespace {
 
 constexpr uint32_t kRouteTile = 32;

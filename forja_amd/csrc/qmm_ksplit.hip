@@ -60,6 +60,14 @@ struct KsplitArgs {
   const uint32_t *sorted_routes, *blocks, *n_blocks;
   uint32_t route_div;
   uint32_t batches_per_tile;
+  // dense pair: what silu(gate) * up of the two stored results becomes
+  uint16_t *activated;
+  uint64_t activated_row_stride;
+  // kNorm: the rows are made here, x = (x + update) normalised; `added` gets x + update, `normed` the rows
+  const uint16_t *update, *norm_weight;
+  uint16_t *added, *normed;
+  uint64_t update_row_stride, added_row_stride, normed_row_stride;
+  float norm_eps;
 };
 
 // A word the whole wave reads from a table no kernel writes while this one runs (the route plan):
@@ -148,12 +156,22 @@ constexpr int resident_waves(int waves, int row_tiles, int groups, bool routed, 
 // three products with a weight operand (exact 16+q in bf16) add up, in the f32 accumulator, to
 // the product with the f32 value itself.  The stationary rows then take three times the
 // registers: one 16-row tile, one workgroup per compute unit.
-template <int WAVES, int G, int RT, bool kPair, bool kRouted, int XP>
+//
+// kNorm (dense, one row tile): the rows are the RMS normalisation the dispatch in front of the product
+// computes from x (+ update), and every workgroup makes them itself from the sums its waves exchange
+// through LDS, while its first weights are on their way; between them they also store what that
+// dispatch stores.  A normalisation of a few rows is a launch of 3 us whose bytes every workgroup can read from
+// L2 in less.  kPair of a dense product: columns c and c + columns of one gate/up matrix, whose
+// silu(gate) * up, the element program behind it, the epilogue stores beside the two.  Measured, with a
+// layer of one row of 1024 against 4096 and 2 x 3072 columns: normalisation + product 2.9 + 7.4 us in two
+// launches and 6.0 in one, normalisation + product + silu 3.2 + 7.4 + 2.5 and 6.7; 23 rows 3.0 + 8.4
+// and 8.3, 4.4 + 9 + 3.8 and 12.3.
+template <int WAVES, int G, int RT, bool kPair, bool kRouted, int XP, bool kNorm, int CT>
 __global__ __launch_bounds__(64 * WAVES, resident_waves(WAVES, RT, G, kRouted, XP)) void qmm_ksplit_kernel(KsplitArgs a) {
   static_assert(XP == 1 || (XP == 3 && RT == 1), "f32 rows: one row tile");
+  static_assert(!kNorm || (XP == 1 && !kRouted), "normalised rows: bf16, dense");
   constexpr int P = kPair ? 2 : 1;
   constexpr int NS = ring_slots(RT, G, kRouted);
-  constexpr int CT = batch_tiles(kPair, G);
   constexpr int kBatchCols = 16 * CT;
   constexpr int Q = (G + 3) / 4;             // f32 matrix steps of the bias term (4 groups each)
   constexpr int W2 = G / 2;                  // words of a lane's scales (or biases) of a column
@@ -177,8 +195,9 @@ __global__ __launch_bounds__(64 * WAVES, resident_waves(WAVES, RT, G, kRouted, X
   constexpr bool kStage = RT == 1;
   constexpr int kSub = P * CT * 2;
   constexpr int kPieces = kSub * 16 * WAVES;          // 2G-byte pieces of a batch (one per column and wave)
-  constexpr int PT = kPieces / (64 * WAVES);          // pieces a thread fetches per batch (1 or 2)
-  static_assert(PT * 64 * WAVES == kPieces, "whole pieces per thread");
+  constexpr int PT = (kPieces + 64 * WAVES - 1) / (64 * WAVES);   // pieces a thread fetches per batch (1 or 2)
+  constexpr bool kSomeIdle = kPieces < 64 * WAVES;    // one 16-column tile: half of the threads fetch nothing they pass on
+  static_assert(kSomeIdle || PT * 64 * WAVES == kPieces, "whole pieces per thread");
   extern __shared__ __attribute__((aligned(16))) float exchange[];   // f32x4 [2][WAVES][kSlots][64]
   uint32_t *scale_lds = (uint32_t *)(exchange + 2 * WAVES * kSlots * 4 * 64);   // [2][kPieces][W2]
   const uint32_t lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
@@ -200,6 +219,124 @@ __global__ __launch_bounds__(64 * WAVES, resident_waves(WAVES, RT, G, kRouted, X
   uint32_t out_rows[RT][4]; // output row of accumulator (row tile, i): tile row 16 rt + 4 g + i
   uint32_t tile_first = 0, tile_count = 0, current_tile = kNoBlock;
   const uint32_t g_perm = 2 * (g & 1) + (g >> 1);
+  auto keep_sums = [&](int rt, const float (&sums)[G]) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      float mine = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (4 * q + i < G && g == (uint32_t)i) mine = sums[4 * q + i];
+      xs[rt][q] = mine;
+    }
+  };
+  // kNorm: the rows' pieces as they lie in memory (requested before the first weights), and what
+  // becomes of them.
+  uint4 raw_x[kNorm ? RT : 1][kNorm ? G : 1][2], raw_u[kNorm ? RT : 1][kNorm ? G : 1][2], raw_w[kNorm ? G : 1][2];
+  auto request_rows = [&] {
+    if constexpr (kNorm) {
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        const uint32_t row = min((uint32_t)(16 * rt) + n, a.rows - 1);
+        const uint32_t at = wave * (G * kGroup) + 16 * g_perm;
+        const uint16_t *xp = (const uint16_t *)a.x + (uint64_t)row * a.x_row_stride + at;
+#pragma unroll
+        for (int j = 0; j < G; ++j)
+#pragma unroll
+          for (int half = 0; half < 2; ++half) raw_x[rt][j][half] = *(const uint4 *)(xp + kGroup * j + 8 * half);
+        if (a.update) {
+          const uint16_t *up = a.update + (uint64_t)row * a.update_row_stride + at;
+#pragma unroll
+          for (int j = 0; j < G; ++j)
+#pragma unroll
+            for (int half = 0; half < 2; ++half) raw_u[rt][j][half] = *(const uint4 *)(up + kGroup * j + 8 * half);
+        } else {   // x + -0 is x, whatever x is
+#pragma unroll
+          for (int j = 0; j < G; ++j)
+#pragma unroll
+            for (int half = 0; half < 2; ++half) raw_u[rt][j][half] = make_uint4(0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < G; ++j)
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+          raw_w[j][half] = *(const uint4 *)(a.norm_weight + wave * (G * kGroup) + 16 * g_perm + kGroup * j + 8 * half);
+    }
+  };
+  auto normalise_rows = [&] {
+    if constexpr (kNorm) {
+      auto value_of = [&](int rt, int j, int half, int i) -> float {
+        const uint4 xv = raw_x[rt][j][half], uv = raw_u[rt][j][half];
+        const uint32_t xw = i / 2 == 0 ? xv.x : i / 2 == 1 ? xv.y : i / 2 == 2 ? xv.z : xv.w;
+        const uint32_t uw = i / 2 == 0 ? uv.x : i / 2 == 1 ? uv.y : i / 2 == 2 ? uv.z : uv.w;
+        return __uint_as_float(i & 1 ? xw & 0xffff0000u : xw << 16) + __uint_as_float(i & 1 ? uw & 0xffff0000u : uw << 16);
+      };
+      // the waves' partial sums of squares meet in the half of the exchange buffer that is not
+      // written before the first batch's barrier has been passed
+      float *squares = exchange + WAVES * kSlots * 4 * 64;
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int j = 0; j < G; ++j)
+#pragma unroll
+          for (int half = 0; half < 2; ++half)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              const float v = value_of(rt, j, half, i);
+              sum += v * v;
+            }
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+        if (g == 0) squares[wave * (16 * RT) + 16 * rt + n] = sum;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) sum += squares[w * (16 * RT) + 16 * rt + n];
+        const float inverse = 1.0f / sqrtf(sum / (float)a.inner + a.norm_eps);
+        const uint32_t row = 16 * rt + n;
+        const uint32_t at = wave * (G * kGroup) + 16 * g_perm;
+        float sums[G];
+#pragma unroll
+        for (int j = 0; j < G; ++j) {
+          float s = 0.0f;
+#pragma unroll
+          for (int half = 0; half < 2; ++half) {
+            const uint4 w = raw_w[j][half];
+            const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
+            uint32_t rows[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              rows[i] = pack_bf16_pair(value_of(rt, j, half, 2 * i) * inverse * __uint_as_float(ww[i] << 16),
+                                       value_of(rt, j, half, 2 * i + 1) * inverse * __uint_as_float(ww[i] & 0xffff0000u));
+            const uint4 normed = make_uint4(rows[0], rows[1], rows[2], rows[3]);
+            // (the pieces of what the normalisation stores are dealt out over the workgroups)
+            const uint32_t storing = (uint32_t)((rt * G + j) * 2 + half) % gridDim.x;
+            if (blockIdx.x == storing && row < a.rows) {
+              *(uint4 *)(a.normed + (uint64_t)row * a.normed_row_stride + at + kGroup * j + 8 * half) = normed;
+              if (a.update) {
+                uint32_t whole[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                  whole[i] = pack_bf16_pair(value_of(rt, j, half, 2 * i), value_of(rt, j, half, 2 * i + 1));
+                *(uint4 *)(a.added + (uint64_t)row * a.added_row_stride + at + kGroup * j + 8 * half) =
+                    make_uint4(whole[0], whole[1], whole[2], whole[3]);
+              }
+            }
+            s += sum8(normed);
+            xa[0][rt][j][half] = permute_slots(normed);
+          }
+          s += __shfl_xor(s, 16, 64);
+          s += __shfl_xor(s, 32, 64);
+          sums[j] = s;
+        }
+        keep_sums(rt, sums);
+      }
+    }
+  };
   auto load_tile = [&](uint32_t tile) {
     current_tile = tile;
     if (kRouted) {
@@ -221,6 +358,7 @@ __global__ __launch_bounds__(64 * WAVES, resident_waves(WAVES, RT, G, kRouted, X
         const uint32_t at = tile_first + (row < tile_count ? row : 0);
         out_rows[rt][i] = kRouted ? a.sorted_routes[at] : at;
       }
+    if constexpr (kNorm) return;   // one tile, made before the loop
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       const uint32_t row = 16 * rt + n;
@@ -272,14 +410,7 @@ __global__ __launch_bounds__(64 * WAVES, resident_waves(WAVES, RT, G, kRouted, X
         s += __shfl_xor(s, 32, 64);
         sums[j] = s;
       }
-#pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        float mine = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (4 * q + i < G && g == (uint32_t)i) mine = sums[4 * q + i];
-        xs[rt][q] = mine;
-      }
+      keep_sums(rt, sums);
       __builtin_amdgcn_sched_barrier(0);   // one row tile's loads in flight at a time (registers)
     }
     // The row ids are used when a batch ends; claim them here, so that the wait for them stands in
@@ -353,6 +484,7 @@ __global__ __launch_bounds__(64 * WAVES, resident_waves(WAVES, RT, G, kRouted, X
   };
   auto write_share = [&](const Share &r, uint32_t half) {
     if constexpr (!kStage) return;
+    if (kSomeIdle && threadIdx.x >= (uint32_t)kPieces) return;
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
       uint32_t *to = scale_lds + ((uint64_t)half * kPieces + threadIdx.x + i * (64 * WAVES)) * W2;
@@ -492,6 +624,16 @@ __global__ __launch_bounds__(64 * WAVES, resident_waves(WAVES, RT, G, kRouted, X
         acc[P * CT - 1][rt][i] = __builtin_fmaf(late_scale, late[rt][i], acc[P * CT - 1][rt][i]);
     // One result: activation of a pair, residual of a dense product, rounding, store.
     auto store_result = [&](float value, float up, uint32_t out_row, uint32_t column, uint32_t residual_bits) {
+      if (kPair && !kRouted) {   // both results are stored, and the element program reads what was stored
+        const uint32_t both = pack_bf16_pair(value, up);
+        uint16_t *row = (uint16_t *)a.out + (uint64_t)out_row * a.out_row_stride + column;
+        row[0] = (uint16_t)(both & 0xffffu);
+        row[a.columns] = (uint16_t)(both >> 16);
+        const float gate = __uint_as_float(both << 16);
+        const float product = gate * (1.0f / (1.0f + expf(-gate))) * __uint_as_float(both & 0xffff0000u);
+        a.activated[(uint64_t)out_row * a.activated_row_stride + column] = (uint16_t)(pack_bf16_pair(product, 0.0f) & 0xffffu);
+        return;
+      }
       if (kPair) value = value * (1.0f / (1.0f + __expf(-value))) * up;
       if (!kRouted && a.residual) value += XP == 1 ? bf16_bits(residual_bits & 0xffffu) : __uint_as_float(residual_bits);
       const uint64_t at = (uint64_t)out_row * a.out_row_stride + column;
@@ -574,6 +716,7 @@ __global__ __launch_bounds__(64 * WAVES, resident_waves(WAVES, RT, G, kRouted, X
   };
 
   if (first_unit >= last_unit) return;
+  request_rows();
   Cursor loading{first_unit, first_unit / a.batches_per_tile, first_unit % a.batches_per_tile, 0};
   loading.expert = expert_of(loading.tile);
   Cursor computing = loading, sharing = loading;
@@ -594,7 +737,12 @@ __global__ __launch_bounds__(64 * WAVES, resident_waves(WAVES, RT, G, kRouted, X
     advance(loading);
   }
   write_share(first_share, 0);
-  if (kStage) __syncthreads();   // the first unit's scales are in LDS
+  if constexpr (kNorm) {
+    load_tile(0);
+    normalise_rows();   // (its barrier covers the first unit's scales)
+  } else if (kStage) {
+    __syncthreads();   // the first unit's scales are in LDS
+  }
   // Whole rounds of the ring first, in a loop without exits in its body (an exit that rejoins the
   // loop would make every wait assume the shortest path, i.e. drain the ring); the last, partial
   // round is a copy of the body that requests nothing.  Unit number i of this workgroup uses ring
@@ -603,7 +751,7 @@ __global__ __launch_bounds__(64 * WAVES, resident_waves(WAVES, RT, G, kRouted, X
   for (; base + NS <= last_unit; base += NS) {
 #pragma unroll
     for (int slot = 0; slot < NS; ++slot) {
-      if (computing.tile != current_tile) load_tile(computing.tile);
+      if (!kNorm && computing.tile != current_tile) load_tile(computing.tile);
       finish_batch(ring[slot], shares[(slot + 1) % NS], computing.batch, buf);
       buf ^= 1u;
       load_share(shares[(slot + 3) % NS], sharing);
@@ -616,7 +764,7 @@ __global__ __launch_bounds__(64 * WAVES, resident_waves(WAVES, RT, G, kRouted, X
 #pragma unroll
   for (int slot = 0; slot < NS - 1; ++slot) {
     if (base + slot >= last_unit) break;
-    if (computing.tile != current_tile) load_tile(computing.tile);
+    if (!kNorm && computing.tile != current_tile) load_tile(computing.tile);
     finish_batch(ring[slot], shares[(slot + 1) % NS], computing.batch, buf);
     buf ^= 1u;
     advance(computing);
@@ -639,12 +787,26 @@ bool ksplit_shape(uint32_t inner, int *waves, int *groups) {
 
 // One launch: as many workgroups as stay resident at once (the runtime's own occupancy figure for
 // this instantiation), never more than there are units of work.
-template <int WAVES, int G, int RT, bool kPair, bool kRouted, int XP>
+template <int WAVES, int G, int RT, bool kPair, bool kRouted, int XP, bool kNorm, int CT = batch_tiles(kPair, G)>
 void launch_one(fh_backend *backend, const KsplitArgs &a, uint64_t most_units) {
-  constexpr int P = kPair ? 2 : 1, CT = batch_tiles(kPair, G);
+  constexpr int P = kPair ? 2 : 1;
+  // Dense products of few columns: batches of one column tile where wide ones would leave compute
+  // units without a workgroup.  Such a launch is one chain of latencies per workgroup, and a narrow batch's is
+  // shorter (1 row: 1024 -> 4096 8.6 us wide and 6.2 narrow, 2048 -> 1024 6.7 and 5.6, 3072 -> 1024 7.7 and
+  // 6.2; 23 rows 1024 -> 4096 16.3 and 10.7).  Beyond two workgroups a compute unit the wide batches' longer
+  // streams win (their fixed costs, and in the 16-row form the coalesced scales, are shared by more columns).
+  if constexpr (!kRouted && CT > 1) {
+    const uint64_t narrow = most_units * CT;
+    if (most_units < backend_compute_units(backend) && narrow <= 2 * backend_compute_units(backend)) {
+      KsplitArgs n = a;
+      n.batches_per_tile = a.batches_per_tile * CT;
+      launch_one<WAVES, G, RT, kPair, kRouted, XP, kNorm, 1>(backend, n, narrow);
+      return;
+    }
+  }
   constexpr uint32_t lds = 2u * WAVES * (CT * P * RT * 4) * 64 * sizeof(float) +   // partial sums
                            (RT == 1 ? 2u * (P * CT * 2 * 16 * WAVES) * (G / 2) * sizeof(uint32_t) : 0u);   // scales and biases
-  const void *kernel = reinterpret_cast<const void *>(&qmm_ksplit_kernel<WAVES, G, RT, kPair, kRouted, XP>);
+  const void *kernel = reinterpret_cast<const void *>(&qmm_ksplit_kernel<WAVES, G, RT, kPair, kRouted, XP, kNorm, CT>);
   static int per_unit = 0;   // set once per process: the dynamic LDS limit and the occupancy
   if (per_unit == 0) {
     (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -655,28 +817,28 @@ void launch_one(fh_backend *backend, const KsplitArgs &a, uint64_t most_units) {
   }
   const uint64_t resident = (uint64_t)backend_compute_units(backend) * (uint32_t)per_unit;
   const uint32_t grid = (uint32_t)(most_units < resident ? most_units : resident);
-  qmm_ksplit_kernel<WAVES, G, RT, kPair, kRouted, XP><<<dim3(grid), 64 * WAVES, lds, backend_stream(backend)>>>(a);
+  qmm_ksplit_kernel<WAVES, G, RT, kPair, kRouted, XP, kNorm, CT><<<dim3(grid), 64 * WAVES, lds, backend_stream(backend)>>>(a);
 }
 
-template <int RT, bool kPair, bool kRouted, int XP>
+template <int RT, bool kPair, bool kRouted, int XP, bool kNorm = false>
 bool launch_shape(fh_backend *backend, const KsplitArgs &a, uint64_t most_units) {
   int waves = 0, groups = 0;
   if (!ksplit_shape(a.inner, &waves, &groups)) return false;
   switch (waves * 16 + groups) {
-  case 4 * 16 + 2: launch_one<4, 2, RT, kPair, kRouted, XP>(backend, a, most_units); return true;
-  case 6 * 16 + 2: launch_one<6, 2, RT, kPair, kRouted, XP>(backend, a, most_units); return true;
-  case 8 * 16 + 2: launch_one<8, 2, RT, kPair, kRouted, XP>(backend, a, most_units); return true;
-  case 6 * 16 + 4: launch_one<6, 4, RT, kPair, kRouted, XP>(backend, a, most_units); return true;
-  case 8 * 16 + 4: launch_one<8, 4, RT, kPair, kRouted, XP>(backend, a, most_units); return true;
+  case 4 * 16 + 2: launch_one<4, 2, RT, kPair, kRouted, XP, kNorm>(backend, a, most_units); return true;
+  case 6 * 16 + 2: launch_one<6, 2, RT, kPair, kRouted, XP, kNorm>(backend, a, most_units); return true;
+  case 8 * 16 + 2: launch_one<8, 2, RT, kPair, kRouted, XP, kNorm>(backend, a, most_units); return true;
+  case 6 * 16 + 4: launch_one<6, 4, RT, kPair, kRouted, XP, kNorm>(backend, a, most_units); return true;
+  case 8 * 16 + 4: launch_one<8, 4, RT, kPair, kRouted, XP, kNorm>(backend, a, most_units); return true;
   default: break;
   }
-  if constexpr (RT == 1 && !kRouted && XP == 1) {   // the long rows of dense decode products
+  if constexpr (!kRouted && XP == 1 && !kPair && !kNorm) {   // the long rows of dense decode products
     if (waves == 8 && groups == 6) {
-      launch_one<8, 6, 1, false, false, 1>(backend, a, most_units);
+      launch_one<8, 6, RT, false, false, 1, false>(backend, a, most_units);
       return true;
     }
-    if (waves == 8 && groups == 8) {
-      launch_one<8, 8, 1, false, false, 1>(backend, a, most_units);
+    if (RT == 1 && waves == 8 && groups == 8) {
+      launch_one<8, 8, 1, false, false, 1, false>(backend, a, most_units);
       return true;
     }
   }
@@ -702,16 +864,29 @@ bool ksplit_dense_supports(uint32_t rows, uint32_t inner, uint32_t columns, bool
   if (!ksplit_supports(inner, columns, false, false)) return false;
   // f32 rows: 16-row tiles of K slices of at most four groups, two passes at most
   if (wide) return groups <= 4 && rows <= 32 && (rows <= 16 || (uint64_t)columns * inner / 2 <= kCachedWeightBytes);
-  const uint32_t tile_rows = rows > 16 && groups <= 4 ? 32 : 16;
+  // (a K slice of six groups holds 32 rows too, in one pass, 23 x 1024 x 3072 9.3 us against 6.7 + 3.7 through
+  // row tiles and the launch that adds their ranges; one of eight does not fit the registers)
+  const uint32_t tile_rows = rows > 16 && (groups <= 4 || (groups == 6 && rows <= 32)) ? 32 : 16;
   // (row tiles of 16, which the long K slices are held to, would take eight passes for 128 rows)
   return rows <= tile_rows || (groups <= 4 && (uint64_t)columns * inner / 2 <= kCachedWeightBytes);
+}
+
+// The fused forms hold their rows in one tile of a K slice of at most four groups.
+bool ksplit_fuses(uint32_t rows, uint32_t inner, uint32_t columns, bool pair) {
+  int waves = 0, groups = 0;
+  if (rows == 0 || rows > 32 || !ksplit_shape(inner, &waves, &groups) || groups > 4) return false;
+  return ksplit_supports(inner, columns, pair, false);
 }
 
 bool launch_ksplit_dense(fh_backend *backend, const KsplitDense &d) {
   int waves = 0, groups = 0;
   if (!ksplit_dense_supports(d.rows, d.inner, d.columns, d.wide) || !ksplit_shape(d.inner, &waves, &groups)) return false;
   if (d.wide && !d.out_f32) return false;
-  const bool wide_tiles = d.rows > 16 && groups <= 4 && !d.wide;
+  if ((d.norm || d.activated) &&
+      (d.wide || d.weight_inner || (d.activated && (d.residual || d.out_f32)) ||
+       !ksplit_fuses(d.rows, d.inner, d.columns, d.activated != nullptr)))
+    return false;
+  const bool wide_tiles = d.rows > 16 && groups <= 6 && !d.wide;
   KsplitArgs a{};
   a.x = d.x;
   a.x_row_stride = d.x_row_stride;
@@ -733,6 +908,36 @@ bool launch_ksplit_dense(fh_backend *backend, const KsplitDense &d) {
   const uint64_t units = (uint64_t)((d.rows + tile_rows - 1) / tile_rows) * a.batches_per_tile;
   KernelTimer timer(backend, FH_KC_QMM_KERNEL);
   if (d.wide) return launch_shape<1, false, false, 3>(backend, a, units);
+  if (d.norm || d.activated) {
+    if (d.norm) {
+      a.x = d.norm->x;
+      a.x_row_stride = d.norm->x_stride;
+      a.update = (const uint16_t *)d.norm->update;
+      a.update_row_stride = d.norm->update_stride;
+      a.norm_weight = (const uint16_t *)d.norm->weight;
+      a.added = (uint16_t *)d.norm->added;
+      a.added_row_stride = d.norm->added_stride;
+      a.normed = (uint16_t *)d.norm->normed;
+      a.normed_row_stride = d.norm->normed_stride;
+      a.norm_eps = d.norm->eps;
+    }
+    if (d.activated) {
+      a.packed[1] = a.packed[0] + (uint64_t)d.columns * (d.inner / 8);
+      a.scales[1] = a.scales[0] + (uint64_t)d.columns * (d.inner / kGroup);
+      a.biases[1] = a.biases[0] + (uint64_t)d.columns * (d.inner / kGroup);
+      a.activated = d.activated;
+      a.activated_row_stride = d.activated_row_stride;
+      const uint32_t pair_cols = 16 * batch_tiles(true, groups);
+      a.batches_per_tile = d.columns / pair_cols;
+      if (d.norm)
+        return wide_tiles ? launch_shape<2, true, false, 1, true>(backend, a, a.batches_per_tile)
+                          : launch_shape<1, true, false, 1, true>(backend, a, a.batches_per_tile);
+      return wide_tiles ? launch_shape<2, true, false, 1>(backend, a, a.batches_per_tile)
+                        : launch_shape<1, true, false, 1>(backend, a, a.batches_per_tile);
+    }
+    return wide_tiles ? launch_shape<2, false, false, 1, true>(backend, a, units)
+                      : launch_shape<1, false, false, 1, true>(backend, a, units);
+  }
   return wide_tiles ? launch_shape<2, false, false, 1>(backend, a, units)
                     : launch_shape<1, false, false, 1>(backend, a, units);
 }

@@ -799,6 +799,56 @@ def test_weighted_sum_followed_by_the_normalisation_of_its_rows(cpu, hip, rows, 
     differential(cpu, hip, build, **({"rel": 3e-2} if form == "weights_in_the_sum" else {}))
 
 
+@pytest.mark.parametrize("rows,n,k", [(1, 1024, 1024), (8, 96, 512), (16, 64, 768), (17, 160, 1536), (32, 256, 2048),
+                                      (5, 32768, 1024), (33, 64, 1024), (3, 72, 1024), (4, 128, 3072)])
+@pytest.mark.parametrize("form", ["norm", "residual_norm", "residual_norm_silu", "silu", "norm_add",
+                                  "sum_added", "over_the_rows", "other_rows", "other_halves"])
+def test_dense_products_with_the_row_programs_around_them(cpu, hip, rows, n, k, form):
+    """A normalisation, the product of its rows and silu of the product's halves, next to each other:
+    the backend may run them as one kernel (up to 32 rows; the last three sizes are beyond what it takes) and the
+    results must be those of the dispatches one by one, also where they are not to be joined: a product
+    that adds the sum the normalisation has just written, one stored over the rows that are normalised,
+    one that reads other rows, halves taken the other way round."""
+    weights = Quantised(35, 1, (n, k))
+    x_values, u_values = normal_bf16(35, 10, (rows, k)), normal_bf16(35, 11, (rows, k))
+    norm_values = 0.02 + 0.002 * normal_bf16(35, 12, (k,))
+
+    def build(backend):
+        x, u = upload(backend, x_values, DType.BF16), upload(backend, u_values, DType.BF16)
+        norm_weight = upload(backend, norm_values, DType.BF16).broadcast((rows, k))
+        added, normed = (backend.alloc(DType.BF16, (rows, k)) for _ in range(2))
+        out, activated = backend.alloc(DType.BF16, (rows, n)), backend.alloc(DType.BF16, (rows, n // 2))
+        commands = CommandList()
+        outputs = [normed, out]
+        if form != "silu":
+            if "residual" in form or form == "sum_added":
+                commands.dispatch_kernel(backend.prepare_program(programs.residual_norm_rows(1e-6)), [x, u, norm_weight],
+                                         [added, normed])
+                outputs.append(added)
+            else:
+                commands.dispatch_kernel(backend.prepare_program(programs.rms_norm_rows(1e-6)), [x, norm_weight], [normed])
+        product = [u if form == "other_rows" else x if form == "silu" else normed, *weights.upload(backend)]
+        if form in ("norm_add", "sum_added"):   # something as wide as the result is added to it
+            extra = upload(backend, normal_bf16(35, 13, (rows, n)), DType.BF16)
+            if form == "sum_added" and n <= k:
+                extra = added.narrow(1, 0, n)
+            commands.dispatch_epilogue(Op.quant_matmul(4, 64), product, out,
+                                       backend.prepare_epilogue(programs.add_elements()), [extra])
+        elif form == "over_the_rows" and n <= k:
+            commands.dispatch(Op.quant_matmul(4, 64), product, x.narrow(1, 0, n))
+            outputs[1] = x
+        else:
+            commands.dispatch(Op.quant_matmul(4, 64), product, out)
+        if form in ("residual_norm_silu", "silu", "other_halves"):
+            halves = [out.narrow(1, 0, n // 2), out.narrow(1, n // 2, n // 2)]
+            commands.dispatch_kernel(backend.prepare_program(programs.silu_mul_elements()),
+                                     halves[::-1] if form == "other_halves" else halves, [activated])
+            outputs.append(activated)
+        return commands, outputs if form != "silu" else outputs[1:]
+    # silu of halves multiplies two results of one ulp each
+    differential(cpu, hip, build, rel=2e-2, abs_=2e-2)
+
+
 @pytest.mark.parametrize("with_residual", [False, True])
 def test_f32_weighted_sum_followed_by_the_normalisation_of_its_rows(cpu, hip, with_residual):
     """The same pair in the engine's dtypes: an 8-row decode batch, everything f32."""
