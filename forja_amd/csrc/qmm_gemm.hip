@@ -274,7 +274,7 @@ __device__ inline void store_tile(const GemmArgs &a, f32x16 (&acc)[kQM / 32][kQN
     float *unscale_of = (float *)(mine + kQM * kOutPitch);   // the quadrant's row factors
     const uint32_t quad_row0 = row0 + kQM * wm, quad_col0 = col0 + kQN * wn;
     const uint32_t piece_row = lane / kPieces, piece_col = 8 * (lane % kPieces);
-    unscale_of[lane] = a.row_unscale[min(quad_row0 + lane, a.rows - 1)];
+    if (kQM >= 64 || lane < kQM) unscale_of[lane] = a.row_unscale[min(quad_row0 + lane, a.rows - 1)];
     if (kQM > 64) unscale_of[64 + lane] = a.row_unscale[min(quad_row0 + 64 + lane, a.rows - 1)];
     if (a.residual) {
 #pragma unroll 4
@@ -923,6 +923,305 @@ __global__ __launch_bounds__(64 * kWM * kWN) void gemm_q4_kernel(GemmArgs a) {
   store_tile<kQM, kQN, kWN>(a, acc, gemm_lds, row0, col0);
 }
 
+// load_to_lds_16 with the address as a wave-uniform base and a 32-bit offset per lane, and LDS by its offset (a
+// pointer's costs five scalar instructions to make one of).
+__device__ inline void load_to_lds_16_at(const void *base, uint32_t offset, uint32_t lds_offset) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_offset) : "memory");
+}
+
+// The same product for outputs of few tiles: eight waves of 64 rows x 64 columns, kWM x kWN of them beside each other
+// and kWK along K, so that a compute unit has two waves per SIMD although its tile is small (2 x 2 x 2: 128 x 128;
+// 2 x 1 x 4: 128 x 64).  Four waves of 64 x 64, one per SIMD, take 2000 cycles a K step of 64 whatever is loaded
+// when (rings of two to five steps measured the same): half of them issuing, in order, 280 instructions that no
+// other wave's overlap, the other half at waits and the barrier.  In a period every wave takes one of the kWK
+// next steps, all of them behind one barrier.  2048 rows x 1024 columns: K 2048 41 -> 29 us, K 3072 54 -> 35, with the rows' preparation
+// (8 and 10 us of it).  What is left of a launch: 8 us before and after the periods, 1.4 us a period of 256 K values,
+// of which the matrix instructions take 0.5 and the loads (72 KB a compute unit) most of the rest.
+//   * Activations and packed words of kSlots periods and scales of two blocks of eight groups in LDS, loaded by
+//     hand (load_to_lds_16_at) in whole lines: a wave that reads its columns' operands from memory itself
+//     touches a line per lane, and doing so for the columns after the inner values alone took 3 us.
+//   * A wave's operands are read two sub-steps ahead of their use: the barrier that says that the next period has
+//     landed stands in the middle of a period, and behind it the period's own slot, of which everything is in
+//     registers, is requested anew.
+//   * At the end the K parts' sums meet in LDS and are added in K order, each part finishing its share of the
+//     blocks.
+template <int kWM, int kWN, int kWK, int kSlots>
+__global__ __launch_bounds__(512, 2) void gemm_q4_split_kernel(GemmArgs a) {
+  const uint32_t refused = a.refused[0];   // looked at before the stores: the loads need not wait for it
+  static_assert(kWM * kWN * kWK == 8 && kSlots >= 2, "eight waves");
+  constexpr int kQ = 64, kMI = 2, kSub = 4;
+  constexpr int kSideM = kQ * kWM, kSideN = kQ * kWN;
+  constexpr int kStepBytes = kSideM * 128;                 // the activations of one step
+  constexpr int kTileBytes = kWK * kStepBytes;             // ... of a period
+  constexpr int kWordRow = 32 * kWK;                       // the packed words of a column and period
+  constexpr int kWordBytes = kSideN * kWordRow;
+  constexpr int kSlotBytes = kTileBytes + kWordBytes;
+  constexpr int kLoads = kTileBytes / 8192, kWordLoads = kWordBytes / 8192;   // instructions per wave and period
+  constexpr int kPieces = kWordRow / 16;                   // 16-byte pieces of a column's words
+  constexpr int kBlockPeriods = 8 / kWK;                   // periods of a block of eight groups
+  extern __shared__ __attribute__((aligned(16))) unsigned char gemm_lds[];   // [kSlots]{[kWK][kSideM][128], [kSideN][kWordRow]}
+  unsigned char *scale_rows = gemm_lds + kSlots * kSlotBytes;                // [2][kSideN][16]
+  const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)gemm_lds;
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // (so numbered that the parts the waves finish at the end lie row by row, see store_tile)
+  const uint32_t wn = kWN == 1 ? 0 : wave % kWN, wk = wave / kWN % kWK, wm = wave / (kWN * kWK);
+  const uint32_t l32 = lane & 31, kh = lane >> 5;
+  auto swizzle_of = [](uint32_t row) { return (row >> 1) & 7u; };
+
+  // Workgroups go round-robin to the eight XCDs: each takes an equal run of tiles.
+  const uint32_t tiles = a.row_tiles * a.column_tiles, share = (tiles + 7) / 8;
+  const uint32_t nth = blockIdx.x / 8, tile = blockIdx.x % 8 * share + nth;
+  if (nth >= share || tile >= tiles) return;
+  const uint32_t band = tile / (a.row_tiles * kBand);
+  const uint32_t band_width = min((uint32_t)kBand, a.column_tiles - band * kBand);
+  const uint32_t in_band = tile - band * a.row_tiles * kBand;
+  const uint32_t row0 = in_band / band_width * kSideM, col0 = (band * kBand + in_band % band_width) * kSideN;
+  const uint32_t main_steps = a.inner / 64, steps = a.kt / 64, groups = main_steps;   // main_steps is a multiple of eight
+  const uint32_t periods = main_steps / kWK;
+
+  // Rows and columns past the end of a matrix reload its last one; what they produce is never stored.
+  uint32_t a_off[kLoads], w_off[kWordLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const uint32_t line = 64 * i + 8 * wave + lane / 8, row = line % kSideM;   // line: (step of the period, row)
+    a_off[i] = (min(row0 + row, a.rows - 1) * a.kt + 64 * (line / kSideM) + 8 * ((lane % 8) ^ swizzle_of(row))) * 2;
+  }
+  // A column's pieces lie in slots piece ^ (swizzle of the column): the 16 lanes that a read serves at once, which
+  // read the same piece of consecutive columns, spread over all banks.
+  auto word_swizzle = [](uint32_t column) { return kPieces == 4 ? (column >> 2) & 3u : (column >> 1) & 7u; };
+#pragma unroll
+  for (int i = 0; i < kWordLoads; ++i) {
+    const uint32_t at = 512 * i + tid, column = at / kPieces;   // 16-byte places of the buffer in order
+    w_off[i] = min(col0 + column, a.columns - 1) * (a.inner / 2) + 16 * ((at % kPieces) ^ word_swizzle(column));
+  }
+  const uint32_t s_off = min(col0 + kQ * wn + lane, a.columns - 1) * groups * 2;
+  auto stage = [&](uint32_t slot, uint32_t period) {
+    const unsigned char *from = (const unsigned char *)a.a + (uint64_t)period * (128 * kWK);
+    const unsigned char *words_from = (const unsigned char *)a.packed + (uint64_t)period * kWordRow;
+    const uint32_t to = lds + slot * kSlotBytes + wave * 1024;
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) load_to_lds_16_at(from, a_off[i], to + i * 8192);
+#pragma unroll
+    for (int i = 0; i < kWordLoads; ++i) load_to_lds_16_at(words_from, w_off[i], to + kTileBytes + i * 8192);
+  };
+  auto stage_scales = [&](uint32_t block) {
+    if (wm != 0 || wk != 0) return;   // one wave for 64 columns
+    const uint32_t bl = min(block, groups / 8 - 1);
+    load_to_lds_16_at((const unsigned char *)a.scales + (uint64_t)bl * 16, s_off,
+                      lds + kSlots * kSlotBytes + (block & 1u) * (kSideN * 16) + wn * 1024);
+  };
+
+  f32x16 acc[kMI][kMI];
+#pragma unroll
+  for (int i = 0; i < kMI; ++i)
+#pragma unroll
+    for (int j = 0; j < kMI; ++j)
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+  // The columns after the inner values are fp16 on both sides: kExtraSteps of their steps take the place of a slot.
+  constexpr int kExtraBytes = (kSideM + kSideN) * 128, kExtraSteps = kSlotBytes / kExtraBytes;
+  static_assert(kExtraSteps >= 1, "a slot holds a step of them");
+  const uint32_t extra_steps = steps - main_steps, extras_width = a.kt - a.inner;
+  uint32_t e_off[kSideN / 64];
+#pragma unroll
+  for (int i = 0; i < kSideN / 64; ++i) {
+    const uint32_t column = 64 * i + 8 * wave + lane / 8;
+    e_off[i] = (min(col0 + column, a.columns - 1) * extras_width + 8 * ((lane % 8) ^ swizzle_of(column))) * 2;
+  }
+  auto stage_extras = [&](uint32_t slot, uint32_t first) {
+#pragma unroll 1
+    for (uint32_t e = 0; e < kExtraSteps && first + e < extra_steps; ++e) {
+      const uint32_t to = lds + slot * kSlotBytes + e * kExtraBytes + wave * 1024;
+#pragma unroll
+      for (int i = 0; i < kSideM / 64; ++i)
+        load_to_lds_16_at((const unsigned char *)a.a + (uint64_t)(main_steps + first + e) * 128, a_off[i], to + i * 8192);
+#pragma unroll
+      for (int i = 0; i < kSideN / 64; ++i)
+        load_to_lds_16_at((const unsigned char *)a.extras + (uint64_t)(first + e) * 128, e_off[i], to + kSideM * 128 + i * 8192);
+    }
+  };
+
+  stage_scales(0);
+#pragma unroll 1
+  for (uint32_t p = 0; p < kSlots; ++p) stage(p, p);
+
+  // Lane half kh contracts K values [32 kh + 8 s, + 8) of a step in sub-step s.
+  f16x8 a_op[kSub][kMI], b_op[2][kMI];
+  const unsigned char *a_at[kSub];
+#pragma unroll
+  for (int s = 0; s < kSub; ++s)
+    a_at[s] = gemm_lds + wk * kStepBytes + (kQ * wm + l32) * 128 + 16 * ((4 * kh + s) ^ swizzle_of(l32));
+  auto read_a = [&](uint32_t slot, int s) {
+#pragma unroll
+    for (int i = 0; i < kMI; ++i)
+      a_op[s][i] = __builtin_bit_cast(f16x8, *(const uint4 *)(a_at[s] + slot * kSlotBytes + 32 * i * 128));
+  };
+  const unsigned char *words_at = gemm_lds + kTileBytes + (kQ * wn + l32) * kWordRow + 16 * ((2 * wk + kh) ^ word_swizzle(l32));
+  const unsigned char *scales_at = scale_rows + (kQ * wn + l32) * 16;
+  uint4 words[kMI], next_words[kMI];
+  uint32_t scale_bits[kMI];
+  auto read_words = [&](uint4 (&to)[kMI], uint32_t slot, uint32_t period) {
+#pragma unroll
+    for (int j = 0; j < kMI; ++j) to[j] = *(const uint4 *)(words_at + slot * kSlotBytes + 32 * j * kWordRow);
+    const uint32_t group = period * kWK + wk;
+#pragma unroll
+    for (int j = 0; j < kMI; ++j)
+      scale_bits[j] = *(const uint16_t *)(scales_at + (group / 8 & 1u) * (kSideN * 16) + (group & 7u) * 2 + 32 * j * 16);
+  };
+  f16x2 scale2[kMI], next_scale2[kMI];
+  auto take_scales = [&](f16x2 (&to)[kMI]) {
+#pragma unroll
+    for (int j = 0; j < kMI; ++j) {
+      const _Float16 h = (_Float16)__uint_as_float(scale_bits[j] << 16);
+      to[j] = f16x2{h, h};
+    }
+  };
+  uint32_t mask = 0x001e001eu, magic = 0x60006000u;
+  asm("" : "+s"(mask), "+v"(magic));   // no instruction: keeps the two constants in registers
+  // the matrix instructions of sub-step s; behind each row of them the operand of a column block for sub-step s + 1
+  auto sub_step = [&](int s, const uint4 (&next_words)[kMI], const f16x2 (&next_scale)[kMI]) {
+#pragma unroll
+    for (int i = 0; i < kMI; ++i) {
+#pragma unroll
+      for (int j = 0; j < kMI; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_op[s][i], b_op[s & 1][j], acc[i][j], 0, 0, 0);
+      const uint4 v = next_words[i];
+      b_op[(s + 1) & 1][i] = dequantise_word(s == 0 ? v.y : s == 1 ? v.z : s == 2 ? v.w : v.x, next_scale[i], mask, magic);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  __builtin_amdgcn_s_waitcnt(wait_vmcnt((kSlots - 1) * (kLoads + kWordLoads)));   // the first period has landed
+  lds_barrier();
+  read_words(words, 0, 0);
+  read_a(0, 0);
+  read_a(0, 1);
+  take_scales(scale2);
+#pragma unroll
+  for (int j = 0; j < kMI; ++j) b_op[0][j] = dequantise_word(words[j].x, scale2[j], mask, magic);
+
+  uint32_t slot = 0;
+#pragma unroll 1
+  for (uint32_t period = 0; period < periods; ++period) {
+    const uint32_t following = slot + 1 == kSlots ? 0 : slot + 1;
+    __builtin_amdgcn_sched_barrier(0);
+    read_a(slot, 2);
+    read_a(slot, 3);
+    __builtin_amdgcn_sched_barrier(0);
+    sub_step(0, words, scale2);
+    sub_step(1, words, scale2);
+    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): this wave has read all of the slot
+    // ... and its requests of the next period have landed; those of the kSlots - 2 periods behind that may be in
+    // flight (the block of scales is requested in front of its period's others)
+    if (kSlots == 2 || period + kSlots > periods)
+      __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));
+    else
+      __builtin_amdgcn_s_waitcnt(wait_vmcnt((kSlots - 2) * (kLoads + kWordLoads)));
+    lds_barrier();
+    read_words(next_words, following, period + 1);   // (behind the last period: nobody's)
+    read_a(following, 0);
+    read_a(following, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (period + kSlots < periods) {
+      if ((period & (kBlockPeriods - 1)) == 0) stage_scales(period / kBlockPeriods + 1);
+      stage(slot, period + kSlots);
+    } else if (period + 2 == periods) {
+      stage_extras(slot, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    sub_step(2, words, scale2);
+    take_scales(next_scale2);
+    sub_step(3, next_words, next_scale2);
+#pragma unroll
+    for (int j = 0; j < kMI; ++j) {
+      words[j] = next_words[j];
+      scale2[j] = next_scale2[j];
+    }
+    slot = following;
+  }
+  // ---- the columns after the inner values: their first steps are in the slot of the last period but one
+  uint32_t from = slot;
+#pragma unroll 1
+  for (int back = 0; back < 2; ++back) from = from == 0 ? kSlots - 1 : from - 1;
+  uint32_t to = from + 1 == kSlots ? 0 : from + 1;
+#pragma unroll 1
+  for (uint32_t first = 0; first < extra_steps; first += kExtraSteps) {
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));
+    lds_barrier();
+    stage_extras(to, first + kExtraSteps);
+#pragma unroll 1
+    for (uint32_t e = 0; e < kExtraSteps && first + e < extra_steps; ++e) {
+      const unsigned char *tile_at = gemm_lds + from * kSlotBytes + e * kExtraBytes;
+#pragma unroll
+      for (int own = 0; own < kSub / kWK; ++own) {   // a K part's share of a step: some of its sub-steps
+        const uint32_t piece = 16 * ((4 * kh + wk * (kSub / kWK) + own) ^ swizzle_of(l32));
+        f16x8 rows[kMI], columns[kMI];
+#pragma unroll
+        for (int i = 0; i < kMI; ++i) {
+          rows[i] = __builtin_bit_cast(f16x8, *(const uint4 *)(tile_at + (kQ * wm + 32 * i + l32) * 128 + piece));
+          columns[i] = __builtin_bit_cast(f16x8, *(const uint4 *)(tile_at + kSideM * 128 + (kQ * wn + 32 * i + l32) * 128 + piece));
+        }
+#pragma unroll
+        for (int i = 0; i < kMI; ++i)
+#pragma unroll
+          for (int j = 0; j < kMI; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(rows[i], columns[j], acc[i][j], 0, 0, 0);
+      }
+    }
+    const uint32_t swap = from;
+    from = to;
+    to = swap;
+  }
+  if (refused != 0) return;   // (uniform: the whole grid)
+  __builtin_amdgcn_s_waitcnt(0xc07f);
+  __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));   // nothing is on its way into LDS any more
+  lds_barrier();
+
+  // ---- the K parts' sums.  Part wk finishes blocks [wk * kOwn, (wk + 1) * kOwn) of its wave's four (row by row).
+  constexpr int kOwn = 4 / kWK;
+  float *parts = (float *)gemm_lds;   // [kWK][kWM * kWN][the 4 - kOwn blocks of others][16][64]
+  auto part_block = [&](uint32_t part, uint32_t block) -> float * {
+    const uint32_t nth_block = block < part * kOwn ? block : block - kOwn;
+    return parts + ((part * kWM * kWN + wm * kWN + wn) * (4 - kOwn) + nth_block) * 1024 + lane;
+  };
+#pragma unroll
+  for (int block = 0; block < 4; ++block) {
+    if ((uint32_t)(block / kOwn) == wk) continue;   // uniform
+    float *to = part_block(wk, block);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) to[64 * r] = acc[block / 2][block % 2][r];
+  }
+  __syncthreads();
+  f32x16 total[1][kOwn];
+#pragma unroll
+  for (int own = 0; own < kOwn; ++own) {
+    f32x16 mine = acc[0][0];   // this part's own block, picked without indexing registers dynamically
+#pragma unroll
+    for (int block = 1; block < 4; ++block)
+      if (wk * kOwn + own == (uint32_t)block) mine = acc[block / 2][block % 2];
+    f32x16 sum = mine;
+#pragma unroll
+    for (int part = 0; part < kWK; ++part) {
+      f32x16 value = mine;
+      if ((uint32_t)part != wk) {   // uniform
+        const float *from = part_block(part, wk * kOwn + own);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) value[r] = from[64 * r];
+      }
+      sum = part == 0 ? value : sum + value;
+    }
+    total[0][own] = sum;
+  }
+  __syncthreads();   // the sums have been read: store_tile reuses LDS
+  store_tile<32, 32 * kOwn, 2>(a, total, gemm_lds, row0, col0);
+}
+
+constexpr int split_lds_bytes(int wm, int wn, int wk, int slots) {
+  return slots * wk * (wm * 64 * 128 + wn * 64 * 32) + 2 * wn * 64 * 16;
+}
+
 }  // namespace
 
 // Whether gemm_q4_kernel takes the product: whole blocks of eight groups per weight row (a lane
@@ -1011,7 +1310,9 @@ bool launch_quant_gemm(fh_backend *backend, const QmmProblem &p, const uint32_t 
         {reinterpret_cast<const void *>(&gemm_f16_wide_kernel<kGemmK>), kWideLds},
         {reinterpret_cast<const void *>(&gemm_f16_kernel<kGemmK, kGemmStages, 64>), gemm_lds_bytes(64)},
         {reinterpret_cast<const void *>(&gemm_q4_kernel<2, 4, 128, 64>), kLargeLds},
-        {reinterpret_cast<const void *>(&gemm_q4_kernel<2, 2, 64, 64>), kSmallLds}};
+        {reinterpret_cast<const void *>(&gemm_q4_kernel<2, 2, 64, 64>), kSmallLds},
+        {reinterpret_cast<const void *>(&gemm_q4_split_kernel<2, 2, 2, 3>), split_lds_bytes(2, 2, 2, 3)},
+        {reinterpret_cast<const void *>(&gemm_q4_split_kernel<2, 1, 4, 2>), split_lds_bytes(2, 1, 4, 2)}};
     for (const auto &limit : limits) {
       if (hipFuncSetAttribute(limit.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, limit.bytes) != hipSuccess)
         return false;
@@ -1038,10 +1339,22 @@ bool launch_quant_gemm(fh_backend *backend, const QmmProblem &p, const uint32_t 
     }
   }
   if (packed_form) {
-    if (small_tiles)
+    // Outputs with fewer small tiles than the device has compute units: the kernel whose waves split K.  More tiles
+    // put two workgroups of four waves on a unit, which hide each other's waits too, without meeting K parts
+    // (microseconds, 128 x 128 tiles of four waves, 128 x 128 and 128 x 64 of eight: 2048 x 1024 x 2048 41.3, 32.0,
+    // 29.2; 300 x 4096 x 1024 22.8, 18.4, 15.1; 600 x 5120 x 17408 258, 186, 220 (400 of 128 x 64); 1000 x 5120 x 5120
+    // 106, 112, 108; 2080 x 5120 x 2048 81, 84, 101).
+    const uint32_t half_tiles = a.row_tiles * ((p.columns + 63) / 64), units = backend_compute_units(backend);
+    if (small_tiles && half_tiles <= units) {
+      a.column_tiles = (p.columns + 63) / 64;
+      gemm_q4_split_kernel<2, 1, 4, 2><<<(half_tiles + 7) / 8 * 8, 512, split_lds_bytes(2, 1, 4, 2), stream>>>(a);
+    } else if (small_tiles && a.row_tiles * a.column_tiles <= units) {
+      gemm_q4_split_kernel<2, 2, 2, 3><<<(a.row_tiles * a.column_tiles + 7) / 8 * 8, 512, split_lds_bytes(2, 2, 2, 3), stream>>>(a);
+    } else if (small_tiles) {
       gemm_q4_kernel<2, 2, 64, 64><<<grid, 256, kSmallLds, stream>>>(a);
-    else
+    } else {
       gemm_q4_kernel<2, 4, 128, 64><<<grid, 512, kLargeLds, stream>>>(a);
+    }
   } else if (small_tiles) {
     gemm_f16_kernel<kGemmK, kGemmStages, 64><<<grid, 256, gemm_lds_bytes(64), stream>>>(a);
   } else {

@@ -475,6 +475,34 @@ def test_quant_matmul_with_f16_scales_and_a_residual_in_other_dtypes(cpu, hip, d
     differential(cpu, hip, build)
 
 
+@pytest.mark.parametrize("rows,n,k", [
+    (129, 72, 512),       # the fewest K steps a part of the split takes, a column tile nearly empty
+    (300, 200, 1536),     # ragged rows and columns
+    (130, 70, 17408),     # more columns of group sums than a slot of LDS holds at a time
+    (200, 8264, 512),     # 128 x 128 tiles, the fewest K steps
+    (257, 5700, 2560),
+])
+@pytest.mark.parametrize("residual", [False, True])
+def test_prefill_products_of_few_tiles(hip, rows, n, k, residual):
+    """Products whose waves split K: against 64 bits.  A result is rounded once to bf16 (2^-9 of it at most), its
+    weights once to f16 (2^-12 of each)."""
+    weights, values, extra = Quantised(62, n + k, (n, k)), normal_bf16(62, 1, (rows, k)), normal_bf16(62, 2, (rows, n))
+    out = hip.alloc(DType.BF16, (rows, n))
+    commands, operands = CommandList(), [upload(hip, values, DType.BF16), *weights.upload(hip)]
+    if residual:
+        commands.dispatch_epilogue(Op.quant_matmul(4, 64), operands, out, hip.prepare_epilogue(programs.add_elements()),
+                                   [upload(hip, extra, DType.BF16)])
+    else:
+        commands.dispatch(Op.quant_matmul(4, 64), operands, out)
+    run(hip, commands)
+    reference = values.astype(np.float64) @ weights.dequantised().T + (extra if residual else 0.0)
+    error = to_f32(hip.read(out), DType.BF16).reshape(rows, n) - reference
+    assert np.linalg.norm(error) <= (2.0 ** -9 + 2.0 ** -12) * np.linalg.norm(reference)
+    # (element by element: the sums' own rounding is that of f16 products of k random values)
+    scale = np.sqrt(np.mean(reference ** 2))
+    assert np.all(np.abs(error) <= 2.0 ** -8 * np.abs(reference) + 2.0 ** -9 * scale)
+
+
 def test_quant_gemm_with_scales_outside_the_fp16_range_and_huge_activations(cpu, hip):
     """Prefill-sized product whose affine parameters are not fp16 normal numbers (tiny scales, a
     zero bias, a large scale) and whose activations exceed the fp16 range in some rows: the
