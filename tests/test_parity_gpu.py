@@ -1017,7 +1017,9 @@ def test_gather_with_an_unrecognised_epilogue_uses_the_interpreter(cpu, hip):
 
 @pytest.mark.parametrize("rows,k,experts,tile", [(256, 8, 128, 16), (128, 8, 128, 32), (7, 3, 5, 2),
                                                 (1, 1, 1, 1), (300, 8, 128, 32), (64, 2, 200, 8),
-                                                (100, 8, 512, 32), (333, 8, 3, 32)])
+                                                (100, 8, 512, 32), (333, 8, 3, 32),
+                                                (2081, 8, 128, 64),     # 17 steps of a wave, the last runs short
+                                                (5003, 8, 40, 32)])     # more routes than LDS puts together
 def test_route_pack_is_bit_exact(cpu, hip, rows, k, experts, tile):
     rng = np.random.default_rng(rows * 31 + k)
     indices = rng.integers(0, experts, (rows, k)).astype(np.uint32)
@@ -1668,6 +1670,30 @@ def test_engine_row_programs(cpu, hip, dtype):
              norm.narrow(2, half, half), pos],
             [rotated.narrow(2, 0, half), rotated.narrow(2, half, half)])
         return commands, [normed, hidden_out, normed2, rotated]
+    differential(cpu, hip, build, abs_=2e-2, bar=DType.F16 if dtype == DType.F32 else None)
+
+
+@pytest.mark.parametrize("rows,heads", [(512, 3), (1029, 24)])
+@pytest.mark.parametrize("dtype", [DType.BF16, DType.F32])
+def test_head_norm_and_rotation_over_many_rows(cpu, hip, rows, heads, dtype):
+    """Four rows to a workgroup, two heads to a wave: an odd number of heads, rows that end inside a workgroup.  f32
+    results are held to the f16 bar, as above."""
+    half = 64
+    qk_values, norm_values = normal_bf16(73, rows, (rows, heads + 1, 2 * half)), 1.0 + 0.1 * normal_bf16(73, 5, (heads, 2 * half))
+    positions = (np.arange(rows) * 7 % 4099).astype(np.float32)
+
+    def build(backend):
+        qk = upload(backend, qk_values, dtype).narrow(1, 1, heads)   # (rows that lie further apart than their heads)
+        norm = upload(backend, norm_values, dtype).broadcast((rows, heads, 2 * half))
+        pos = upload(backend, positions, DType.F32).reshape((rows, 1, 1)).broadcast((rows, heads, half))
+        rotated = backend.alloc(dtype, (rows, heads, 2 * half))
+        commands = CommandList()
+        commands.dispatch_kernel(
+            backend.prepare_program(programs.qk_norm_rope_rows(128.0, 1e-6, 1e6)),
+            [qk.narrow(2, 0, half), qk.narrow(2, half, half), norm.narrow(2, 0, half),
+             norm.narrow(2, half, half), pos],
+            [rotated.narrow(2, 0, half), rotated.narrow(2, half, half)])
+        return commands, [rotated]
     differential(cpu, hip, build, abs_=2e-2, bar=DType.F16 if dtype == DType.F32 else None)
 
 
