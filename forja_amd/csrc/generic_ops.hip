@@ -46,6 +46,13 @@ __global__ __launch_bounds__(256) void copy_flat_kernel(const uint4 *in, uint4 *
     out[i] = in[i];
 }
 
+// A few kilobytes from or to pinned host memory, in pieces of the widest size that addresses and length allow.
+template <typename Piece>
+__global__ __launch_bounds__(256) void move_bytes_kernel(const Piece *from, Piece *to, uint32_t pieces) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i < pieces) to[i] = from[i];
+}
+
 // ---------------------------------------------------------------- scalar programs
 
 __device__ inline uint32_t saturating_u32(float value) {
@@ -1094,6 +1101,18 @@ void launch_fill_seeded(hipStream_t s, const View &out, uint64_t elements, uint3
 void launch_fill_u32(hipStream_t s, uint32_t *ptr, uint64_t count, uint32_t value) {
   if (count == 0) return;
   fill_u32_kernel<<<grid_for(count), kBlock, 0, s>>>(ptr, count, value);
+}
+
+void launch_move_bytes(hipStream_t s, void *to, const void *from, uint32_t bytes) {
+  if (bytes == 0) return;
+  const uint64_t all = (uint64_t)(uintptr_t)to | (uint64_t)(uintptr_t)from | bytes;
+  auto blocks = [&](uint32_t size) { return (bytes / size + 255) / 256; };
+  if (all % 16 == 0)
+    move_bytes_kernel<uint4><<<blocks(16), 256, 0, s>>>((const uint4 *)from, (uint4 *)to, bytes / 16);
+  else if (all % 4 == 0)
+    move_bytes_kernel<uint32_t><<<blocks(4), 256, 0, s>>>((const uint32_t *)from, (uint32_t *)to, bytes / 4);
+  else
+    move_bytes_kernel<uint8_t><<<blocks(1), 256, 0, s>>>((const uint8_t *)from, (uint8_t *)to, bytes);
 }
 
 void launch_init_errors(hipStream_t s, ErrorSlot *slots, uint32_t count) {
