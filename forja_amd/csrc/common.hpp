@@ -118,6 +118,28 @@ __device__ inline int32_t total_key(float value) {
   return bits ^ (int32_t)(((uint32_t)(bits >> 31)) >> 1);
 }
 
+// 64 lanes x 16 bytes from memory straight into LDS at `lds_base` + 16 * lane, issued as an
+// instruction the compiler does not see: while it knows of such a load in flight it waits for ALL
+// outstanding LDS reads wherever it has to wait for one (it cannot tell the load's LDS write from
+// the wave's own LDS traffic), i.e. also for the operand reads just issued for the next sub-step,
+// and it drains every such load at a __syncthreads().  Callers order these loads by hand (vmcnt).
+__device__ inline void load_to_lds_16_at(const void *from, uint32_t lds_address) {
+  // (uniform by construction; the intrinsic tells the compiler so)
+  const uint32_t at = __builtin_amdgcn_readfirstlane(lds_address);
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(at) : "memory");   // (m0 is the compiler's only for its own such loads: kernels that use this have none)
+}
+
+__device__ inline uint32_t lds_address(const void *in_lds) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) unsigned char *)in_lds;
+}
+
+__device__ inline void load_to_lds_16(const void *from, unsigned char *lds_base) {
+  load_to_lds_16_at(from, lds_address(lds_base));
+}
+
+// A barrier alone: the caller has waited for what it needs (a __syncthreads() drains more).
+__device__ inline void lds_barrier() { asm volatile("s_barrier" ::: "memory"); }
+
 #endif  // __HIPCC__
 
 }  // namespace fh

@@ -4,6 +4,7 @@
 // the lane's new K/V rows were stored at its q_start (execute_paged_append,
 // crates/forja-cpu/src/lib.rs:262-306).  Pools are [P, page_tokens, Hkv, D]; a table entry is
 // (physical page, generation) and is valid iff page < P and generations[page] == generation.
+#include <algorithm>
 #include <cstdlib>
 
 #include "fast_kernels.hpp"
@@ -273,6 +274,9 @@ constexpr uint32_t kFillingGroups = 512, kFilledSplitTokens = 512;
 constexpr uint32_t kPrefillSplitTokens = 2048;
 constexpr uint32_t kTargetItems = 1024;  // (token, split) items wanted per launch of grouped tokens
 constexpr uint32_t kTile = 32;          // tokens per inner step
+// Prefill workgroups per compute unit at most (it holds two); what is left of the items' list, whose length
+// only the device knows, they walk on.
+constexpr uint32_t kPrefillGrid = 8;
 
 struct TokenPlan {
   uint32_t lane, attended, chunk, splits;  // splits == 0: token produces zeros
@@ -301,7 +305,7 @@ struct FastRagged {
   // sizes the splits so that the items fill these places once.
   uint32_t item_slots;
   // Query tokens of one lane are processed `group_tokens` at a time (they share the lane's K/V
-  // stream): 1 for decode batches (a wave per kv head), kSharedWaves * kSharedTiles * (16 / group)
+  // stream): 1 for decode batches (a wave per kv head), kPrefillRows / group
   // for prefill batches (a workgroup per kv head).
   uint32_t group_tokens;
   float scale_log2;
@@ -687,87 +691,71 @@ struct Softmax {
   float m, l;
 };
 
-// Scores, online softmax and the value product for one tile of 32 keys against NT query tiles
-// (16 query rows each: this lane holds row hl of every tile).  `limit[nt]` is the first key the
-// lane's row of tile nt may NOT attend (0 for an unused row); with kMasked false every key of
-// the tile is below every limit.
-template <int NT, bool kMasked, bool kHalf>
-__device__ inline void consume_tile(const TileRegs &cur, const uint4 (&q_reg)[NT][4],
-                                    f32x4 (&o)[NT][8], Softmax (&sm)[NT], uint32_t tile0,
-                                    const uint32_t (&limit)[NT], float scale_log2, uint32_t g) {
-  uint4 p_reg[NT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    float s_val[8];
-    for (int sub = 0; sub < 2; ++sub) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-      for (int step = 0; step < 4; ++step)
-        acc = mfma_16x16x32<kHalf>(cur.k[sub][step], q_reg[nt][step], acc);
-      for (int j = 0; j < 4; ++j) {
-        s_val[4 * sub + j] = acc[j] * scale_log2;
-        if (kMasked && tile0 + 16 * sub + 4 * g + j >= limit[nt]) s_val[4 * sub + j] = -__builtin_inff();
-      }
+// Scores, online softmax and the value product for one tile of 32 keys against 16 query rows (this lane
+// holds row hl).  `limit` is the first key the rows may NOT attend; with kMasked false every key of the
+// tile is below it.
+template <bool kMasked, bool kHalf>
+__device__ inline void consume_tile(const TileRegs &cur, const uint4 (&q_reg)[4], f32x4 (&o)[8], Softmax &sm,
+                                    uint32_t tile0, uint32_t limit, float scale_log2, uint32_t g) {
+  float s_val[8];
+  for (int sub = 0; sub < 2; ++sub) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int step = 0; step < 4; ++step)
+      acc = mfma_16x16x32<kHalf>(cur.k[sub][step], q_reg[step], acc);
+    for (int j = 0; j < 4; ++j) {
+      s_val[4 * sub + j] = acc[j] * scale_log2;
+      if (kMasked && tile0 + 16 * sub + 4 * g + j >= limit) s_val[4 * sub + j] = -__builtin_inff();
     }
-    float tile_max = s_val[0];
-    for (int i = 1; i < 8; ++i) tile_max = fmaxf(tile_max, s_val[i]);
-    tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, 64));
-    tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, 64));
-    const float m_new = fmaxf(sm[nt].m, tile_max);
-    // a row with nothing to attend yet keeps m = -inf; subtract 0 instead so that exp2(-inf) = 0
-    const float m_safe = (kMasked && m_new == -__builtin_inff()) ? 0.0f : m_new;
-    float p_val[8], p_sum = 0.0f;
-    for (int i = 0; i < 8; ++i) {
-      p_val[i] = __builtin_amdgcn_exp2f(s_val[i] - m_safe);
-      p_sum += p_val[i];
-    }
-    // The running maximum settles after a few tiles; skip the rescale when no lane's moved.
-    if (__any(m_new != sm[nt].m)) {
-      const float alpha = __builtin_amdgcn_exp2f(sm[nt].m - m_safe);   // 0 while m is -inf
-      sm[nt].l *= alpha;
-      for (int mt = 0; mt < 8; ++mt)
-        for (int j = 0; j < 4; ++j) o[nt][mt][j] *= alpha;
-      sm[nt].m = m_new;
-    }
-    sm[nt].l += p_sum;
-    p_reg[nt] = make_uint4(pack_operand<kHalf>(p_val[0], p_val[1]), pack_operand<kHalf>(p_val[2], p_val[3]),
-                           pack_operand<kHalf>(p_val[4], p_val[5]), pack_operand<kHalf>(p_val[6], p_val[7]));
   }
-  // O^T += V^T . P^T.  Tile mt takes element mt of each of the lane's 8 token pieces; the
-  // transposed value operand serves all NT query tiles.
+  float tile_max = s_val[0];
+  for (int i = 1; i < 8; ++i) tile_max = fmaxf(tile_max, s_val[i]);
+  tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, 64));
+  tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, 64));
+  const float m_new = fmaxf(sm.m, tile_max);
+  // a row with nothing to attend yet keeps m = -inf; subtract 0 instead so that exp2(-inf) = 0
+  const float m_safe = (kMasked && m_new == -__builtin_inff()) ? 0.0f : m_new;
+  float p_val[8], p_sum = 0.0f;
+  for (int i = 0; i < 8; ++i) {
+    p_val[i] = __builtin_amdgcn_exp2f(s_val[i] - m_safe);
+    p_sum += p_val[i];
+  }
+  // The running maximum settles after a few tiles; skip the rescale when no lane's moved.
+  if (__any(m_new != sm.m)) {
+    const float alpha = __builtin_amdgcn_exp2f(sm.m - m_safe);   // 0 while m is -inf
+    sm.l *= alpha;
+    for (int mt = 0; mt < 8; ++mt)
+      for (int j = 0; j < 4; ++j) o[mt][j] *= alpha;
+    sm.m = m_new;
+  }
+  sm.l += p_sum;
+  const uint4 p_reg = make_uint4(pack_operand<kHalf>(p_val[0], p_val[1]), pack_operand<kHalf>(p_val[2], p_val[3]),
+                                 pack_operand<kHalf>(p_val[4], p_val[5]), pack_operand<kHalf>(p_val[6], p_val[7]));
+  // O^T += V^T . P^T.  Tile mt takes element mt of each of the lane's 8 token pieces.
   for (int mt = 0; mt < 8; ++mt) {
     const uint32_t selector = (mt & 1) ? 0x07060302u : 0x05040100u;
     uint32_t a_words[4];
     for (int pair = 0; pair < 4; ++pair)
       a_words[pair] = __builtin_amdgcn_perm(dword_of(cur.v[2 * pair + 1], mt >> 1),
                                             dword_of(cur.v[2 * pair], mt >> 1), selector);
-    const uint4 a_reg = make_uint4(a_words[0], a_words[1], a_words[2], a_words[3]);
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-      o[nt][mt] = mfma_16x16x32<kHalf>(a_reg, p_reg[nt], o[nt][mt]);
+    o[mt] = mfma_16x16x32<kHalf>(make_uint4(a_words[0], a_words[1], a_words[2], a_words[3]), p_reg, o[mt]);
   }
 }
 
-// NT query tiles of 16 rows per wave: row hl of tile nt is (query token nt * per_tile + hl / group
-// of the item's group, head hl % group of the kv head), per_tile = 16 / group.
-template <int NT, bool kHalf, bool kMixed>
-__device__ inline void ragged_attention_body(const FastRagged &p, ErrorSlot *error) {
-  // a workgroup is one work item; its waves take one kv head each, so the slices of a K/V page
-  // (one 256-byte piece of every token row per kv head) are requested close together in time
-  const uint32_t lane = threadIdx.x & 63, hl = lane & 15, g = lane >> 4;
-  const uint32_t item = blockIdx.x, kv_head = blockIdx.y * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (item >= p.item_count[0] || kv_head >= p.kv_heads) return;
+// One split of a group of one query token, for one kv head, by one wave: the head's `group` query rows
+// (lane's row hl; rows from `group` on are padding) attend keys streamed straight into registers.
+template <bool kHalf, bool kMixed>
+__device__ inline void attend_one_token(const FastRagged &p, ErrorSlot *error, uint32_t item, uint32_t kv_head) {
+  uint32_t lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));   // what follows from it is not kept in registers from item to item
+  const uint32_t hl = lane & 15, g = lane >> 4;
   const uint2 work = p.items[item];
   const uint32_t leader = work.x, split = work.y;
   const TokenPlan plan = p.plans[leader];
-  const uint32_t members = NT == 1 ? 1 : plan.members;
-  // the group's split layout is sized for its last member
-  const uint32_t longest =
-      (NT == 1 || p.fixed_attended) ? plan.attended : plan.attended + members - 1;
   const uint32_t begin = split * plan.chunk;
-  const uint32_t end = min(longest, begin + plan.chunk);
+  const uint32_t end = min(plan.attended, begin + plan.chunk);
   const uint32_t pt = p.page_tokens;
   const uint32_t *table = p.tables + (uint64_t)plan.lane * p.table_pages * 2;
-  if (NT == 1 && p.append_in_kernel &&
+  if (p.append_in_kernel &&
       (split + 1 == plan.splits || (p.row_twice != nullptr && p.row_twice[0] != 0))) {
     // This wave's kv head of the lane's new row goes into the pool before anything is read: the
     // row sits at the last attended position, which only the last split's range contains.
@@ -805,37 +793,16 @@ __device__ inline void ragged_attention_body(const FastRagged &p, ErrorSlot *err
   lc.k_offset = (hl * p.kv_heads + kv_head) * 128 + 8 * g;
   lc.v_offset = (4 * g * p.kv_heads + kv_head) * 128 + 8 * hl;
 
-  // Query operands and causal limits of this lane's rows.
-  const uint32_t per_tile = NT == 1 ? 1 : 16 / p.group;
-  uint4 q_reg[NT][4];
-  uint32_t limit[NT], member_of[NT];
-  const uint32_t head = kv_head * p.group + (NT == 1 ? hl : hl % p.group);
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    member_of[nt] = NT == 1 ? 0 : nt * per_tile + hl / p.group;
-    const bool used = hl < per_tile * p.group && member_of[nt] < members;
-    // (a decode row that is only padding keeps the uniform limit: its query is zero anyway)
-    limit[nt] = NT == 1 ? end
-                        : (!used ? 0
-                                 : min(end, p.fixed_attended ? plan.attended
-                                                             : plan.attended + member_of[nt]));
-    const uint64_t q_row = (uint64_t)(leader + member_of[nt]) * p.q_stride_t +
-                           (uint64_t)head * p.q_stride_h;
-    for (int step = 0; step < 4; ++step) {  // same head-dim slice per (step, g) as the K operand
-      q_reg[nt][step] = make_uint4(0, 0, 0, 0);
-      if (used) q_reg[nt][step] = load_query<kHalf, kMixed>(p, q_row + 32 * step + 8 * g);
-    }
-    if (NT > 1 && !used) member_of[nt] = 0xffffffffu;
+  uint4 q_reg[4];
+  const uint32_t head = kv_head * p.group + hl;
+  const uint64_t q_row = (uint64_t)leader * p.q_stride_t + (uint64_t)head * p.q_stride_h;
+  for (int step = 0; step < 4; ++step) {  // same head-dim slice per (step, g) as the K operand
+    q_reg[step] = make_uint4(0, 0, 0, 0);
+    if (hl < p.group) q_reg[step] = load_query<kHalf, kMixed>(p, q_row + 32 * step + 8 * g);
   }
-  // keys below `unmasked_end` are attended by every used row
-  const uint32_t unmasked_end = NT == 1 ? end : min(end, plan.attended);
-  f32x4 o[NT][8];
-  Softmax sm[NT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    for (int mt = 0; mt < 8; ++mt) o[nt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    sm[nt] = Softmax{-__builtin_inff(), 0.0f};
-  }
+  f32x4 o[8];
+  for (int mt = 0; mt < 8; ++mt) o[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  Softmax sm{-__builtin_inff(), 0.0f};
 
   const uint32_t first_page = begin / pt, last_page = (end - 1) / pt;
   for (uint32_t page0 = first_page; page0 <= last_page; page0 += 64) {
@@ -851,188 +818,300 @@ __device__ inline void ragged_attention_body(const FastRagged &p, ErrorSlot *err
     if (bad_mask) {
       if (lane == (uint32_t)__ffsll((long long)bad_mask) - 1) {
         report_error(error + (uint64_t)leader * p.error_stride, my_page);
-        for (uint32_t member = 0; member < members; ++member) p.bad[leader + member] = 1;
+        p.bad[leader] = 1;
       }
-      if (plan.splits == 1) zero_head_rows<kMixed>(p, leader, members, kv_head, lane);
+      if (plan.splits == 1) zero_head_rows<kMixed>(p, leader, 1, kv_head, lane);
       return;
     }
     const uint32_t tok_lo = max(begin, page0 * pt);
     const uint32_t tok_hi = (uint32_t)min((uint64_t)end, ((uint64_t)page0 + 64) * pt);
-    // Tiles wholly below unmasked_end need no bounds logic at all; the rest (at most a few
-    // around the causal diagonal and the end of the split) take the masked forms.
-    const uint32_t plain_keys = unmasked_end > tok_lo ? min(tok_hi, unmasked_end) - tok_lo : 0;
-    const uint32_t full_hi = tok_lo + plain_keys / kTile * kTile;
-    TileRegs cur;
-    if (tok_lo + kTile <= tok_hi)
+    const uint32_t full_hi = tok_lo + (tok_hi - tok_lo) / kTile * kTile;
+    // Two tiles in registers, one on its way while the other is consumed.  The loop requests whole tiles
+    // only, so that the wait in front of a tile's products is for that tile alone: with a choice between
+    // whole and masked requests inside, the compiler waits for both tiles there.
+    const bool tail = full_hi < tok_hi;   // plain tiles are followed by at most one masked tile
+    TileRegs cur, nxt;
+    if (full_hi > tok_lo) {
       load_tile<false>(p, cur, tok_lo, end, page0, physical, lc, hl, g);
-    else
-      load_tile<true>(p, cur, tok_lo, end, page0, physical, lc, hl, g);
-    // Software pipeline: the next tile's loads are in flight while this one is consumed.
-    if constexpr (NT == 1) {
-      // a decode split is plain tiles followed by at most one masked tile
-      for (uint32_t tile0 = tok_lo; tile0 < full_hi; tile0 += kTile) {
-        TileRegs nxt;
-        const uint32_t next0 = tile0 + kTile;
-        if (next0 < full_hi)
-          load_tile<false>(p, nxt, next0, end, page0, physical, lc, hl, g);
-        else if (next0 < tok_hi)
-          load_tile<true>(p, nxt, next0, end, page0, physical, lc, hl, g);
-        consume_tile<NT, false, kHalf>(cur, q_reg, o, sm, tile0, limit, p.scale_log2, g);
-        if (next0 < tok_hi) cur = nxt;
+      uint32_t tile0 = tok_lo;   // the tile in `cur`
+      for (; tile0 + kTile < full_hi; tile0 += kTile) {
+        load_tile<false>(p, nxt, tile0 + kTile, end, page0, physical, lc, hl, g);
+        __builtin_amdgcn_sched_barrier(0);
+        consume_tile<false, kHalf>(cur, q_reg, o, sm, tile0, end, p.scale_log2, g);
+        __builtin_amdgcn_sched_barrier(0);
+        cur = nxt;
       }
-      if (full_hi < tok_hi)
-        consume_tile<NT, true, kHalf>(cur, q_reg, o, sm, full_hi, limit, p.scale_log2, g);
+      if (tail) load_tile<true>(p, nxt, full_hi, end, page0, physical, lc, hl, g);
+      consume_tile<false, kHalf>(cur, q_reg, o, sm, tile0, end, p.scale_log2, g);
     } else {
-      for (uint32_t tile0 = tok_lo; tile0 < tok_hi; tile0 += kTile) {
-        TileRegs nxt;
-        const uint32_t next0 = tile0 + kTile;
-        if (next0 + kTile <= tok_hi)
-          load_tile<false>(p, nxt, next0, end, page0, physical, lc, hl, g);
-        else if (next0 < tok_hi)
-          load_tile<true>(p, nxt, next0, end, page0, physical, lc, hl, g);
-        if (tile0 < full_hi)
-          consume_tile<NT, false, kHalf>(cur, q_reg, o, sm, tile0, limit, p.scale_log2, g);
-        else
-          consume_tile<NT, true, kHalf>(cur, q_reg, o, sm, tile0, limit, p.scale_log2, g);
-        if (next0 < tok_hi) cur = nxt;
-      }
+      load_tile<true>(p, nxt, full_hi, end, page0, physical, lc, hl, g);
     }
+    if (tail) consume_tile<true, kHalf>(nxt, q_reg, o, sm, full_hi, end, p.scale_log2, g);
   }
-  // Lane (row hl, group g) holds value columns 32g + 8j + mt of its rows.
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    float m_run = sm[nt].m, l_run = sm[nt].l;
-    l_run += __shfl_xor(l_run, 16, 64);
-    l_run += __shfl_xor(l_run, 32, 64);
-    if (NT == 1 ? hl >= p.group : member_of[nt] == 0xffffffffu) continue;
-    const uint32_t token = leader + member_of[nt];
-    if (plan.splits == 1) {
-      float inv = 1.0f / l_run;
-      const uint64_t out_row = (uint64_t)token * p.out_stride_t + (uint64_t)head * p.out_stride_h;
-      for (int j = 0; j < 4; ++j) {
-        store_out4<kHalf, kMixed>(p, out_row + 32 * g + 8 * j, o[nt][0][j] * inv, o[nt][1][j] * inv,
-                   o[nt][2][j] * inv, o[nt][3][j] * inv);
-        store_out4<kHalf, kMixed>(p, out_row + 32 * g + 8 * j + 4, o[nt][4][j] * inv, o[nt][5][j] * inv,
-                   o[nt][6][j] * inv, o[nt][7][j] * inv);
-      }
-      continue;
-    }
-    uint64_t slot = ((uint64_t)token * p.max_splits + split) * p.query_heads + head;
-    float *po = p.partial_o + slot * 128 + 32 * g;
+  // Lane (row hl, group g) holds value columns 32g + 8j + mt of its row.
+  sm.l += __shfl_xor(sm.l, 16, 64);
+  sm.l += __shfl_xor(sm.l, 32, 64);
+  if (hl >= p.group) return;
+  if (plan.splits == 1) {
+    float inv = 1.0f / sm.l;
+    const uint64_t out_row = (uint64_t)leader * p.out_stride_t + (uint64_t)head * p.out_stride_h;
     for (int j = 0; j < 4; ++j) {
-      *(float4 *)(po + 8 * j) = make_float4(o[nt][0][j], o[nt][1][j], o[nt][2][j], o[nt][3][j]);
-      *(float4 *)(po + 8 * j + 4) = make_float4(o[nt][4][j], o[nt][5][j], o[nt][6][j], o[nt][7][j]);
+      store_out4<kHalf, kMixed>(p, out_row + 32 * g + 8 * j, o[0][j] * inv, o[1][j] * inv, o[2][j] * inv, o[3][j] * inv);
+      store_out4<kHalf, kMixed>(p, out_row + 32 * g + 8 * j + 4, o[4][j] * inv, o[5][j] * inv, o[6][j] * inv,
+                                o[7][j] * inv);
     }
-    if (g == 0) p.partial_ml[slot] = make_float2(m_run, l_run);
+    return;
   }
+  uint64_t slot = ((uint64_t)leader * p.max_splits + split) * p.query_heads + head;
+  float *po = p.partial_o + slot * 128 + 32 * g;
+  for (int j = 0; j < 4; ++j) {
+    *(float4 *)(po + 8 * j) = make_float4(o[0][j], o[1][j], o[2][j], o[3][j]);
+    *(float4 *)(po + 8 * j + 4) = make_float4(o[4][j], o[5][j], o[6][j], o[7][j]);
+  }
+  if (g == 0) p.partial_ml[slot] = make_float2(sm.m, sm.l);
 }
 
 // ---- prefill: K/V tiles staged in LDS and shared by the four waves of a workgroup -------------
 //
-// A work item of a prefill batch is (up to kSharedWaves * kSharedTiles * (16 / group) consecutive query
-// tokens of a lane, split); blockIdx.y is the kv head.  Wave w owns the w-th slice of those tokens
-// (one 16-row query tile: 16 / group tokens x group heads) and all waves walk the same keys, so a
-// K/V tile is fetched from memory once per workgroup: each wave moves its share of the tile
-// straight into LDS (global_load_lds), double buffered, one barrier per tile.  The softmax is
-// vector-ALU and latency heavy, so the kernel is built for occupancy rather than for long
-// software pipelines: one query tile per wave keeps it at 168 registers, three waves per SIMD
-// (three workgroups per CU).  Rows are 256 bytes (one head of one
-// token); the 16-byte piece p of row r sits in slot p ^ (r & 15), which keeps both operand read
-// patterns (a K row piece per lane, a V column piece of eight tokens per lane) free of bank
-// conflicts.  Keys past the end of the split are staged from its last valid token and masked.
-constexpr uint32_t kSharedWaves = 4;    // waves of a prefill workgroup
-constexpr int kSharedTiles = 1;          // 16-row query tiles per wave
+// A work item of a prefill batch is (up to 128 / group consecutive query tokens of a lane, split) and a
+// kv head: 128 query rows (token-major, the group's heads inside), 32 to a wave.  All waves walk the same
+// keys in tiles of 64, moved straight into LDS while the tile before is attended, one barrier per tile.
+// The moves are issued behind the compiler's back (load_to_lds_16_at): it waits for every one it knows of
+// in front of the next read of LDS, which puts the moves and the arithmetic one after the other.
+// What bounds it: the tiles' way in (alone 72 of 95 us where 2048 rows in three chunks behind 1024 keys and 32 decode
+// rows attend with 32 heads) and the chain of one wave's tile, scores, softmax and value product (alone
+// 75 us), of which two waves per SIMD overlap a part.  Hence 32 x 32 products (a tile's LDS bytes serve
+// twice the rows of 16 x 16 ones), one query row to a lane pair (a maximum is 31 comparisons and one
+// exchange), operands read from LDS four products ahead, V transposed on the way out of LDS.
+// Against 16-row waves that waited for each tile: that batch 186 -> 92 us, 8192 rows in six chunks with 64
+// decode rows (40 heads) 567 -> 235, 512 rows of f32 (32 heads) 44 -> 21, 2000 rows in four chunks with 48
+// decode rows (16 heads) 89 -> 66.
+// Eight waves of 32 rows and four tiles in LDS (three on their way) took 99, 265, 27 and 88 us: the decode rows of a
+// batch keep one wave busy, and one workgroup per compute unit leaves nothing beside it.
+//
+// Rows are 256 bytes (one head of one token).  The 16-byte piece p of K row r sits in slot p ^ (r & 15):
+// 16 rows read at one piece use all banks once.  Piece p of V row r sits in slot
+// p ^ ((r & 3) << 2 | (r >> 2 & 3)): the transposing read takes 4 rows x 4 pieces at once, which the
+// first term spreads over the banks.  Keys past the end of the split are staged from a valid row and
+// masked.
+constexpr uint32_t kPrefillWaves = 4, kPrefillRows = 32 * kPrefillWaves, kPrefillTile = 64;
 
-struct SharedTiles {
-  uint4 rows[2][2][kTile][16];   // [buffer][K, V][token][slot]
+typedef __attribute__((ext_vector_type(4))) short s16x4;
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+
+// A staged tile in LDS: K rows, V rows.  Tiles are named by their LDS address.
+constexpr uint32_t kPrefillRow = 256, kPrefillValues = kPrefillTile * kPrefillRow, kPrefillTileBytes = 2 * kPrefillValues;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+typedef __attribute__((address_space(3))) s16x4 *LdsPiece;
+typedef const __attribute__((address_space(3))) u32x4 *LdsWords;
+
+template <bool kHalf>
+__device__ inline f32x16 mfma_32x32x16(const uint4 &a, const uint4 &b, const f32x16 &c) {
+  if constexpr (kHalf)
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// Where a wave's next 16 rows are: index into the 64 pages held and token slot in that page.
+struct StageCursor {
+  uint32_t page, slot;
 };
 
-__device__ inline void stage_tile(const FastRagged &p, SharedTiles &lds, uint32_t buffer,
-                                  uint32_t tile0, uint32_t end, uint32_t page0, uint32_t physical,
-                                  uint32_t kv_head, uint32_t wave, uint32_t lane) {
-  const uint32_t pt = p.page_tokens;
-  constexpr int kPerWave = kTile / 4 / kSharedWaves;   // instructions per wave and operand
+// Moves this wave's 16 rows of K and V of the tile at `tile0` into LDS.  Rows from `end` on are taken from
+// a valid row.
+__device__ inline void stage_tile(const FastRagged &p, uint32_t tile, uint32_t tile0, uint32_t end,
+                                  const StageCursor &at, uint32_t physical, const uint32_t (&offset_k)[4],
+                                  const uint32_t (&offset_v)[4], uint32_t kv_head, uint32_t wave,
+                                  uint32_t lane) {
+  const uint32_t block = tile0 + 16 * wave, row_elems = p.kv_heads * 128;
+  const uint32_t page = __builtin_amdgcn_readlane(physical, at.page);
+  const uint64_t base = ((uint64_t)page * p.page_tokens + at.slot) * row_elems + kv_head * 128;
+  const uint16_t *k_base = p.key_pool + base, *v_base = p.value_pool + base;
+  const uint32_t to = tile + 16 * kPrefillRow * wave;
+  if (block + 16 <= end) {
 #pragma unroll
-  for (int j = 0; j < kPerWave; ++j) {
-    const uint32_t row = 4 * kPerWave * wave + 4 * j + (lane >> 4);
-    const uint32_t token = min(tile0 + row, end - 1);
-    const uint32_t page = (uint32_t)__shfl((int)physical, (int)(token / pt - page0), 64);
-    const uint64_t element = (((uint64_t)page * pt + token % pt) * p.kv_heads + kv_head) * 128 +
-                             8 * ((lane & 15) ^ (row & 15));
-    __builtin_amdgcn_global_load_lds(
-        (const __attribute__((address_space(1))) void *)(p.key_pool + element),
-        (__attribute__((address_space(3))) void *)&lds.rows[buffer][0][4 * kPerWave * wave + 4 * j][0], 16, 0, 0);
-    __builtin_amdgcn_global_load_lds(
-        (const __attribute__((address_space(1))) void *)(p.value_pool + element),
-        (__attribute__((address_space(3))) void *)&lds.rows[buffer][1][4 * kPerWave * wave + 4 * j][0], 16, 0, 0);
+    for (int j = 0; j < 4; ++j) {
+      load_to_lds_16_at(k_base + offset_k[j], to + 4 * kPrefillRow * j);
+      load_to_lds_16_at(v_base + offset_v[j], to + kPrefillValues + 4 * kPrefillRow * j);
+    }
+  } else {
+    const uint32_t last = block < end ? end - 1 - block : 0;   // past the end: the cursor stayed behind
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t row = 4 * j + (lane >> 4), back = (row - min(row, last)) * row_elems;
+      load_to_lds_16_at(k_base + (offset_k[j] - back), to + 4 * kPrefillRow * j);
+      load_to_lds_16_at(v_base + (offset_v[j] - back), to + kPrefillValues + 4 * kPrefillRow * j);
+    }
   }
 }
 
-// The register image load_tile would have produced, read from the staged tile.
-__device__ inline void read_tile(const SharedTiles &lds, uint32_t buffer, TileRegs &r, uint32_t hl,
-                                 uint32_t g) {
+// Scores, online softmax and the value product of one tile for a wave's 32 query rows; this lane holds
+// row (lane & 31) and, of each 8 keys, the four of its half.  `limit` is the first key the row may not
+// attend (0: unused row), `wave_end` the first none of the wave's rows may; `masked` false: every key of
+// the tile is below every limit.  k_at / v_at: byte offsets of the lane's operand pieces in a tile.
+// scale_log2 is positive.
+template <bool kHalf>
+__device__ inline void attend_tile(uint32_t tile, const uint4 (&q)[8], f32x16 (&o)[4], Softmax &sm,
+                                   bool masked, uint32_t tile0, uint32_t limit, uint32_t wave_end, float scale_log2,
+                                   uint32_t k_at, uint32_t v_at, uint32_t half) {
+  f32x16 s[2];
 #pragma unroll
-  for (int sub = 0; sub < 2; ++sub) {
-    const uint32_t k_row = 16 * sub + hl;
+  for (int b = 0; b < 2; ++b)
+    for (int i = 0; i < 16; ++i) s[b][i] = 0.0f;
+  // operands four steps ahead of their products
+  uint4 keys[4][2];
+  auto read_keys = [&](int step) {
 #pragma unroll
-    for (int step = 0; step < 4; ++step) r.k[sub][step] = lds.rows[buffer][0][k_row][(4 * step + g) ^ hl];
+    for (int b = 0; b < 2; ++b)
+      keys[step & 3][b] =
+          __builtin_bit_cast(uint4, *(LdsWords)(tile + (k_at ^ (32 * step)) + 32 * kPrefillRow * b));
+  };
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t v_row = 16 * sub + 4 * g + i;
-      r.v[4 * sub + i] = lds.rows[buffer][1][v_row][hl ^ (v_row & 15)];
-    }
+  for (int step = 0; step < 4; ++step) read_keys(step);
+#pragma unroll
+  for (int step = 0; step < 8; ++step) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) s[b] = mfma_32x32x16<kHalf>(keys[step & 3][b], q[step], s[b]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (step < 4) read_keys(step + 4);
   }
+  // (Steps past wave_end have zero weights; what they multiply is read again from the step before it: a V
+  // row that no row of the wave attends may hold a NaN.)
+  const uint32_t last_step = min(wave_end - 1 - tile0, kPrefillTile - 1) / 16;
+  auto read_values = [&](uint32_t step, int c) {
+    const uint32_t from = tile + kPrefillValues + 16 * kPrefillRow * min(step, last_step);
+    const s16x4 low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsPiece)(from + (v_at ^ (64 * c))));
+    const s16x4 high =
+        __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsPiece)(from + 8 * kPrefillRow + (v_at ^ (64 * c) ^ 32)));
+    const uint2 low_words = __builtin_bit_cast(uint2, low), high_words = __builtin_bit_cast(uint2, high);
+    return make_uint4(low_words.x, low_words.y, high_words.x, high_words.y);
+  };
+  uint4 values[4];   // operands four products ahead
+#pragma unroll
+  for (int c = 0; c < 4; ++c) values[c] = read_values(0, c);
+  __builtin_amdgcn_sched_barrier(0);
+  if (masked) {
+    const uint32_t below = limit > tile0 + 4 * half ? limit - tile0 - 4 * half : 0;
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+      for (int i = 0; i < 16; ++i)
+        if (32 * b + 8 * (i >> 2) + (i & 3) >= below) s[b][i] = -__builtin_inff();
+  }
+  float tile_max = s[0][0];
+#pragma unroll
+  for (int i = 1; i < 32; ++i) tile_max = fmaxf(tile_max, s[i >> 4][i & 15]);
+  tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, 64)) * scale_log2;
+  // The running maximum may lag behind by 2^kLag: the weights stay exact multiples of what they would
+  // be, and the rescale of the 64 sums per lane is seldom needed.
+  constexpr float kLag = 6.0f;
+  if (__any(tile_max > sm.m + kLag)) {
+    const float m_new = fmaxf(sm.m, tile_max);
+    const float alpha = m_new == -__builtin_inff() ? 1.0f : __builtin_amdgcn_exp2f(sm.m - m_new);
+    sm.l *= alpha;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      for (int i = 0; i < 16; ++i) o[c][i] *= alpha;
+    sm.m = m_new;
+  }
+  // a row with nothing to attend yet keeps m = -inf; subtract 0 instead so that exp2(-inf) = 0
+  const float m_safe = sm.m == -__builtin_inff() ? 0.0f : sm.m;
+  float sum[2] = {0.0f, 0.0f};
+  uint4 weights[4];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    uint32_t words[8];
+#pragma unroll
+    for (int i = 0; i < 16; i += 2) {
+      const float x = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][i], scale_log2, -m_safe));
+      const float y = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][i + 1], scale_log2, -m_safe));
+      sum[0] += x;
+      sum[1] += y;
+      words[i / 2] = pack_operand<kHalf>(x, y);
+    }
+    weights[2 * b] = make_uint4(words[0], words[1], words[2], words[3]);
+    weights[2 * b + 1] = make_uint4(words[4], words[5], words[6], words[7]);
+  }
+  sm.l += sum[0] + sum[1];
+  // O^T += V^T . P^T, 16 keys a step in the order the scores left them: half h takes keys 4h..4h+3 and
+  // 8 + 4h..8 + 4h + 3 of the 16.
+#pragma unroll
+  for (int step = 0; step < 4; ++step)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      o[c] = mfma_32x32x16<kHalf>(values[c], weights[step], o[c]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (step < 3) values[c] = read_values(step + 1, c);
+    }
 }
 
 template <bool kHalf, bool kMixed>
-__global__ __launch_bounds__(64 * kSharedWaves) __attribute__((amdgpu_waves_per_eu(3, 3))) void ragged_attention_prefill_kernel(
-    FastRagged p, ErrorSlot *error) {
-  constexpr int NT = kSharedTiles;
-  __shared__ SharedTiles lds;
-  const uint32_t lane = threadIdx.x & 63, hl = lane & 15, g = lane >> 4;
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t item = blockIdx.x, kv_head = blockIdx.y;
-  if (item >= p.item_count[0]) return;
+__device__ inline void attend_item(const FastRagged &p, ErrorSlot *error, uint32_t tiles, uint32_t item,
+                                   uint32_t kv_head) {
+  uint32_t lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));   // what follows from it is not kept in registers from item to item
+  const uint32_t half = lane >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint2 work = p.items[item];
   const uint32_t leader = work.x, split = work.y;
   const TokenPlan plan = p.plans[leader];
-  const uint32_t per_tile = 16 / p.group, per_wave = NT * per_tile;
-  const uint32_t first = wave * per_wave;                       // this wave's first member
-  const uint32_t members = plan.members > first ? min(plan.members - first, per_wave) : 0;
-  // the item's split layout is sized for its last member; a wave stops at its own last member
+  // the item's split layout is sized for its last member
   const uint32_t longest = p.fixed_attended ? plan.attended : plan.attended + plan.members - 1;
   const uint32_t begin = split * plan.chunk;
   const uint32_t end = min(longest, begin + plan.chunk);
-  const uint32_t own_end =
-      members == 0 ? begin : min(end, p.fixed_attended ? plan.attended : plan.attended + first + members - 1);
   const uint32_t pt = p.page_tokens;
   const uint32_t *table = p.tables + (uint64_t)plan.lane * p.table_pages * 2;
 
-  uint4 q_reg[NT][4];
-  uint32_t limit[NT], member_of[NT];
-  const uint32_t head = kv_head * p.group + hl % p.group;
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    member_of[nt] = first + nt * per_tile + hl / p.group;
-    const bool used = hl < per_tile * p.group && member_of[nt] < plan.members;
-    limit[nt] = !used ? 0 : min(end, p.fixed_attended ? plan.attended : plan.attended + member_of[nt]);
-    const uint64_t q_row = (uint64_t)(leader + (used ? member_of[nt] : 0)) * p.q_stride_t +
-                           (uint64_t)head * p.q_stride_h;
-    for (int step = 0; step < 4; ++step) {
-      q_reg[nt][step] = make_uint4(0, 0, 0, 0);
-      if (used) q_reg[nt][step] = load_query<kHalf, kMixed>(p, q_row + 32 * step + 8 * g);
-    }
-    if (!used) member_of[nt] = 0xffffffffu;
+  // This lane's query row, and the keys of this wave's rows: none at or past wave_end, all below plain_end.
+  const uint32_t rows = plan.members * p.group, row = 32 * wave + (lane & 31);
+  const bool used = row < rows;
+  const uint32_t member = used ? row / p.group : 0, head = kv_head * p.group + (used ? row % p.group : 0);
+  const uint32_t own_limit = !used ? 0 : min(end, p.fixed_attended ? plan.attended : plan.attended + member);
+  uint32_t wave_end = begin, plain_end = begin;
+  if (32 * wave < rows) {
+    const uint32_t last = (min(32 * wave + 32, rows) - 1) / p.group, first = 32 * wave / p.group;
+    wave_end = min(end, p.fixed_attended ? plan.attended : plan.attended + last);
+    plain_end = min(end, p.fixed_attended ? plan.attended : plan.attended + first);
   }
-  // keys below `unmasked_end` are attended by every used row of this wave
-  const uint32_t unmasked_end = min(own_end, p.fixed_attended ? plan.attended : plan.attended + first);
-  f32x4 o[NT][8];
-  Softmax sm[NT];
+  const float scale_log2 = p.scale_log2 == 0.0f ? 1.0f : fabsf(p.scale_log2);
+  // (An unused row takes the item's first: its keys are all masked and nothing of it is stored.)
+  const uint64_t q_row = (uint64_t)(leader + member) * p.q_stride_t + (uint64_t)head * p.q_stride_h + 8 * half;
+  uint4 q[8];
+  if (!kMixed || p.q_dtype != FH_F32) {
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    for (int mt = 0; mt < 8; ++mt) o[nt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    sm[nt] = Softmax{-__builtin_inff(), 0.0f};
+    for (int step = 0; step < 8; ++step) q[step] = load_query<kHalf, false>(p, q_row + 16 * step);
+  } else {
+#pragma unroll
+    for (int step = 0; step < 8; ++step) q[step] = load_query<kHalf, true>(p, q_row + 16 * step);
   }
+  if (!(p.scale_log2 > 0.0f)) {
+    // A negative scale goes into the queries' signs, a zero one into their values: the largest product is
+    // then the largest score, and a masked one stays -inf.
+    const uint32_t flip = p.scale_log2 < 0.0f ? 0x80008000u : 0, keep = p.scale_log2 == 0.0f ? 0 : 0xffffffffu;
+#pragma unroll
+    for (int step = 0; step < 8; ++step)
+      q[step] = make_uint4((q[step].x ^ flip) & keep, (q[step].y ^ flip) & keep, (q[step].z ^ flip) & keep,
+                           (q[step].w ^ flip) & keep);
+  }
+  f32x16 o[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    for (int i = 0; i < 16; ++i) o[c][i] = 0.0f;
+  Softmax sm{-__builtin_inff(), 0.0f};
+
+  const uint32_t row_elems = p.kv_heads * 128;
+  uint32_t offset_k[4], offset_v[4];   // elements from a wave's first row of a tile to what this lane moves
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t r = 4 * j + (lane >> 4);
+    offset_k[j] = r * row_elems + 8 * ((lane & 15) ^ r);
+    offset_v[j] = r * row_elems + 8 * ((lane & 15) ^ ((r & 3) << 2 | r >> 2));
+  }
+  const uint32_t k_row = lane & 31, v_row = (lane & 15) >> 2;   // v_row: of the four that a read transposes
+  const uint32_t k_at = 256 * k_row + 16 * (half ^ (k_row & 15));
+  const uint32_t v_at = 256 * (4 * half + v_row) + 8 * (lane & 1) +
+                        16 * ((2 * (lane >> 4 & 1) + (lane >> 1 & 1)) ^ v_row << 2 ^ half);
 
   const uint32_t first_page = begin / pt, last_page = (end - 1) / pt;
   for (uint32_t page0 = first_page; page0 <= last_page; page0 += 64) {
@@ -1049,65 +1128,87 @@ __global__ __launch_bounds__(64 * kSharedWaves) __attribute__((amdgpu_waves_per_
     if (bad_mask) {
       if (wave == 0 && lane == (uint32_t)__ffsll((long long)bad_mask) - 1) {
         report_error(error + (uint64_t)leader * p.error_stride, my_page);
-        for (uint32_t member = 0; member < plan.members; ++member) p.bad[leader + member] = 1;
+        for (uint32_t m = 0; m < plan.members; ++m) p.bad[leader + m] = 1;
       }
-      if (plan.splits == 1) zero_head_rows<kMixed>(p, leader + first, members, kv_head, lane);
+      if (plan.splits == 1 && wave == 0) zero_head_rows<kMixed>(p, leader, plan.members, kv_head, lane);
       return;
     }
     const uint32_t tok_lo = max(begin, page0 * pt);
     const uint32_t tok_hi = (uint32_t)min((uint64_t)end, ((uint64_t)page0 + 64) * pt);
-    stage_tile(p, lds, 0, tok_lo, end, page0, physical, kv_head, wave, lane);
+    const uint32_t limit = min(own_limit, tok_hi), group_end = min(wave_end, tok_hi);
+    const uint32_t start = min(tok_lo + 16 * wave, (tok_hi - 1) & ~15u);
+    StageCursor at{start / pt - page0, start % pt};
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the queries are here, only the tiles' loads are waited for below
+    stage_tile(p, tiles, tok_lo, tok_hi, at, physical, offset_k, offset_v, kv_head, wave, lane);
     uint32_t buffer = 0;
-    for (uint32_t tile0 = tok_lo; tile0 < tok_hi; tile0 += kTile, buffer ^= 1) {
+    for (uint32_t tile0 = tok_lo; tile0 < tok_hi; tile0 += kPrefillTile, buffer ^= kPrefillTileBytes) {
       __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): this wave's share of the tile has landed
       __syncthreads();                      // everybody's has, and the other buffer is free
-      if (tile0 + kTile < tok_hi)
-        stage_tile(p, lds, buffer ^ 1, tile0 + kTile, end, page0, physical, kv_head, wave, lane);
-      if (tile0 < own_end) {
-        TileRegs cur;
-        read_tile(lds, buffer, cur, hl, g);
-        if (tile0 + kTile <= unmasked_end)
-          consume_tile<NT, false, kHalf>(cur, q_reg, o, sm, tile0, limit, p.scale_log2, g);
-        else
-          consume_tile<NT, true, kHalf>(cur, q_reg, o, sm, tile0, limit, p.scale_log2, g);
+      const uint32_t next0 = tile0 + kPrefillTile;
+      if (next0 < tok_hi) {
+        if (next0 + 16 * wave < tok_hi) {
+          at.slot += kPrefillTile;
+          while (at.slot >= pt) {
+            at.slot -= pt;
+            ++at.page;
+          }
+        }
+        stage_tile(p, tiles + kPrefillTileBytes - buffer, next0, tok_hi, at, physical, offset_k, offset_v, kv_head, wave, lane);
       }
+      if (tile0 < group_end)
+        attend_tile<kHalf>(tiles + buffer, q, o, sm, next0 > min(plain_end, tok_hi), tile0, limit, group_end,
+                           scale_log2, k_at, v_at, half);
     }
-    __builtin_amdgcn_s_waitcnt(0x0f70);
-    __syncthreads();   // the next group's first tile goes into buffer 0
+    __syncthreads();   // the next tile staged goes into the first buffer
   }
+  sm.l += __shfl_xor(sm.l, 32, 64);
+  if (!used) return;
+  const uint32_t token = leader + member;
+  // This lane holds value columns 32c + 8n + 4 * half + 0..3 of its row in o[c][4n..4n + 3].
+  if (plan.splits == 1) {
+    const float inv = 1.0f / sm.l;
+    const uint64_t out_row = (uint64_t)token * p.out_stride_t + (uint64_t)head * p.out_stride_h + 4 * half;
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    float m_run = sm[nt].m, l_run = sm[nt].l;
-    l_run += __shfl_xor(l_run, 16, 64);
-    l_run += __shfl_xor(l_run, 32, 64);
-    if (member_of[nt] == 0xffffffffu) continue;
-    const uint32_t token = leader + member_of[nt];
-    if (plan.splits == 1) {
-      float inv = 1.0f / l_run;
-      const uint64_t out_row = (uint64_t)token * p.out_stride_t + (uint64_t)head * p.out_stride_h;
-      for (int j = 0; j < 4; ++j) {
-        store_out4<kHalf, kMixed>(p, out_row + 32 * g + 8 * j, o[nt][0][j] * inv, o[nt][1][j] * inv,
-                   o[nt][2][j] * inv, o[nt][3][j] * inv);
-        store_out4<kHalf, kMixed>(p, out_row + 32 * g + 8 * j + 4, o[nt][4][j] * inv, o[nt][5][j] * inv,
-                   o[nt][6][j] * inv, o[nt][7][j] * inv);
-      }
-      continue;
-    }
-    uint64_t slot = ((uint64_t)token * p.max_splits + split) * p.query_heads + head;
-    float *po = p.partial_o + slot * 128 + 32 * g;
-    for (int j = 0; j < 4; ++j) {
-      *(float4 *)(po + 8 * j) = make_float4(o[nt][0][j], o[nt][1][j], o[nt][2][j], o[nt][3][j]);
-      *(float4 *)(po + 8 * j + 4) = make_float4(o[nt][4][j], o[nt][5][j], o[nt][6][j], o[nt][7][j]);
-    }
-    if (g == 0) p.partial_ml[slot] = make_float2(m_run, l_run);
+    for (int c = 0; c < 4; ++c)
+      for (int n = 0; n < 4; ++n)
+        store_out4<kHalf, kMixed>(p, out_row + 32 * c + 8 * n, o[c][4 * n] * inv, o[c][4 * n + 1] * inv,
+                                  o[c][4 * n + 2] * inv, o[c][4 * n + 3] * inv);
+    return;
   }
+  const uint64_t slot = ((uint64_t)token * p.max_splits + split) * p.query_heads + head;
+  float *po = p.partial_o + slot * 128 + 4 * half;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    for (int n = 0; n < 4; ++n)
+      *(float4 *)(po + 32 * c + 8 * n) =
+          make_float4(o[c][4 * n], o[c][4 * n + 1], o[c][4 * n + 2], o[c][4 * n + 3]);
+  if (half == 0) p.partial_ml[slot] = make_float2(sm.m, sm.l);
+}
+
+// Items longest first, the kv heads of an item side by side: with 8 (or 4, 2, 1) kv heads a head's items
+// meet in the L2 of one XCD, as workgroups go to the XCDs in turn, and the launch ends on its shortest.
+// (8192 prompt rows in six chunks and 64 decode rows, 8 kv heads: 241 us, and 447 us where workgroups
+// take the next entry wherever they are.)
+template <bool kHalf, bool kMixed>
+__global__ __launch_bounds__(64 * kPrefillWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void ragged_attention_prefill_kernel(
+    FastRagged p, ErrorSlot *error) {
+  __shared__ uint4 tiles[2 * kPrefillTileBytes / 16];
+  const uint32_t listed = p.item_count[0] * p.kv_heads;
+  for (uint32_t entry = blockIdx.x; entry < listed; entry += gridDim.x)
+    attend_item<kHalf, kMixed>(p, error, lds_address(tiles), entry / p.kv_heads, entry % p.kv_heads);
 }
 
 // Decode batches: one query token per wave, two waves per SIMD to hide the K/V stream's latency.
 template <bool kHalf, bool kMixed>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void ragged_attention_mfma_kernel(
     FastRagged p, ErrorSlot *error) {
-  ragged_attention_body<1, kHalf, kMixed>(p, error);
+  // a workgroup is one work item; its waves take one kv head each, so the slices of a K/V page
+  // (one 256-byte piece of every token row per kv head) are requested close together in time
+  const uint32_t kv_head = blockIdx.y * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const uint32_t items = p.item_count[0];
+  if (kv_head >= p.kv_heads) return;
+  for (uint32_t item = blockIdx.x; item < items; item += gridDim.x)
+    attend_one_token<kHalf, kMixed>(p, error, item, kv_head);
 }
 
 // Merges the per-split partials of one (token, head): out = sum_s O_s 2^(m_s-M) / sum_s l_s
@@ -1324,22 +1425,25 @@ uint32_t decode_item_slots(fh_backend *backend, const FastRagged &f) {
 }
 
 void launch_fast(fh_backend *backend, hipStream_t stream, const FastRagged &f, ErrorSlot *error) {
-  uint64_t groups = f.group_tokens > 1 ? f.tokens / f.group_tokens + f.lanes : f.tokens;
-  uint64_t blocks = groups * f.max_splits;
+  const uint64_t groups = f.group_tokens > 1 ? f.tokens / f.group_tokens + f.lanes : f.tokens;
+  const uint64_t items = groups * f.max_splits;   // at most
   const bool mixed = mixed_dtypes(f);
   {
     KernelTimer timer(backend, FH_KC_ATTENTION_KERNEL);
     // one workgroup per work item, up to 8 (decode) or 4 (prefill) kv heads of it per workgroup
     if (f.group_tokens > 1) {
-      const dim3 grid((unsigned)blocks, f.kv_heads);
+      const uint64_t most = (uint64_t)kPrefillGrid * backend_compute_units(backend);
+      const dim3 grid((unsigned)std::min(items * f.kv_heads, most));
       auto *kernel = f.pool_half ? (mixed ? ragged_attention_prefill_kernel<true, true>
                                           : ragged_attention_prefill_kernel<true, false>)
                                  : (mixed ? ragged_attention_prefill_kernel<false, true>
                                           : ragged_attention_prefill_kernel<false, false>);
-      kernel<<<grid, 64 * kSharedWaves, 0, stream>>>(f, error);
+      kernel<<<grid, 64 * kPrefillWaves, 0, stream>>>(f, error);
     } else {
       const uint32_t waves = decode_waves(f);
-      const dim3 grid((unsigned)blocks, (f.kv_heads + waves - 1) / waves);
+      // The items mostly fill the device's places once (see the plan); what is left they walk on.  An
+      // empty workgroup costs its place about 1 us.
+      const dim3 grid((unsigned)std::min<uint64_t>(items, 2 * (uint64_t)f.item_slots), (f.kv_heads + waves - 1) / waves);
       decode_kernel(f)<<<grid, 64 * waves, 0, stream>>>(f, error);
     }
   }
@@ -1368,7 +1472,7 @@ bool try_fast_lane_attention(fh_backend *backend, const LaneAttention &lane, Err
   f.table_pages = lane.logical_pages;
   f.max_splits = splits_for(f.tokens);
   fit_splits(backend, &f, true);
-  f.group_tokens = f.tokens > 1 ? kSharedWaves * kSharedTiles * (16 / group) : 1;
+  f.group_tokens = f.tokens > 1 ? kPrefillRows / group : 1;
   f.scale_log2 = lane.scale * 1.4426950408889634f;
   f.one_start = lane.query_start;
   f.fixed_attended = lane.causal ? 0 : lane.key_length;
@@ -1409,7 +1513,7 @@ bool run_ragged_attention(fh_backend *backend, const RaggedAttention &p, ErrorSl
     f.query_heads = p.query_heads;
     f.kv_heads = p.kv_heads;
     f.group = p.query_heads / p.kv_heads;
-    f.group_tokens = p.tokens > p.lanes ? kSharedWaves * kSharedTiles * (16 / f.group) : 1;
+    f.group_tokens = p.tokens > p.lanes ? kPrefillRows / f.group : 1;
     f.page_tokens = p.page_tokens;
     f.physical_pages = p.physical_pages;
     f.table_pages = p.table_pages;

@@ -470,20 +470,6 @@ __global__ __launch_bounds__(256) void gemm_f16_kernel(GemmArgs a) {
   store_tile<kQ, kQ, 2>(a, acc, gemm_lds, row0, col0);
 }
 
-
-// 64 lanes x 16 bytes from memory straight into LDS at `lds_base` + 16 * lane, issued as an
-// instruction the compiler does not see: while it knows of such a load in flight it waits for ALL
-// outstanding LDS reads wherever it has to wait for one (it cannot tell the load's LDS write from
-// the wave's own LDS traffic), i.e. also for the operand reads just issued for the next sub-step,
-// and it drains every such load at a __syncthreads().  Callers order these loads by hand (vmcnt).
-__device__ inline void load_to_lds_16(const void *from, unsigned char *lds_base) {
-  // (uniform by construction; the intrinsic tells the compiler so)
-  const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds_base);
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(at) : "memory");   // (m0 is the compiler's only for its own such loads: kernels that use this have none)
-}
-
-__device__ inline void lds_barrier() { asm volatile("s_barrier" ::: "memory"); }
-
 // The same GEMM with eight waves to a 256 x 256 tile (two per SIMD), each owning 128 rows x 64
 // columns (128 accumulator registers): while one wave of a SIMD waits for its operands or at the
 // barrier the other one feeds the matrix pipe.

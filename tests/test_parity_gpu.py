@@ -1399,6 +1399,43 @@ def test_decode_rows_beside_prefill_groups_that_fill_the_device(cpu, hip, contex
     assert cpu.read(cpu_out[1]) == hip.read(hip_out[1]) and cpu.read(cpu_out[2]) == hip.read(hip_out[2])
 
 
+@pytest.mark.parametrize("contexts,counts,hq,hkv,pt,scale", [
+    # groups of 128 query rows, waves of 32, tiles of 64 keys: one row less, the edge, one more
+    ([0, 1, 63, 64], [63, 64, 65, 2], 16, 8, 16, 0.09),      # 64 tokens to a group
+    ([31, 0, 960], [25, 26, 51], 40, 8, 16, 0.09),           # 25 tokens, rows that share a wave unevenly
+    ([0, 32], [17, 130], 24, 3, 48, -0.09),                  # three kv heads, a negative scale
+    ([5], [130], 4, 4, 16, 0.0),                             # 128 tokens to a group, every key alike
+    ([1100, 2048, 3070], [70, 3, 2], 32, 2, 16, 0.09),       # page numbers in rounds of 64, two splits
+    ([3071, 3100], [40, 9], 16, 8, 48, 0.09)])
+def test_prefill_attention_at_the_edges_of_its_tiles(cpu, hip, contexts, counts, hq, hkv, pt, scale):
+    def build(backend):
+        t, inputs = ragged_case(backend, contexts, counts, hq, hkv, pt, seed=63)
+        commands = CommandList()
+        commands.dispatch_many(Op.paged_attention_ragged(scale, pt), inputs, [t["out"], t["keys"], t["values"]])
+        return commands, [t["out"], t["keys"], t["values"]]
+    (cpu_out, _), (hip_out, _) = differential(cpu, hip, build)
+    assert cpu.read(cpu_out[1]) == hip.read(hip_out[1]) and cpu.read(cpu_out[2]) == hip.read(hip_out[2])
+
+
+def test_a_value_without_a_number_reaches_later_rows_only(cpu, hip):
+    """Token 69 of a chunk stores a value row of NaNs: rows whose 16-key blocks end before it (here: the
+    first 64 tokens, four waves of a group) do not meet it."""
+    def build(backend):
+        t, inputs = ragged_case(backend, [0], [70], 16, 8, 16, seed=64)
+        values = normal_bf16(64, 5, (70, 8, 128)).astype(np.float32)
+        values[69] = np.nan
+        inputs[2] = upload(backend, values, DType.BF16)
+        commands = CommandList()
+        commands.dispatch_many(Op.paged_attention_ragged(0.09, 16), inputs, [t["out"], t["keys"], t["values"]])
+        backend.submit(commands).wait()
+        return to_f32(backend.read(t["out"]), DType.BF16).reshape(70, 16, 128)
+    want, got = build(cpu), build(hip)
+    assert np.isfinite(want[:69]).all() and np.isnan(want[69]).all()
+    # both round a sum of at most 70 weighted values to bf16; weights are rounded to bf16 on the device
+    assert np.abs(got[:64] - want[:64]).max() <= 2.0 ** -7 * np.abs(want[:64]).max()
+    assert np.isnan(got[69]).all()
+
+
 DTYPE_MIXES = [
     # query and new rows, pools, output
     (DType.F32, DType.F16, DType.F32),      # the qwen3-coder engine
