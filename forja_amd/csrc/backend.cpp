@@ -1888,21 +1888,38 @@ fh_status run_lane_group(fh_backend *b, const LaneRun &run, ErrorSlot *errors, b
   problem.attention_error_offset = head.attention_at;
   problem.one_row_per_lane = 1;   // by construction: every member is one query row of its own lane
   problem.row_twice = lanes == 1 ? cu + lanes + 1 : nullptr;
-  if (!run_ragged_attention(b, problem, errors)) return FH_ALLOCATION_FAILED;
-
-  for (uint32_t base = 0; base < lanes; base += kLaneChunk) {
-    uint32_t chunk = std::min<uint32_t>(kLaneChunk, lanes - base);
-    LaneRows targets{};
+  // Where the members' rows go, a chunk of lanes at a time.
+  auto targets_of = [&](uint32_t base, uint32_t chunk, LaneRows *targets) -> fh_status {
     for (uint32_t local = 0; local < chunk; ++local) {
       const LaneMember &m = run.members[base + local];
       View row;
       if ((status = make_view(b, m.out, true, &row)) != FH_OK) return status;
-      targets.first[local] = row.base + row.offset * dtype_size(row.dtype);
+      targets->first[local] = row.base + row.offset * dtype_size(row.dtype);
       if (m.has_copy) {
         if ((status = make_view(b, m.copy_target, true, &row)) != FH_OK) return status;
-        targets.second[local] = row.base + row.offset * dtype_size(row.dtype);
+        targets->second[local] = row.base + row.offset * dtype_size(row.dtype);
       }
     }
+    return FH_OK;
+  };
+  LaneRows targets{};
+  bool placed = false;
+  if (lanes <= kLaneChunk) {
+    if ((status = targets_of(0, lanes, &targets)) != FH_OK) return status;
+    const uint64_t four = 4 * dtype_size(out0.dtype);
+    bool aligned = true;
+    for (uint32_t lane = 0; lane < lanes; ++lane)
+      aligned = aligned && (uint64_t)targets.first[lane] % four == 0 && (uint64_t)targets.second[lane] % four == 0;
+    if (aligned) {
+      problem.lane_rows = &targets;
+      problem.rows_placed = &placed;
+    }
+  }
+  if (!run_ragged_attention(b, problem, errors)) return FH_ALLOCATION_FAILED;
+  for (uint32_t base = 0; base < lanes && !placed; base += kLaneChunk) {
+    const uint32_t chunk = std::min<uint32_t>(kLaneChunk, lanes - base);
+    targets = LaneRows{};
+    if ((status = targets_of(base, chunk, &targets)) != FH_OK) return status;
     launch_scatter_lane_rows(b->stream, targets, rows, base, chunk, (uint32_t)row_bytes);
   }
   b->fused_runs += 1;

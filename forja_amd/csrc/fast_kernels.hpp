@@ -267,6 +267,11 @@ struct RaggedAttention {
   // Null, or (one lane, whose table nothing has checked) a device word: non-zero where the table names the
   // page of the new row at an earlier position too, so that the row is to be stored before anything is read.
   const uint32_t *row_twice;
+  // Null, or where each token's attended rows go ([query_heads, value_width], dense, of the output's dtype,
+  // aligned to four elements), instead of `out`; one_row_per_lane, at most kLaneChunk tokens.  Done only
+  // where a merge kernel runs anyway: `*rows_placed` says so, and if not, the rows are in `out`.
+  const LaneRows *lane_rows;
+  bool *rows_placed;
 };
 // Always handles the problem (specialised kernel when the layout allows, generic otherwise);
 // false only when workspace allocation fails.

@@ -6,6 +6,7 @@
 // (physical page, generation) and is valid iff page < P and generations[page] == generation.
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 #include "fast_kernels.hpp"
 
@@ -330,6 +331,7 @@ struct FastRagged {
   // before it reads: the split that meets it at the other position sees it, as after an append of its own.
   const uint32_t *row_twice;
   uint32_t promised;   // one query row per lane, vouched for by the caller: verified by the plan
+  uint32_t merge_all;  // every token goes through the merge, one of a single split too
 };
 
 // Splits of a group whose longest member attends `longest` (> 0) keys: as few as keep each within
@@ -582,7 +584,7 @@ __global__ __launch_bounds__(kPlanThreads) void ragged_plan_kernel(FastRagged p,
     p.plans[token] = plan;
     if (plan.leader == token && plan.splits) atomicAdd(&class_items[class_of(plan)], plan.splits);
     // tokens with a single split are finished by the attention kernel itself
-    if (plan.splits != 1 || bad) p.merge_tokens[atomicAdd(&merge_count, 1u)] = token;
+    if (plan.splits != 1 || bad || p.merge_all) p.merge_tokens[atomicAdd(&merge_count, 1u)] = token;
   }
   __syncthreads();
   if (wave == 0) {   // class counts -> first item of each class, longest class first
@@ -655,19 +657,24 @@ __device__ inline uint4 load_query(const FastRagged &p, uint64_t element) {
 // kMixed false: queries and outputs are of the pools' dtype, known when the kernel is compiled
 // (the attention kernels have no registers to spare for the choice).
 template <bool kHalf, bool kMixed>
-__device__ inline void store_out4(const FastRagged &p, uint64_t element, float a, float b, float c,
+__device__ inline void store_four(void *out, uint32_t out_dtype, uint64_t element, float a, float b, float c,
                                   float d) {
   if (!kMixed) {
-    *(uint2 *)((uint16_t *)p.out + element) =
+    *(uint2 *)((uint16_t *)out + element) =
         make_uint2(pack_operand<kHalf>(a, b), pack_operand<kHalf>(c, d));
     return;
   }
-  if (p.out_dtype == FH_F32)
-    *(float4 *)((float *)p.out + element) = make_float4(a, b, c, d);
-  else if (p.out_dtype == FH_F16)
-    *(uint2 *)((uint16_t *)p.out + element) = make_uint2(pack_f16(a, b), pack_f16(c, d));
+  if (out_dtype == FH_F32)
+    *(float4 *)((float *)out + element) = make_float4(a, b, c, d);
+  else if (out_dtype == FH_F16)
+    *(uint2 *)((uint16_t *)out + element) = make_uint2(pack_f16(a, b), pack_f16(c, d));
   else
-    *(uint2 *)((uint16_t *)p.out + element) = make_uint2(pack_bf16(a, b), pack_bf16(c, d));
+    *(uint2 *)((uint16_t *)out + element) = make_uint2(pack_bf16(a, b), pack_bf16(c, d));
+}
+template <bool kHalf, bool kMixed>
+__device__ inline void store_out4(const FastRagged &p, uint64_t element, float a, float b, float c,
+                                  float d) {
+  store_four<kHalf, kMixed>(p.out, p.out_dtype, element, a, b, c, d);
 }
 
 __device__ inline uint32_t dword_of(const uint4 &v, int index) {
@@ -867,7 +874,7 @@ __device__ inline void attend_one_token(const FastRagged &p, ErrorSlot *error, u
         report_error(error + (uint64_t)leader * p.error_stride, my_page);
         p.bad[leader] = 1;
       }
-      if (plan.splits == 1) zero_head_rows<kMixed>(p, leader, 1, kv_head, lane);
+      if (plan.splits == 1 && !p.merge_all) zero_head_rows<kMixed>(p, leader, 1, kv_head, lane);
       return;
     }
     const uint32_t tok_lo = max(begin, page0 * pt);
@@ -899,7 +906,7 @@ __device__ inline void attend_one_token(const FastRagged &p, ErrorSlot *error, u
   sm.l += __shfl_xor(sm.l, 16, 64);
   sm.l += __shfl_xor(sm.l, 32, 64);
   if (hl >= p.group) return;
-  if (plan.splits == 1) {
+  if (plan.splits == 1 && !p.merge_all) {
     float inv = 1.0f / sm.l;
     const uint64_t out_row = (uint64_t)leader * p.out_stride_t + (uint64_t)head * p.out_stride_h;
     for (int j = 0; j < 4; ++j) {
@@ -1263,7 +1270,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // table was refused.  Four waves: every wave finds M and the weights from one (m, l) load per
 // lane (a token has at most 64 splits), then wave w folds splits 2w+half, 2w+half+8, ... of its
 // lanes' four columns, all loads in flight at once, and the waves' sums meet in LDS.
-__global__ __launch_bounds__(256) void ragged_reduce_kernel(FastRagged p) {
+// kPlaced: token t's rows go to targets.first[t] and, unless null, second[t] instead of `out`: the copies that a lane by
+// lane recording makes of every attended row cost a launch of 3.3 us (one lane) to 4.7 us (eight) of their own.
+struct InPlace {};   // nothing to pass: the rows go to `out`
+template <bool kPlaced>
+__global__ __launch_bounds__(256) void ragged_reduce_kernel(FastRagged p, std::conditional_t<kPlaced, LaneRows, InPlace> targets) {
   __shared__ float4 folded[3][32];
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t column = (lane & 31) * 4, half = lane >> 5;
@@ -1274,9 +1285,19 @@ __global__ __launch_bounds__(256) void ragged_reduce_kernel(FastRagged p) {
     const uint32_t token = p.merge_tokens[entry];
     const TokenPlan plan = p.plans[token];
     const bool zero = plan.splits == 0 || p.bad[token] != 0;
-    const uint64_t dst = (uint64_t)token * p.out_stride_t + (uint64_t)head * p.out_stride_h + column;
+    auto store = [&](float a, float b, float c, float d) {
+      if constexpr (kPlaced) {
+        const uint64_t element = (uint64_t)head * 128 + column;
+        store_four<false, true>(targets.first[token], p.out_dtype, element, a, b, c, d);
+        if (targets.second[token])
+          store_four<false, true>(targets.second[token], p.out_dtype, element, a, b, c, d);
+      } else {
+        store_out4<false, true>(p, (uint64_t)token * p.out_stride_t + (uint64_t)head * p.out_stride_h + column, a, b,
+                                c, d);
+      }
+    };
     if (zero) {
-      if (threadIdx.x < 32) store_out4<false, true>(p, dst, 0.0f, 0.0f, 0.0f, 0.0f);
+      if (threadIdx.x < 32) store(0.0f, 0.0f, 0.0f, 0.0f);
       continue;
     }
     const uint64_t base = (uint64_t)token * p.max_splits * p.query_heads + head;
@@ -1315,7 +1336,7 @@ __global__ __launch_bounds__(256) void ragged_reduce_kernel(FastRagged p) {
         acc.w += part.w;
       }
       const float inv = 1.0f / l_all;
-      store_out4<false, true>(p, dst, acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+      store(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
     }
   }
 }
@@ -1476,7 +1497,8 @@ uint32_t decode_item_slots(fh_backend *backend, const FastRagged &f) {
   return slots ? slots : 1;
 }
 
-void launch_fast(fh_backend *backend, hipStream_t stream, const FastRagged &f, ErrorSlot *error) {
+void launch_fast(fh_backend *backend, hipStream_t stream, const FastRagged &f, ErrorSlot *error,
+                 const LaneRows *placed = nullptr) {
   const uint64_t groups = f.group_tokens > 1 ? f.tokens / f.group_tokens + f.lanes : f.tokens;
   const uint64_t items = groups * f.max_splits;   // at most
   const bool mixed = mixed_dtypes(f);
@@ -1499,7 +1521,11 @@ void launch_fast(fh_backend *backend, hipStream_t stream, const FastRagged &f, E
       decode_kernel(f)<<<grid, 64 * waves, 0, stream>>>(f, error);
     }
   }
-  ragged_reduce_kernel<<<dim3(f.query_heads, f.tokens < 1024 ? f.tokens : 1024), 256, 0, stream>>>(f);
+  const dim3 merge(f.query_heads, f.tokens < 1024 ? f.tokens : 1024);
+  if (placed)
+    ragged_reduce_kernel<true><<<merge, 256, 0, stream>>>(f, *placed);
+  else
+    ragged_reduce_kernel<false><<<merge, 256, 0, stream>>>(f, InPlace{});
 }
 
 }  // namespace
@@ -1593,10 +1619,11 @@ bool run_ragged_attention(fh_backend *backend, const RaggedAttention &p, ErrorSl
     key.address[4] = (uint64_t)f.generations;
     f.promised = p.one_row_per_lane;
     f.append_in_kernel = p.one_row_per_lane && append_in_kernel_possible(p);
-    const uint32_t params[13] = {f.tokens, f.lanes, f.group_tokens, f.page_tokens, f.physical_pages,
+    f.merge_all = p.lane_rows != nullptr && f.append_in_kernel;
+    const uint32_t params[14] = {f.tokens, f.lanes, f.group_tokens, f.page_tokens, f.physical_pages,
                                  f.table_pages, f.max_splits, forced_split_tokens(), f.kv_heads,
-                                 f.query_heads, f.append_in_kernel, f.promised, f.item_slots};
-    for (int i = 0; i < 13; ++i) key.params[i] = params[i];
+                                 f.query_heads, f.append_in_kernel, f.promised, f.item_slots, f.merge_all};
+    for (int i = 0; i < 14; ++i) key.params[i] = params[i];
     bool reuse = false;
     char *plan_storage = backend_attention_plan(backend, key, plan_storage_bytes(f), &reuse);
     if (!plan_storage || !carve_partials(backend, &f, plan_storage)) return false;
@@ -1619,7 +1646,8 @@ bool run_ragged_attention(fh_backend *backend, const RaggedAttention &p, ErrorSl
     if (!reuse) launch_plan(stream, f, error);
   }
   if (fast && f.append_in_kernel) {
-    launch_fast(backend, stream, f, error);
+    launch_fast(backend, stream, f, error, f.merge_all ? p.lane_rows : nullptr);
+    if (f.merge_all) *p.rows_placed = true;
     return true;
   }
   // Whether cu_seqlens was refused: the work plan records it; without a plan a kernel of its own
