@@ -115,6 +115,33 @@ CASES = [
 ]
 
 
+@pytest.mark.parametrize("pad", [0, 2, 4])
+@pytest.mark.parametrize("contexts", [[0], [5, 40, 700, 31], [3 + lane % 29 for lane in range(128)]])
+def test_lane_rows_go_where_the_copies_put_them(cpu, hip, contexts, pad):
+    """Destinations whose rows are `pad` elements apart: aligned to four elements (0, 4) or not (2); lanes of
+    one split and of several; as many lanes as one launch takes."""
+    def build(backend):
+        batch = LaneBatch(backend, contexts, 8, 2, 16, seed=74)
+        width = batch.hq * WIDTH
+        placed = backend.alloc(DType.BF16, (batch.lanes, width + pad))
+        backend.write_array(placed, np.zeros(batch.lanes * (width + pad), np.uint16))
+        commands = CommandList()
+        rows = []
+        for lane in range(batch.lanes):
+            row = backend.alloc(DType.BF16, (1, batch.hq, WIDTH))
+            commands.dispatch_many(Op.paged_sdpa_append(0.09, contexts[lane], 16),
+                                   [batch.q.narrow(0, lane, 1).permute([1, 0, 2]), batch.k.narrow(0, lane, 1),
+                                    batch.v.narrow(0, lane, 1), batch.tables[lane], batch.generations],
+                                   [row.permute([1, 0, 2]), *batch.pools[0]])
+            commands.dispatch(Op.copy(), [row.reshape((1, width))], placed.narrow(0, lane, 1).narrow(1, 0, width))
+            rows.append(row)
+        run(backend, commands)
+        return [placed, *batch.pools[0], rows[0], rows[-1]]
+    before = hip.fusion_stats()
+    check(cpu, hip, build(cpu), build(hip), exact=(1, 2))
+    assert hip.fusion_stats() != before
+
+
 @pytest.mark.parametrize("idiom", ["append", "copies"])
 @pytest.mark.parametrize("contexts,hq,hkv,pt", CASES)
 def test_lane_by_lane_batch_equals_serial_execution(cpu, hip, contexts, hq, hkv, pt, idiom):
