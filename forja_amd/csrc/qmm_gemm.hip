@@ -127,65 +127,86 @@ __device__ inline void split_f16(float v, float *head, float *tail) {
 // brings its largest magnitude into [2^14, 2^15) (unscale[row] is the inverse); every 8 values are
 // stored in the order (0,4,1,5,2,6,3,7); after the inner values come, for every group g of 64,
 // (head, tail, head) of S_g / 64 with S_g the f32 sum of the group's scaled values, then zeros.
-// One wave per row.
+// What bounds it: the bytes where rows are many (2.05 times the activations), a chain of three round trips
+// where they are few.  A row is in the registers of its kThreads threads (kPieces of eight values each), all
+// loads at once: read a second time for the conversion it came from memory again (one wave a row holds no
+// long one), and a short row's chain was one trip longer.  (8256 x 17408 169 -> 100 us, x 5120 42 -> 29, 95 x 5120 9.3
+// -> 4.8, 2080 x 4096 12.8 -> 9.3, 2048 x 3072 8.5 -> 7.6, x 1024 and x 2048 6.3 and 6.5 as before.)
+template <int kThreads, int kPieces>
 __global__ __launch_bounds__(256) void prepare_rows_kernel(const uint16_t *x, uint64_t x_row_stride,
                                                            uint32_t rows, uint32_t inner, uint32_t kt,
                                                            uint16_t *out, float *unscale,
                                                            uint32_t *refused) {
-  __shared__ float sums[4][kMaxGroups];
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const uint32_t row = blockIdx.x * 4 + wave;
+  constexpr int kRows = 256 / kThreads;   // of a workgroup
+  constexpr int kRowGroups = kThreads * kPieces / 8;
+  __shared__ float sums[kRows][kRowGroups];
+  __shared__ uint32_t tops[4];
+  const uint32_t lane = threadIdx.x & 63, in_row = threadIdx.x % kThreads, local = threadIdx.x / kThreads;
+  const uint32_t wanted = blockIdx.x * kRows + local, row = min(wanted, rows - 1);
+  const bool live = wanted < rows;
   // the refusal flag of this product starts clear (prepare_weights_kernel, launched next, sets it)
   if (blockIdx.x == 0 && threadIdx.x == 0) refused[0] = 0;
-  if (row >= rows) return;   // no workgroup-wide barrier below
-  const uint16_t *in_row = x + (uint64_t)row * x_row_stride;
-  uint32_t top = 0;   // largest magnitude bits (bf16 without sign) in the row
-  for (uint32_t piece = lane; piece < inner / 8; piece += 64) {
-    const uint4 v = *(const uint4 *)(in_row + 8 * piece);
-    const uint32_t words[4] = {v.x, v.y, v.z, v.w};
+  const uint16_t *from = x + (uint64_t)row * x_row_stride;
+  const uint32_t pieces = inner / 8;
+  uint4 held[kPieces];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t lo = words[i] & 0x7fffu, hi = (words[i] >> 16) & 0x7fffu;
+  for (int i = 0; i < kPieces; ++i) {
+    const uint32_t piece = i * kThreads + in_row;
+    held[i] = piece < pieces ? *(const uint4 *)(from + 8 * piece) : make_uint4(0, 0, 0, 0);
+  }
+  uint32_t top = 0;   // largest magnitude bits (bf16 without sign) in the row
+#pragma unroll
+  for (int i = 0; i < kPieces; ++i) {
+    const uint32_t words[4] = {held[i].x, held[i].y, held[i].z, held[i].w};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const uint32_t lo = words[w] & 0x7fffu, hi = (words[w] >> 16) & 0x7fffu;
       // NaN and infinity (exponent 255) pass through the conversion unchanged; leave them out
       if (lo < 0x7f80u) top = max(top, lo);
       if (hi < 0x7f80u) top = max(top, hi);
     }
   }
   for (int offset = 32; offset > 0; offset >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, offset, 64));
+  if constexpr (kThreads > 64) {
+    if (lane == 0) tops[threadIdx.x >> 6] = top;
+    __syncthreads();
+    for (int w = 0; w < kThreads / 64; ++w) top = max(top, tops[local * (kThreads / 64) + w]);
+  }
   const int exponent = (int)(top >> 7) - 127;                    // floor(log2(max |x|))
   int down = exponent - 14;                                      // scale by 2^-down
   if (down < -100) down = -100;                                  // rows of zeros and denormals
   const float scale = __uint_as_float((uint32_t)(127 - down) << 23);
-  if (lane == 0) unscale[row] = __uint_as_float((uint32_t)(127 + down) << 23);
+  if (live && in_row == 0) unscale[row] = __uint_as_float((uint32_t)(127 + down) << 23);
   uint16_t *out_row = out + (uint64_t)row * kt;
-  for (uint32_t piece = lane; piece < inner / 8; piece += 64) {
-    const uint4 v = *(const uint4 *)(in_row + 8 * piece);
-    const uint32_t words[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int i = 0; i < kPieces; ++i) {
+    const uint32_t piece = i * kThreads + in_row;
+    const uint32_t words[4] = {held[i].x, held[i].y, held[i].z, held[i].w};
     float f[8];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      f[2 * i] = __uint_as_float(words[i] << 16) * scale;
-      f[2 * i + 1] = __uint_as_float(words[i] & 0xffff0000u) * scale;
+    for (int w = 0; w < 4; ++w) {
+      f[2 * w] = __uint_as_float(words[w] << 16) * scale;
+      f[2 * w + 1] = __uint_as_float(words[w] & 0xffff0000u) * scale;
     }
-    *(uint4 *)(out_row + 8 * piece) = make_uint4(pack_f16(f[0], f[4]), pack_f16(f[1], f[5]),
-                                                 pack_f16(f[2], f[6]), pack_f16(f[3], f[7]));
+    if (live && piece < pieces)
+      *(uint4 *)(out_row + 8 * piece) = make_uint4(pack_f16(f[0], f[4]), pack_f16(f[1], f[5]),
+                                                   pack_f16(f[2], f[6]), pack_f16(f[3], f[7]));
     // eight consecutive pieces (= lanes) make one group; the scaled values are exact in f32
     float sum = ((f[0] + f[1]) + (f[2] + f[3])) + ((f[4] + f[5]) + (f[6] + f[7]));
     sum += __shfl_xor(sum, 1, 64);
     sum += __shfl_xor(sum, 2, 64);
     sum += __shfl_xor(sum, 4, 64);
-    if ((piece & 7) == 0) sums[wave][piece >> 3] = sum;
+    if ((piece & 7) == 0) sums[local][piece >> 3] = sum;
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  __syncthreads();
+  if (!live) return;
   const uint32_t groups = inner / 64;
-  for (uint32_t extra = lane; extra < kt - inner; extra += 64) {
+  for (uint32_t extra = in_row; extra < kt - inner; extra += kThreads) {
     const uint32_t group = extra / 3, kind = extra % 3;
     float value = 0.0f;
     if (group < groups) {
       float head, tail;
-      split_f16(sums[wave][group] * (1.0f / 64.0f), &head, &tail);
+      split_f16(sums[local][group] * (1.0f / 64.0f), &head, &tail);
       value = kind == 1 ? tail : head;
     }
     out_row[inner + extra] = f16_bits(value);
@@ -1306,7 +1327,14 @@ bool launch_quant_gemm(fh_backend *backend, const QmmProblem &p, const uint32_t 
     configured = true;
   }
   const uint32_t grid = (a.row_tiles * a.column_tiles + 255) / 256 * 256;
-  prepare_rows_kernel<<<(p.rows + 3) / 4, 256, 0, stream>>>(
+  // The fewest threads that hold a row in four pieces each, then more pieces.
+  auto *prepare_rows = p.inner <= 2048    ? prepare_rows_kernel<64, 4>
+                       : p.inner <= 4096  ? prepare_rows_kernel<128, 4>
+                       : p.inner <= 8192  ? prepare_rows_kernel<256, 4>
+                       : p.inner <= 20480 ? prepare_rows_kernel<256, 10>
+                                          : prepare_rows_kernel<256, kMaxGroups / 32>;
+  const uint32_t rows_each = p.inner <= 2048 ? 4 : p.inner <= 4096 ? 2 : 1;
+  prepare_rows<<<(p.rows + rows_each - 1) / rows_each, 256, 0, stream>>>(
       (const uint16_t *)p.x.base + p.x.offset, p.x.stride[0], p.rows, p.inner, kt, (uint16_t *)ws,
       (float *)after, flag);
   if (!kept || fresh) {

@@ -481,6 +481,8 @@ def test_quant_matmul_with_f16_scales_and_a_residual_in_other_dtypes(cpu, hip, d
     (130, 70, 17408),     # more columns of group sums than a slot of LDS holds at a time
     (200, 8264, 512),     # 128 x 128 tiles, the fewest K steps
     (257, 5700, 2560),
+    # rows held by 64, 128 and 256 threads, in four, ten and sixteen pieces each
+    (133, 72, 2048), (133, 72, 4096), (131, 72, 8192), (129, 72, 8704), (129, 72, 20992),
 ])
 @pytest.mark.parametrize("residual", [False, True])
 def test_prefill_products_of_few_tiles(hip, rows, n, k, residual):
