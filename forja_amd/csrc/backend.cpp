@@ -1420,10 +1420,48 @@ bool find_norm_tail(fh_backend *b, const fh_dispatch &d, const fh_dispatch &next
 // one of them writes is read or written by another in any other way, since the workgroups of one
 // kernel do it all in no order.
 //
+// A product of a few long f32 rows and the residual normalisation that takes its result: the product's two halves in
+// one launch, their sum in the normalisation's.  Two launches one after the other, so that all that matters is
+// that nothing the normalisation writes lies in the product's result, which now is written beside it, and that
+// it reads the result as one of its terms only.
+uint32_t run_product_of_halves(fh_backend *b, const fh_dispatch *d, uint32_t first) {
+  const fh_dispatch &product = d[first], &norm = d[first + 1];
+  if (product.n_outputs != 1 || product.n_inputs != 4 || product.epilogue != 0 || product.inputs[0].rank != 2 ||
+      product.inputs[0].shape[0] > 16 || norm.op != FH_OP_PROGRAM || norm.n_inputs != 3 || norm.n_outputs != 2)
+    return 0;
+  auto program = b->programs.find(norm.program);
+  if (program == b->programs.end() || program->second.fast.kind != kProgramResidualNorm) return 0;
+  const fh_tensor &out = product.outputs[0];
+  uint32_t reads = 0;
+  for (uint32_t i = 0; i < 3; ++i) reads += may_overlap(out, norm.inputs[i]);
+  if (reads != 1 || may_overlap(out, norm.outputs[0]) || may_overlap(out, norm.outputs[1])) return 0;
+  View views[4], made, in[3], normed[2];
+  for (uint32_t i = 0; i < 4; ++i)
+    if (make_view(b, product.inputs[i], false, &views[i]) != FH_OK) return 0;
+  if (make_view(b, out, true, &made) != FH_OK) return 0;
+  for (uint32_t i = 0; i < 3; ++i)
+    if (make_view(b, norm.inputs[i], false, &in[i]) != FH_OK) return 0;
+  for (uint32_t i = 0; i < 2; ++i)
+    if (make_view(b, norm.outputs[i], true, &normed[i]) != FH_OK) return 0;
+  ProgramArgs args;
+  if (bind_program(b, program->second, norm.inputs, norm.n_inputs, in, norm.outputs, norm.n_outputs, normed,
+                   norm.outputs[0].shape, norm.outputs[0].rank, &args) != FH_OK ||
+      !norm_takes_halves(program->second.fast, args, made))
+    return 0;
+  const QmmProblem problem{views[0], views[1], views[2], views[3], made, product.inputs[0].shape[0],
+                           product.inputs[0].shape[1], out.shape[1], product.bits, product.group_size};
+  const float *halves = launch_wide_halves(b, problem);
+  if (!halves) return 0;
+  launch_norm_of_halves(b->stream, program->second.fast, args, made, halves);
+  return 2;
+}
+
 // Executes the normalisation, product and element program that start at `first` in one launch and
 // returns how many dispatches that were (2 or 3), or returns 0 having done nothing.
 uint32_t run_dense_group(fh_backend *b, const fh_dispatch *d, uint32_t count, uint32_t first) {
   if (b->static_mode || first + 1 >= count) return 0;
+  if (d[first].op == FH_OP_QUANT_MATMUL && d[first].n_inputs > 0 && d[first].inputs[0].dtype == FH_F32)
+    return run_product_of_halves(b, d, first);
   auto program_at = [&](uint32_t at, int kind_a, int kind_b) -> Program * {
     if (at >= count || d[at].op != FH_OP_PROGRAM) return nullptr;
     auto it = b->programs.find(d[at].program);

@@ -162,8 +162,13 @@ struct KsplitRouted {
   const uint32_t *sorted_routes, *blocks, *n_blocks;
   uint32_t max_blocks, tile_rows, route_div;
   bool wide;                // f32 activations and results (launch_ksplit_routed: tiles of 16 routes only)
+  uint32_t weight_inner;    // 0, or "expert" e is the e-th part of K (inner long) of one matrix of so long rows
 };
 bool launch_ksplit_routed(fh_backend *backend, const KsplitRouted &problem);
+
+// A dense product of at most 16 f32 rows of 4096 values as two sums of 2048 products each, [rows][2][columns] in the
+// workspace, in one launch; whoever reads them adds the two.  Null: nothing was launched.
+const float *launch_wide_halves(fh_backend *backend, const QmmProblem &problem);
 
 // ---- qmm_rows.hip: products over up to 64 activation rows per weight, weights unpacked once for
 // all of them.  Operands as above, K a multiple of 256, columns of 16; rows of bf16, or f32 (`wide`: f32 residual
@@ -313,6 +318,12 @@ void launch_combine_routes_norm(hipStream_t stream, const float *partial, const 
                                 uint64_t residual_row_stride, void *out, uint64_t out_row_stride,
                                 uint32_t rows, uint32_t routes, uint32_t columns, uint32_t experts,
                                 const NormTail &tail);
+
+// The residual normalisation of f32 rows whose sum takes `produced`, a product's result, given as the two halves
+// of launch_wide_halves: it adds them, stores the product's rows, and goes on with those.
+bool norm_takes_halves(const ProgramClass &cls, const ProgramArgs &args, const View &produced);
+void launch_norm_of_halves(hipStream_t stream, const ProgramClass &cls, const ProgramArgs &args, const View &produced,
+                           const float *halves);
 
 // Epilogue recognisers: `acc + extra` and `silu(acc0) * acc1` in the instruction orders the SDK
 // emits (crates/forja-sdk/src/nn/blocks.rs:406-416) and commuted variants.

@@ -65,20 +65,37 @@ struct RowArgs {
   uint64_t x_stride, update_stride, weight_stride, out0_stride, out1_stride;
   uint32_t width;
   float eps;
+  // kHalves: the update is the sum of two rows here, which is stored where the product's rows go
+  const float *halves;
+  float *produced;
+  uint64_t produced_stride;
 };
 
 // out = x * rsqrt(mean(x^2) + eps) * w            (kResidual = false)
 // value = x + update; out0 = value; out1 = value * rsqrt(mean(value^2) + eps) * w
-template <bool kResidual, bool kWide>
+// kHalves: f32 decode rows behind a product of 4096 values a row, which came in two launches of 6.9 us because
+// three pieces of so long a slice do not fit the registers.  One launch of both halves leaves two sums and this kernel, whose
+// 3 us are latency, adds them: 13.8 -> 7.8 us a layer for one lane.
+template <bool kResidual, bool kWide, bool kHalves = false>
 __global__ __launch_bounds__(256) void norm_rows_kernel(RowArgs a) {
   __shared__ float scratch[4];
   const uint64_t row = blockIdx.x;
   const uint64_t x_at = row * a.x_stride, u_at = row * a.update_stride, w_at = row * a.weight_stride;
+  auto load_update = [&](uint32_t c, float (&u)[8]) {
+    if constexpr (kHalves) {
+      float second[8];
+      load8<true>(a.halves, 2 * row * a.width + c, u);
+      load8<true>(a.halves, (2 * row + 1) * a.width + c, second);
+      for (int i = 0; i < 8; ++i) u[i] += second[i];
+    } else if constexpr (kResidual) {
+      load8<kWide>(a.update, u_at + c, u);
+    }
+  };
   float acc = 0.0f;
   for (uint32_t c = threadIdx.x * 8; c < a.width; c += 256 * 8) {
     float v[8], u[8];
     load8<kWide>(a.x, x_at + c, v);
-    if (kResidual) load8<kWide>(a.update, u_at + c, u);
+    load_update(c, u);
     for (int i = 0; i < 8; ++i) {
       const float value = kResidual ? v[i] + u[i] : v[i];
       acc += value * value;
@@ -90,7 +107,8 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(RowArgs a) {
     float v[8], u[8], w[8], normed[8];
     load8<kWide>(a.x, x_at + c, v);
     load8<kWide>(a.weight, w_at + c, w);
-    if (kResidual) load8<kWide>(a.update, u_at + c, u);
+    load_update(c, u);
+    if constexpr (kHalves) store8<true>(a.produced, row * a.produced_stride + c, u);
     for (int i = 0; i < 8; ++i) {
       if (kResidual) v[i] += u[i];
       normed[i] = v[i] * inverse * w[i];
@@ -646,6 +664,45 @@ bool norm_tail_of(const ProgramClass &cls, const ProgramArgs &p, const View &pro
   tail->eps = cls.c[0];
   tail->wide = dtype == FH_F32;
   return true;
+}
+
+namespace {
+
+// Which input of the residual normalisation is `produced`, element for element: 0 or 1, or -1.
+int halves_input(const ProgramArgs &p, const View &produced) {
+  int found = -1;
+  for (int i = 0; i < 2; ++i) {
+    const View &v = p.inputs[i];
+    if (v.base != produced.base || v.offset != produced.offset || v.dtype != produced.dtype) continue;
+    if (found >= 0 || v.stride[0] != produced.stride[0]) return -1;
+    found = i;
+  }
+  return found;
+}
+
+}  // namespace
+
+bool norm_takes_halves(const ProgramClass &cls, const ProgramArgs &p, const View &produced) {
+  RowArgs a{};
+  bool residual = false, wide = false;
+  if (!norm_rows_args(cls, p, &a, &residual, &wide) || !residual || !wide) return false;
+  return produced.rank == 2 && produced.shape[0] == p.shape[0] && produced.shape[1] == p.shape[1] &&
+         halves_input(p, produced) >= 0;
+}
+
+void launch_norm_of_halves(hipStream_t stream, const ProgramClass &cls, const ProgramArgs &p, const View &produced,
+                           const float *halves) {
+  RowArgs a{};
+  bool residual = false, wide = false;
+  if (!norm_rows_args(cls, p, &a, &residual, &wide)) return;   // (norm_takes_halves has said that it does)
+  if (halves_input(p, produced) == 0) {   // x + update is update + x
+    a.x = a.update;
+    a.x_stride = a.update_stride;
+  }
+  a.halves = halves;
+  a.produced = (float *)produced.base + produced.offset;
+  a.produced_stride = produced.stride[0];
+  norm_rows_kernel<true, true, true><<<dim3(p.shape[0]), 256, 0, stream>>>(a);
 }
 
 void launch_combine_routes_norm(hipStream_t stream, const float *partial, const View &indices,

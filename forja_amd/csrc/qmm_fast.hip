@@ -1126,7 +1126,57 @@ bool try_wide_quant_matmul(fh_backend *backend, const QmmProblem &p) {
   return true;
 }
 
+// The plan of launch_wide_halves for 1 to 16 rows: half h of row m is input row 2m + h (of half the length), and
+// result row 2m + h.  First the rows of the two tiles, then two tiles (half, first row, rows) for each number
+// of rows, then how many tiles.
+struct WideHalvesPlan {
+  uint32_t routes[32], tiles[16][6], count;
+  constexpr WideHalvesPlan() : routes(), tiles(), count(2) {
+    for (uint32_t i = 0; i < 32; ++i) routes[i] = 2 * (i & 15) + (i >> 4);
+    for (uint32_t rows = 1; rows <= 16; ++rows) {
+      tiles[rows - 1][2] = rows;
+      tiles[rows - 1][3] = 1;
+      tiles[rows - 1][4] = 16;
+      tiles[rows - 1][5] = rows;
+    }
+  }
+};
+__device__ WideHalvesPlan wide_halves_plan = WideHalvesPlan();   // (not const: used by its address alone, it would not be kept)
+
 }  // namespace
+
+const float *launch_wide_halves(fh_backend *backend, const QmmProblem &p) {
+  constexpr uint32_t kInner = 4096, kHalf = kInner / 2;
+  if (p.x.dtype != FH_F32 || p.out.dtype != FH_F32 || p.out.stride[1] != 1 || p.residual) return nullptr;
+  if (p.inner != kInner || p.bits != 4 || p.rows == 0 || p.rows > 16) return nullptr;
+  if (!weights_eligible(p.packed, p.scales, p.biases, 2, p.inner, p.bits, p.group, 4)) return nullptr;
+  if (p.x.stride[1] != 1 || p.x.offset % 4 != 0 || (p.rows > 1 && p.x.stride[0] != kInner)) return nullptr;
+  if (!ksplit_supports(kHalf, p.columns, false, true)) return nullptr;
+  float *halves = (float *)backend_workspace(backend, (uint64_t)p.rows * 2 * p.columns * sizeof(float));
+  void *plan = nullptr;
+  if (!halves || hipGetSymbolAddress(&plan, HIP_SYMBOL(wide_halves_plan)) != hipSuccess) return nullptr;
+  const WideHalvesPlan *at = (const WideHalvesPlan *)plan;
+  KsplitRouted r{};
+  r.x = (const float *)p.x.base + p.x.offset;
+  r.x_row_stride = kHalf;
+  r.packed[0] = u32_ptr(p.packed);
+  r.scales[0] = u16_ptr(p.scales);
+  r.biases[0] = u16_ptr(p.biases);
+  r.out = halves;
+  r.out_f32 = 1;
+  r.inner = kHalf;
+  r.weight_inner = kInner;
+  r.columns = p.columns;
+  r.sorted_routes = at->routes;
+  r.blocks = at->tiles[p.rows - 1];
+  r.n_blocks = &at->count;
+  r.max_blocks = 2;
+  r.tile_rows = 16;
+  r.route_div = 1;
+  r.wide = true;
+  KernelTimer timer(backend, FH_KC_QMM_KERNEL);
+  return launch_ksplit_routed(backend, r) ? halves : nullptr;
+}
 
 bool try_fast_quant_matmul(fh_backend *backend, const QmmProblem &p) {
   hipStream_t stream = backend_stream(backend);

@@ -795,9 +795,9 @@ void launch_one(fh_backend *backend, const KsplitArgs &a, uint64_t most_units) {
   // shorter (1 row: 1024 -> 4096 8.6 us wide and 6.2 narrow, 2048 -> 1024 6.7 and 5.6, 3072 -> 1024 7.7 and
   // 6.2; 23 rows 1024 -> 4096 16.3 and 10.7).  Beyond two workgroups a compute unit the wide batches' longer
   // streams win (their fixed costs, and in the 16-row form the coalesced scales, are shared by more columns).
-  if constexpr (!kRouted && CT > 1) {
+  if constexpr ((!kRouted || (XP == 3 && !kPair && G == 4 && WAVES == 8)) && CT > 1) {
     const uint64_t narrow = most_units * CT;
-    if (most_units < backend_compute_units(backend) && narrow <= 2 * backend_compute_units(backend)) {
+    if ((!kRouted || a.weight_inner != a.inner) && most_units < backend_compute_units(backend) && narrow <= 2 * backend_compute_units(backend)) {
       KsplitArgs n = a;
       n.batches_per_tile = a.batches_per_tile * CT;
       launch_one<WAVES, G, RT, kPair, kRouted, XP, kNorm, 1>(backend, n, narrow);
@@ -962,6 +962,11 @@ bool launch_ksplit_routed(fh_backend *backend, const KsplitRouted &r) {
   a.out_f32 = r.out_f32;
   a.inner = r.inner;
   a.weight_inner = r.inner;
+  if (r.weight_inner) {
+    a.weight_inner = r.weight_inner;
+    a.expert_words = r.inner / 8;
+    a.expert_groups = r.inner / kGroup;
+  }
   a.columns = r.columns;
   a.sorted_routes = r.sorted_routes;
   a.blocks = r.blocks;

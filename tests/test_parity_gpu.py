@@ -879,6 +879,39 @@ def test_dense_products_with_the_row_programs_around_them(cpu, hip, rows, n, k, 
     differential(cpu, hip, build, rel=2e-2, abs_=2e-2)
 
 
+@pytest.mark.parametrize("rows,n", [(1, 2048), (8, 2048), (16, 96), (17, 96), (3, 40)])
+@pytest.mark.parametrize("product_first", [False, True])
+def test_f32_product_of_long_rows_and_the_residual_normalisation_behind_it(cpu, hip, rows, n, product_first):
+    """A product over K = 4096, whose two halves the normalisation adds: the oracle's results, and bit for bit
+    those of the two dispatches submitted one by one; 17 rows and columns of no whole batch take the launches apart."""
+    k, weights = 4096, Quantised(75, n, (n, 4096))
+    x_values = orc.fill_normal_f32(75, 1, rows * k).reshape(rows, k)
+    other_values = orc.fill_normal_f32(75, 2, rows * n).reshape(rows, n)
+    norm_values = orc.fill_normal_f32(75, 3, n)
+
+    def record(backend):
+        x, other = upload(backend, x_values, DType.F32), upload(backend, other_values, DType.F32)
+        norm_weight = upload(backend, norm_values, DType.F32).broadcast((rows, n))
+        product, summed, normed = (backend.alloc(DType.F32, (rows, n)) for _ in range(3))
+        first, second = CommandList(), CommandList()
+        terms = [product, other] if product_first else [other, product]
+        program = backend.prepare_program(programs.residual_norm_rows(1e-6))
+        operands = [x, *weights.upload(backend)]
+        joined = CommandList()
+        for product_list, norm_list in ((first, second), (joined, joined)):
+            product_list.dispatch(Op.quant_matmul(4, 64), operands, product)
+            norm_list.dispatch_kernel(program, [*terms, norm_weight], [summed, normed])
+        return joined, [first, second], [product, summed, normed]
+
+    differential(cpu, hip, lambda backend: record(backend)[::2])
+    joined, apart, tensors = record(hip)
+    run(hip, joined)
+    together = [hip.read(t) for t in tensors]
+    for commands in apart:
+        run(hip, commands)
+    assert together == [hip.read(t) for t in tensors]
+
+
 @pytest.mark.parametrize("with_residual", [False, True])
 def test_f32_weighted_sum_followed_by_the_normalisation_of_its_rows(cpu, hip, with_residual):
     """The same pair in the engine's dtypes: an 8-row decode batch, everything f32."""
