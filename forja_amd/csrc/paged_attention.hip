@@ -288,6 +288,13 @@ struct TokenPlan {
   uint32_t leader, members;                // first token of this token's group, group size
 };
 
+// One split of a group of tokens, with what its workgroup has to know of the group's plan: one load in front
+// of the page table's instead of two that follow each other.
+struct alignas(16) WorkItem {
+  uint32_t leader, split, lane, attended;   // attended: by the leader
+  uint32_t chunk, splits, members, unused;
+};
+
 struct FastRagged {
   const void *q;       // q_dtype elements
   const uint16_t *key_pool, *value_pool;
@@ -299,7 +306,7 @@ struct FastRagged {
   float2 *partial_ml;  // [T, S, Hq]
   uint32_t *bad;       // [T]
   TokenPlan *plans;    // [T]
-  uint2 *items;        // [T * S] (group leader token, split) of every live split, compacted
+  WorkItem *items;     // [T * S] every live split, compacted
   uint32_t *item_count;   // [0] work items, [1] tokens the merge kernel has work for,
                           // [2] non-zero: cu_seqlens was refused
   uint32_t *merge_tokens; // [T] those tokens (several splits, or a zero row to write)
@@ -610,7 +617,8 @@ __global__ __launch_bounds__(kPlanThreads) void ragged_plan_kernel(FastRagged p,
     const TokenPlan plan = p.plans[token];
     if (plan.leader != token || plan.splits == 0) continue;
     const uint32_t first = atomicAdd(&class_items[class_of(plan)], plan.splits);
-    for (uint32_t s = 0; s < plan.splits; ++s) p.items[first + s] = make_uint2(token, s);
+    for (uint32_t s = 0; s < plan.splits; ++s)
+      p.items[first + s] = WorkItem{token, s, plan.lane, plan.attended, plan.chunk, plan.splits, plan.members, 0};
   }
 }
 
@@ -798,13 +806,11 @@ __device__ inline void consume_tile(const TileRegs &cur, const uint4 (&q_reg)[4]
 // One split of a group of one query token, for one kv head, by one wave: the head's `group` query rows
 // (lane's row hl; rows from `group` on are padding) attend keys streamed straight into registers.
 template <bool kHalf, bool kMixed>
-__device__ inline void attend_one_token(const FastRagged &p, ErrorSlot *error, uint32_t item, uint32_t kv_head) {
+__device__ inline void attend_one_token(const FastRagged &p, ErrorSlot *error, const WorkItem &plan, uint32_t kv_head) {
   uint32_t lane = threadIdx.x & 63;
   asm volatile("" : "+v"(lane));   // what follows from it is not kept in registers from item to item
   const uint32_t hl = lane & 15, g = lane >> 4;
-  const uint2 work = p.items[item];
-  const uint32_t leader = work.x, split = work.y;
-  const TokenPlan plan = p.plans[leader];
+  const uint32_t leader = plan.leader, split = plan.split;
   const uint32_t begin = split * plan.chunk;
   const uint32_t end = min(plan.attended, begin + plan.chunk);
   const uint32_t pt = p.page_tokens;
@@ -1107,9 +1113,8 @@ __device__ inline void attend_item(const FastRagged &p, ErrorSlot *error, uint32
   uint32_t lane = threadIdx.x & 63;
   asm volatile("" : "+v"(lane));   // what follows from it is not kept in registers from item to item
   const uint32_t half = lane >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint2 work = p.items[item];
-  const uint32_t leader = work.x, split = work.y;
-  const TokenPlan plan = p.plans[leader];
+  const WorkItem plan = p.items[item];
+  const uint32_t leader = plan.leader, split = plan.split;
   // the item's split layout is sized for its last member
   const uint32_t longest = p.fixed_attended ? plan.attended : plan.attended + plan.members - 1;
   const uint32_t begin = split * plan.chunk;
@@ -1259,10 +1264,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // a workgroup is one work item; its waves take one kv head each, so the slices of a K/V page
   // (one 256-byte piece of every token row per kv head) are requested close together in time
   const uint32_t kv_head = blockIdx.y * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  // (the first item comes with the count: there is room for as many as there are workgroups)
+  WorkItem work = p.items[blockIdx.x];
   const uint32_t items = p.item_count[0];
+  asm volatile("" : "+s"(work.leader), "+s"(work.chunk));   // loaded here, not where it is used
   if (kv_head >= p.kv_heads) return;
-  for (uint32_t item = blockIdx.x; item < items; item += gridDim.x)
-    attend_one_token<kHalf, kMixed>(p, error, item, kv_head);
+  for (uint32_t item = blockIdx.x; item < items;) {
+    attend_one_token<kHalf, kMixed>(p, error, work, kv_head);
+    item += gridDim.x;
+    if (item < items) work = p.items[item];
+  }
 }
 
 // Merges the per-split partials of one (token, head): out = sum_s O_s 2^(m_s-M) / sum_s l_s
@@ -1278,11 +1289,11 @@ __global__ __launch_bounds__(256) void ragged_reduce_kernel(FastRagged p, std::c
   __shared__ float4 folded[3][32];
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t column = (lane & 31) * 4, half = lane >> 5;
-  const uint32_t head = blockIdx.x, listed = p.item_count[1];
+  const uint32_t head = blockIdx.x, listed = kPlaced ? p.tokens : p.item_count[1];
   // blockIdx.y walks the list of tokens that need the merge (the plan kernel compiled it; the
   // bad-page flags an attention wave may have raised since are re-read here)
   for (uint32_t entry = blockIdx.y; entry < listed; entry += gridDim.y) {
-    const uint32_t token = p.merge_tokens[entry];
+    const uint32_t token = kPlaced ? entry : p.merge_tokens[entry];   // (placed: every token is listed)
     const TokenPlan plan = p.plans[token];
     const bool zero = plan.splits == 0 || p.bad[token] != 0;
     auto store = [&](float a, float b, float c, float d) {
@@ -1399,7 +1410,7 @@ uint64_t round_256(uint64_t bytes) { return (bytes + 255) / 256 * 256; }
 uint64_t plan_storage_bytes(const FastRagged &f) {
   uint64_t slots = (uint64_t)f.tokens * f.max_splits;
   return 2 * round_256((uint64_t)f.tokens * 4) + round_256((uint64_t)f.tokens * sizeof(TokenPlan)) +
-         round_256(slots * sizeof(uint2)) + 256;
+         round_256(slots * sizeof(WorkItem)) + 256;
 }
 
 char *carve_plan(FastRagged *f, char *ws) {
@@ -1410,8 +1421,8 @@ char *carve_plan(FastRagged *f, char *ws) {
   ws += round_256((uint64_t)f->tokens * 4);
   f->plans = (TokenPlan *)ws;
   ws += round_256((uint64_t)f->tokens * sizeof(TokenPlan));
-  f->items = (uint2 *)ws;
-  ws += round_256(slots * sizeof(uint2));
+  f->items = (WorkItem *)ws;
+  ws += round_256(slots * sizeof(WorkItem));
   f->item_count = (uint32_t *)ws;
   return ws + 256;
 }
