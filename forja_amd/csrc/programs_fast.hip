@@ -134,25 +134,45 @@ __global__ __launch_bounds__(256) void combine_routes_norm_kernel(
   const uint32_t row = blockIdx.x, column = 8 * threadIdx.x;
   const bool live = column < columns;
   float value[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  float r[8], w[8];
   if (live) {
+    // Everything is asked for at once, with no branch in between (a route that is skipped has a row of its own too,
+    // whatever it holds, and past the last one the last is read again): with the weights' dtype asked
+    // per route the eight came one round trip after the other.  (2080 rows 30.2 -> 26.3 us, 128 rows
+    // 7.4 -> 6.2, one f32 row 5.0 -> 4.6.)
     float weight[8];
     float4 part[8][2];
+    uint32_t expert[8];
 #pragma unroll
-    for (int slot = 0; slot < 8; ++slot) {
-      weight[slot] = 0.0f;
-      part[slot][0] = part[slot][1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      if ((uint32_t)slot < routes) {
-        const uint32_t expert = load_u32_at(indices, indices.offset + row * indices.stride[0] +
-                                                         slot * indices.stride[1]);
-        if (expert < experts) {
-          weight[slot] = load_float_at(weights, weights.offset + row * weights.stride[0] +
-                                                    slot * weights.stride[1]);
-          const float4 *from = (const float4 *)(partial + ((uint64_t)row * routes + slot) * columns + column);
-          part[slot][0] = from[0];
-          part[slot][1] = from[1];
-        }
-      }
+    for (uint32_t slot = 0; slot < 8; ++slot) {
+      const uint32_t route = min(slot, routes - 1);
+      const float4 *from = (const float4 *)(partial + ((uint64_t)row * routes + route) * columns + column);
+      part[slot][0] = from[0];
+      part[slot][1] = from[1];
+      expert[slot] = load_u32_at(indices, indices.offset + row * indices.stride[0] + route * indices.stride[1]);
     }
+    load8<kWide>(tail.weight, (uint64_t)row * tail.weight_stride + column, w);
+    if (residual) load8<kWide>(residual, (uint64_t)row * residual_row_stride + column, r);
+    const uint64_t first_weight = weights.offset + row * weights.stride[0];
+    if (weights.dtype == FH_F32) {
+#pragma unroll
+      for (uint32_t slot = 0; slot < 8; ++slot)
+        weight[slot] = ((const float *)weights.base)[first_weight + min(slot, routes - 1) * weights.stride[1]];
+    } else {
+      uint16_t bits[8];
+#pragma unroll
+      for (uint32_t slot = 0; slot < 8; ++slot)
+        bits[slot] = ((const uint16_t *)weights.base)[first_weight + min(slot, routes - 1) * weights.stride[1]];
+#pragma unroll
+      for (uint32_t slot = 0; slot < 8; ++slot)
+        weight[slot] = weights.dtype == FH_F16 ? f16_to_f32(bits[slot]) : bf16_to_f32(bits[slot]);
+    }
+#pragma unroll
+    for (uint32_t slot = 0; slot < 8; ++slot)
+      if (slot >= routes || expert[slot] >= experts) {
+        weight[slot] = 0.0f;
+        part[slot][0] = part[slot][1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      }
 #pragma unroll
     for (int slot = 0; slot < 8; ++slot) {   // a skipped route adds +0 * 0: no effect
       value[0] += weight[slot] * part[slot][0].x;
@@ -164,11 +184,8 @@ __global__ __launch_bounds__(256) void combine_routes_norm_kernel(
       value[6] += weight[slot] * part[slot][1].z;
       value[7] += weight[slot] * part[slot][1].w;
     }
-    if (residual) {
-      float r[8];
-      load8<kWide>(residual, (uint64_t)row * residual_row_stride + column, r);
+    if (residual)
       for (int i = 0; i < 8; ++i) value[i] += r[i];
-    }
     store8<kWide>(out, (uint64_t)row * out_row_stride + column, value);
     // the normalisation reads what was stored
     if (!kWide)
@@ -179,8 +196,7 @@ __global__ __launch_bounds__(256) void combine_routes_norm_kernel(
   const float total = block_sum(acc, scratch);
   const float inverse = 1.0f / sqrtf(total / (float)columns + tail.eps);
   if (live) {
-    float w[8], normed[8];
-    load8<kWide>(tail.weight, (uint64_t)row * tail.weight_stride + column, w);
+    float normed[8];
     for (int i = 0; i < 8; ++i) normed[i] = value[i] * inverse * w[i];
     store8<kWide>(tail.out, (uint64_t)row * tail.out_stride + column, normed);
   }
