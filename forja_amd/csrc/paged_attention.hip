@@ -103,11 +103,12 @@ struct TokenPlan {
   uint32_t leader, members;                // first token of this token's group, group size
 };
 
-// The same append for rows and pools of one 2-byte dtype whose head rows are 16-byte aligned: a
-// thread moves eight elements.
+// The same append for pools of a 2-byte dtype and rows of that dtype or (kWide) f32, rounded as a store into the
+// pool rounds, whose head rows are 16-byte aligned: a thread moves eight elements.
 // What bounds it: a chain of memory round trips.  The row itself is asked for first; where there is a work plan
 // (`plans`, else null) a token's lane and position are one load instead of a binary search, its start
 // and its lane's first token.  (2048 rows of 8 kv heads 9.5 -> 6.6 us, 8256 35.7 -> 21.8, 2080 of 4 8.9 -> 6.0.)
+template <bool kWide>
 __global__ __launch_bounds__(256) void ragged_append_pieces_kernel(RaggedAttention p, ErrorSlot *error,
                                                                    const uint32_t *malformed,
                                                                    const TokenPlan *plans) {
@@ -124,8 +125,15 @@ __global__ __launch_bounds__(256) void ragged_append_pieces_kernel(RaggedAttenti
   const uint32_t head = 8 * local / row_width, c = 8 * local % row_width;
   const View &src = key ? p.k_new : p.v_new;
   const View &pool = key ? p.key_pool : p.value_pool;
-  const uint4 value = *(const uint4 *)((const uint16_t *)src.base + src.offset +
-                                       (uint64_t)token * src.stride[0] + head * src.stride[1] + c);
+  const uint64_t from = src.offset + (uint64_t)token * src.stride[0] + head * src.stride[1] + c;
+  uint4 value;
+  float4 wide[2];
+  if constexpr (kWide) {
+    wide[0] = *(const float4 *)((const float *)src.base + from);
+    wide[1] = *(const float4 *)((const float *)src.base + from + 4);
+  } else {
+    value = *(const uint4 *)((const uint16_t *)src.base + from);
+  }
   const uint32_t planned_lane = plans ? plans[token].lane : 0, planned = plans ? plans[token].attended : 0;
   if (malformed[0]) return;   // cu_seqlens refused: nothing is stored
   uint32_t lane, slot;
@@ -160,15 +168,23 @@ __global__ __launch_bounds__(256) void ragged_append_pieces_kernel(RaggedAttenti
     return;
   }
   const uint64_t pool_row = (uint64_t)physical * p.page_tokens + slot;
+  if constexpr (kWide) {
+    const bool half = pool.dtype == FH_F16;
+    auto pair = [&](float lo, float hi) {
+      return half ? f32_to_f16(lo) | (uint32_t)f32_to_f16(hi) << 16 : f32_to_bf16(lo) | (uint32_t)f32_to_bf16(hi) << 16;
+    };
+    value = make_uint4(pair(wide[0].x, wide[0].y), pair(wide[0].z, wide[0].w), pair(wide[1].x, wide[1].y),
+                       pair(wide[1].z, wide[1].w));
+  }
   *(uint4 *)((uint16_t *)pool.base + pool.offset + pool_row * ((uint64_t)p.kv_heads * row_width) +
              8 * local) = value;
 }
 
 bool append_by_pieces(const RaggedAttention &p) {
-  const uint32_t dtype = p.key_pool.dtype;
-  if (dtype != FH_BF16 && dtype != FH_F16) return false;
+  const uint32_t dtype = p.key_pool.dtype, rows = p.k_new.dtype;
+  if ((dtype != FH_BF16 && dtype != FH_F16) || (rows != dtype && rows != FH_F32)) return false;
   for (const View *v : {&p.k_new, &p.v_new})
-    if (v->dtype != dtype || v->stride[2] != 1 || v->stride[0] % 8 || v->stride[1] % 8 || v->offset % 8)
+    if (v->dtype != rows || v->stride[2] != 1 || v->stride[0] % 8 || v->stride[1] % 8 || v->offset % 8)
       return false;
   for (const View *v : {&p.key_pool, &p.value_pool})
     if (v->dtype != dtype || v->offset % 8) return false;
@@ -1690,12 +1706,14 @@ bool run_ragged_attention(fh_backend *backend, const RaggedAttention &p, ErrorSl
   }
   uint64_t append_work =
       (uint64_t)p.tokens * (p.kv_heads * p.width + p.kv_heads * p.value_width);
-  if (append_by_pieces(p))
-    ragged_append_pieces_kernel<<<dim3((unsigned)((append_work / 8 + 255) / 256)), 256, 0, stream>>>(
+  if (append_by_pieces(p)) {
+    auto *append = p.k_new.dtype == FH_F32 ? ragged_append_pieces_kernel<true> : ragged_append_pieces_kernel<false>;
+    append<<<dim3((unsigned)((append_work / 8 + 255) / 256)), 256, 0, stream>>>(
         p, append_error, malformed, fast ? f.plans : nullptr);
-  else
+  } else {
     ragged_append_kernel<<<dim3((unsigned)((append_work + 255) / 256)), 256, 0, stream>>>(
         p, append_error, malformed);
+  }
   if (fast) {
     launch_fast(backend, stream, f, error);
     return true;
