@@ -602,30 +602,48 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
   }
 }
 
-// out[r, c..c+4) = residual? + the K ranges' partial sums, added in order.
+// out[r, c..c+4) = residual? + the K ranges' partial sums, added in order.  Bound by its bytes, and of few rows by the
+// launch: what a thread reads it asks for at once, and its four results are one store where rows and residual are
+// `aligned` to four elements (four ranges of 512 x 5120: 10.3 -> 9.1 us).
 __global__ __launch_bounds__(256) void sum_ranges_kernel(const float *partials, uint32_t splits, uint32_t rows,
                                                          uint32_t columns, void *out, uint64_t out_row_stride,
                                                          uint32_t out_f32, const void *residual,
-                                                         uint64_t residual_row_stride, uint32_t residual_f32) {
+                                                         uint64_t residual_row_stride, uint32_t residual_f32,
+                                                         uint32_t aligned) {
   const uint64_t at = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * 4, plane = (uint64_t)rows * columns;
   if (at >= plane) return;
+  const uint64_t row = plane <= 0xffffffffull ? (uint32_t)at / columns : at / columns, column = at - row * columns;
+  f32x4 added = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (residual) {
+    const uint64_t from = row * residual_row_stride + column;
+    if (aligned && residual_f32) {
+      added = *(const f32x4 *)((const float *)residual + from);
+    } else if (aligned) {
+      const uint2 words = *(const uint2 *)((const uint16_t *)residual + from);
+      added = f32x4{low_bf16(words.x), high_bf16(words.x), low_bf16(words.y), high_bf16(words.y)};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        added[i] = residual_f32 ? ((const float *)residual)[from + i] : low_bf16(((const uint16_t *)residual)[from + i]);
+    }
+  }
   f32x4 total = *(const f32x4 *)(partials + at);
 #pragma unroll 4
   for (uint32_t s = 1; s < splits; ++s) total += *(const f32x4 *)(partials + s * plane + at);
-  const uint64_t row = at / columns, column = at % columns;
-  if (residual) {
-    const uint64_t from = row * residual_row_stride + column;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      total[i] += residual_f32 ? ((const float *)residual)[from + i] : low_bf16(((const uint16_t *)residual)[from + i]);
-  }
+  if (residual) total += added;
   const uint64_t to = row * out_row_stride + column;
+  if (aligned && out_f32) {
+    *(f32x4 *)((float *)out + to) = total;
+  } else if (aligned) {
+    *(uint2 *)((uint16_t *)out + to) = make_uint2(pack_bf16(total[0], total[1]), pack_bf16(total[2], total[3]));
+  } else {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if (out_f32)
-      ((float *)out)[to + i] = total[i];
-    else
-      ((uint16_t *)out)[to + i] = (uint16_t)pack_bf16(total[i], 0.0f);
+    for (int i = 0; i < 4; ++i) {
+      if (out_f32)
+        ((float *)out)[to + i] = total[i];
+      else
+        ((uint16_t *)out)[to + i] = (uint16_t)pack_bf16(total[i], 0.0f);
+    }
   }
 }
 
@@ -716,10 +734,11 @@ bool launch_rows_dense(fh_backend *backend, const RowsDense &d) {
     default: launch_rows<1, 4, 4, 2, 2, false, false>(stream, a, grid); break;
     }
   }
+  const bool residual_aligned = !d.residual || ((uintptr_t)d.residual % (d.wide ? 16 : 8) == 0 && d.residual_row_stride % 4 == 0);
   if (a.splits > 1)
     sum_ranges_kernel<<<dim3((unsigned)(((uint64_t)d.rows * d.columns / 4 + 255) / 256)), 256, 0, stream>>>(
         (const float *)a.out, a.splits, d.rows, d.columns, d.out, d.out_row_stride, d.out_f32, d.residual,
-        d.residual_row_stride, d.wide);
+        d.residual_row_stride, d.wide, a.out_aligned && residual_aligned);
   return true;
 }
 
