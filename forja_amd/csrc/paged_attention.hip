@@ -1093,28 +1093,36 @@ __device__ inline void attend_tile(uint32_t tile, const uint4 (&q)[8], f32x16 (&
       for (int i = 0; i < 16; ++i)
         if (32 * b + 8 * (i >> 2) + (i & 3) >= below) s[b][i] = -__builtin_inff();
   }
-  float tile_max = s[0][0];
+  // The sums follow every new maximum, of 32 keys at a time: the weight of the largest score is then exactly 1, which
+  // 16 bits hold.  (Errors against 64 bits, f32 queries and f16 pools: 512 rows from scratch 1.41e-4, with one maximum for the
+  // 64 keys 1.43e-4, with one that may lag by 2^6 1.53e-4; 260 rows behind 3071 keys, peaked, 2.9e-5 and 8.7e-5 with the lag.)
+  float maxima[2];
 #pragma unroll
-  for (int i = 1; i < 32; ++i) tile_max = fmaxf(tile_max, s[i >> 4][i & 15]);
-  tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, 64)) * scale_log2;
-  // The running maximum may lag behind by 2^kLag: the weights stay exact multiples of what they would
-  // be, and the rescale of the 64 sums per lane is seldom needed.
-  constexpr float kLag = 6.0f;
-  if (__any(tile_max > sm.m + kLag)) {
-    const float m_new = fmaxf(sm.m, tile_max);
+  for (int b = 0; b < 2; ++b) {
+    maxima[b] = s[b][0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) maxima[b] = fmaxf(maxima[b], s[b][i]);
+    maxima[b] = fmaxf(maxima[b], __shfl_xor(maxima[b], 32, 64)) * scale_log2;
+  }
+  auto raise = [&](float m_new) {
+    if (!__any(m_new > sm.m)) return;
     const float alpha = m_new == -__builtin_inff() ? 1.0f : __builtin_amdgcn_exp2f(sm.m - m_new);
     sm.l *= alpha;
 #pragma unroll
     for (int c = 0; c < 4; ++c)
       for (int i = 0; i < 16; ++i) o[c][i] *= alpha;
     sm.m = m_new;
-  }
-  // a row with nothing to attend yet keeps m = -inf; subtract 0 instead so that exp2(-inf) = 0
-  const float m_safe = sm.m == -__builtin_inff() ? 0.0f : sm.m;
-  float sum[2] = {0.0f, 0.0f};
+  };
+  maxima[0] = fmaxf(sm.m, maxima[0]);
+  maxima[1] = fmaxf(maxima[0], maxima[1]);
+  raise(maxima[0]);
+  float sums[2];
   uint4 weights[4];
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
+    // a row with nothing to attend yet keeps m = -inf; subtract 0 instead so that exp2(-inf) = 0
+    const float m_safe = maxima[b] == -__builtin_inff() ? 0.0f : maxima[b];
+    float sum[2] = {0.0f, 0.0f};
     uint32_t words[8];
 #pragma unroll
     for (int i = 0; i < 16; i += 2) {
@@ -1124,20 +1132,24 @@ __device__ inline void attend_tile(uint32_t tile, const uint4 (&q)[8], f32x16 (&
       sum[1] += y;
       words[i / 2] = pack_operand<kHalf>(x, y);
     }
+    sums[b] = sum[0] + sum[1];
     weights[2 * b] = make_uint4(words[0], words[1], words[2], words[3]);
     weights[2 * b + 1] = make_uint4(words[4], words[5], words[6], words[7]);
   }
-  sm.l += sum[0] + sum[1];
+  sm.l += sums[0];
   // O^T += V^T . P^T, 16 keys a step in the order the scores left them: half h takes keys 4h..4h+3 and
   // 8 + 4h..8 + 4h + 3 of the 16.
 #pragma unroll
-  for (int step = 0; step < 4; ++step)
+  for (int step = 0; step < 4; ++step) {
+    if (step == 2) raise(maxima[1]);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       o[c] = mfma_32x32x16<kHalf>(values[c], weights[step], o[c]);
       __builtin_amdgcn_sched_barrier(0);
       if (step < 3) values[c] = read_values(step + 1, c);
     }
+  }
+  sm.l += sums[1];
 }
 
 template <bool kHalf, bool kMixed>

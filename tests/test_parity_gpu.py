@@ -1471,6 +1471,30 @@ def test_a_value_without_a_number_reaches_later_rows_only(cpu, hip):
     assert np.isnan(got[69]).all()
 
 
+@pytest.mark.parametrize("pool", [DType.F16, DType.BF16])
+@pytest.mark.parametrize("lead", [1.3, 4.7, 5.9])
+def test_prefill_weight_of_the_largest_score_is_not_rounded(hip, pool, lead):
+    """Key 64, the first of a second tile, leads key 0 by 2^lead and all others by far more; only its value is not
+    zero.  Weights are relative to the largest score, so that its own is 1 in any format and a row's result has the
+    errors of 32-bit sums alone: of the score (2^-24 of at most 8, doubled by the scale's rounding) and the division."""
+    tokens = 130
+    t, inputs = ragged_case(hip, [0], [tokens], 2, 2, 16, seed=66, dtype=DType.F32, pool_dtype=pool)
+    q, keys, values = (np.zeros((tokens, 2, 128), np.float32) for _ in range(3))
+    q[:, :, 0] = 1.0
+    keys[:, :, 0] = -60.0
+    keys[0, :, 0], keys[64, :, 0] = 0.0, to_f32(from_f32(np.array([lead]), pool), pool)[0]
+    values[64] = 1.0
+    inputs[:3] = [upload(hip, v, DType.F32) for v in (q, keys, values)]
+    commands = CommandList()
+    commands.dispatch_many(Op.paged_attention_ragged(float(np.log(2.0)), 16), inputs, [t["out"], t["keys"], t["values"]])
+    run(hip, commands)
+    got = to_f32(hip.read(t["out"]), DType.F32).reshape(tokens, 2, 128).astype(np.float64)
+    scores = keys[:, 0, 0].astype(np.float64)
+    for row in range(64, tokens):
+        weights = np.exp2(scores[:row + 1])
+        assert np.abs(got[row] / (weights[64] / weights.sum()) - 1.0).max() <= 2.0 ** -18
+
+
 DTYPE_MIXES = [
     # query and new rows, pools, output
     (DType.F32, DType.F16, DType.F32),      # the qwen3-coder engine
