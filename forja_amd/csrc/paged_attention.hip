@@ -1190,13 +1190,19 @@ __device__ inline void attend_item(const FastRagged &p, ErrorSlot *error, uint32
     for (int step = 0; step < 8; ++step) q[step] = load_query<kHalf, true>(p, q_row + 16 * step);
   }
   if (!(p.scale_log2 > 0.0f)) {
-    // A negative scale goes into the queries' signs, a zero one into their values: the largest product is
-    // then the largest score, and a masked one stays -inf.
-    const uint32_t flip = p.scale_log2 < 0.0f ? 0x80008000u : 0, keep = p.scale_log2 == 0.0f ? 0 : 0xffffffffu;
+    // A negative scale goes into the queries' signs, a zero one into their values (an infinity becomes the NaN that
+    // zero times it is): the largest product is then the largest score, and a masked one stays -inf.
+    const bool zero = p.scale_log2 == 0.0f;
+    const uint32_t flip = p.scale_log2 < 0.0f ? 0x80008000u : 0;
+    auto scaled = [&](uint32_t w) {
+      if (!zero) return w ^ flip;
+      constexpr uint32_t kExponent = kHalf ? 0x7c00u : 0x7f80u;
+      const bool lo = (w & kExponent) == kExponent, hi = (w >> 16 & kExponent) == kExponent;
+      return (lo ? 0x7fffu : 0u) | (hi ? 0x7fff0000u : 0u);
+    };
 #pragma unroll
     for (int step = 0; step < 8; ++step)
-      q[step] = make_uint4((q[step].x ^ flip) & keep, (q[step].y ^ flip) & keep, (q[step].z ^ flip) & keep,
-                           (q[step].w ^ flip) & keep);
+      q[step] = make_uint4(scaled(q[step].x), scaled(q[step].y), scaled(q[step].z), scaled(q[step].w));
   }
   f32x16 o[4];
 #pragma unroll

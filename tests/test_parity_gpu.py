@@ -1495,6 +1495,26 @@ def test_prefill_weight_of_the_largest_score_is_not_rounded(hip, pool, lead):
         assert np.abs(got[row] / (weights[64] / weights.sum()) - 1.0).max() <= 2.0 ** -18
 
 
+@pytest.mark.parametrize("dtype,pool", [(DType.BF16, DType.BF16), (DType.F32, DType.F16)])
+def test_prefill_with_a_zero_scale_keeps_queries_without_a_number(cpu, hip, dtype, pool):
+    """Every finite score is zero; zero times a NaN or an infinity is a NaN, and so is that row of that head.  (f32
+    queries beyond the f16 range of their pool are held at its largest number, infinities too: only the NaN there.)"""
+    infinities = dtype == pool
+    def build(backend):
+        t, inputs = ragged_case(backend, [3], [70], 16, 8, 16, seed=67, dtype=dtype, pool_dtype=pool)
+        queries = normal_bf16(67, 3, (70, 16, 128)).astype(np.float32)
+        queries[5, 2, 17] = np.nan
+        if infinities:
+            queries[40, 9, 126], queries[69, 0, 0] = np.inf, -np.inf
+        inputs[0] = upload(backend, queries, dtype)
+        commands = CommandList()
+        commands.dispatch_many(Op.paged_attention_ragged(0.0, 16), inputs, [t["out"], t["keys"], t["values"]])
+        return commands, [t["out"]]
+    (cpu_out, _), _ = differential(cpu, hip, build, bar=DType.F16 if dtype == DType.F32 else None)
+    nan = np.isnan(to_f32(cpu.read(cpu_out[0]), dtype).reshape(70, 16, 128))
+    assert nan[5, 2].all() and nan.sum() == (3 if infinities else 1) * 128
+
+
 DTYPE_MIXES = [
     # query and new rows, pools, output
     (DType.F32, DType.F16, DType.F32),      # the qwen3-coder engine
