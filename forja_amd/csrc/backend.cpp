@@ -581,7 +581,10 @@ fh_status bind_program(fh_backend *b, Program &p, const fh_tensor *inputs, uint3
       }
     } else {
       void *ptr = nullptr;
-      if (hipMalloc(&ptr, bytes) != hipSuccess) return FH_ALLOCATION_FAILED;
+      if (hipMalloc(&ptr, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return FH_ALLOCATION_FAILED;
+      }
       if (hipMemcpy(ptr, typed, bytes, hipMemcpyHostToDevice) != hipSuccess)
         return FH_DEVICE_EXECUTION_FAILED;
       device = (DInst *)ptr;
@@ -2660,6 +2663,8 @@ fh_status fh_write(fh_backend *b, fh_buffer buffer, uint64_t byte_offset, const 
         b->ring = (char *)ptr;
         b->ring_bytes = kRingBytes;
         b->ring_head = 0;
+      } else {
+        (void)hipGetLastError();
       }
     }
     if (b->ring) {
@@ -2672,10 +2677,9 @@ fh_status fh_write(fh_backend *b, fh_buffer buffer, uint64_t byte_offset, const 
       char *stage = b->ring + b->ring_head;
       memcpy(stage, bytes, len);
       b->ring_head += need;
-      if (len <= kMovedBytes) {
-        launch_move_bytes(b->stream, it->second.ptr + byte_offset, stage, (uint32_t)len);
-        return hipGetLastError() == hipSuccess ? FH_OK : FH_DEVICE_EXECUTION_FAILED;
-      }
+      if (len <= kMovedBytes &&
+          launch_move_bytes(b->stream, it->second.ptr + byte_offset, stage, (uint32_t)len) == hipSuccess)
+        return FH_OK;
       if (hipMemcpyAsync(it->second.ptr + byte_offset, stage, len, hipMemcpyHostToDevice,
                          b->stream) != hipSuccess)
         return FH_DEVICE_EXECUTION_FAILED;
@@ -2864,6 +2868,7 @@ fh_status fh_submission_profile(fh_submission *s, fh_dispatch_timing *out, uint3
 
 static fh_status submit_locked(fh_backend *b, const fh_dispatch *dispatches, uint32_t count, bool profiled,
                                fh_submission **out) {
+  (void)hipGetLastError();   // what stood before is not this submission's
   b->reap_dead_prepared();
   // Validate the whole list before anything is enqueued (lib.rs:1423-1432).
   for (uint32_t i = 0; i < count; ++i) {
@@ -2895,6 +2900,7 @@ static fh_status submit_locked(fh_backend *b, const fh_dispatch *dispatches, uin
     uint32_t capacity = std::max<uint32_t>(slots, 1024);
     if (hipMalloc(&dev, capacity * sizeof(ErrorSlot)) != hipSuccess ||
         hipHostMalloc(&host, capacity * sizeof(ErrorSlot), hipHostMallocCoherent) != hipSuccess) {
+      (void)hipGetLastError();
       if (dev) (void)hipFree(dev);
       if (host) (void)hipHostFree(host);
       delete s;
@@ -3027,6 +3033,7 @@ fh_status fh_submit_static(fh_backend *b, const fh_dispatch *dispatches, uint32_
   if ((uint64_t)count * sizeof(ErrorSlot) > kStaticErrorBytes) return fail(FH_QUOTA_EXCEEDED, count);
   std::lock_guard<std::mutex> lock(b->mutex);
   (void)hipSetDevice(b->device);
+  (void)hipGetLastError();   // what stood before is not this call's
   // From here on no allocator may run: scratch needs beyond the fixed regions fail instead.
   struct Regions {
     char *workspace, *accumulators, *route_plan, *attention_plan;

@@ -1116,16 +1116,18 @@ void launch_fill_u32(hipStream_t s, uint32_t *ptr, uint64_t count, uint32_t valu
   fill_u32_kernel<<<grid_for(count), kBlock, 0, s>>>(ptr, count, value);
 }
 
-void launch_move_bytes(hipStream_t s, void *to, const void *from, uint32_t bytes) {
-  if (bytes == 0) return;
+hipError_t launch_move_bytes(hipStream_t s, void *to, const void *from, uint32_t bytes) {
+  if (bytes == 0) return hipSuccess;
   const uint64_t all = (uint64_t)(uintptr_t)to | (uint64_t)(uintptr_t)from | bytes;
-  auto blocks = [&](uint32_t size) { return (bytes / size + 255) / 256; };
-  if (all % 16 == 0)
-    move_bytes_kernel<uint4><<<blocks(16), 256, 0, s>>>((const uint4 *)from, (uint4 *)to, bytes / 16);
-  else if (all % 4 == 0)
-    move_bytes_kernel<uint32_t><<<blocks(4), 256, 0, s>>>((const uint32_t *)from, (uint32_t *)to, bytes / 4);
-  else
-    move_bytes_kernel<uint8_t><<<blocks(1), 256, 0, s>>>((const uint8_t *)from, (uint8_t *)to, bytes);
+  const uint32_t size = all % 16 == 0 ? 16 : all % 4 == 0 ? 4 : 1;
+  const void *kernel = size == 16  ? reinterpret_cast<const void *>(&move_bytes_kernel<uint4>)
+                       : size == 4 ? reinterpret_cast<const void *>(&move_bytes_kernel<uint32_t>)
+                                   : reinterpret_cast<const void *>(&move_bytes_kernel<uint8_t>);
+  uint32_t pieces = bytes / size;
+  void *args[] = {&from, &to, &pieces};
+  const hipError_t status = hipLaunchKernel(kernel, dim3((pieces + 255) / 256), dim3(256), args, 0, s);
+  if (status != hipSuccess) (void)hipGetLastError();   // the caller has it
+  return status;
 }
 
 void launch_init_errors(hipStream_t s, ErrorSlot *slots, uint32_t count) {

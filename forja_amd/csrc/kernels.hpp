@@ -82,8 +82,8 @@ void launch_fill_seeded(hipStream_t s, const View &out, uint64_t elements, uint3
                         uint64_t seed, uint64_t stream, uint64_t first, float lo, float hi);
 void launch_fill_u32(hipStream_t s, uint32_t *ptr, uint64_t count, uint32_t value);
 void launch_init_errors(hipStream_t s, ErrorSlot *slots, uint32_t count);
-// Copies between device memory and pinned host memory (either side may be either).
-void launch_move_bytes(hipStream_t s, void *to, const void *from, uint32_t bytes);
+// Copies between device memory and pinned host memory (either side may be either).  Returns the launch's own status.
+hipError_t launch_move_bytes(hipStream_t s, void *to, const void *from, uint32_t bytes);
 
 // ---- moe.hip ----
 // counts [E], offsets [E+1], sorted_routes [R*k], blocks [max_blocks,3], n_blocks [1].

@@ -1,0 +1,55 @@
+"""What the library does on the host, on a HIP runtime without a device (fake_hip.cpp): kernels are only named, and a
+launch can be refused.  Each case runs in a process of its own, where that runtime stands in front of the real one."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PREAMBLE = """
+import ctypes, sys
+sys.path.insert(0, {root!r})
+fake = ctypes.CDLL({fake!r}, mode=ctypes.RTLD_GLOBAL)
+fake.fake_launched.restype = ctypes.c_char_p
+import numpy as np
+from forja_amd import programs
+from forja_amd.core import BackendError, CommandList, DType, Op
+from forja_amd.hip_backend import HipBackend, load_library
+hip = HipBackend(0)
+
+def launched():
+    names = fake.fake_launched().decode().split()
+    fake.fake_forget()
+    return names
+
+def refuse(part):
+    fake.fake_refuse(part.encode())
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    library = str(tmp_path_factory.mktemp("fake_hip") / "libfake_hip.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(ROOT, "tests", "fake_hip.cpp"), "-o", library], check=True)
+
+    def run(body):
+        script = PREAMBLE.format(root=ROOT, fake=library) + body
+        result = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True, timeout=120)
+        assert result.returncode == 0, result.stdout + result.stderr
+    return run
+
+
+def test_an_error_that_stood_before_a_call_is_not_its_own(fake):
+    """A HIP call that failed elsewhere in the program leaves its error until someone asks."""
+    fake("""
+t = hip.alloc(DType.U32, (4,))
+for call in (lambda: hip.write_array(t, np.arange(4, dtype=np.uint32)),
+             lambda: hip.submit(CommandList()).wait(),
+             lambda: hip.submit_static(CommandList())):
+    fake.fake_fail()
+    call()
+assert np.frombuffer(hip.read_buffer_range(t.buffer, 0, 16), np.uint32).tolist() == [0, 1, 2, 3]
+""")
