@@ -2703,8 +2703,8 @@ fh_status fh_read(fh_backend *b, fh_buffer buffer, uint64_t byte_offset, void *b
     return FH_INVALID_INPUT;
   if (len == 0) return FH_OK;
   (void)hipSetDevice(b->device);
-  if (char *stage = len <= kMovedBytes ? read_stage(b) : nullptr) {
-    launch_move_bytes(b->stream, stage, it->second.ptr + byte_offset, (uint32_t)len);
+  char *stage = len <= kMovedBytes ? read_stage(b) : nullptr;
+  if (stage && launch_move_bytes(b->stream, stage, it->second.ptr + byte_offset, (uint32_t)len) == hipSuccess) {
     if (hipStreamSynchronize(b->stream) != hipSuccess) return FH_DEVICE_EXECUTION_FAILED;
     memcpy(bytes, stage, len);
     return FH_OK;
@@ -2741,7 +2741,9 @@ fh_status fh_read_tensor(fh_backend *b, const fh_tensor *tensor, void *bytes, ui
     // 16-bit payloads are moved as raw bits by viewing them as u16 pairs is not possible with
     // arbitrary strides; the float path round-trips exactly (f16/bf16 -> f32 -> same dtype).
   }
+  (void)hipGetLastError();
   launch_copy(b->stream, source, flat, elements);
+  if (hipGetLastError() != hipSuccess) return FH_DEVICE_EXECUTION_FAILED;   // nothing has been gathered
   if (stage) {
     if (hipStreamSynchronize(b->stream) != hipSuccess) return FH_DEVICE_EXECUTION_FAILED;
     memcpy(bytes, stage, elements * size);
@@ -2995,19 +2997,21 @@ static fh_status submit_locked(fh_backend *b, const fh_dispatch *dispatches, uin
     }
     i += consumed;
   }
-  if (slots * sizeof(ErrorSlot) <= kMovedBytes)
-    launch_move_bytes(b->stream, s->host_errors, s->device_errors, slots * (uint32_t)sizeof(ErrorSlot));
-  else
-    (void)hipMemcpyAsync(s->host_errors, s->device_errors, slots * sizeof(ErrorSlot),
-                         hipMemcpyDeviceToHost, b->stream);
-  (void)hipEventRecord(s->end, b->stream);
+  hipError_t launch_error = hipGetLastError();
+  if (slots * sizeof(ErrorSlot) > kMovedBytes ||
+      launch_move_bytes(b->stream, s->host_errors, s->device_errors, slots * (uint32_t)sizeof(ErrorSlot)) != hipSuccess) {
+    const hipError_t copy_error =
+        hipMemcpyAsync(s->host_errors, s->device_errors, slots * sizeof(ErrorSlot), hipMemcpyDeviceToHost, b->stream);
+    if (launch_error == hipSuccess) launch_error = copy_error;
+  }
+  const hipError_t record_error = hipEventRecord(s->end, b->stream);
+  if (launch_error == hipSuccess) launch_error = record_error;
   if (status != FH_OK) {
     (void)hipStreamSynchronize(b->stream);
     recycle_submission(b, s);
     delete s;
     return status;
   }
-  hipError_t launch_error = hipGetLastError();
   if (launch_error != hipSuccess) {
     s->result = FH_DEVICE_EXECUTION_FAILED;
     s->error.code = FH_DEVICE_EXECUTION_FAILED;

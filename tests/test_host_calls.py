@@ -53,3 +53,28 @@ for call in (lambda: hip.write_array(t, np.arange(4, dtype=np.uint32)),
     call()
 assert np.frombuffer(hip.read_buffer_range(t.buffer, 0, 16), np.uint32).tolist() == [0, 1, 2, 3]
 """)
+
+
+def test_a_refused_move_is_noticed(fake):
+    """Bytes read are the buffer's, and a submission's error records are looked at, also where the kernel that moves
+    them is refused.  A gather that is refused fails the read, a dispatch the submission."""
+    fake("""
+t = hip.alloc(DType.U32, (64,))
+values = np.arange(64, dtype=np.uint32)
+for first in (0, 100):
+    refuse("" if first == 0 else "move_bytes")
+    hip.write_array(t, values + first)
+    assert np.frombuffer(hip.read_buffer_range(t.buffer, 0, 256), np.uint32).tolist() == (values + first).tolist()
+    hip.submit(CommandList()).wait()
+    assert fake.fake_standing() == 0
+copies = CommandList()
+copies.dispatch(Op.copy(), [t], hip.alloc(DType.U32, (64,)))
+for part, call in (("copy", lambda: hip.read(t)), ("copy", lambda: hip.submit(copies).wait()),
+                   ("kernel", lambda: hip.submit(copies).wait())):
+    refuse(part)
+    try:
+        call()
+        raise SystemExit("a refused kernel has not been noticed")
+    except BackendError:
+        pass
+""")
