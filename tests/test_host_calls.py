@@ -78,3 +78,28 @@ for part, call in (("copy", lambda: hip.read(t)), ("copy", lambda: hip.submit(co
     except BackendError:
         pass
 """)
+
+
+def test_which_reads_and_writes_a_kernel_moves(fake):
+    """Up to 16 KiB, in the widest pieces that address and length allow; the copies of the runtime beyond."""
+    fake("""
+t = hip.alloc(DType.U32, (1 << 15,))
+expected = bytearray(hip.read_buffer_range(t.buffer, 0, 1 << 17))
+lib, rng = load_library(), np.random.default_rng(3)
+widths = {16: "15HIP_vector_type", 4: "Ij", 1: "Ih"}
+for first, length in ((0, 16), (16, 4080), (4, 20), (32, 36), (1, 16), (16, 3), (0, 16384), (4, 16380), (7, 16377), (0, 16385),
+                      (8, 16388), (4, 65536), (0, 65537), (12, 100000)):
+    data = rng.bytes(length)
+    hip.synchronize()
+    launched()
+    assert lib.fh_write(hip._handle, t.buffer, first, data, length) == 0
+    wrote = launched()
+    expected[first:first + length] = data
+    assert hip.read_buffer_range(t.buffer, first, first + length) == data
+    read = launched()
+    width = next(w for w in widths if (first | length) % w == 0)
+    for names in (wrote, read):
+        assert len(names) == (length <= 16384), (first, length, names)
+        assert all(widths[width] in name and "move_bytes_kernel" in name for name in names), (first, length, names)
+assert hip.read_buffer_range(t.buffer, 0, 1 << 17) == bytes(expected)
+""")

@@ -81,6 +81,40 @@ def test_device_is_gfx950_and_storage_round_trips(hip):
         hip.read(t)                                             # released allocation
 
 
+@pytest.mark.parametrize("first,length", [(0, 16), (4, 20), (1, 16), (16, 3), (7, 16377), (0, 16384), (0, 16385), (4, 24572),
+                                          (8, 65528), (0, 65536), (3, 65537)])
+def test_bytes_moved_to_and_from_a_buffer(hip, first, length):
+    """Pieces of 16, 4 and 1 bytes by alignment, and both sides of the sizes that a kernel moves."""
+    t = hip.alloc(DType.U32, (1 << 15,))
+    rng = np.random.default_rng(length)
+    expected = bytearray(rng.bytes(1 << 17))
+    hip.write(t, bytes(expected))
+    data = rng.bytes(length)
+    assert hip._lib.fh_write(hip._handle, t.buffer, first, data, length) == 0
+    expected[first:first + length] = data
+    assert hip.read_buffer_range(t.buffer, first, first + length) == data
+    assert hip.read_buffer_range(t.buffer, 0, 1 << 17) == bytes(expected)
+    view = t.narrow(0, first, (length + 3) // 4)   # (gathered on the device)
+    assert hip.read(view) == bytes(expected[4 * first:4 * (first + (length + 3) // 4)])
+    hip.release(t)
+
+
+def test_error_records_are_clear_again_after_an_error(hip):
+    """Records of a submission without an error are used again as they are, those of one that raised one are cleared."""
+    ids, out, table = hip.alloc(DType.U32, (1,)), hip.alloc(DType.BF16, (1, 64)), Quantised(68, 0, (4, 64)).upload(hip)
+    commands = CommandList()
+    for _ in range(3):
+        commands.dispatch(Op.quant_embed(4, 64), [*table, ids], out)
+    for index in (3, 9, 2, 1, 7, 8, 0):
+        hip.write_array(ids, np.array([index], np.uint32))
+        if index < 4:
+            run(hip, commands)
+            continue
+        with pytest.raises(BackendError) as info:
+            run(hip, commands)
+        assert info.value.status == Status.INDEX_OUT_OF_RANGE and info.value.index == index and info.value.dispatch == 0
+
+
 def test_submit_refuses_foreign_tensors_and_bad_shapes(hip):
     x = hip.alloc(DType.BF16, (4, 64))
     out = hip.alloc(DType.BF16, (4, 8))
