@@ -143,8 +143,9 @@ struct KsplitDense {
   uint16_t *activated;
   uint64_t activated_row_stride;
 };
-// Whether the fused forms of the dense kernel take a product (columns: of one half with `pair`).
-bool ksplit_fuses(uint32_t rows, uint32_t inner, uint32_t columns, bool pair);
+// Whether the dense kernel is to take a product together with the silu behind it (`pair`; columns: of one half) and
+// the normalisation in front of it (`norm`, or null).
+bool ksplit_fuses(fh_backend *backend, uint32_t rows, uint32_t inner, uint32_t columns, bool pair, const NormHead *norm);
 // Whether launch_ksplit_dense takes a product of `rows` rows: at most 128, in row tiles of 16 or
 // 32, and more than one tile only for weights small enough to stay cached between the tiles.
 bool ksplit_dense_supports(uint32_t rows, uint32_t inner, uint32_t columns, bool wide = false);

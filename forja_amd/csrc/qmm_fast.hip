@@ -1269,7 +1269,7 @@ bool try_fused_quant_matmul(fh_backend *backend, const QmmProblem &p, const Norm
   if (!weights_eligible(p.packed, p.scales, p.biases, 2, p.inner, p.bits, p.group)) return false;
   if (p.x.stride[1] != 1 || p.x.stride[0] % 8 != 0 || p.x.offset % 8 != 0 || p.out.stride[1] != 1) return false;
   const uint32_t columns = activated ? p.columns / 2 : p.columns;
-  if (!ksplit_fuses(p.rows, p.inner, columns, activated != nullptr)) return false;
+  if (!ksplit_fuses(backend, p.rows, p.inner, columns, activated != nullptr, norm)) return false;
   KsplitDense d{};
   d.x = u16_ptr(p.x);
   d.x_row_stride = p.x.stride[0];

@@ -157,19 +157,16 @@ constexpr int resident_waves(int waves, int row_tiles, int groups, bool routed, 
 // the product with the f32 value itself.  The stationary rows then take three times the
 // registers: one 16-row tile, one workgroup per compute unit.
 //
-// kNorm (dense, one row tile): the rows are the RMS normalisation the dispatch in front of the product
-// computes from x (+ update), and every workgroup makes them itself from the sums its waves exchange
-// through LDS, while its first weights are on their way; between them they also store what that
-// dispatch stores.  A normalisation of a few rows is a launch of 3 us whose bytes every workgroup can read from
-// L2 in less.  kPair of a dense product: columns c and c + columns of one gate/up matrix, whose
-// silu(gate) * up, the element program behind it, the epilogue stores beside the two.  Measured, with a
-// layer of one row of 1024 against 4096 and 2 x 3072 columns: normalisation + product 2.9 + 7.4 us in two
-// launches and 6.0 in one, normalisation + product + silu 3.2 + 7.4 + 2.5 and 6.7; 23 rows 3.0 + 8.4
-// and 8.3, 4.4 + 9 + 3.8 and 12.3.
+// kNorm (dense, up to 32 rows, K slices of two groups): the rows are the RMS normalisation the dispatch in
+// front of the product computes from x (+ update), and every workgroup makes them itself from the sums its
+// waves exchange through LDS, while its first weights are on their way; between them they also store what
+// that dispatch stores.  A normalisation of a few rows is a launch of 3 us whose bytes every workgroup can
+// read from L2 in less (ksplit_fuses: where it does).  kPair of a dense product: columns c and c + columns of
+// one gate/up matrix, whose silu(gate) * up, the element program behind it, the epilogue stores beside the two.
 template <int WAVES, int G, int RT, bool kPair, bool kRouted, int XP, bool kNorm, int CT>
 __global__ __launch_bounds__(64 * WAVES, resident_waves(WAVES, RT, G, kRouted, XP)) void qmm_ksplit_kernel(KsplitArgs a) {
   static_assert(XP == 1 || (XP == 3 && RT == 1), "f32 rows: one row tile");
-  static_assert(!kNorm || (XP == 1 && !kRouted), "normalised rows: bf16, dense");
+  static_assert(!kNorm || (XP == 1 && !kRouted && G == 2), "normalised rows: bf16, dense, short");
   constexpr int P = kPair ? 2 : 1;
   constexpr int NS = ring_slots(RT, G, kRouted);
   constexpr int kBatchCols = 16 * CT;
@@ -785,19 +782,24 @@ bool ksplit_shape(uint32_t inner, int *waves, int *groups) {
   }
 }
 
+// Dense products of few columns: batches of one column tile where wide ones (of `tiles`) would leave compute
+// units without a workgroup.  Such a launch is one chain of latencies per workgroup, and a narrow batch's is
+// shorter (1 row: 1024 -> 4096 8.6 us wide and 6.2 narrow, 2048 -> 1024 6.7 and 5.6, 3072 -> 1024 7.7 and
+// 6.2; 23 rows 1024 -> 4096 16.3 and 10.7).  Beyond two workgroups a compute unit the wide batches' longer
+// streams win (their fixed costs, and in the 16-row form the coalesced scales, are shared by more columns).
+bool narrow_batches(fh_backend *backend, uint64_t wide, uint32_t tiles) {
+  const uint64_t compute_units = backend_compute_units(backend);
+  return wide < compute_units && wide * tiles <= 2 * compute_units;
+}
+
 // One launch: as many workgroups as stay resident at once (the runtime's own occupancy figure for
 // this instantiation), never more than there are units of work.
 template <int WAVES, int G, int RT, bool kPair, bool kRouted, int XP, bool kNorm, int CT = batch_tiles(kPair, G)>
 void launch_one(fh_backend *backend, const KsplitArgs &a, uint64_t most_units) {
   constexpr int P = kPair ? 2 : 1;
-  // Dense products of few columns: batches of one column tile where wide ones would leave compute
-  // units without a workgroup.  Such a launch is one chain of latencies per workgroup, and a narrow batch's is
-  // shorter (1 row: 1024 -> 4096 8.6 us wide and 6.2 narrow, 2048 -> 1024 6.7 and 5.6, 3072 -> 1024 7.7 and
-  // 6.2; 23 rows 1024 -> 4096 16.3 and 10.7).  Beyond two workgroups a compute unit the wide batches' longer
-  // streams win (their fixed costs, and in the 16-row form the coalesced scales, are shared by more columns).
   if constexpr ((!kRouted || (XP == 3 && !kPair && G == 4 && WAVES == 8)) && CT > 1) {
     const uint64_t narrow = most_units * CT;
-    if ((!kRouted || a.weight_inner != a.inner) && most_units < backend_compute_units(backend) && narrow <= 2 * backend_compute_units(backend)) {
+    if ((!kRouted || a.weight_inner != a.inner) && narrow_batches(backend, most_units, CT)) {
       KsplitArgs n = a;
       n.batches_per_tile = a.batches_per_tile * CT;
       launch_one<WAVES, G, RT, kPair, kRouted, XP, kNorm, 1>(backend, n, narrow);
@@ -828,9 +830,17 @@ bool launch_shape(fh_backend *backend, const KsplitArgs &a, uint64_t most_units)
   case 4 * 16 + 2: launch_one<4, 2, RT, kPair, kRouted, XP, kNorm>(backend, a, most_units); return true;
   case 6 * 16 + 2: launch_one<6, 2, RT, kPair, kRouted, XP, kNorm>(backend, a, most_units); return true;
   case 8 * 16 + 2: launch_one<8, 2, RT, kPair, kRouted, XP, kNorm>(backend, a, most_units); return true;
-  case 6 * 16 + 4: launch_one<6, 4, RT, kPair, kRouted, XP, kNorm>(backend, a, most_units); return true;
-  case 8 * 16 + 4: launch_one<8, 4, RT, kPair, kRouted, XP, kNorm>(backend, a, most_units); return true;
   default: break;
+  }
+  if constexpr (!kNorm) {
+    if (waves * 16 + groups == 6 * 16 + 4) {
+      launch_one<6, 4, RT, kPair, kRouted, XP, false>(backend, a, most_units);
+      return true;
+    }
+    if (waves * 16 + groups == 8 * 16 + 4) {
+      launch_one<8, 4, RT, kPair, kRouted, XP, false>(backend, a, most_units);
+      return true;
+    }
   }
   if constexpr (!kRouted && XP == 1 && !kPair && !kNorm) {   // the long rows of dense decode products
     if (waves == 8 && groups == 6) {
@@ -871,11 +881,34 @@ bool ksplit_dense_supports(uint32_t rows, uint32_t inner, uint32_t columns, bool
   return rows <= tile_rows || (groups <= 4 && (uint64_t)columns * inner / 2 <= kCachedWeightBytes);
 }
 
-// The fused forms hold their rows in one tile of a K slice of at most four groups.
-bool ksplit_fuses(uint32_t rows, uint32_t inner, uint32_t columns, bool pair) {
+// The silu behind a gate/up product is always the cheaper in the product's epilogue (microseconds together and
+// apart: 1 row of 1024 against 2 x 3072 columns 6.2 and 8.9, 32 rows 8.9 and 14.0; 2048 against 2 x 6144 11.2 and 14.1, 15.6 and
+// 18.4).  The normalisation in front gains a launch and costs every workgroup the rows' bytes, registers and
+// arithmetic before its first product, twice as much with a residual sum:
+//   * K beyond 1024: the rows' raw words do not fit beside the weights in flight (K 2048, 5120 columns: 1 row 13.3
+//     together and 8.8 apart, 32 rows with the sum 17.5 and 13.0).
+//   * the sum over two row tiles: apart (32 rows, K 1024, 4096 columns 10.2 and 8.6), but for K 512 (7.3 and 7.6; with
+//     silu behind 8.0 in one, 7.7 with the normalisation alone apart, 9.6 in three).
+//   * the sum over one, and nothing behind the product to save a second launch: two workgroups that share a
+//     compute unit make the rows twice there.  Narrow batches from 5 rows on (K 1024, 6144 columns: 4 rows 7.6 and 7.8, 8
+//     rows 8.4 and 8.1, 16 rows 9.6 and 8.7; 4096 columns, one workgroup, 6.9 and 7.6), wide ones from 9 on (32768
+//     columns: 8 rows 12.5 and 13.0, 16 rows 13.7 and 13.4), until each has many (65536: 0.98 of the time apart); K 512
+//     gains anywhere.
+bool ksplit_fuses(fh_backend *backend, uint32_t rows, uint32_t inner, uint32_t columns, bool pair, const NormHead *norm) {
   int waves = 0, groups = 0;
   if (rows == 0 || rows > 32 || !ksplit_shape(inner, &waves, &groups) || groups > 4) return false;
-  return ksplit_supports(inner, columns, pair, false);
+  if (!ksplit_supports(inner, columns, pair, false)) return false;
+  if (!norm) return true;
+  if (groups > 2) return false;
+  if (!norm->update) return true;
+  if (inner <= 512) return true;
+  if (rows > 16) return false;
+  if (pair) return true;
+  const uint64_t compute_units = backend_compute_units(backend);
+  const uint32_t tiles = batch_tiles(false, groups);
+  const uint64_t wide = columns / (16 * tiles);
+  if (narrow_batches(backend, wide, tiles)) return wide * tiles <= compute_units || rows <= 4;
+  return wide <= compute_units || wide >= 4 * compute_units || rows <= 8;
 }
 
 bool launch_ksplit_dense(fh_backend *backend, const KsplitDense &d) {
@@ -884,7 +917,7 @@ bool launch_ksplit_dense(fh_backend *backend, const KsplitDense &d) {
   if (d.wide && !d.out_f32) return false;
   if ((d.norm || d.activated) &&
       (d.wide || d.weight_inner || (d.activated && (d.residual || d.out_f32)) ||
-       !ksplit_fuses(d.rows, d.inner, d.columns, d.activated != nullptr)))
+       !ksplit_fuses(backend, d.rows, d.inner, d.columns, d.activated != nullptr, d.norm)))
     return false;
   const bool wide_tiles = d.rows > 16 && groups <= 6 && !d.wide;
   KsplitArgs a{};

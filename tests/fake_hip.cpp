@@ -1,6 +1,6 @@
 // A HIP runtime without a device, for tests of what the library does on the host: which kernels it launches, and what
 // becomes of a launch that is refused.  Memory is the host's, streams finish at once, and of the kernels only those
-// that move bytes do anything.  An event's time is the number of launches and asynchronous copies before it, in ms.
+// that move bytes and clear error records do anything.  An event's time is the number of launches and asynchronous copies before it, in ms.
 #include <hip/hip_runtime_api.h>
 
 #include <cstdlib>
@@ -67,6 +67,7 @@ hipError_t hipLaunchKernel(const void *host, dim3 grid, dim3, void **args, size_
   if (name.find("move_bytes_kernelIh") != std::string::npos) move<uint8_t>(args);
   else if (name.find("move_bytes_kernelIj") != std::string::npos) move<uint32_t>(args);
   else if (name.find("move_bytes_kernel") != std::string::npos) move<uint32_t[4]>(args);
+  else if (name.find("init_errors_kernel") != std::string::npos) memset(*(void **)args[0], 0, *(uint32_t *)args[1] * 8);   // {flag, value}
   return hipSuccess;
 }
 hipError_t hipGetLastError() {

@@ -103,3 +103,41 @@ for first, length in ((0, 16), (16, 4080), (4, 20), (32, 36), (1, 16), (16, 3), 
         assert all(widths[width] in name and "move_bytes_kernel" in name for name in names), (first, length, names)
 assert hip.read_buffer_range(t.buffer, 0, 1 << 17) == bytes(expected)
 """)
+
+
+@pytest.mark.parametrize("rows,n,k,form,expected", [
+    # the normalisation in front: K up to 1024 ..
+    (1, 6144, 1024, "norm", [2]), (16, 4096, 1024, "norm", [2]), (32, 4096, 768, "norm", [2]), (33, 4096, 1024, "norm", [1, 1]),
+    (8, 5120, 2048, "norm", [1, 1]), (1, 2560, 1536, "res", [1, 1]),
+    # .. with the residual sum over one row tile where a compute unit has one workgroup, rows are few or batches many
+    (16, 4096, 768, "res", [2]), (16, 8192, 512, "res", [2]), (17, 4096, 768, "res", [1, 1]), (32, 1024, 512, "res", [2]),
+    (4, 4160, 1024, "res", [2]), (5, 4160, 1024, "res", [1, 1]), (16, 8192, 1024, "res", [1, 1]), (16, 8256, 1024, "res", [2]),
+    (16, 16384, 1024, "res", [2]), (8, 16448, 1024, "res", [2]), (9, 16448, 1024, "res", [1, 1]), (16, 65536, 1024, "res", [2]),
+    # silu behind: wherever the kernel takes the product
+    (16, 6144, 1024, "res-silu", [3]), (32, 6144, 1024, "norm-silu", [3]), (17, 6144, 1024, "res-silu", [1, 2]),
+    (17, 6144, 512, "res-silu", [3]), (8, 6144, 2048, "norm-silu", [1, 2]), (32, 4096, 1536, "silu", [2]),
+    (33, 6144, 1024, "res-silu", [1, 1, 1]), (4, 6144, 3072, "norm-silu", [1, 1, 1]), (4, 1008, 1024, "norm-silu", [1, 1, 1]),
+    # not the rows the product reads, or not the halves of what it makes
+    (4, 4096, 1024, "other-rows", [1, 1]), (4, 4096, 1024, "norm-other-halves", [2, 1])])
+def test_which_row_programs_a_dense_product_takes_in(fake, rows, n, k, form, expected):
+    """Dispatches of a joined group share one entry of the profile."""
+    fake(f"""
+rows, n, k, form, expected = {rows}, {n}, {k}, {form!r}, {expected}
+x, u, normed, added, other = (hip.alloc(DType.BF16, (rows, k)) for _ in range(5))
+w = hip.alloc(DType.BF16, (k,)).broadcast((rows, k))
+weights = [hip.alloc(DType.U32, (n, k // 8)), *(hip.alloc(DType.BF16, (n, k // 64)) for _ in range(2))]
+out, activated = hip.alloc(DType.BF16, (rows, n)), hip.alloc(DType.BF16, (rows, n // 2))
+commands = CommandList()
+if "res" in form:
+    commands.dispatch_kernel(hip.prepare_program(programs.residual_norm_rows(1e-6)), [x, u, w], [added, normed])
+elif form != "silu":
+    commands.dispatch_kernel(hip.prepare_program(programs.rms_norm_rows(1e-6)), [x, w], [normed])
+commands.dispatch(Op.quant_matmul(4, 64), [other if form == "other-rows" else normed, *weights], out)
+if "silu" in form or "halves" in form:
+    halves = [out.narrow(1, 0, n // 2), out.narrow(1, n // 2, n // 2)]
+    commands.dispatch_kernel(hip.prepare_program(programs.silu_mul_elements()), halves if "silu" in form else halves[::-1], [activated])
+submission = hip.submit_profiled(commands)
+submission.wait()
+got = [entry[1] for entry in submission.profile()]
+assert got == expected, got
+""")

@@ -911,6 +911,18 @@ def test_dense_products_with_the_row_programs_around_them(cpu, hip, rows, n, k, 
         return commands, outputs if form != "silu" else outputs[1:]
     # silu of halves multiplies two results of one ulp each
     differential(cpu, hip, build, rel=2e-2, abs_=2e-2)
+    # dispatches that run as one share an entry of the profile
+    takes_rows = (rows, n, k) in ((1, 1024, 1024), (16, 64, 768), (5, 32768, 1024))
+    takes_silu = (rows, n, k) in ((1, 1024, 1024), (32, 256, 2048), (5, 32768, 1024))
+    groups = {"norm": [2] if takes_rows else [1, 1], "residual_norm": [2] if takes_rows else [1, 1],
+              "residual_norm_silu": [3] if takes_rows and takes_silu else [1, 2] if takes_silu else [2, 1] if takes_rows
+              else [1, 1, 1],
+              "silu": [2] if takes_silu else [1, 1], "norm_add": [2] if takes_rows else [1, 1], "sum_added": [2] if takes_rows and n > k else [1, 1],
+              "over_the_rows": [2] if takes_rows and n > k else [1, 1], "other_rows": [1, 1],
+              "other_halves": [2, 1] if takes_rows else [1, 1, 1]}
+    submission = hip.submit_profiled(build(hip)[0])
+    submission.wait()
+    assert [entry[1] for entry in submission.profile()] == groups[form]
 
 
 @pytest.mark.parametrize("rows,n", [(1, 2048), (8, 2048), (16, 96), (17, 96), (3, 40)])
@@ -944,6 +956,9 @@ def test_f32_product_of_long_rows_and_the_residual_normalisation_behind_it(cpu, 
     for commands in apart:
         run(hip, commands)
     assert together == [hip.read(t) for t in tensors]
+    submission = hip.submit_profiled(joined)
+    submission.wait()
+    assert [entry[1] for entry in submission.profile()] == ([1, 1] if (rows, n) in ((17, 96), (3, 40)) else [2])
 
 
 @pytest.mark.parametrize("with_residual", [False, True])
