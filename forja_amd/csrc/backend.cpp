@@ -2942,6 +2942,7 @@ static fh_status submit_locked(fh_backend *b, const fh_dispatch *dispatches, uin
     uint32_t consumed = 1;
     LaneRun run;
     const uint32_t op = dispatches[i].op;
+    uint32_t timed_as = op;
     const bool candidate = b->lane_fusion && (op == FH_OP_PAGED_SDPA_APPEND || op == FH_OP_PAGED_COPY) &&
                            i >= no_run_before;
     // a run that brings prefill chunks first (it takes one-row members too), else one of one-row members
@@ -2973,6 +2974,7 @@ static fh_status submit_locked(fh_backend *b, const fh_dispatch *dispatches, uin
     } else if (const uint32_t together = op == FH_OP_PROGRAM || op == FH_OP_QUANT_MATMUL
                                              ? run_dense_group(b, dispatches, count, i) : 0) {
       consumed = together;
+      timed_as = FH_OP_QUANT_MATMUL;   // whatever comes first
       for (uint32_t member = 1; member < consumed; ++member) s->ops[i + member] = dispatches[i + member].op;
     } else {
       NormTail tail;
@@ -2996,7 +2998,7 @@ static fh_status submit_locked(fh_backend *b, const fh_dispatch *dispatches, uin
       if (profiled)
         s->spans.push_back({i, consumed, dispatches[i].op, t0, t1});
       else
-        b->timed.push_back({t0, t1, fused ? (uint32_t)FH_KC_ATTENTION : kernel_class_of(dispatches[i].op)});
+        b->timed.push_back({t0, t1, fused ? (uint32_t)FH_KC_ATTENTION : kernel_class_of(timed_as)});
     }
     i += consumed;
   }

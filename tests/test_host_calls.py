@@ -141,3 +141,16 @@ submission.wait()
 got = [entry[1] for entry in submission.profile()]
 assert got == expected, got
 """)
+
+
+def test_a_product_joined_with_its_normalisation_is_timed_as_a_product(fake):
+    fake("""
+x, normed, out = (hip.alloc(DType.BF16, (4, 1024)) for _ in range(3))
+weights = [hip.alloc(DType.U32, (1024, 128)), *(hip.alloc(DType.BF16, (1024, 16)) for _ in range(2))]
+commands = CommandList()
+commands.dispatch_kernel(hip.prepare_program(programs.rms_norm_rows(1e-6)), [x, hip.alloc(DType.BF16, (1024,)).broadcast((4, 1024))], [normed])
+commands.dispatch(Op.quant_matmul(4, 64), [normed, *weights], out)
+hip.profile_enable(2)
+hip.submit(commands).wait()
+assert [hip.profile_read(kernel_class)[1] for kernel_class in (0, 1)] == [0, 1]   # other, products
+""")
