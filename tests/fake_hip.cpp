@@ -75,13 +75,13 @@ hipError_t hipGetLastError() {
   standing = hipSuccess;
   return code;
 }
-hipError_t hipMalloc(void **ptr, size_t bytes) { return (*ptr = aligned_alloc(256, (bytes + 255) / 256 * 256)) ? hipSuccess : fails(hipErrorOutOfMemory); }
-hipError_t hipFree(void *ptr) { return free(ptr), hipSuccess; }
-hipError_t hipHostMalloc(void **ptr, size_t bytes, unsigned int) {
-  if (hipMalloc(ptr, bytes) != hipSuccess) return hipErrorOutOfMemory;
-  memset(*ptr, 0, bytes);
-  return hipSuccess;
+hipError_t hipMalloc(void **ptr, size_t bytes) {
+  bytes = (bytes + 255) / 256 * 256;
+  *ptr = aligned_alloc(256, bytes);
+  return *ptr ? memset(*ptr, 0, bytes), hipSuccess : fails(hipErrorOutOfMemory);
 }
+hipError_t hipFree(void *ptr) { return free(ptr), hipSuccess; }
+hipError_t hipHostMalloc(void **ptr, size_t bytes, unsigned int) { return hipMalloc(ptr, bytes); }
 hipError_t hipHostFree(void *ptr) { return free(ptr), hipSuccess; }
 hipError_t hipMemcpy(void *to, const void *from, size_t bytes, hipMemcpyKind) { return memcpy(to, from, bytes), hipSuccess; }
 hipError_t hipMemcpyAsync(void *to, const void *from, size_t bytes, hipMemcpyKind, hipStream_t) {

@@ -154,3 +154,29 @@ hip.profile_enable(2)
 hip.submit(commands).wait()
 assert [hip.profile_read(kernel_class)[1] for kernel_class in (0, 1)] == [0, 1]   # other, products
 """)
+
+
+@pytest.mark.parametrize("lanes,pad,placed", [(1, 0, True), (4, 4, True), (4, 2, False), (128, 0, True), (129, 0, False)])
+def test_who_places_the_lanes_rows(fake, lanes, pad, placed):
+    """The merge where the destinations are aligned to four elements and one launch takes the lanes, else a scatter."""
+    fake(f"""
+lanes, pad, placed = {lanes}, {pad}, {placed}
+from tests.test_lane_fusion_gpu import LaneBatch
+batch = LaneBatch(hip, [5 + lane % 7 for lane in range(lanes)], 8, 2, 16, seed=1)
+width = 8 * 128
+target = hip.alloc(DType.BF16, (lanes, width + pad))
+commands = CommandList()
+for lane in range(lanes):
+    row = hip.alloc(DType.BF16, (1, 8, 128))
+    commands.dispatch_many(Op.paged_sdpa_append(0.09, 5 + lane % 7, 16),
+                           [batch.q.narrow(0, lane, 1).permute([1, 0, 2]), batch.k.narrow(0, lane, 1),
+                            batch.v.narrow(0, lane, 1), batch.tables[lane], batch.generations],
+                           [row.permute([1, 0, 2]), *batch.pools[0]])
+    commands.dispatch(Op.copy(), [row.reshape((1, width))], target.narrow(0, lane, 1).narrow(1, 0, width))
+launched()
+hip.submit(commands).wait()
+assert hip.fusion_stats() == (1, 2 * lanes)
+names = launched()
+assert sum("ragged_reduce_kernelILb1" in name for name in names) == placed, names
+assert any("scatter_lane_rows" in name for name in names) == (not placed), names
+""")
