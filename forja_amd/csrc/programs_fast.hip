@@ -289,7 +289,7 @@ __device__ inline void store2(void *base, uint64_t element, float a, float b) {
 
 template <bool kWide>
 __global__ __launch_bounds__(256) void qk_norm_rope_rows_kernel(QkArgs a) {
-  __shared__ float2 turns[64];
+  __shared__ __attribute__((aligned(16))) float2 turns[64];
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane >> 5, at = 2 * (lane & 31);
   const uint64_t row = blockIdx.x;
   constexpr int kAhead = 5;
