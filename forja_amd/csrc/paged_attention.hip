@@ -307,7 +307,7 @@ typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 constexpr uint32_t kMinSplitTokens = 128, kMaxSplitTokens = 1024;  // split length bounds
-// see ragged_plan_kernel (512 groups: two for each of the 256 compute units)
+// see ragged_plan_kernel (512 groups: two for each of the 256 compute units that an MI355X has)
 constexpr uint32_t kFillingGroups = 512, kFilledSplitTokens = 512;
 // Groups of several query tokens (prefill) are many and each split of theirs costs a merge of
 // `members x heads` partial rows: they are split only beyond this many keys.
@@ -509,7 +509,8 @@ __global__ __launch_bounds__(kPlanThreads) void ragged_plan_kernel(FastRagged p,
     }
   }
   if (threadIdx.x == 0) p.item_count[2] = 0;
-  // Every token's record, `chunk` holding the keys of its group; a thread reads back its own only.
+  // Every token's record, `chunk` holding the keys of its group; a thread reads back its own, and the
+  // search for the split length, behind a barrier, those beyond what LDS holds.
   {
     unsigned long long mine = 0;
     uint32_t mine_longest = 0, mine_group = 0, mine_groups = 0;
@@ -974,13 +975,13 @@ __device__ inline void attend_one_token(const FastRagged &p, ErrorSlot *error, c
 // What bounds it: the tiles' way in (alone 72 of 95 us where 2048 rows in three chunks behind 1024 keys and 32 decode
 // rows attend with 32 heads) and the chain of one wave's tile, scores, softmax and value product (alone
 // 75 us), of which two waves per SIMD overlap a part.  Hence 32 x 32 products (a tile's LDS bytes serve
-// twice the rows of 16 x 16 ones), one query row to a lane pair (a maximum is 31 comparisons and one
-// exchange), operands read from LDS four products ahead, V transposed on the way out of LDS.
-// Against 16-row waves that waited for each tile: that batch 186 -> 92 us, 8192 rows in six chunks with 64
-// decode rows (40 heads) 567 -> 235, 512 rows of f32 (32 heads) 44 -> 21, 2000 rows in four chunks with 48
-// decode rows (16 heads) 89 -> 66.
-// Eight waves of 32 rows and four tiles in LDS (three on their way) took 99, 265, 27 and 88 us: the decode rows of a
-// batch keep one wave busy, and one workgroup per compute unit leaves nothing beside it.
+// twice the rows of 16 x 16 ones), one query row to a lane pair (the maximum of 32 keys is 15 comparisons and
+// one exchange), operands read from LDS four products ahead, V transposed on the way out of LDS.
+// Against 16-row waves that waited for each tile: that batch 186 -> 99 us, 8192 rows in six chunks with 64
+// decode rows (40 heads) 567 -> 260, 512 rows of f32 (32 heads) 44 -> 23, 2000 rows in four chunks with 48
+// decode rows (16 heads) 89 -> 65.  (With maxima that lag, which rounds the largest weights: 95, 240, 21 and 64.)
+// Eight waves of 32 rows and four tiles in LDS (three on their way) took 99, 265, 27 and 88 us with lagging maxima:
+// the decode rows of a batch keep one wave busy, and one workgroup per compute unit leaves nothing beside it.
 //
 // Rows are 256 bytes (one head of one token).  The 16-byte piece p of K row r sits in slot p ^ (r & 15):
 // 16 rows read at one piece use all banks once.  Piece p of V row r sits in slot
@@ -1297,8 +1298,8 @@ __device__ inline void attend_item(const FastRagged &p, ErrorSlot *error, uint32
 
 // Items longest first, the kv heads of an item side by side: with 8 (or 4, 2, 1) kv heads a head's items
 // meet in the L2 of one XCD, as workgroups go to the XCDs in turn, and the launch ends on its shortest.
-// (8192 prompt rows in six chunks and 64 decode rows, 8 kv heads: 241 us, and 447 us where workgroups
-// take the next entry wherever they are.)
+// (8192 prompt rows in six chunks and 64 decode rows, 8 kv heads, lagging maxima: 241 us, and 447 us where
+// workgroups take the next entry wherever they are.)
 template <bool kHalf, bool kMixed>
 __global__ __launch_bounds__(64 * kPrefillWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void ragged_attention_prefill_kernel(
     FastRagged p, ErrorSlot *error) {
@@ -1566,7 +1567,7 @@ void launch_fast(fh_backend *backend, hipStream_t stream, const FastRagged &f, E
   const bool mixed = mixed_dtypes(f);
   {
     KernelTimer timer(backend, FH_KC_ATTENTION_KERNEL);
-    // one workgroup per work item, up to 8 (decode) or 4 (prefill) kv heads of it per workgroup
+    // decode: a workgroup takes up to 8 kv heads of an item; prefill: one kv head of one
     if (f.group_tokens > 1) {
       const uint64_t most = (uint64_t)kPrefillGrid * backend_compute_units(backend);
       const dim3 grid((unsigned)std::min(items * f.kv_heads, most));

@@ -609,7 +609,9 @@ bool try_fast_program(hipStream_t stream, const ProgramClass &cls, const Program
     a.eps = cls.c[1];
     a.theta = cls.c[2];
     a.exponent_scale = cls.c[3];
-    // From two workgroups for every compute unit on (below, a wave to a head is the shorter chain).
+    // Many rows: a workgroup to a row, its angles formed once.  Few: a wave to a head is the shorter chain (us, by rows
+    // and by heads: bf16, 24 heads, 64 rows 4.4 and 3.5, 256 4.5 and 5.4, 512 4.9 and 8.1; 48 heads 6.0 and 3.8, 6.4 and
+    // 8.0, 7.3 and 11.1; f32 the same within 1.5).  The two meet near 200 rows.
     bool pairs = a.width == 64 && a.pos_s[1] == 0 && a.rows >= 512;
     for (const View *v : {&p.inputs[0], &p.inputs[1], &p.inputs[2], &p.inputs[3], &p.outputs[0], &p.outputs[1]})
       pairs = pairs && v->offset % 2 == 0 && v->stride[0] % 2 == 0 && v->stride[1] % 2 == 0;

@@ -232,13 +232,15 @@ FH_API fh_status fh_submit_static(fh_backend *backend, const fh_dispatch *dispat
                            fh_error *error);
 /* Submission::wait / wait_timeout (backend.rs:609-647).  timeout_ns 0 = no deadline. */
 FH_API fh_status fh_wait(fh_submission *submission, uint64_t timeout_ns, fh_error *error);
-/* Submission::gpu_time: device time between the first and last kernel, in ns (0 before wait). */
+/* Submission::gpu_time: device time from the first kernel to the end of the last, in ns (0 before wait).  The
+ * last is the one that moves the submission's error records into host memory, about 2 us. */
 FH_API uint64_t fh_gpu_time_ns(fh_submission *submission);
 FH_API void fh_submission_free(fh_submission *submission);
 
 /* Backend::submit_profiled_retained (backend.rs:813-857): fh_submit with one device timer
  * around every dispatch it executes.  A run of dispatches executed together (per-lane attention
- * fused into one ragged launch, a weighted sum with the normalisation that follows it) gets one
+ * fused into one ragged launch, a weighted sum with the normalisation that follows it, a product of a
+ * few rows with the normalisation in front of it, the silu or the residual normalisation behind it) gets one
  * timer.  The timers cost two event records per dispatch on the stream. */
 FH_API fh_status fh_submit_profiled(fh_backend *backend, const fh_dispatch *dispatches, uint32_t count,
                              fh_submission **out);

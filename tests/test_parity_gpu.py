@@ -1841,8 +1841,8 @@ def test_engine_row_programs(cpu, hip, dtype):
 @pytest.mark.parametrize("rows,heads", [(512, 3), (1029, 24)])
 @pytest.mark.parametrize("dtype", [DType.BF16, DType.F32])
 def test_head_norm_and_rotation_over_many_rows(cpu, hip, rows, heads, dtype):
-    """Four rows to a workgroup, two heads to a wave: an odd number of heads, rows that end inside a workgroup.  f32
-    results are held to the f16 bar, as above."""
+    """From 512 rows on a workgroup takes a row and a wave two heads: an odd number of heads, rows that lie further apart
+    than their heads.  f32 results are held to the f16 bar, as above."""
     half = 64
     qk_values, norm_values = normal_bf16(73, rows, (rows, heads + 1, 2 * half)), 1.0 + 0.1 * normal_bf16(73, 5, (heads, 2 * half))
     positions = (np.arange(rows) * 7 % 4099).astype(np.float32)
