@@ -2425,14 +2425,14 @@ fh_status failure_of(uint32_t op, uint32_t index, uint64_t serial, const ErrorSl
   return result;
 }
 
-// Up to so many bytes a kernel moves between the device and pinned host memory by itself: a copy command of the
-// runtime takes barriers and a signal of its own.  Error records and writes, whose both sides are the library's and which
-// nobody waits for, and the gather of fh_read_tensor, which is a kernel anyway, up to kMovedBytes (a submission of one
-// dispatch 18.4 us against 19.2 and, with an event of its own for the copy, 25.5; a write between two submissions, 16 KiB
-// 2.5 us against 2.6, 24 KiB 2.7 against 9.5, 64 KiB 3.5 against 10.0; a tensor of 512 bytes 12.0 against 22.5, of 64 KiB 14.6
-// against 24.9).  fh_read, which is waited for, up to kMovedRead, where the runtime's own way changes (512 bytes 12.3 us
-// against 21.6, 16 KiB 13.0 against 27.6, 24 KiB 13.8 against 10.4).
-constexpr uint64_t kMovedBytes = 64 * 1024, kMovedRead = 16 * 1024;
+// Up to this many bytes a kernel moves between the device and pinned host memory by itself: a copy command of the
+// runtime takes barriers and a signal of its own, which tells behind a submission.  Microseconds, moved and copied: a
+// submission of one dispatch 18.4 and 19.2 (25.5 with an event of its own for the copy of the error records); a write
+// between two submissions 16 KiB 2.5 and 2.6, 24 KiB 2.7 and 9.5, 64 KiB 3.5 and 10.0; a read behind a submission that has been
+// waited for 24 KiB 29 and 45, 64 KiB 31 and 38, not waited for 24 KiB 12 and 44, 64 KiB 13 and 37; a tensor of 512 bytes
+// 12.0 and 22.5, of 64 KiB 14.6 and 24.9.  Only reads of an idle device, one after the other, are copied the faster from
+// 20 KiB on (512 bytes 12.3 and 21.6, 16 KiB 13.0 and 27.6, 24 KiB 13.8 and 10.4, 64 KiB 15.0 and 12.4).
+constexpr uint64_t kMovedBytes = 64 * 1024;
 
 // Pinned memory for one small read at a time (under the backend's mutex); null when there is none.
 char *read_stage(fh_backend *b) {
@@ -2707,7 +2707,7 @@ fh_status fh_read(fh_backend *b, fh_buffer buffer, uint64_t byte_offset, void *b
     return FH_INVALID_INPUT;
   if (len == 0) return FH_OK;
   (void)hipSetDevice(b->device);
-  char *stage = len <= kMovedRead ? read_stage(b) : nullptr;
+  char *stage = len <= kMovedBytes ? read_stage(b) : nullptr;
   if (stage && launch_move_bytes(b->stream, stage, it->second.ptr + byte_offset, (uint32_t)len) == hipSuccess) {
     if (hipStreamSynchronize(b->stream) != hipSuccess) return FH_DEVICE_EXECUTION_FAILED;
     memcpy(bytes, stage, len);

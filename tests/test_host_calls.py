@@ -81,8 +81,7 @@ for part, call in (("copy", lambda: hip.read(t)), ("copy", lambda: hip.submit(co
 
 
 def test_which_reads_and_writes_a_kernel_moves(fake):
-    """Reads up to 16 KiB and writes up to 64 KiB, in the widest pieces that address and length allow; the copies of the
-    runtime beyond."""
+    """Up to 64 KiB, in the widest pieces that address and length allow; the copies of the runtime beyond."""
     fake("""
 t = hip.alloc(DType.U32, (1 << 15,))
 expected = bytearray(hip.read_buffer_range(t.buffer, 0, 1 << 17))
@@ -99,8 +98,8 @@ for first, length in ((0, 16), (16, 4080), (4, 20), (32, 36), (1, 16), (16, 3), 
     assert hip.read_buffer_range(t.buffer, first, first + length) == data
     read = launched()
     width = next(w for w in widths if (first | length) % w == 0)
-    for names, limit in ((wrote, 65536), (read, 16384)):
-        assert len(names) == (length <= limit), (first, length, names)
+    for names in (wrote, read):
+        assert len(names) == (length <= 65536), (first, length, names)
         assert all(widths[width] in name and "move_bytes_kernel" in name for name in names), (first, length, names)
 assert hip.read_buffer_range(t.buffer, 0, 1 << 17) == bytes(expected)
 """)
