@@ -11,11 +11,11 @@
 //     too coarse for the stated tolerance on outputs that cancel, fp16 (11 bits) is not, and the
 //     matrix cores run both at the same rate.  bf16 activations convert to fp16 exactly once a row
 //     is scaled by a power of two into the fp16 range (undone exactly when the result is stored).
-//   * Weights are centred: w = scale * q - c with c = 7.5 * scale, which halves their magnitude
-//     and so their rounding error; at the deepest contraction (K = 17408) the uncentred form does
-//     not meet the tolerance.  What centring takes out, (bias + c) * sum of the group's
+//   * Weights are centred: w = scale * (q - 8).  That is a number of fp16 exactly (a scale has eight significant bits,
+//     q - 8 at most three or is a power of two), where scale * q rounded once misses the tolerance at the deepest
+//     contraction (K = 17408).  What centring takes out, (bias + 8 * scale) * sum of the group's
 //     activations, is put back through the same GEMM: both operands get three more K columns per
-//     quantisation group, holding S/64 and 64 * (bias + c) each split in an fp16 head and tail
+//     quantisation group, holding S/64 and 64 * (bias + 8 * scale) each split in an fp16 head and tail
 //     (head*head + tail*head + head*tail, about 22 significant bits), so the kernel needs no
 //     side channel for it.  The contraction grows by 3/64.
 //   * prepare_rows_kernel writes the activation operand [rows, Kt], Kt = K + 3K/64 rounded up to
@@ -64,7 +64,8 @@ constexpr int gemm_lds_bytes(int quadrant) {
   return pipeline > output ? pipeline : output;
 }
 constexpr int gemm_q4_lds_bytes(int side, int waves, int part_rows, int part_columns) {
-  const int pipeline = 4 * side * 2 * kGemmK + 2 * side * 64;   // two tiles a side + packed words of two pairs of K steps
+  // activations of two steps, a tile of the weights' extra columns, packed words of two pairs of K steps, two blocks of scales
+  const int pipeline = 3 * side * 2 * kGemmK + 2 * side * 64 + 2 * side * 16;
   const int output = waves * (part_rows * out_pitch(part_columns) + 4 * part_rows);
   return pipeline > output ? pipeline : output;
 }
@@ -216,12 +217,12 @@ __global__ __launch_bounds__(256) void prepare_rows_kernel(const uint16_t *x, ui
 // Scales and biases this scheme can take: every centred weight and 64 * (bias + centre) must
 // stay inside the fp16 range.  False for NaN too.
 __device__ inline bool f16_safe(float scale, float bias) {
-  return fabsf(scale) <= 4000.0f && fabsf(bias + 7.5f * scale) <= 900.0f;
+  return fabsf(scale) <= 2700.0f && fabsf(bias + 8.0f * scale) <= 900.0f;
 }
 
-// packed/scales/biases [columns, inner] -> fp16 [columns, kt]: scale * q - 7.5 * scale (one
-// rounding, from f32) in the order (0,4,1,5,2,6,3,7) inside every 8, then per group (head, head,
-// tail) of 64 * (bias + 7.5 * scale), then zeros.  Eight threads per 64-value chunk, one packed
+// packed/scales/biases [columns, inner] -> fp16 [columns, kt]: scale * (q - 8)
+// in the order (0,4,1,5,2,6,3,7) inside every 8, then per group (head, head,
+// tail) of 64 * (bias + 8 * scale), then zeros.  Eight threads per 64-value chunk, one packed
 // word each; refused[0] is set when a group is out of range.
 __global__ __launch_bounds__(256) void prepare_weights_kernel(const uint32_t *packed,
                                                               const uint16_t *scales,
@@ -240,7 +241,7 @@ __global__ __launch_bounds__(256) void prepare_weights_kernel(const uint32_t *pa
     const float scale = bf16_bits_to_f32(s_row[chunk]), bias = bf16_bits_to_f32(b_row[chunk]);
     if (part == 0 && !f16_safe(scale, bias)) refused[0] = 1;
     const uint32_t w = packed[(uint64_t)column * (inner / 8) + 8 * chunk + part];
-    const float centre = 7.5f * scale;
+    const float centre = 8.0f * scale;
     float v[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = __builtin_fmaf(scale, (float)((w >> (4 * i)) & 15u), -centre);
@@ -257,7 +258,7 @@ __global__ __launch_bounds__(256) void prepare_weights_kernel(const uint32_t *pa
     if (group < groups) {
       const float scale = bf16_bits_to_f32(s_row[group]), bias = bf16_bits_to_f32(b_row[group]);
       float head, tail;
-      split_f16(64.0f * (bias + 7.5f * scale), &head, &tail);
+      split_f16(64.0f * (bias + 8.0f * scale), &head, &tail);
       value = kind == 2 ? tail : head;
     }
     values[i] = f16_bits(value);
@@ -595,7 +596,7 @@ __global__ __launch_bounds__(512) void gemm_f16_wide_kernel(GemmArgs a) {
 }
 
 // packed/scales/biases [columns, inner] -> the columns an operand row holds after its inner
-// values, fp16 [columns, kt - inner]: per group (head, head, tail) of 64 * (bias + 7.5 * scale),
+// values, fp16 [columns, kt - inner]: per group (head, head, tail) of 64 * (bias + 8 * scale),
 // then zeros.  One thread per 8 values; refused[0] is set when a group is out of range.
 __global__ __launch_bounds__(256) void prepare_extras_kernel(const uint16_t *scales, const uint16_t *biases,
                                                              uint32_t columns, uint32_t inner, uint32_t kt,
@@ -616,7 +617,7 @@ __global__ __launch_bounds__(256) void prepare_extras_kernel(const uint16_t *sca
       // the GEMM multiplies by the scale as an fp16 number: it must be one exactly
       if (kind == 0 && (!f16_safe(scale, bias) || (scale != 0.0f && fabsf(scale) < 6.103515625e-5f))) refused[0] = 1;
       float head, tail;
-      split_f16(64.0f * (bias + 7.5f * scale), &head, &tail);
+      split_f16(64.0f * (bias + 8.0f * scale), &head, &tail);
       value = kind == 2 ? tail : head;
     }
     values[i] = f16_bits(value);
@@ -626,20 +627,33 @@ __global__ __launch_bounds__(256) void prepare_extras_kernel(const uint16_t *sca
                  values[4] | ((uint32_t)values[5] << 16), values[6] | ((uint32_t)values[7] << 16));
 }
 
-// Eight nibbles of `w` as the centred weights scale * (q - 7.5) in fp16, in the order
-// (0,4)(1,5)(2,6)(3,7).  A nibble lands in mantissa bits 1..4 of 512.0 (whose unit in the last
-// place is 0.5), giving 512 + q exactly; 519.5 is taken off exactly and the product with the
-// scale is rounded once, like a weight formed in f32 and rounded.  scale2 = (scale, scale).
-__device__ inline f16x8 dequantise_word(uint32_t w, f16x2 scale2, uint32_t mask, uint32_t magic) {
-  const f16x2 centre = {(_Float16)519.5f, (_Float16)519.5f};
-  uint32_t bits[4] = {((w << 1) & mask) | magic, ((w >> 3) & mask) | magic, ((w >> 7) & mask) | magic,
-                      ((w >> 11) & mask) | magic};
+// What a group's scale is multiplied in as, exact in fp16: 16 times and -24 times the scale.
+__device__ inline f16x2 scale_factors(float scale) { return f16x2{(_Float16)(16.0f * scale), (_Float16)(-24.0f * scale)}; }
+
+// Eight nibbles of `w` as the centred weights scale * (q - 8) in fp16, in the order
+// (0,4)(1,5)(2,6)(3,7).  A nibble lands in the upper four mantissa bits of 1.0, giving 1 + q/16; times 16 scale less
+// 24 scale that is scale * (q - 8), exactly: a scale of eight significant bits times at most 7 takes eleven, and 8 is a
+// power of two.  Three instructions a pair of nibbles.  (Around 7.5, which needs a twelfth bit, a subtraction and a rounded
+// product took four.)
+__device__ inline f16x8 dequantise_word(uint32_t w, f16x2 factors, uint32_t mask, uint32_t magic) {
+  const f16x2 by = {factors[0], factors[0]}, less = {factors[1], factors[1]};
+  const uint32_t bits[4] = {((w << 6) & mask) | magic, ((w << 2) & mask) | magic, ((w >> 2) & mask) | magic,
+                            ((w >> 6) & mask) | magic};
   uint4 r;
-  r.x = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(f16x2, bits[0]) - centre) * scale2);
-  r.y = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(f16x2, bits[1]) - centre) * scale2);
-  r.z = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(f16x2, bits[2]) - centre) * scale2);
-  r.w = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(f16x2, bits[3]) - centre) * scale2);
+  r.x = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, bits[0]), by, less));
+  r.y = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, bits[1]), by, less));
+  r.z = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, bits[2]), by, less));
+  r.w = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, bits[3]), by, less));
   return __builtin_bit_cast(f16x8, r);
+}
+
+// load_to_lds_16 with the address as a wave-uniform base and a 32-bit offset per lane, and LDS by its offset (a
+// pointer's costs five scalar instructions to make one of).
+__device__ inline void load_to_lds_16_at(const void *base, uint32_t offset, uint32_t lds_offset) {
+  const uint64_t address = (uint64_t)base;   // (uniform by construction; the intrinsics tell the compiler so)
+  base = (const void *)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(address >> 32)) << 32) |
+                        (uint32_t)__builtin_amdgcn_readfirstlane((int)address));
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_offset) : "memory");
 }
 
 // The GEMM with the weights dequantised on their way into LDS.
@@ -653,19 +667,25 @@ __device__ inline f16x8 dequantise_word(uint32_t w, f16x2 scale2, uint32_t mask,
 //   * Weights: the packed words themselves go from memory into LDS the same way (64 bytes = two K
 //     steps of a column per request, half a byte per weight instead of two), and from there into
 //     the operand registers: a lane reads the 16 bytes that hold its 32 weights of a K step (a
-//     column, half a group) and turns one word into one matrix operand per sub-step (per nibble
-//     pair two integer and two packed fp16 instructions).  The dequantised weights never exist in
+//     column, half a group) and turns one word into one matrix operand per sub-step
+//     (dequantise_word).  The dequantised weights never exist in
 //     LDS: per K step a workgroup moves 40 KB from memory instead of 64 and reads 150 KB of LDS
 //     instead of 190.
 //   * The columns after the inner values (the bias term, see the head of this file) are plain fp16
 //     on both sides: for the last few K steps the weights' tile is loaded from `extras`.
-//   * Scales: a thread keeps the bf16 scales of eight groups of its column in registers (one
-//     16-byte load per eight K steps).
+//   * Scales: eight groups of a column at a time in LDS, two blocks of them.  In registers, loaded under the branch that
+//     every eighth step takes, they were waited for as soon as they were asked for, and cost what spilled.
+//   * A sub-step's words are unpacked between its matrix instructions, a word behind a row of them, also behind the
+//     barrier: left to itself the compiler puts the last sub-step's unpacking behind all of its matrix instructions, where
+//     both waves of a SIMD, which the barrier has just aligned, do it at once.
+//   * Measured with these and the shorter dequantise_word, before and after: 8256 x 34816 x 5120 2870 -> 2610 us, 8256 x 5120 x 17408
+//     1675 -> 1550, 2048 x 151936 x 1024 769 -> 721; 128 x 128 tiles: 2080 x 2048 x 4096 82 -> 70, 2080 x 5120 x 2048 81 -> 74,
+//     95 x 34816 x 5120 110 -> 95.
 //   * Every load into LDS is issued as inline assembly and ordered by the waits written here
 //     (see load_to_lds_16, lds_barrier): what the compiler knows of are the operand reads, whose
 //     waits it then counts exactly.
-// LDS: activations [2][side][128 B], fp16 weights of the extra columns [2][side][128 B], packed words of two pairs of K
-// steps [2][side][64 B].  A column's four 16-byte quarters of a pair sit in slots
+// LDS: activations [2][side][128 B], fp16 weights of the extra columns [side][128 B], packed words of two pairs of K
+// steps [2][side][64 B] (behind the inner steps a second tile of the extra columns), scales [2][side][16 B].  A column's four 16-byte quarters of a pair sit in slots
 // quarter ^ ((column >> 2) & 3), which spreads the 16 lanes a read serves at once over all banks.
 template <int kWM, int kWN, int kQM, int kQN>
 __global__ __launch_bounds__(64 * kWM * kWN) void gemm_q4_kernel(GemmArgs a) {
@@ -684,8 +704,12 @@ __global__ __launch_bounds__(64 * kWM * kWN) void gemm_q4_kernel(GemmArgs a) {
   constexpr int kPairLoads = kSide / 16 / kWaves;   // instructions per wave and pair (16 columns each)
   extern __shared__ __attribute__((aligned(16))) unsigned char gemm_lds[];
   unsigned char *a_tiles = gemm_lds;                 // [2][kSide][128]
+  // The fp16 tiles of the weights' extra columns: one of their own, and that of the packed words, which are used up by then.
   unsigned char *b_tiles = gemm_lds + 2 * kTile;     // [2][kSide][128]
-  unsigned char *pairs = gemm_lds + 4 * kTile;       // [2][kSide][64]
+  unsigned char *pairs = gemm_lds + 3 * kTile;       // [2][kSide][64]
+  static_assert(2 * kPair == kTile, "the packed words leave room for a tile");
+  unsigned char *scale_rows = gemm_lds + 4 * kTile;  // [2][kSide][16]
+  const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)gemm_lds;
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t wm = wave / kWN, wn = wave % kWN;
@@ -721,18 +745,18 @@ __global__ __launch_bounds__(64 * kWM * kWN) void gemm_q4_kernel(GemmArgs a) {
   auto stage_a = [&](uint32_t buffer, uint32_t step, int i) {
     const uint32_t st = min(step, steps - 1);   // past the end: the last tile again, never used
     const unsigned char *from = (const unsigned char *)a.a + (uint64_t)st * (kBK * 2);
-    load_to_lds_16(from + a_off[i], a_tiles + buffer * kTile + (kStaged * wave + 8 * i) * kRowBytes);
+    load_to_lds_16_at(from, a_off[i], lds + buffer * kTile + (kStaged * wave + 8 * i) * kRowBytes);
   };
   // the weights' fp16 tile of step `step`, one of the steps after the inner ones
   auto stage_extras = [&](uint32_t buffer, uint32_t step, int i) {
     const uint32_t st = min(step, steps - 1) - main_steps;
     const unsigned char *from = (const unsigned char *)a.extras + (uint64_t)st * (kBK * 2);
-    load_to_lds_16(from + e_off[i], b_tiles + buffer * kTile + (kStaged * wave + 8 * i) * kRowBytes);
+    load_to_lds_16_at(from, e_off[i], lds + (2 + buffer) * kTile + (kStaged * wave + 8 * i) * kRowBytes);
   };
   auto stage_pair = [&](uint32_t pair, int i) {
     const uint32_t pr = min(pair, main_steps / 2 - 1);   // past the end: into the buffer nobody reads
     const unsigned char *from = (const unsigned char *)a.packed + (uint64_t)pr * 64;
-    load_to_lds_16(from + p_off[i], pairs + (pair & 1u) * kPair + 16 * (kPairLoads * wave + i) * 64);
+    load_to_lds_16_at(from, p_off[i], lds + 3 * kTile + (pair & 1u) * kPair + 16 * (kPairLoads * wave + i) * 64);
   };
 
   f32x16 acc[kMIR][kMIC];
@@ -764,7 +788,7 @@ __global__ __launch_bounds__(64 * kWM * kWN) void gemm_q4_kernel(GemmArgs a) {
   // column and K step (the half kh of the step's group), one word per sub-step, and the columns'
   // scales
   const uint32_t quarter_swizzle = (l32 >> 2) & 3u;
-  uint4 words[kMIC], next_words[kMIC];
+  uint4 words[2][kMIC];   // by the step's parity
   auto read_words = [&](uint4 (&to)[kMIC], uint32_t step) {
     const unsigned char *from = pairs + ((step >> 1) & 1u) * kPair + (kQN * wn + l32) * 64 +
                                 16 * ((2 * (step & 1u) + kh) ^ quarter_swizzle);
@@ -772,46 +796,42 @@ __global__ __launch_bounds__(64 * kWM * kWN) void gemm_q4_kernel(GemmArgs a) {
     for (int j = 0; j < kMIC; ++j) to[j] = *(const uint4 *)(from + 32 * j * 64);
   };
   const uint32_t groups = a.inner / 64;
-  uint32_t scale_off[kMIC];
-#pragma unroll
-  for (int j = 0; j < kMIC; ++j) scale_off[j] = min(col0 + kQN * wn + 32 * j + l32, a.columns - 1) * groups * 2;
-  uint4 scale_block[kMIC], next_block[kMIC];   // bf16 scales of eight groups per column
-  auto load_scales = [&](uint4 (&to)[kMIC], uint32_t block) {
+  const uint32_t s_off = min(col0 + kQN * (wave % kWN) + lane, a.columns - 1) * groups * 2;
+  static_assert(kQN == 64, "a wave's lanes bring the scales of its columns");
+  auto stage_scales = [&](uint32_t block) {   // of eight groups, by one row of waves
+    if (wm != 0) return;
     const uint32_t bl = min(block, groups / 8 - 1);
-    const unsigned char *from = (const unsigned char *)a.scales + (uint64_t)bl * 16;
-#pragma unroll
-    for (int j = 0; j < kMIC; ++j) to[j] = *(const uint4 *)(from + scale_off[j]);
+    load_to_lds_16_at((const unsigned char *)a.scales + (uint64_t)bl * 16, s_off, lds + 4 * kTile + (block & 1u) * (kSide * 16) + wn * 1024);
   };
-  f16x2 scale2[kMIC], next_scale2[kMIC];
-  auto pick_scales = [&](f16x2 (&to)[kMIC], uint32_t step) {
-    const uint32_t e = step & 7u;   // uniform
+  f16x2 factors[2][kMIC];
+  uint32_t scale_bits[kMIC];
+  auto read_scales = [&](uint32_t step) {
 #pragma unroll
-    for (int j = 0; j < kMIC; ++j) {
-      const uint4 v = scale_block[j];
-      const uint32_t word = e < 4 ? (e < 2 ? v.x : v.y) : (e < 6 ? v.z : v.w);
-      const float scale = __uint_as_float((e & 1u) ? (word & 0xffff0000u) : (word << 16));
-      const _Float16 h = (_Float16)scale;
-      to[j] = f16x2{h, h};
-    }
+    for (int j = 0; j < kMIC; ++j)
+      scale_bits[j] = *(const uint16_t *)(scale_rows + (step / 8 & 1u) * (kSide * 16) + (kQN * wn + 32 * j + l32) * 16 + (step & 7u) * 2);
   };
-  uint32_t mask = 0x001e001eu, magic = 0x60006000u;
+  auto take_scales = [&](f16x2 (&to)[kMIC]) {
+#pragma unroll
+    for (int j = 0; j < kMIC; ++j) to[j] = scale_factors(__uint_as_float(scale_bits[j] << 16));
+  };
+  uint32_t mask = 0x03c003c0u, magic = 0x3c003c00u;
   asm("" : "+s"(mask), "+v"(magic));   // no instruction: keeps the two constants in registers
 
-  // ---- prologue: activations of step 0, packed words of steps 0..1, scales of groups 0..15;
+  // ---- prologue: activations of step 0, packed words of steps 0..1, scales of groups 0..7;
   // then the operands of the first sub-step
+  stage_scales(0);
 #pragma unroll
   for (int i = 0; i < kLoads; ++i) stage_a(0, 0, i);
 #pragma unroll
   for (int i = 0; i < kPairLoads; ++i) stage_pair(0, i);
-  load_scales(scale_block, 0);
-  load_scales(next_block, 1);
   __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));
   lds_barrier();
-  read_words(words, 0);
-  pick_scales(scale2, 0);
+  read_words(words[0], 0);
+  read_scales(0);
+  take_scales(factors[0]);
   read_a(0, 0, 0);
 #pragma unroll
-  for (int j = 0; j < kMIC; ++j) b_op[0][j] = dequantise_word(words[j].x, scale2[j], mask, magic);
+  for (int j = 0; j < kMIC; ++j) b_op[0][j] = dequantise_word(words[0][j].x, factors[0][j], mask, magic);
   // One inner step.  On entry the operands of its first sub-step are in registers (set 0).  kOdd:
   // the step's parity (= the LDS buffer its activations are in); kLast: the last inner step, which
   // requests the first fp16 tile of the weights' side and prepares no weights for a next step.
@@ -824,14 +844,10 @@ __global__ __launch_bounds__(64 * kWM * kWN) void gemm_q4_kernel(GemmArgs a) {
     constexpr bool kOdd = decltype(odd_tag)::value, kLast = decltype(last_tag)::value;
     constexpr uint32_t buffer = kOdd ? 1u : 0u;
     if (!kLast) {
-      if (kOdd && ((step + 1) & 7u) == 0) {   // the next step opens a block of eight groups
-#pragma unroll
-        for (int j = 0; j < kMIC; ++j) scale_block[j] = next_block[j];
-        load_scales(next_block, (step + 1) / 8 + 1);
-      }
-      pick_scales(next_scale2, step + 1);
-      read_words(next_words, step + 1);
+      read_words(words[kOdd ? 0 : 1], step + 1);
+      read_scales(step + 1);
     }
+    if (!kOdd && (step & 7u) == 0) stage_scales(step / 8 + 1);
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) stage_a(buffer ^ 1u, step + 1, i);
     if (kLast) {
@@ -852,10 +868,11 @@ __global__ __launch_bounds__(64 * kWM * kWN) void gemm_q4_kernel(GemmArgs a) {
         for (int j = 0; j < kMIC; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_op[s & 1][i], b_op[s & 1][j], acc[i][j], 0, 0, 0);
         if (i < kMIC) {   // behind row i: the operand of column block i for the next sub-step
-          const uint4 v = words[i];
+          const uint4 v = words[buffer][i];
           const uint32_t w = s == 0 ? v.y : s == 1 ? v.z : v.w;
-          b_op[(s + 1) & 1][i] = dequantise_word(w, scale2[i], mask, magic);
+          b_op[(s + 1) & 1][i] = dequantise_word(w, factors[buffer][i], mask, magic);
         }
+        if (!kLast && s == kSub - 2 && i == kMIR - 1) take_scales(factors[buffer ^ 1u]);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -871,15 +888,8 @@ __global__ __launch_bounds__(64 * kWM * kWN) void gemm_q4_kernel(GemmArgs a) {
 #pragma unroll
       for (int j = 0; j < kMIC; ++j)
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_op[1][i], b_op[1][j], acc[i][j], 0, 0, 0);
-      if (!kLast && i < kMIC) b_op[0][i] = dequantise_word(next_words[i].x, next_scale2[i], mask, magic);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    if (!kLast) {
-#pragma unroll
-      for (int j = 0; j < kMIC; ++j) {
-        words[j] = next_words[j];
-        scale2[j] = next_scale2[j];
-      }
+      if (!kLast && i < kMIC) b_op[0][i] = dequantise_word(words[buffer ^ 1u][i].x, factors[buffer ^ 1u][i], mask, magic);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
   typedef std::integral_constant<bool, false> no;
@@ -928,12 +938,6 @@ __global__ __launch_bounds__(64 * kWM * kWN) void gemm_q4_kernel(GemmArgs a) {
   __builtin_amdgcn_s_waitcnt(0xc07f);
   lds_barrier();   // the last reads are done before the tile's stores reuse LDS
   store_tile<kQM, kQN, kWN>(a, acc, gemm_lds, row0, col0);
-}
-
-// load_to_lds_16 with the address as a wave-uniform base and a 32-bit offset per lane, and LDS by its offset (a
-// pointer's costs five scalar instructions to make one of).
-__device__ inline void load_to_lds_16_at(const void *base, uint32_t offset, uint32_t lds_offset) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_offset) : "memory");
 }
 
 // The same product for outputs of few tiles: eight waves of 64 rows x 64 columns, kWM x kWN of them beside each other
@@ -1080,11 +1084,10 @@ __global__ __launch_bounds__(512, 2) void gemm_q4_split_kernel(GemmArgs a) {
   auto take_scales = [&](f16x2 (&to)[kMI]) {
 #pragma unroll
     for (int j = 0; j < kMI; ++j) {
-      const _Float16 h = (_Float16)__uint_as_float(scale_bits[j] << 16);
-      to[j] = f16x2{h, h};
+      to[j] = scale_factors(__uint_as_float(scale_bits[j] << 16));
     }
   };
-  uint32_t mask = 0x001e001eu, magic = 0x60006000u;
+  uint32_t mask = 0x03c003c0u, magic = 0x3c003c00u;
   asm("" : "+s"(mask), "+v"(magic));   // no instruction: keeps the two constants in registers
   // the matrix instructions of sub-step s; behind each row of them the operand of a column block for sub-step s + 1
   auto sub_step = [&](int s, const uint4 (&next_words)[kMI], const f16x2 (&next_scale)[kMI]) {
