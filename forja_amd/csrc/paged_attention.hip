@@ -750,36 +750,30 @@ struct LaneConst {
   uint32_t row_elems; // elements per pool token row (Hkv * 128)
 };
 
-// Issues the 16 loads of one 32-token tile.  `physical` holds this lane's authenticated page of
-// the current 64-page group; a 16-token half never straddles a page, so each half is addressed
-// as a wave-uniform base plus a per-lane 32-bit offset.  kMasked tiles (the last, partial tile
-// of a split) load zeros past `end`: unused pool slots may hold anything and 0 * NaN would
-// poison the sum.
-template <bool kMasked>
+// Issues the 16 loads of one 32-token tile.  `physical` holds this lane's authenticated page of the current
+// 64-page group; a 16-token half never straddles a page, so each half is a buffer of its rows up to `end` and a
+// per-lane 32-bit offset.  What lies past a buffer's length reads as zeros and is not fetched: unused pool slots
+// may hold anything, and 0 * NaN would poison the sum.  Without a condition all 16 loads are on their way at
+// once; with one around each, the compiler waits for each by itself (eight round trips for a partial tile).
+__device__ inline uint4 load_row_piece(__amdgpu_buffer_rsrc_t rows, uint32_t element) {
+  typedef __attribute__((ext_vector_type(4))) uint32_t words;
+  const words v = __builtin_amdgcn_raw_buffer_load_b128(rows, (int)(2 * element), 0, 2 /* as stream_load */);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+
 __device__ inline void load_tile(const FastRagged &p, TileRegs &r, uint32_t tile0, uint32_t end,
-                                 uint32_t page0, uint32_t physical, const LaneConst &lc,
-                                 uint32_t hl, uint32_t g) {
+                                 uint32_t page0, uint32_t physical, const LaneConst &lc) {
   const uint32_t pt = p.page_tokens;
   for (int sub = 0; sub < 2; ++sub) {
-    const uint32_t tok0 = tile0 + 16 * sub;
-    if (kMasked && tok0 >= end) {
-      for (int step = 0; step < 4; ++step) r.k[sub][step] = make_uint4(0, 0, 0, 0);
-      for (int i = 0; i < 4; ++i) r.v[4 * sub + i] = make_uint4(0, 0, 0, 0);
-      continue;
-    }
-    const uint32_t page =
-        __builtin_amdgcn_readfirstlane(__shfl(physical, (int)(tok0 / pt - page0), 64));
-    const uint64_t row0 = (uint64_t)page * pt + tok0 % pt;
-    const uint16_t *k_base = p.key_pool + row0 * lc.row_elems;
-    const uint16_t *v_base = p.value_pool + row0 * lc.row_elems;
-    for (int step = 0; step < 4; ++step) {
-      r.k[sub][step] = stream_load(k_base + lc.k_offset + 32 * step);
-      if (kMasked && tok0 + hl >= end) r.k[sub][step] = make_uint4(0, 0, 0, 0);
-    }
-    for (int i = 0; i < 4; ++i) {
-      r.v[4 * sub + i] = stream_load(v_base + lc.v_offset + i * lc.row_elems);
-      if (kMasked && tok0 + 4 * g + i >= end) r.v[4 * sub + i] = make_uint4(0, 0, 0, 0);
-    }
+    const uint32_t tok0 = tile0 + 16 * sub, rows = end > tok0 ? min(end - tok0, 16u) : 0;
+    const uint32_t token = min(tok0, (end - 1) & ~15u);   // a half past the end has no rows: any page will do
+    const uint32_t page = __builtin_amdgcn_readlane(physical, __builtin_amdgcn_readfirstlane(token / pt - page0));
+    const uint64_t row0 = (uint64_t)page * pt + __builtin_amdgcn_readfirstlane(token % pt);
+    const int bytes = __builtin_amdgcn_readfirstlane(2 * rows * lc.row_elems);
+    const auto k_rows = __builtin_amdgcn_make_buffer_rsrc((void *)(p.key_pool + row0 * lc.row_elems), 0, bytes, 0x27000);
+    const auto v_rows = __builtin_amdgcn_make_buffer_rsrc((void *)(p.value_pool + row0 * lc.row_elems), 0, bytes, 0x27000);
+    for (int step = 0; step < 4; ++step) r.k[sub][step] = load_row_piece(k_rows, lc.k_offset + 32 * step);
+    for (int i = 0; i < 4; ++i) r.v[4 * sub + i] = load_row_piece(v_rows, lc.v_offset + i * lc.row_elems);
   }
 }
 
@@ -919,28 +913,33 @@ __device__ inline void attend_one_token(const FastRagged &p, ErrorSlot *error, c
     }
     const uint32_t tok_lo = max(begin, page0 * pt);
     const uint32_t tok_hi = (uint32_t)min((uint64_t)end, ((uint64_t)page0 + 64) * pt);
-    const uint32_t full_hi = tok_lo + (tok_hi - tok_lo) / kTile * kTile;
-    // Two tiles in registers, one on its way while the other is consumed.  The loop requests whole tiles
-    // only, so that the wait in front of a tile's products is for that tile alone: with a choice between
-    // whole and masked requests inside, the compiler waits for both tiles there.
-    const bool tail = full_hi < tok_hi;   // plain tiles are followed by at most one masked tile
-    TileRegs cur, nxt;
-    if (full_hi > tok_lo) {
-      load_tile<false>(p, cur, tok_lo, end, page0, physical, lc, hl, g);
-      uint32_t tile0 = tok_lo;   // the tile in `cur`
-      for (; tile0 + kTile < full_hi; tile0 += kTile) {
-        load_tile<false>(p, nxt, tile0 + kTile, end, page0, physical, lc, hl, g);
-        __builtin_amdgcn_sched_barrier(0);
-        consume_tile<false, kHalf>(cur, q_reg, o, sm, tile0, end, p.scale_log2, g);
-        __builtin_amdgcn_sched_barrier(0);
-        cur = nxt;
-      }
-      if (tail) load_tile<true>(p, nxt, full_hi, end, page0, physical, lc, hl, g);
-      consume_tile<false, kHalf>(cur, q_reg, o, sm, tile0, end, p.scale_log2, g);
-    } else {
-      load_tile<true>(p, nxt, full_hi, end, page0, physical, lc, hl, g);
+    // Two tiles in registers, in turns: one is requested while the other is on its way, and neither is moved (a
+    // move waits for it, and with it for every load before).  Only the last tile may be partial.  Bound by HBM where
+    // items fill the device, by one wave's chain where they do not: 23 lanes of 60 to 3000 keys (16 heads) 22.7 -> 21.0 us,
+    // one lane of 500 keys 10.0 -> 8.5, 48 lanes (40 heads) 43.0 -> 41.6, 128 lanes of up to 32768 keys 288 -> 284, against
+    // one tile that was moved between registers, and partial tiles of loads under a condition.
+    uint32_t tile0 = tok_lo, left = (tok_hi - tok_lo + kTile - 1) / kTile;
+    TileRegs a, b;
+    load_tile(p, a, tile0, end, page0, physical, lc);
+    for (; left > 2; left -= 2, tile0 += 2 * kTile) {
+      load_tile(p, b, tile0 + kTile, end, page0, physical, lc);
+      __builtin_amdgcn_sched_barrier(0);
+      consume_tile<false, kHalf>(a, q_reg, o, sm, tile0, end, p.scale_log2, g);
+      __builtin_amdgcn_sched_barrier(0);
+      load_tile(p, a, tile0 + 2 * kTile, end, page0, physical, lc);
+      __builtin_amdgcn_sched_barrier(0);
+      consume_tile<false, kHalf>(b, q_reg, o, sm, tile0 + kTile, end, p.scale_log2, g);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    if (tail) consume_tile<true, kHalf>(nxt, q_reg, o, sm, full_hi, end, p.scale_log2, g);
+    if (left == 2) {
+      load_tile(p, b, tile0 + kTile, end, page0, physical, lc);
+      __builtin_amdgcn_sched_barrier(0);
+      consume_tile<false, kHalf>(a, q_reg, o, sm, tile0, end, p.scale_log2, g);
+      __builtin_amdgcn_sched_barrier(0);
+      consume_tile<true, kHalf>(b, q_reg, o, sm, tile0 + kTile, end, p.scale_log2, g);
+    } else {
+      consume_tile<true, kHalf>(a, q_reg, o, sm, tile0, end, p.scale_log2, g);
+    }
   }
   // Lane (row hl, group g) holds value columns 32g + 8j + mt of its row.
   sm.l += __shfl_xor(sm.l, 16, 64);

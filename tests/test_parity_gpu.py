@@ -1468,6 +1468,36 @@ def test_ragged_attention_equals_the_per_lane_sequence(cpu, hip, contexts, count
     assert cpu.read(cpu_out[1]) == hip.read(hip_out[1]) and cpu.read(cpu_out[2]) == hip.read(hip_out[2])
 
 
+@pytest.mark.parametrize("pt,hq,hkv,dtype", [(16, 16, 8, DType.BF16), (48, 5, 1, DType.F16), (64, 32, 2, DType.F32)])
+def test_decode_reads_no_slot_past_its_keys(cpu, hip, pt, hq, hkv, dtype):
+    """Every length of a last tile and both parities of the tiles in front of it, one split and several; all slots
+    that hold no key are NaNs (bf16 and f16 pools; f32 queries read an f16 one)."""
+    contexts = list(range(0, 66)) + [94, 95, 96, 127, 128, 159, 160, 161, 64 * pt - 2, 64 * pt, 64 * pt + 33, 4000]
+    pool_dtype = DType.F16 if dtype is DType.F32 else dtype
+    pools = {}
+
+    def build(backend):
+        t, inputs = ragged_case(backend, contexts, [1] * len(contexts), hq, hkv, pt, seed=67, dtype=dtype,
+                                pool_dtype=pool_dtype)
+        tables = np.frombuffer(backend.read(t["tables"]), np.uint32).reshape(len(contexts), -1, 2)
+        for name in ("keys", "values"):
+            pool = np.frombuffer(backend.read(t[name]), np.uint16).reshape(-1, pt, hkv * 128)
+            held = np.full_like(pool, 0x7fff)
+            for lane, keys in enumerate(contexts):
+                for first in range(0, keys, pt):
+                    page, rows = tables[lane, first // pt, 0], min(pt, keys - first)
+                    held[page, :rows] = pool[page, :rows]
+            backend.write(t[name], held.tobytes())
+        commands = CommandList()
+        commands.dispatch_many(Op.paged_attention_ragged(0.09, pt), inputs, [t["out"], t["keys"], t["values"]])
+        pools[backend] = t["keys"], t["values"]
+        return commands, [t["out"]]
+    _, (hip_out, _) = differential(cpu, hip, build, bar=pool_dtype)
+    assert np.isfinite(to_f32(hip.read(hip_out[0]), dtype)).all()
+    for want, got in zip(pools[cpu], pools[hip]):
+        assert cpu.read(want) == hip.read(got)
+
+
 @pytest.mark.parametrize("contexts,counts", [
     # six tokens to a group of five heads, eight kv heads: 63 and 64 groups, the second with decode rows
     # in items of the longest group's length, the third with groups shorter than the shortest items
