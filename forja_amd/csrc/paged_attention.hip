@@ -306,7 +306,11 @@ typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-constexpr uint32_t kMinSplitTokens = 128, kMaxSplitTokens = 1024;  // split length bounds
+constexpr uint32_t kMinSplitTokens = 128, kMaxSplitTokens = 1024;  // split length bounds beside prompt rows
+// Of a decode batch that fits the device at once: with two tiles a wave requests its whole item before it waits.  Steps of
+// the small model with items of 64 keys against 128: 3 lanes 1459 / 1616 us, 8 lanes 1507 / 1663, 14 lanes 1578 / 1730,
+// 30 lanes 1840 / 2008; of the mixture model 1 and 2 lanes 0.97 to 1.00; items of 32: equal to 0.98, but more to merge.
+constexpr uint32_t kMinDecodeSplit = 64;
 // see ragged_plan_kernel (512 groups: two for each of the 256 compute units that an MI355X has)
 constexpr uint32_t kFillingGroups = 512, kFilledSplitTokens = 512;
 // Groups of several query tokens (prefill) are many and each split of theirs costs a merge of
@@ -565,7 +569,7 @@ __global__ __launch_bounds__(kPlanThreads) void ragged_plan_kernel(FastRagged p,
       // alone at the end: then the even share of a place is the length.
       const unsigned long long share = (total_attended + p.item_slots - 1) / p.item_slots;
       uint32_t even = (uint32_t)((share + kTile - 1) / kTile * kTile);
-      if (even < kMinSplitTokens) even = kMinSplitTokens;
+      if (even < kMinDecodeSplit) even = kMinDecodeSplit;
       uint32_t low = even / kTile, high = max(longest_keys, even) / kTile;   // in tiles
       while (low < high) {   // smallest length in [low, high] with at most item_slots items: one try per wave
         const uint32_t tried = low + (uint32_t)((uint64_t)(high - low) * (wave + 1) / (kWaves + 1));
