@@ -920,7 +920,7 @@ __device__ inline void attend_one_token(const FastRagged &p, ErrorSlot *error, c
     // Two tiles in registers, in turns: one is requested while the other is on its way, and neither is moved (a
     // move waits for it, and with it for every load before).  Only the last tile may be partial.  Bound by HBM where
     // items fill the device, by one wave's chain where they do not: 23 lanes of 60 to 3000 keys (16 heads) 22.7 -> 21.0 us,
-    // one lane of 500 keys 10.0 -> 8.5, 48 lanes (40 heads) 43.0 -> 41.6, 128 lanes of up to 32768 keys 288 -> 284, against
+    // one lane of 500 keys 9.7 -> 8.5, 48 lanes (40 heads) 43.0 -> 41.6, 128 lanes of up to 32768 keys 288 -> 284, against
     // one tile that was moved between registers, and partial tiles of loads under a condition.
     uint32_t tile0 = tok_lo, left = (tok_hi - tok_lo + kTile - 1) / kTile;
     TileRegs a, b;
