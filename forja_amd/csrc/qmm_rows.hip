@@ -28,6 +28,14 @@
 // x 2048 284 -> 62, 512 x 2048 x 4096 231 -> 45, 8 bits 512 x 128 x 2048 93 -> 16; routed, 128 experts of 768 x 2048,
 // gate/up and down together: bf16 16640 routes 435 -> 324, f32 4096 routes 1027 -> 220.
 //
+// The activations come in by rows, eight lanes to a row's 128 bytes of a group: sixteen bytes of another row in every lane
+// (operand order) cost the compute unit's address unit 65 cycles a load against 18, and a third of all loads were of
+// that kind; the chunks find their operand places on the way into LDS, and a group's sum is three exchanges within eight
+// lanes.  A lane quarter reads the scales and biases of one column tile for all four.  Against operand-order loads
+// by every quarter: bf16 48 x 34816 x 5120 67 -> 61 us, 48 x 151936 x 5120 209 -> 193, 64 x 34816 x 5120 83 -> 75; f32 512 x 5120 x 2048
+// 60 -> 54; routed as above, bf16 24000 routes 457 -> 434, f32 8192 routes 388 -> 371; launches of one or two quads
+// a workgroup, whose length is their latency, 0 to 1 us longer (8 bits 512 x 128 x 2048 12.8 -> 13.7).
+//
 // The bias term rides on the matrix cores too: the group sums are split into their three exact
 // bf16 pieces, one per lane quarter, and the operand against them is the column's scales and
 // biases as they lie in memory (both exact in bf16), so that one instruction per 16 x 16 block and
@@ -148,6 +156,12 @@ constexpr uint32_t part_bytes() { return XP * RT * 4 * 1024 + RT * 1024 + (XP ==
 template <int XP, int RT, int WK>
 constexpr uint32_t staged_bytes() { return 2u * WK * part_bytes<XP, RT>(); }
 
+// The value of another lane of the same eight: its neighbour, of the other pair of its four, of the other four (any of them:
+// for sums that the four already share).
+constexpr int kOther = 0xb1, kOtherPair = 0x4e, kOtherFour = 0x141;   // quad_perm 1,0,3,2 and 2,3,0,1; row_half_mirror
+template <int kWay>
+__device__ inline int across(int v) { return __builtin_amdgcn_update_dpp(0, v, kWay, 0xf, 0xf, true); }
+
 // XP: pieces of an activation (1: bf16 rows as they are, 3: f32 rows in f16).  BITS: 4 or 8 (f32 rows only).  RT: 16-row tiles.
 // WC waves side by side (64 columns each; of a pair 32 of either projection), WK waves along K.
 template <int XP, int BITS, int RT, int WC, int WK, bool kPair, bool kRouted>
@@ -195,15 +209,29 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
   const uint32_t first_quad = split * quads / a.splits, last_quad = (split + 1) * quads / a.splits;
   const uint32_t rounds = (last_quad - first_quad + WK - 1) / WK;
 
-  // ---- the activations this wave stages: for each of its pieces, lane (row n, quarter g) brings
-  // values [8g, 8g+8) and [32+8g, 32+8g+8) of one row and group.
-  uint32_t x_lane[kTasks];   // bytes
+  // ---- the activations this wave stages: for each of its pieces, lane (row e, chunk c) brings values [8c, 8c+8) of
+  // rows e and 8 + e of one group: neighbouring lanes read neighbouring addresses.  (Sixteen bytes of another row
+  // in every lane take the address unit 65 cycles a load, whole lines of a row 18.)
+  const uint32_t chunk = lane & 7, e = lane >> 3;
+  constexpr uint32_t kValue = XP == 1 ? 2 : 4;
+  // Bytes.  Dense: one lane offset for every row, from a buffer that ends with the last row (past it zeros, never
+  // stored); routed: each row's own.  (Tiles of 64 dense rows, too: there the buffers' scalars push nine registers out, 85
+  // us against 76 for 64 x 34816 x 5120; of 48 rows the offsets do, 66 against 61 for 48 x 34816 x 5120.)
+  constexpr bool kOwnOffsets = kRouted || RT == 4;
+  uint32_t x_lane[kOwnOffsets ? kTasks : 1][2];
+  const uint32_t x_bytes = (uint32_t)(((uint64_t)(a.rows - 1) * a.x_row_stride + a.inner) * kValue);
+  if constexpr (kOwnOffsets) {
 #pragma unroll
-  for (int t = 0; t < kTasks; ++t) {
-    const uint32_t task = wc + t * WC, row = 16 * (task / 2) + n;
-    const uint32_t safe = row < tile_count ? row : 0;     // rows past the tile: computed, never stored
-    const uint64_t in_row = kRouted ? a.sorted_routes[tile_first + safe] / a.route_div : tile_first + safe;
-    x_lane[t] = (uint32_t)(in_row * a.x_row_stride + kGroup * (task % 2) + 8 * g) * (XP == 1 ? 2 : 4);
+    for (int t = 0; t < kTasks; ++t)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const uint32_t task = wc + t * WC, row = 16 * (task / 2) + 8 * i + e;
+        const uint32_t safe = row < tile_count ? row : 0;     // rows past the tile: computed, never stored
+        const uint64_t in_row = kRouted ? a.sorted_routes[tile_first + safe] / a.route_div : tile_first + safe;
+        x_lane[t][i] = (uint32_t)(in_row * a.x_row_stride + kGroup * (task % 2) + 8 * chunk) * kValue;
+      }
+  } else {
+    x_lane[0][0] = (uint32_t)(e * a.x_row_stride + 8 * chunk) * kValue;
   }
   uint32_t xr[kTasks][2][XW];
   auto load_rows = [&](uint32_t quad, int pair) {   // (a quad past the end reads the last one)
@@ -211,29 +239,41 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
 #pragma unroll
     for (int t = 0; t < kTasks; ++t)
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        const global_bytes from = uniform((const char *)a.x + at * (XP == 1 ? 2 : 4));
+      for (int i = 0; i < 2; ++i) {
+        u32x4 eight[XW / 4];
+        if constexpr (kOwnOffsets) {
+          const global_bytes from = uniform((const char *)a.x + at * kValue);
+#pragma unroll
+          for (int v = 0; v < XW / 4; ++v) eight[v] = load_at<u32x4>(from, x_lane[t][i] + 16 * v);
+        } else {
+          const uint32_t task = wc + t * WC;
+          const uint64_t skip = ((tile_first + 16 * (task / 2) + 8 * i) * a.x_row_stride + at + kGroup * (task % 2)) * kValue;
+          const auto rows = __builtin_amdgcn_make_buffer_rsrc((char *)const_cast<void *>(a.x) + skip, 0,
+                                                              (int)(skip < x_bytes ? x_bytes - (uint32_t)skip : 0u), 0x27000);
+#pragma unroll
+          for (int v = 0; v < XW / 4; ++v) eight[v] = __builtin_amdgcn_raw_buffer_load_b128(rows, (int)x_lane[0][0] + 16 * v, 0, 0);
+        }
 #pragma unroll
         for (int v = 0; v < XW / 4; ++v) {
-          const u32x4 four = load_at<u32x4>(from, x_lane[t] + 32 * half * (XP == 1 ? 2 : 4) + 16 * v);
-          xr[t][half][4 * v] = four.x, xr[t][half][4 * v + 1] = four.y;
-          xr[t][half][4 * v + 2] = four.z, xr[t][half][4 * v + 3] = four.w;
+          const u32x4 four = eight[v];
+          xr[t][i][4 * v] = four.x, xr[t][i][4 * v + 1] = four.y;
+          xr[t][i][4 * v + 2] = four.z, xr[t][i][4 * v + 3] = four.w;
         }
       }
   };
   // Where a chunk of eight values lies in operand order: chunk c of a group belongs to quarter
-  // g' = c / 2 of the lanes and operand half c % 2; with 4-bit weights the half-wave swaps leave
+  // c / 2 of the lanes and operand half c % 2; with 4-bit weights the half-wave swaps leave
   // quarter q of the lanes holding the nibbles of values [16 q', 16 q' + 16), q' = (0,2,1,3)[q].
-  auto slot_of = [&](uint32_t chunk) -> uint32_t {
-    const uint32_t quarter = chunk / 2;
-    const uint32_t at = BITS == 4 ? 2 * (quarter & 1) + (quarter >> 1) : quarter;
-    return (chunk % 2) * 1024 + (16 * at + n) * 16;
-  };
-  const uint32_t slot[2] = {slot_of(g), slot_of(g + 4)};
+  // A row's place within its quarter is turned by twice the quarter and half, so that the sixteen lanes of a store,
+  // two rows of eight chunks, meet different banks.
+  auto turn_of = [](uint32_t at, uint32_t half) { return 2 * (2 * at + half); };
+  const uint32_t quarter = chunk / 2, at_quarter = BITS == 4 ? 2 * (quarter & 1) + (quarter >> 1) : quarter;
+  const uint32_t slot0 = (chunk % 2) * 1024 + (16 * at_quarter + (e ^ turn_of(at_quarter, chunk % 2))) * 16;
+  const uint32_t slot[2] = {slot0, slot0 ^ 128};   // rows e and 8 + e
   uint32_t sum_mask[3];
 #pragma unroll
   for (int piece = 0; piece < 3; ++piece) {
-    sum_mask[piece] = g == (uint32_t)piece ? 0xffffffffu : 0u;
+    sum_mask[piece] = chunk % 4 == (uint32_t)piece ? 0xffffffffu : 0u;
     asm("" : "+v"(sum_mask[piece]));
   }
   // `parity`: which of the two sets of group sums (by quad)
@@ -243,40 +283,36 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
 #pragma unroll
     for (int t = 0; t < kTasks; ++t) {
       const uint32_t task = wc + t * WC, row_tile = task / 2, group = task % 2;
-      float s = 0.0f;
-      if constexpr (XP == 1) {
+      float s[2] = {0.0f, 0.0f};
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-          const uint4 v = make_uint4(xr[t][half][0], xr[t][half][1], xr[t][half][2], xr[t][half][3]);
+      for (int i = 0; i < 2; ++i) {
+        if constexpr (XP == 1) {
+          const uint4 v = make_uint4(xr[t][i][0], xr[t][i][1], xr[t][i][2], xr[t][i][3]);
           const uint32_t words[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, words[i]), __builtin_bit_cast(bf16x2, 0x3f803f80u), s, false);
-          *(uint4 *)(part + (row_tile * 4 + group * 2) * 1024 + slot[half]) = permute_slots(v);
-        }
-      } else {
-        // A power of two takes the largest of the row's group into [2^14, 2^15); then three f16
-        // pieces, each the leading eleven bits of what the ones before left, make up every value to
-        // 2^-38 of that largest: the smallest step of f16 is 2^-24 (pieces are cut off, not rounded, so that
-        // the rest is exact).
-        uint32_t largest = 0;
-#pragma unroll
-        for (int half = 0; half < 2; ++half)
+          for (int w = 0; w < 4; ++w)
+            s[i] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, words[w]), __builtin_bit_cast(bf16x2, 0x3f803f80u), s[i], false);
+          *(uint4 *)(part + (row_tile * 4 + group * 2) * 1024 + slot[i]) = permute_slots(v);
+        } else {
+          // A power of two takes the largest of the row's group into [2^14, 2^15); then three f16
+          // pieces, each the leading eleven bits of what the ones before left, make up every value to
+          // 2^-38 of that largest: the smallest step of f16 is 2^-24 (pieces are cut off, not rounded, so that
+          // the rest is exact).
+          uint32_t largest = 0;
 #pragma unroll
           for (int v = 0; v < 8; ++v) {
-            s += __uint_as_float(xr[t][half][v]);
-            largest = max(largest, xr[t][half][v] & 0x7fffffffu);
+            s[i] += __uint_as_float(xr[t][i][v]);
+            largest = max(largest, xr[t][i][v] & 0x7fffffffu);
           }
-        largest = max(largest, (uint32_t)__shfl_xor((int)largest, 16, 64));
-        largest = max(largest, (uint32_t)__shfl_xor((int)largest, 32, 64));
-        const uint32_t exponent = max(largest >> 23, 15u);
-        const float up = __uint_as_float((268u - exponent) << 23);   // exponent - 127 + 14, undone: 141 - exponent + 127
-        if (g == 0) ((float *)(part + kFragments * 1024 + RT * 1024))[group * 16 * RT + 16 * row_tile + n] = __uint_as_float((exponent - 14u) << 23);
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
+          largest = max(largest, (uint32_t)across<kOther>((int)largest));
+          largest = max(largest, (uint32_t)across<kOtherPair>((int)largest));
+          largest = max(largest, (uint32_t)across<kOtherFour>((int)largest));
+          const uint32_t exponent = max(largest >> 23, 15u);
+          const float up = __uint_as_float((268u - exponent) << 23);   // exponent - 127 + 14, undone: 141 - exponent + 127
+          if (chunk == 0) ((float *)(part + kFragments * 1024 + RT * 1024))[group * 16 * RT + 16 * row_tile + 8 * i + e] = __uint_as_float((exponent - 14u) << 23);
           float value[8];
 #pragma unroll
-          for (int v = 0; v < 8; ++v) value[v] = __uint_as_float(xr[t][half][v]) * up;
+          for (int v = 0; v < 8; ++v) value[v] = __uint_as_float(xr[t][i][v]) * up;
 #pragma unroll
           for (int piece = XP - 1; piece >= 0; --piece) {   // piece 0 holds the low bits, added first
             uint4 packed;
@@ -288,23 +324,26 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
               value[2 * v + 1] -= (float)two[1];
               words[v] = __builtin_bit_cast(uint32_t, two);
             }
-            *(uint4 *)(part + ((piece * RT + row_tile) * 4 + group * 2) * 1024 + slot[half]) =
+            *(uint4 *)(part + ((piece * RT + row_tile) * 4 + group * 2) * 1024 + slot[i]) =
                 BITS == 4 ? permute_slots(packed) : packed;
           }
         }
+        // the eight chunks of the row's group
+        s[i] += __int_as_float(across<kOther>(__float_as_int(s[i])));
+        s[i] += __int_as_float(across<kOtherPair>(__float_as_int(s[i])));
+        s[i] += __int_as_float(across<kOtherFour>(__float_as_int(s[i])));
       }
-      s += __shfl_xor(s, 16, 64);   // the four quarters of the row's group
-      s += __shfl_xor(s, 32, 64);
-      // quarter g stores the g-th piece of the sum (high, middle, low, nothing): slots 0..3 stand
-      // against the quad's four scales, 4..7 against its biases
-      const float high = __uint_as_float(__float_as_uint(s) & 0xffff0000u);
-      const float rest = s - high, middle = __uint_as_float(__float_as_uint(rest) & 0xffff0000u);
+      // Chunks 0..3 store the four pieces of row e's sum (high, middle, low, nothing), 4..7 those of row 8 + e: slots
+      // 0..3 of a lane quarter's operand stand against the quad's four scales, 4..7 against its biases.
+      const float sum = chunk < 4 ? s[0] : s[1];
+      const float high = __uint_as_float(__float_as_uint(sum) & 0xffff0000u);
+      const float rest = sum - high, middle = __uint_as_float(__float_as_uint(rest) & 0xffff0000u);
       const float low = rest - middle;
       // (by masks: written as a choice it becomes branches, which the contraction would be split by)
       const float mine = __uint_as_float((__float_as_uint(high) & sum_mask[0]) | (__float_as_uint(middle) & sum_mask[1]) |
                                          (__float_as_uint(low) & sum_mask[2]));
       const float offset = (XP == 1 ? -16.0f : BITS == 4 ? 8.0f : 128.0f) * mine;
-      uint16_t *to = (uint16_t *)(sums + row_tile * 1024 + lane * 16) + 2 * pair + group;
+      uint16_t *to = (uint16_t *)(sums + row_tile * 1024 + (16 * (chunk % 4) + 8 * (chunk / 4) + e) * 16) + 2 * pair + group;
       to[0] = (uint16_t)(__float_as_uint(offset) >> 16);
       to[4] = (uint16_t)(__float_as_uint(mine) >> 16);
     }
@@ -316,20 +355,28 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
   constexpr int LPP = BITS / 4;                  // loads per pair of groups and column tile
   // The tile's base address is uniform and stays in scalar registers (a tile past the last column
   // reads the last one); one offset per lane serves every tile.
-  const char *w_from[kColTiles], *s_from[kColTiles], *b_from[kColTiles];
-  const uint32_t w_lane = (n * words_per_row + 4 * g) * 4, s_lane = n * groups_per_row * 2;
+  const char *w_from[kColTiles];
+  const uint32_t w_lane = (n * words_per_row + 4 * g) * 4;
 #pragma unroll
   for (int tp = 0; tp < kColTiles; ++tp) {
     const int pj = tp / CT, ct = tp % CT;
     const uint32_t column = min(col_block * kBlockCols + (wc * CT + ct) * 16, a.columns - 16);
     w_from[tp] = (const char *)(a.packed[pj] + expert * a.expert_words + (uint64_t)column * words_per_row);
-    s_from[tp] = (const char *)(a.scales[pj] + expert * a.expert_groups + (uint64_t)column * groups_per_row);
-    b_from[tp] = (const char *)(a.biases[pj] + expert * a.expert_groups + (uint64_t)column * groups_per_row);
+  }
+  // Scales and biases: lane (n, g) reads those of column n of tile g, one load for the four tiles.
+  const char *s_from, *b_from;
+  {
+    const uint32_t column = min(col_block * kBlockCols + (wc * CT + g % CT) * 16, a.columns - 16) + n;
+    const uint64_t at = expert * a.expert_groups + (uint64_t)column * groups_per_row;
+    const uint16_t *s0 = a.scales[0], *s1 = a.scales[P - 1], *b0 = a.biases[0], *b1 = a.biases[P - 1];
+    asm("" : "+s"(s0), "+s"(s1), "+s"(b0), "+s"(b1));   // (chosen from registers, not loaded by lane)
+    s_from = (const char *)((g / CT ? s1 : s0) + at);
+    b_from = (const char *)((g / CT ? b1 : b0) + at);
   }
   // Requested ahead: the weights one pair of groups, the scales one quad, the biases from the
   // start of their quad to its end.
   u32x4 w[kColTiles][LPP];
-  u32x2 scale4[kColTiles], next_scale4[kColTiles], bias4[kColTiles];
+  u32x2 scale4[kColTiles], next_scales, biases;
   auto load_weights = [&](uint32_t quad, int pair) {
     const uint32_t at = (min(quad, quads - 1) * 2 + pair) * (LPP * 64);
 #pragma unroll
@@ -337,11 +384,16 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
 #pragma unroll
       for (int l = 0; l < LPP; ++l) w[tp][l] = load_at<u32x4>(uniform(w_from[tp] + at), w_lane + 64 * l);
   };
-  auto load_params = [&](u32x2 (&to)[kColTiles], const char *const (&from)[kColTiles], uint32_t quad) {
-    const uint32_t at = min(quad, quads - 1) * 8;
-#pragma unroll
-    for (int tp = 0; tp < kColTiles; ++tp) to[tp] = load_at<u32x2>(uniform(from[tp] + at), s_lane);
+  auto load_params = [&](const char *from, uint32_t quad) { return *(const u32x2 *)(from + min(quad, quads - 1) * 8); };
+  // Tile t's values from lane quarter t to all four quarters.
+  auto spread = [](uint32_t v, uint32_t (&to)[kColTiles]) {
+    const auto even_odd = __builtin_amdgcn_permlane16_swap(v, v, false, false);   // quarters 0 0 2 2 and 1 1 3 3
+    const uint32_t even = even_odd[0], odd = even_odd[1];
+    const auto low = __builtin_amdgcn_permlane32_swap(even, even, false, false);
+    const auto high = __builtin_amdgcn_permlane32_swap(odd, odd, false, false);
+    to[0] = low[0], to[1] = high[0], to[2] = low[1], to[3] = high[1];
   };
+  static_assert(kColTiles == 4, "a tile for each quarter of the lanes");
 
   f32x4 acc[kColTiles][RT];
 #pragma unroll
@@ -356,8 +408,9 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
     else
       return __builtin_amdgcn_mfma_f32_16x16x32_f16(rows, weights, sum, 0, 0, 0);
   };
-  auto contract = [&](uint32_t buffer, int pair, uint32_t next_quad, uint32_t keep) {
-    const char *part = staged + (buffer * WK + wk) * kPartBytes + lane * 16;
+  const uint32_t read_slot[2] = {(16 * g + (n ^ turn_of(g, 0))) * 16, (16 * g + (n ^ turn_of(g, 1))) * 16};
+  auto contract = [&](uint32_t buffer, int pair, uint32_t next_quad) {
+    const char *part = staged + (buffer * WK + wk) * kPartBytes;
     const char *factors = staged + (buffer * WK + wk) * kPartBytes + kFragments * 1024 + RT * 1024 + 16 * g;   // rows 4g..4g+3
     u32x2 first[kColTiles], second[kColTiles];
     if constexpr (BITS == 4) {
@@ -376,7 +429,7 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
       for (int piece = 0; piece < XP; ++piece)
 #pragma unroll
         for (int half = 0; half < 2; ++half)
-          rows[unit % 2][piece][half] = *(const Operand *)(part + ((piece * RT + unit % RT) * 4 + unit / RT * 2 + half) * 1024);
+          rows[unit % 2][piece][half] = *(const Operand *)(part + read_slot[half] + ((piece * RT + unit % RT) * 4 + unit / RT * 2 + half) * 1024);
     };
     if (kAhead) read_rows(0);
 #pragma unroll
@@ -398,7 +451,7 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
           b[tp][0] = unpack_bytes_f16(v.x, v.y);
           b[tp][1] = unpack_bytes_f16(v.z, v.w);
         }
-        const uint32_t word = (pair ? scale4[tp].y : scale4[tp].x) & keep;
+        const uint32_t word = pair ? scale4[tp].y : scale4[tp].x;
         scale[tp] = j ? high_bf16(word) : low_bf16(word);
       }
 #pragma unroll
@@ -434,12 +487,15 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
   };
   auto add_bias = [&](uint32_t parity, uint32_t keep) {
     const char *sums = staged + (parity * WK + wk) * kPartBytes + kFragments * 1024 + lane * 16;
+    uint32_t bias_x[kColTiles], bias_y[kColTiles];
+    spread(biases.x & keep, bias_x);
+    spread(biases.y & keep, bias_y);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       const bf16x8 rows = *(const bf16x8 *)(sums + rt * 1024);
 #pragma unroll
       for (int tp = 0; tp < kColTiles; ++tp) {
-        const uint4 params = make_uint4(scale4[tp].x & keep, scale4[tp].y & keep, bias4[tp].x & keep, bias4[tp].y & keep);
+        const uint4 params = make_uint4(scale4[tp].x, scale4[tp].y, bias_x[tp], bias_y[tp]);
         acc[tp][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rows, __builtin_bit_cast(bf16x8, params), acc[tp][rt], 0, 0, 0);
       }
     }
@@ -447,25 +503,30 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
 
   const uint32_t my_first = first_quad + wk;
   load_rows(my_first, 0);
-  load_params(next_scale4, s_from, my_first);
+  next_scales = load_params(s_from, my_first);
   load_weights(my_first, 0);
   uint32_t buffer = 0;
   for (uint32_t round = 0; round < rounds; ++round) {
     const uint32_t quad = my_first + round * WK;
     const uint32_t parity = round & 1;
-#pragma unroll
-    for (int tp = 0; tp < kColTiles; ++tp) scale4[tp] = next_scale4[tp];
-    load_params(bias4, b_from, quad);
+    biases = load_params(b_from, quad);   // (requested before the scales are waited for)
     // A wave whose part of the range is a quad short contracts a quad of another range with all
     // scales and biases zero: under a branch its loads would be waited for where the paths meet.
     const uint32_t keep = WK == 1 || quad < last_quad ? 0xffffffffu : 0u;
-    load_params(next_scale4, s_from, quad + WK);
+    {
+      uint32_t x[kColTiles], y[kColTiles];
+      spread(next_scales.x & keep, x);
+      spread(next_scales.y & keep, y);
+#pragma unroll
+      for (int tp = 0; tp < kColTiles; ++tp) scale4[tp] = u32x2{x[tp], y[tp]};
+    }
+    next_scales = load_params(s_from, quad + WK);
 #pragma unroll
     for (int pair = 0; pair < 2; ++pair) {
       stage_rows(buffer, parity, pair);
       load_rows(pair ? quad + WK : quad, pair ^ 1);
       __syncthreads();
-      contract(buffer, pair, pair ? quad + WK : quad, keep);
+      contract(buffer, pair, pair ? quad + WK : quad);
       if (pair == 1) add_bias(parity, keep);
       if (BITS == 8) load_weights(pair ? quad + WK : quad, pair ^ 1);
       buffer ^= 1;

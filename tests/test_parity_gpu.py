@@ -319,6 +319,25 @@ def test_quant_matmul_in_row_tiles(cpu, hip, rows, n, k, bits, dtype, padded):
     differential(cpu, hip, build)
 
 
+@pytest.mark.parametrize("rows,dtype", [(1, DType.BF16), (9, DType.BF16), (24, DType.BF16), (41, DType.BF16), (57, DType.BF16),
+                                        (97, DType.BF16), (9, DType.F32), (40, DType.F32)])
+def test_row_tiles_of_rows_with_something_between_them(cpu, hip, rows, dtype):
+    """Rows of a wider tensor: NaNs behind each row's values and in the rows that follow (tiles of 16 to 64 rows, each with
+    rows past the last one in its first or second eight)."""
+    weights = Quantised(27, 5, (1040, 1280))
+    values = np.full((rows + 64, 1280 + 64), np.nan, np.float32)
+    values[:rows, :1280] = normal_bf16(27, 3, (rows, 1280))
+
+    def build(backend):
+        x = upload(backend, values, dtype).narrow(0, 0, rows).narrow(1, 0, 1280)
+        out = backend.alloc(dtype, (rows, 1040))
+        commands = CommandList()
+        commands.dispatch(Op.quant_matmul(4, 64), [x, *weights.upload(backend)], out)
+        return commands, [out]
+    _, (hip_out, _) = differential(cpu, hip, build)
+    assert np.isfinite(to_f32(hip.read(hip_out[0]), dtype)).all()
+
+
 @pytest.mark.parametrize("rows,n,k,dtype", [(17, 272, 6400, DType.BF16), (64, 400, 3328, DType.BF16),
                                             (33, 16, 256, DType.BF16), (40, 272, 1280, DType.F32)])
 def test_row_tiles_under_an_epilogue_that_is_not_fused(cpu, hip, rows, n, k, dtype):
