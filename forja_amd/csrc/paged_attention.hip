@@ -1657,7 +1657,8 @@ bool run_ragged_attention(fh_backend *backend, const RaggedAttention &p, ErrorSl
     f.query_heads = p.query_heads;
     f.kv_heads = p.kv_heads;
     f.group = p.query_heads / p.kv_heads;
-    f.group_tokens = p.tokens > p.lanes ? kPrefillRows / f.group : 1;
+    // (under the promise of one row a lane, rows beyond the lanes belong to none)
+    f.group_tokens = p.tokens > p.lanes && !p.one_row_per_lane ? kPrefillRows / f.group : 1;
     f.page_tokens = p.page_tokens;
     f.physical_pages = p.physical_pages;
     f.table_pages = p.table_pages;

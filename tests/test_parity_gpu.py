@@ -1803,6 +1803,25 @@ def test_ragged_attention_refuses_malformed_cu_seqlens(cpu, hip, hq, hkv, pt, co
             assert np.frombuffer(backend.read(t["out"]), np.uint16).any()
 
 
+@pytest.mark.parametrize("promise", [False, True])
+def test_rows_of_no_lane_leave_the_promised_rows_stored(cpu, hip, promise):
+    """More rows than lanes, the last ones of no lane, under the promise of one row a lane: the lanes' new rows are stored
+    and attended, the others read zeros."""
+    def build(backend):
+        t, inputs = ragged_case(backend, [33, 70, 5], [1, 1, 1], 8, 4, 16, seed=70)
+        tables = np.frombuffer(backend.read(t["tables"]), np.uint32).reshape(3, -1, 2)
+        inputs[3] = upload(backend, tables[:2], DType.U32)
+        inputs[5] = upload(backend, np.array([0, 1, 2]), DType.U32)
+        inputs[6] = upload(backend, np.array([33, 70]), DType.U32)
+        commands = CommandList()
+        commands.dispatch_many(Op.paged_attention_ragged(0.09, 16, one_row_per_lane=promise), inputs,
+                               [t["out"], t["keys"], t["values"]])
+        return commands, [t["out"], t["keys"], t["values"]]
+    (cpu_out, _), (hip_out, _) = differential(cpu, hip, build)
+    assert cpu.read(cpu_out[1]) == hip.read(hip_out[1]) and cpu.read(cpu_out[2]) == hip.read(hip_out[2])
+    assert not to_f32(hip.read(hip_out[0]), DType.BF16).reshape(3, -1)[2].any()
+
+
 def test_ragged_attention_skips_inactive_lanes(cpu, hip):
     def build(backend):
         t, inputs = ragged_case(backend, [33, 70, 5], [1, 1, 1], 8, 4, 16, seed=62, activity=[1, 0, 1])
