@@ -918,31 +918,32 @@ __device__ inline void attend_one_token(const FastRagged &p, ErrorSlot *error, c
     const uint32_t tok_lo = max(begin, page0 * pt);
     const uint32_t tok_hi = (uint32_t)min((uint64_t)end, ((uint64_t)page0 + 64) * pt);
     // Two tiles in registers, in turns: one is requested while the other is on its way, and neither is moved (a
-    // move waits for it, and with it for every load before).  Only the last tile may be partial.  Bound by HBM where
+    // move waits for it, and with it for every load before).  Only the last tile may be partial: that of the item, and with
+    // pages of an odd multiple of 16 tokens that of 64 pages, whose other half begins the next 64.  Bound by HBM where
     // items fill the device, by one wave's chain where they do not: 23 lanes of 60 to 3000 keys (16 heads) 22.7 -> 21.0 us,
     // one lane of 500 keys 9.7 -> 8.5, 48 lanes (40 heads) 43.0 -> 41.6, 128 lanes of up to 32768 keys 288 -> 284, against
     // one tile that was moved between registers, and partial tiles of loads under a condition.
     uint32_t tile0 = tok_lo, left = (tok_hi - tok_lo + kTile - 1) / kTile;
     TileRegs a, b;
-    load_tile(p, a, tile0, end, page0, physical, lc);
+    load_tile(p, a, tile0, tok_hi, page0, physical, lc);
     for (; left > 2; left -= 2, tile0 += 2 * kTile) {
-      load_tile(p, b, tile0 + kTile, end, page0, physical, lc);
+      load_tile(p, b, tile0 + kTile, tok_hi, page0, physical, lc);
       __builtin_amdgcn_sched_barrier(0);
-      consume_tile<false, kHalf>(a, q_reg, o, sm, tile0, end, p.scale_log2, g);
+      consume_tile<false, kHalf>(a, q_reg, o, sm, tile0, tok_hi, p.scale_log2, g);
       __builtin_amdgcn_sched_barrier(0);
-      load_tile(p, a, tile0 + 2 * kTile, end, page0, physical, lc);
+      load_tile(p, a, tile0 + 2 * kTile, tok_hi, page0, physical, lc);
       __builtin_amdgcn_sched_barrier(0);
-      consume_tile<false, kHalf>(b, q_reg, o, sm, tile0 + kTile, end, p.scale_log2, g);
+      consume_tile<false, kHalf>(b, q_reg, o, sm, tile0 + kTile, tok_hi, p.scale_log2, g);
       __builtin_amdgcn_sched_barrier(0);
     }
     if (left == 2) {
-      load_tile(p, b, tile0 + kTile, end, page0, physical, lc);
+      load_tile(p, b, tile0 + kTile, tok_hi, page0, physical, lc);
       __builtin_amdgcn_sched_barrier(0);
-      consume_tile<false, kHalf>(a, q_reg, o, sm, tile0, end, p.scale_log2, g);
+      consume_tile<false, kHalf>(a, q_reg, o, sm, tile0, tok_hi, p.scale_log2, g);
       __builtin_amdgcn_sched_barrier(0);
-      consume_tile<true, kHalf>(b, q_reg, o, sm, tile0 + kTile, end, p.scale_log2, g);
+      consume_tile<true, kHalf>(b, q_reg, o, sm, tile0 + kTile, tok_hi, p.scale_log2, g);
     } else {
-      consume_tile<true, kHalf>(a, q_reg, o, sm, tile0, end, p.scale_log2, g);
+      consume_tile<true, kHalf>(a, q_reg, o, sm, tile0, tok_hi, p.scale_log2, g);
     }
   }
   // Lane (row hl, group g) holds value columns 32g + 8j + mt of its row.

@@ -1822,6 +1822,25 @@ def test_rows_of_no_lane_leave_the_promised_rows_stored(cpu, hip, promise):
     assert not to_f32(hip.read(hip_out[0]), DType.BF16).reshape(3, -1)[2].any()
 
 
+def test_decode_item_of_more_than_64_pages(cpu, hip):
+    """Pages of an odd multiple of sixteen tokens: the 64 that a wave looks up at once may end within a tile of 32 keys, whose
+    other half belongs to the next 64.  6000 rows leave a lane two items: the second begins at key 3232, its first page at
+    3216, and its 64 pages end at 6288, in the middle of a tile."""
+    contexts = [6463, 80, 0]
+
+    def build(backend):
+        t, inputs = ragged_case(backend, contexts, [1, 1, 5998], 2, 1, 48, seed=71)
+        tables = np.frombuffer(backend.read(t["tables"]), np.uint32).reshape(3, -1, 2)
+        inputs[3] = upload(backend, tables[:2], DType.U32)
+        inputs[5] = upload(backend, np.array([0, 1, 2]), DType.U32)
+        inputs[6] = upload(backend, np.array(contexts[:2]), DType.U32)
+        commands = CommandList()
+        commands.dispatch_many(Op.paged_attention_ragged(0.09, 48, one_row_per_lane=True), inputs,
+                               [t["out"], t["keys"], t["values"]])
+        return commands, [t["out"]]
+    differential(cpu, hip, build)
+
+
 def test_ragged_attention_skips_inactive_lanes(cpu, hip):
     def build(backend):
         t, inputs = ragged_case(backend, [33, 70, 5], [1, 1, 1], 8, 4, 16, seed=62, activity=[1, 0, 1])
