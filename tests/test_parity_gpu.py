@@ -1825,12 +1825,16 @@ def test_rows_of_no_lane_leave_the_promised_rows_stored(cpu, hip, promise):
 def test_decode_item_of_more_than_64_pages(cpu, hip):
     """Pages of an odd multiple of sixteen tokens: the 64 that a wave looks up at once may end within a tile of 32 keys, whose
     other half belongs to the next 64.  6000 rows leave a lane two items: the second begins at key 3232, its first page at
-    3216, and its 64 pages end at 6288, in the middle of a tile."""
+    3216, and its 64 pages end at 6288, in the middle of a tile.  Were that half read through the first page, the values of
+    page 67, a hundred times the others, would count twice."""
     contexts = [6463, 80, 0]
 
     def build(backend):
         t, inputs = ragged_case(backend, contexts, [1, 1, 5998], 2, 1, 48, seed=71)
         tables = np.frombuffer(backend.read(t["tables"]), np.uint32).reshape(3, -1, 2)
+        values = to_f32(backend.read(t["values"]), DType.BF16).reshape(-1, 48, 128).copy()
+        values[tables[0, 67, 0]] *= 100.0
+        backend.write(t["values"], orc.f32_to_bf16(values).tobytes())
         inputs[3] = upload(backend, tables[:2], DType.U32)
         inputs[5] = upload(backend, np.array([0, 1, 2]), DType.U32)
         inputs[6] = upload(backend, np.array(contexts[:2]), DType.U32)
