@@ -31,10 +31,11 @@
 // The activations come in by rows, eight lanes to a row's 128 bytes of a group: sixteen bytes of another row in every lane
 // (operand order) cost the compute unit's address unit 65 cycles a load against 18, and a third of all loads were of
 // that kind; the chunks find their operand places on the way into LDS, and a group's sum is three exchanges within eight
-// lanes.  A lane quarter reads the scales and biases of one column tile for all four.  Against operand-order loads
-// by every quarter: bf16 48 x 34816 x 5120 67 -> 61 us, 48 x 151936 x 5120 209 -> 193, 64 x 34816 x 5120 83 -> 75; f32 512 x 5120 x 2048
-// 60 -> 54; routed as above, bf16 24000 routes 457 -> 434, f32 8192 routes 388 -> 371; launches of one or two quads
-// a workgroup, whose length is their latency, 0 to 1 us longer (8 bits 512 x 128 x 2048 12.8 -> 13.7).
+// lanes.  A lane quarter reads the scales and biases of one column tile for all four, by global loads: through pointers
+// that may point to LDS every wait for LDS waited for them and for all loads before (48 x 34816 x 5120 57.7 us for 56.1,
+// 8 bits 512 x 128 x 2048 13.5 for 12.3).  Against operand-order loads by every quarter: bf16 48 x 34816 x 5120 63 -> 56 us,
+// 48 x 151936 x 5120 183 -> 164, 64 x 34816 x 5120 75 -> 70, 20 x 34816 x 5120 49 -> 47; f32 512 x 5120 x 2048 57 -> 52, 8 bits
+// 512 x 128 x 2048 12.7 -> 12.3 (back to back, weights from memory).
 //
 // The bias term rides on the matrix cores too: the group sums are split into their three exact
 // bf16 pieces, one per lane quarter, and the operand against them is the column's scales and
@@ -364,14 +365,16 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
     w_from[tp] = (const char *)(a.packed[pj] + expert * a.expert_words + (uint64_t)column * words_per_row);
   }
   // Scales and biases: lane (n, g) reads those of column n of tile g, one load for the four tiles.
-  const char *s_from, *b_from;
+  global_bytes s_from, b_from;
   {
     const uint32_t column = min(col_block * kBlockCols + (wc * CT + g % CT) * 16, a.columns - 16) + n;
     const uint64_t at = expert * a.expert_groups + (uint64_t)column * groups_per_row;
-    const uint16_t *s0 = a.scales[0], *s1 = a.scales[P - 1], *b0 = a.biases[0], *b1 = a.biases[P - 1];
-    asm("" : "+s"(s0), "+s"(s1), "+s"(b0), "+s"(b1));   // (chosen from registers, not loaded by lane)
-    s_from = (const char *)((g / CT ? s1 : s0) + at);
-    b_from = (const char *)((g / CT ? b1 : b0) + at);
+    // (uniform: chosen from registers, not loaded by lane; and known to be global: a load from a pointer that may
+    // point to LDS waits for, and is waited for with, every access to LDS)
+    const global_bytes s0 = uniform((const char *)a.scales[0]), s1 = uniform((const char *)a.scales[P - 1]);
+    const global_bytes b0 = uniform((const char *)a.biases[0]), b1 = uniform((const char *)a.biases[P - 1]);
+    s_from = (g / CT ? s1 : s0) + 2 * at;
+    b_from = (g / CT ? b1 : b0) + 2 * at;
   }
   // Requested ahead: the weights one pair of groups, the scales one quad, the biases from the
   // start of their quad to its end.
@@ -384,7 +387,9 @@ __global__ __launch_bounds__(64 * WC * WK, 2) void qmm_rows_kernel(RowsArgs a) {
 #pragma unroll
       for (int l = 0; l < LPP; ++l) w[tp][l] = load_at<u32x4>(uniform(w_from[tp] + at), w_lane + 64 * l);
   };
-  auto load_params = [&](const char *from, uint32_t quad) { return *(const u32x2 *)(from + min(quad, quads - 1) * 8); };
+  auto load_params = [&](global_bytes from, uint32_t quad) {
+    return *(const __attribute__((address_space(1))) u32x2 *)(from + min(quad, quads - 1) * 8);
+  };
   // Tile t's values from lane quarter t to all four quarters.
   auto spread = [](uint32_t v, uint32_t (&to)[kColTiles]) {
     const auto even_odd = __builtin_amdgcn_permlane16_swap(v, v, false, false);   // quarters 0 0 2 2 and 1 1 3 3
