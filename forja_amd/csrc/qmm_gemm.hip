@@ -12,7 +12,8 @@
 //     matrix cores run both at the same rate.  bf16 activations convert to fp16 exactly once a row
 //     is scaled by a power of two into the fp16 range (undone exactly when the result is stored).
 //   * Weights are centred: w = scale * (q - 8).  That is a number of fp16 exactly (a scale has eight significant bits,
-//     q - 8 at most three or is a power of two), where scale * q rounded once misses the tolerance at the deepest
+//     q - 8 at most three or is a power of two; scales below 2^-14, which only the whole fp16 operand admits, lose the bits
+//     that fall below fp16's smallest), where scale * q rounded once misses the tolerance at the deepest
 //     contraction (K = 17408).  What centring takes out, (bias + 8 * scale) * sum of the group's
 //     activations, is put back through the same GEMM: both operands get three more K columns per
 //     quantisation group, holding S/64 and 64 * (bias + 8 * scale) each split in an fp16 head and tail
@@ -214,10 +215,16 @@ __global__ __launch_bounds__(256) void prepare_rows_kernel(const uint16_t *x, ui
   }
 }
 
-// Scales and biases this scheme can take: every centred weight and 64 * (bias + centre) must
-// stay inside the fp16 range.  False for NaN too.
+// Scales and biases this scheme can take: every centred weight (8 * scale) and 64 * (bias + 8 * scale) must
+// stay inside the fp16 range.  (Of a bias near -7.5 * scale the second is the narrower one: scales up to 1800.)  False
+// for NaN too.
 __device__ inline bool f16_safe(float scale, float bias) {
-  return fabsf(scale) <= 2700.0f && fabsf(bias + 8.0f * scale) <= 900.0f;
+  return fabsf(scale) <= 4000.0f && fabsf(bias + 8.0f * scale) <= 900.0f;
+}
+// ... and what unpacking the words needs of a scale besides (dequantise_word): 24 times a scale inside the fp16 range, and
+// the scale itself, one of eight significant bits, no smaller than a normal number of fp16.
+__device__ inline bool f16_unpackable(float scale) {
+  return fabsf(scale) <= 2700.0f && (scale == 0.0f || fabsf(scale) >= 6.103515625e-5f);
 }
 
 // packed/scales/biases [columns, inner] -> fp16 [columns, kt]: scale * (q - 8)
@@ -614,8 +621,7 @@ __global__ __launch_bounds__(256) void prepare_extras_kernel(const uint16_t *sca
     float value = 0.0f;
     if (group < groups) {
       const float scale = bf16_bits_to_f32(s_row[group]), bias = bf16_bits_to_f32(b_row[group]);
-      // the GEMM multiplies by the scale as an fp16 number: it must be one exactly
-      if (kind == 0 && (!f16_safe(scale, bias) || (scale != 0.0f && fabsf(scale) < 6.103515625e-5f))) refused[0] = 1;
+      if (kind == 0 && (!f16_safe(scale, bias) || !f16_unpackable(scale))) refused[0] = 1;
       float head, tail;
       split_f16(64.0f * (bias + 8.0f * scale), &head, &tail);
       value = kind == 2 ? tail : head;

@@ -587,6 +587,48 @@ def test_quant_gemm_with_scales_outside_the_fp16_range_and_huge_activations(cpu,
     differential(cpu, hip, build)
 
 
+@pytest.mark.parametrize("k,scale,bias,taken", [
+    # words unpacked in the GEMM (whole blocks of eight groups): 24 scale within fp16, the scale a normal number of it
+    (512, 2688.0, -8.0, True), (512, 2704.0, -8.0, False), (512, -2688.0, -8.0, True),
+    (512, 2.0 ** -14, -8.0, True), (512, 2.0 ** -14 - 2.0 ** -22, -8.0, False), (512, 0.0, 0.0, True),
+    (512, 1792.0, -7.5, True), (512, 1920.0, -7.5, False),      # 64 (bias + 8 scale) within fp16
+    # fp16 weights written once
+    (768, 2704.0, -8.0, True), (768, 4000.0, -8.0, True), (768, 4016.0, -8.0, False), (768, 2.0 ** -15, -8.0, True),
+    (768, 1792.0, -7.5, True), (768, 1920.0, -7.5, False),
+])
+def test_prefill_products_at_the_limits_of_a_scale(k, scale, bias, taken):
+    """One group's scale and bias (a multiple of it) at either side of what the GEMM takes.  Refused weights go to the
+    kernel of any range, and no operand of theirs is kept.  Each column against 64 bits: results are rounded once, by at
+    most 2^-8 of each; what the sums themselves and one group of weights below fp16's normal numbers add is far less."""
+    from forja_amd.hip_backend import HipBackend
+    own = HipBackend(0)
+    try:
+        rows, n = 140, 80
+        weights, values = Quantised(63, k, (n, k)), normal_bf16(63, 1, (rows, k))
+        for held, value in ((weights.scales, scale), (weights.biases, bias * scale)):
+            raw = orc.f32_to_bf16(np.array([value], np.float32))
+            assert orc.bf16_to_f32(raw)[0] == value
+            held[37, 5] = raw[0]
+        out = own.alloc(DType.BF16, (rows, n))
+        commands, x, triple = CommandList(), upload(own, values, DType.BF16), weights.upload(own)
+        commands.dispatch(Op.quant_matmul(4, 64), [x, *triple], out)
+        prepared = n * (64 if k == 512 else 832) * 2    # 3 columns a group (or all with them), in whole steps of 64
+        held = []
+        for _ in range(2):      # the first product prepares, the second knows
+            run(own, commands)
+            held.append(own.memory_usage())
+            reference = values.astype(np.float64) @ weights.dequantised().T
+            error = to_f32(own.read(out), DType.BF16).reshape(rows, n) - reference
+            assert np.all(np.linalg.norm(error, axis=0) <= 2.0 ** -8 * np.linalg.norm(reference, axis=0))
+        assert held[0] == held[1]
+        for tensor in triple:   # releasing the weights gives back what was kept of them
+            own.release(tensor)
+        kept = held[1] - own.memory_usage() - sum(t.layout.buffer_len for t in triple)
+        assert kept == (prepared + 256 if taken else 0)
+    finally:
+        own.close()
+
+
 def test_quant_matmul_on_strided_views_with_bias_epilogue(cpu, hip):
     """Every operand sliced with step 2 (crates/forja-metal/tests/quant_matmul/shared.rs:95-107)
     plus a fused epilogue that adds a broadcast bias."""
