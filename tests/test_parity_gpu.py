@@ -1529,10 +1529,23 @@ def test_ragged_attention_equals_the_per_lane_sequence(cpu, hip, contexts, count
     assert cpu.read(cpu_out[1]) == hip.read(hip_out[1]) and cpu.read(cpu_out[2]) == hip.read(hip_out[2])
 
 
+def keep_only_keys(backend, t, contexts, pt, hkv):
+    """Every slot of the pools that holds no key of `contexts` becomes a NaN."""
+    tables = np.frombuffer(backend.read(t["tables"]), np.uint32).reshape(t["tables"].shape)
+    for name in ("keys", "values"):
+        pool = np.frombuffer(backend.read(t[name]), np.uint16).reshape(-1, pt, hkv * 128)
+        held = np.full_like(pool, 0x7fff)
+        for lane, keys in enumerate(contexts):
+            for first in range(0, keys, pt):
+                page, rows = tables[lane, first // pt, 0], min(pt, keys - first)
+                held[page, :rows] = pool[page, :rows]
+        backend.write(t[name], held.tobytes())
+
+
 @pytest.mark.parametrize("pt,hq,hkv,dtype", [(16, 16, 8, DType.BF16), (48, 5, 1, DType.F16), (64, 32, 2, DType.F32)])
 def test_decode_reads_no_slot_past_its_keys(cpu, hip, pt, hq, hkv, dtype):
-    """Every length of a last tile and both parities of the tiles in front of it, one split and several; all slots
-    that hold no key are NaNs (bf16 and f16 pools; f32 queries read an f16 one)."""
+    """Every length of a last tile, one split and several (of one or two tiles, most of them); all slots that hold no key
+    are NaNs (bf16 and f16 pools; f32 queries read an f16 one)."""
     contexts = list(range(0, 66)) + [94, 95, 96, 127, 128, 159, 160, 161, 64 * pt - 2, 64 * pt, 64 * pt + 33, 4000]
     pool_dtype = DType.F16 if dtype is DType.F32 else dtype
     pools = {}
@@ -1540,17 +1553,40 @@ def test_decode_reads_no_slot_past_its_keys(cpu, hip, pt, hq, hkv, dtype):
     def build(backend):
         t, inputs = ragged_case(backend, contexts, [1] * len(contexts), hq, hkv, pt, seed=67, dtype=dtype,
                                 pool_dtype=pool_dtype)
-        tables = np.frombuffer(backend.read(t["tables"]), np.uint32).reshape(len(contexts), -1, 2)
-        for name in ("keys", "values"):
-            pool = np.frombuffer(backend.read(t[name]), np.uint16).reshape(-1, pt, hkv * 128)
-            held = np.full_like(pool, 0x7fff)
-            for lane, keys in enumerate(contexts):
-                for first in range(0, keys, pt):
-                    page, rows = tables[lane, first // pt, 0], min(pt, keys - first)
-                    held[page, :rows] = pool[page, :rows]
-            backend.write(t[name], held.tobytes())
+        keep_only_keys(backend, t, contexts, pt, hkv)
         commands = CommandList()
         commands.dispatch_many(Op.paged_attention_ragged(0.09, pt), inputs, [t["out"], t["keys"], t["values"]])
+        pools[backend] = t["keys"], t["values"]
+        return commands, [t["out"]]
+    _, (hip_out, _) = differential(cpu, hip, build, bar=pool_dtype)
+    assert np.isfinite(to_f32(hip.read(hip_out[0]), dtype)).all()
+    for want, got in zip(pools[cpu], pools[hip]):
+        assert cpu.read(want) == hip.read(got)
+
+
+@pytest.mark.parametrize("pt,hq,hkv,dtype", [(16, 4, 2, DType.BF16), (48, 5, 1, DType.F16), (64, 4, 1, DType.F32)])
+def test_decode_items_of_many_tiles_read_no_slot_past_their_keys(cpu, hip, pt, hq, hkv, dtype):
+    """Items of one to seven tiles of 32 keys, so that either of the kernel's two tiles in flight ends one, with last tiles
+    of one key to all of them; all slots that hold no key are NaNs.  A batch of so many rows has room for one split a lane
+    (16384 // rows), whatever length splits have: an item is a lane's keys."""
+    rows = 8200
+    assert 16384 // rows == 1
+    contexts = [32 * tiles + last - 1 for tiles in range(7) for last in (1, 15, 16, 17, 31, 32)]
+    lanes = len(contexts)
+    pool_dtype = DType.F16 if dtype is DType.F32 else dtype
+    pools = {}
+
+    def build(backend):
+        t, inputs = ragged_case(backend, contexts + [0], [1] * lanes + [rows - lanes], hq, hkv, pt, seed=72, dtype=dtype,
+                                pool_dtype=pool_dtype)
+        keep_only_keys(backend, t, contexts, pt, hkv)
+        tables = np.frombuffer(backend.read(t["tables"]), np.uint32).reshape(t["tables"].shape)
+        inputs[3] = upload(backend, tables[:lanes], DType.U32)     # the other rows belong to no lane
+        inputs[5] = upload(backend, np.arange(lanes + 1), DType.U32)
+        inputs[6] = upload(backend, np.array(contexts), DType.U32)
+        commands = CommandList()
+        commands.dispatch_many(Op.paged_attention_ragged(0.09, pt, one_row_per_lane=True), inputs,
+                               [t["out"], t["keys"], t["values"]])
         pools[backend] = t["keys"], t["values"]
         return commands, [t["out"]]
     _, (hip_out, _) = differential(cpu, hip, build, bar=pool_dtype)
