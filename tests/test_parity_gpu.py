@@ -540,8 +540,8 @@ def test_quant_matmul_with_f16_scales_and_a_residual_in_other_dtypes(cpu, hip, d
 ])
 @pytest.mark.parametrize("residual", [False, True])
 def test_prefill_products_of_few_tiles(hip, rows, n, k, residual):
-    """Products whose waves split K: against 64 bits.  A result is rounded once to bf16 (2^-9 of it at most), its
-    weights once to f16 (2^-12 of each)."""
+    """Products whose waves split K: against 64 bits.  A result is rounded once to bf16 (2^-9 of all of them together);
+    what the products' operands are held to is in the test of their exactness."""
     weights, values, extra = Quantised(62, n + k, (n, k)), normal_bf16(62, 1, (rows, k)), normal_bf16(62, 2, (rows, n))
     out = hip.alloc(DType.BF16, (rows, n))
     commands, operands = CommandList(), [upload(hip, values, DType.BF16), *weights.upload(hip)]
@@ -557,6 +557,34 @@ def test_prefill_products_of_few_tiles(hip, rows, n, k, residual):
     # (element by element: the sums' own rounding is that of f16 products of k random values)
     scale = np.sqrt(np.mean(reference ** 2))
     assert np.all(np.abs(error) <= 2.0 ** -8 * np.abs(reference) + 2.0 ** -9 * scale)
+
+
+@pytest.mark.parametrize("rows,n,k", [
+    (140, 72, 512), (140, 136, 17408),      # 128 x 64 tiles, K over four parts of a workgroup's waves
+    (600, 5120, 1024),                      # 128 x 128 tiles, two parts
+    (1030, 5120, 512),                      # 128 x 128 tiles of four waves
+    (2100, 6200, 512),                      # 256 x 256 tiles
+    (140, 72, 768), (2100, 6200, 256),      # fp16 weights written once
+])
+def test_prefill_products_hold_weights_and_rows_exactly(hip, rows, n, k):
+    """What is left of a product beside the bf16 numbers nearest to it in 64 bits (added before the one rounding, of at most
+    2^-8 of what is left, itself at most 2^-8 of the product).  Rows and weights are exact; group sums and the biases against
+    them are held to 2^-22, and the sums are those of f32.  Weights rounded to f16 would be off by 2^-12.3 of the
+    product."""
+    weights, values = Quantised(64, n + k, (n, k)), normal_bf16(64, 1, (rows, k))
+    centred = -7.5 * orc.bf16_to_f32(weights.scales)    # weights of no common sign
+    weights.biases = orc.f32_to_bf16(centred.ravel()).reshape(centred.shape)
+    reference = values.astype(np.float64) @ weights.dequantised().T
+    nearest = orc.bf16_to_f32(orc.f32_to_bf16(-reference.astype(np.float32).ravel())).reshape(rows, n)
+    out = hip.alloc(DType.BF16, (rows, n))
+    commands = CommandList()
+    commands.dispatch_epilogue(Op.quant_matmul(4, 64), [upload(hip, values, DType.BF16), *weights.upload(hip)], out,
+                               hip.prepare_epilogue(programs.add_elements()), [upload(hip, nearest, DType.BF16)])
+    run(hip, commands)
+    left = reference + nearest
+    error = to_f32(hip.read(out), DType.BF16).reshape(rows, n) - left
+    assert np.linalg.norm(error) <= 2.0 ** -16 * np.linalg.norm(reference)
+    assert np.linalg.norm(left) >= 2.0 ** -10 * np.linalg.norm(reference)
 
 
 def test_quant_gemm_with_scales_outside_the_fp16_range_and_huge_activations(cpu, hip):
