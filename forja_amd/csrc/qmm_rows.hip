@@ -753,24 +753,30 @@ bool launch_rows_dense(fh_backend *backend, const RowsDense &d) {
   a.row_blocks = row_blocks;
   a.col_blocks = (d.columns + block_cols - 1) / block_cols;
   a.splits = 1;
-  // K over workgroups where that shortens the launch.  Measured (microseconds, 48 x 5120 x 17408 and
-  // 48 x 34816 x 5120 bf16, 512 x 5120 x 2048 f32): a workgroup alone on its compute unit takes
-  // `alone` per quad of its longest K wave and 2.4 beyond that, two that share one take `shared` each
-  // (bf16 rows gain nothing from sharing; f32 rows, which meet at two
-  // barriers a pair of groups, do).  Splits cost their partial sums and the launch that adds them.
+  // K over workgroups where that shortens the launch, estimated for the XCD that gets the most of them (units go round
+  // the eight: 220 tiles of 350 x 5120 put 33 on each of four XCDs, which take a third longer than 32 would).  In microseconds:
+  // a workgroup alone on its compute unit takes `alone` per quad of its longest K wave (measured, K = 17408: rows of
+  // 16, 32, 48 and 64 2.0, 2.5, 2.9 and 3.5; f32 rows 4.4), two that share one `shared`, a round of those 2 besides;
+  // splits cost their partial sums and the launch that adds them.  What is not measured by itself is chosen so that of 109
+  // products of 9 to 128 bf16 rows (K 2048 to 17408) and 63 of 33 to 1024 f32 rows, each timed with one to ten splits, the
+  // chosen number is 0.14 and 0.6 % off the fastest on average, 4 and 7 % at most.  (Counted for the whole device, with
+  // constants from operand-order loads: 1.0 and 4 %, 13 and 40 % at most; 95 x 5120 x 17408 51 -> 46 us with six splits
+  // for three, 330 f32 rows x 5120 x 2048 58 -> 41 with two for one.)
   const uint32_t quads = d.inner / kQuad, waves_k = d.wide ? 1 : 2;
-  const uint64_t tiles = (uint64_t)a.row_blocks * a.col_blocks, units_cu = backend_compute_units(backend);
+  const uint64_t places = 2 * std::max<uint32_t>(1, backend_compute_units(backend) / 8);   // of an XCD
   const uint64_t plane = (uint64_t)d.rows * d.columns * sizeof(float);
   if (d.columns % 4 == 0) {
-    const double alone = d.wide ? 4.5 : 1.0 + 0.9 * tile_rows / 16, shared = d.wide ? 1.65 * alone : 2.0 * alone;
+    const double alone = d.wide ? 4.4 : 1.45 + 0.5 * tile_rows / 16, shared = (d.wide ? 1.55 : 1.65) * alone;
+    const double bytes_per_us = d.wide ? 4.5e6 : 3e6;
     const uint64_t most = std::min<uint64_t>(std::max<uint32_t>(1, quads / waves_k), backend_workspace_limit(backend) / plane);
     uint64_t best = 1;
     double best_us = 0.0;
     for (uint64_t splits = 1; splits == 1 || splits <= most; ++splits) {
       const uint64_t range = (quads + splits - 1) / splits, rounds = (range + waves_k - 1) / waves_k;
-      const uint64_t groups = tiles * splits, whole = groups / (2 * units_cu), rest = groups % (2 * units_cu);
-      double us = (whole + (rest > units_cu)) * (rounds * shared + 4.8) + (rest && rest <= units_cu ? rounds * alone + 2.4 : 0.0);
-      if (splits > 1) us += splits * plane / 5e6 + 4.0;
+      const uint64_t groups = (a.col_blocks * splits + 7) / 8 * a.row_blocks, whole = groups / places, rest = groups % places;
+      double us = (whole + (2 * rest > places)) * (rounds * shared + 2.0);
+      if (rest && 2 * rest <= places) us += rounds * alone;
+      if (splits > 1) us += splits * plane / bytes_per_us + 3.0;
       if (splits == 1 || us < best_us) best = splits, best_us = us;
     }
     if (best > 1) {
