@@ -308,8 +308,9 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 constexpr uint32_t kMinSplitTokens = 128, kMaxSplitTokens = 1024;  // split length bounds beside prompt rows
 // Of a decode batch that fits the device at once: with two tiles a wave requests its whole item before it waits.  Steps of
-// the small model with items of 64 keys against 128: 3 lanes 1459 / 1616 us, 8 lanes 1507 / 1663, 14 lanes 1578 / 1730,
-// 30 lanes 1840 / 2008; of the mixture model 1 and 2 lanes 0.97 to 1.00; items of 32: equal to 0.98, but more to merge.
+// the small model with items of 32, 64 and 128 keys: 8 lanes 1470, 1466, 1633 us, 14 lanes 1646, 1541, 1700; of the
+// mixture model one and two lanes 766, 765, 772 and 799, 798, 813.  (Where places are plenty, one tile to an item is better
+// still: see ragged_plan_kernel.  Where they are not, the plan's own length is: 23 lanes 1888 against 2013, 2087, 1964.)
 constexpr uint32_t kMinDecodeSplit = 64;
 // see ragged_plan_kernel (512 groups: two for each of the 256 compute units that an MI355X has)
 constexpr uint32_t kFillingGroups = 512, kFilledSplitTokens = 512;
@@ -555,10 +556,10 @@ __global__ __launch_bounds__(kPlanThreads) void ragged_plan_kernel(FastRagged p,
       if (split_tokens > kMaxSplitTokens) split_tokens = kMaxSplitTokens;
     } else if (longest_keys <= p.max_splits * kTile &&
                2 * (total_attended / kTile + p.tokens) <= p.item_slots) {
-      // Few keys in all: one tile to an item.  What such a launch takes is the chain of one wave, and
-      // an item of a single tile never enters the pipelined loop (one lane of 400 keys: 9.5 us against
-      // 19 us with items of two to four tiles; with more items than half the places the shorter chain
-      // is lost again to their number).
+      // Few keys in all: one tile to an item.  What such a launch takes is the chain of one wave, and every further tile
+      // lengthens it (one to three lanes of 60 to 3000 keys, the kernel by itself: 8.6 us, 12 with items of two tiles, 18 with
+      // four; the merge of more items 4.1 -> 5; steps of one and three lanes 1252 and 1341 us against 1333 and 1400 with items
+      // of two); with more items than half the places the shorter chain is lost again to their number.
       split_tokens = kTile;
     } else {
       // Decode batches: the shortest split length whose items all find a place on the device at

@@ -1217,13 +1217,14 @@ bool try_fast_quant_matmul(fh_backend *backend, const QmmProblem &p) {
     if (launch_ksplit_dense(backend, d)) return true;
   }
   // More rows, or a longer K, than the K-split kernels hold: row tiles, the weights unpacked once for
-  // all rows of a tile.  (48 x 34816 x 5120 66 us against 101 through the streaming kernel, 48 x 5120 x
-  // 17408 33 against 75 through the tile product; 1 row against 34816 x 5120 43 and 64; 128 x 2048 x 4096
-  // with the launch that adds its K ranges 17.6 against 19.0, in the decode step's trace 11.8 + 4.6 against 17.9.)
+  // all rows of a tile.  (48 x 34816 x 5120 56 us against 101 through the streaming kernel, 48 x 5120 x
+  // 17408 30 against 75 through the tile product; 1 row against 34816 x 5120 37 and 64; 128 x 2048 x 4096
+  // with the launch that adds its K ranges 15.5 against 19.0, in the decode step's trace 11.1 + 4.6 against 17.9.)
   // Two shapes go elsewhere: vocabulary-sized matrices at more than 64 rows, which the GEMM's 128-row tiles
-  // read once (128 x 151936 x 2048 127 us against 175); and at most 8 rows against so little weight that a
-  // launch's fixed costs are most of the time: there the two are close (1 x 5120 x 5120 11.8 us through the
-  // tile product and 11.2 through row tiles, 8 rows 13.4 and 11.7), and one
+  // read once (128 x 151936 x 2048 113 us against 136, 95 rows of K = 5120 245 against 268; the line lies low for few
+  // row tiles of fewer columns: 65, 95 and 128 x 34816 x 5120 84, 85, 87 against 76, 81, 96); and at most 8 rows against so
+  // little weight that a launch's fixed costs are most of the time: there the two are close (1 and 8 x 5120 x 5120 10.4 and
+  // 11.6 us through the tile product, 9.4 and 9.7 through row tiles, x 7168 11.7 and 12.9 against 12.6 and 13.1), and one
   // launch needs no room for partial sums.
   const bool vocabulary = p.rows > 64 && p.columns >= 32768;
   const bool little = p.rows <= 8 && p.inner <= 6144 && (p.columns + 31) / 32 <= backend_compute_units(backend);

@@ -948,10 +948,10 @@ __global__ __launch_bounds__(64 * kWM * kWN) void gemm_q4_kernel(GemmArgs a) {
 
 // The same product for outputs of few tiles: eight waves of 64 rows x 64 columns, kWM x kWN of them beside each other
 // and kWK along K, so that a compute unit has two waves per SIMD although its tile is small (2 x 2 x 2: 128 x 128;
-// 2 x 1 x 4: 128 x 64).  Four waves of 64 x 64, one per SIMD, take 2000 cycles a K step of 64 whatever is loaded
-// when (rings of two to five steps measured the same): half of them issuing, in order, 280 instructions that no
-// other wave's overlap, the other half at waits and the barrier.  In a period every wave takes one of the kWK
-// next steps, all of them behind one barrier.  2048 rows x 1024 columns: K 2048 41 -> 29 us, K 3072 54 -> 35, with the rows' preparation
+// 2 x 1 x 4: 128 x 64).  Four waves of 64 x 64, one per SIMD, take 1500 cycles a K step of 64 (2000 before their unpacking
+// was shortened, whatever was loaded when: rings of two to five steps measured the same), issuing, in order, instructions
+// that no other wave's overlap, and at waits and the barrier.  In a period every wave takes one of the kWK
+// next steps, all of them behind one barrier.  2048 rows x 1024 columns: K 2048 39.7 -> 28.5 us, K 3072 50.4 -> 34.8, with the rows' preparation
 // (8 and 10 us of it).  What is left of a launch: 8 us before and after the periods, 1.4 us a period of 256 K values,
 // of which the matrix instructions take 0.5 and the loads (72 KB a compute unit) most of the rest.
 //   * Activations and packed words of kSlots periods and scales of two blocks of eight groups in LDS, loaded by
@@ -1364,9 +1364,10 @@ bool launch_quant_gemm(fh_backend *backend, const QmmProblem &p, const uint32_t 
   if (packed_form) {
     // Outputs with fewer small tiles than the device has compute units: the kernel whose waves split K.  More tiles
     // put two workgroups of four waves on a unit, which hide each other's waits too, without meeting K parts
-    // (microseconds, 128 x 128 tiles of four waves, 128 x 128 and 128 x 64 of eight: 2048 x 1024 x 2048 41.3, 32.0,
-    // 29.2; 300 x 4096 x 1024 22.8, 18.4, 15.1; 600 x 5120 x 17408 258, 186, 220 (400 of 128 x 64); 1000 x 5120 x 5120
-    // 106, 112, 108; 2080 x 5120 x 2048 81, 84, 101).
+    // (microseconds with the rows' preparation, 128 x 128 tiles of four waves, 128 x 128 and 128 x 64 of eight: 2048 x 1024 x
+    // 2048 39.7, 30.5, 28.5; 300 x 4096 x 1024 21.6, 18.2, 15.4; 600 x 5120 x 17408 207, 157, 201 (400 of 128 x 64); 1000 x 5120 x
+    // 5120, 320 tiles, 99.6 all three; 1400 x 3072 x 2048, 264 tiles, 44, 53, 54; 2080 x 5120 x 2048 74, 80, 98; 2080 x 2048 x 4096
+    // 71, 85, 82; 95 x 34816 x 5120 90, 100, 104).
     const uint32_t half_tiles = a.row_tiles * ((p.columns + 63) / 64), units = backend_compute_units(backend);
     if (small_tiles && half_tiles <= units) {
       a.column_tiles = (p.columns + 63) / 64;

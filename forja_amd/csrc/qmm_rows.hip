@@ -12,10 +12,8 @@
 // 2.7e-7 (the vector-ALU kernels, value by value: 2.9e-7 both; bf16 pieces against 16 + q: 5.2e-7, 2.5e-6).
 //
 // No one unit bounds such a product (48 x 34816 x 5120, counters: while two waves share a SIMD, its vector ALU is
-// busy 0.46 of the cycles and its matrix cores 0.22, and a wave issues for a third of its life, is ready but not
-// issued for half and waits for the rest; taking out the loads, the staging or the matrix instructions
-// alone each gains a tenth to a quarter; and its 544 workgroups are 32 more than have a place at once, which
-// costs little less than half of the 61 us).  A weight is used for 16 to 64 rows, so its unpacking (8
+// busy 0.57 of the cycles and its matrix cores 0.26, and a wave issues for 0.41 of its life, is ready but not issued for
+// 0.40 and waits for the rest).  A weight is used for 16 to 64 rows, so its unpacking (8
 // instructions a word) and its share of activation traffic have to be spread over all of them.  A wave therefore owns 64 weight columns and every row of the tile: the weights go
 // straight from memory to the wave's registers, 16 rows x 64 bytes per load, a pair of groups ahead of
 // the arithmetic, and are unpacked once; the activations, which the column waves of a workgroup share,
@@ -24,9 +22,9 @@
 // output has too few tiles for the device, over workgroups whose f32 partial sums a second launch
 // adds in order.
 // Measured, before (streaming, tile-product and vector-ALU kernels) and now: bf16 48 x 34816 x 5120 101 ->
-// 66 us, 48 x 5120 x 17408 75 -> 34, 90 rows in 48-row tiles 5120 x 5120 and 17408 69 -> 30 on average; f32 512 x 5120
-// x 2048 284 -> 62, 512 x 2048 x 4096 231 -> 45, 8 bits 512 x 128 x 2048 93 -> 16; routed, 128 experts of 768 x 2048,
-// gate/up and down together: bf16 16640 routes 435 -> 324, f32 4096 routes 1027 -> 220.
+// 56 us, 48 x 5120 x 17408 75 -> 30; f32 512 x 5120 x 2048 284 -> 52, 512 x 2048 x 4096 231 -> 42, 8 bits 512 x 128 x 2048
+// 93 -> 12; routed, 128 experts of 768 x 2048, gate/up and down together: bf16 16640 routes 435 -> 294, f32 4096 routes
+// 1027 -> 232 (in steps, where their weights come from memory).
 //
 // The activations come in by rows, eight lanes to a row's 128 bytes of a group: sixteen bytes of another row in every lane
 // (operand order) cost the compute unit's address unit 65 cycles a load against 18, and a third of all loads were of
